@@ -123,22 +123,32 @@ def _values(case, shape, dtype, gen):
     return x.uniform_(-1.0, 1.0, generator=gen)
 
 
-def prepare(case, seed):
-    ck = package()
+def _operands(case, seed):
+    """A, B (as the launcher takes it) and C (None: not read)."""
     gen = torch.Generator(device="cuda")
     gen.manual_seed(seed)
     M, N, K, dtype = case["M"], case["N"], case["K"], case["dtype"]
-    code = {"f16": ck.DT_F16, "bf16": ck.DT_BF16, "f32": ck.DT_F32, "i32": ck.DT_I32}[dtype]
-    s = {"kind": case["kind"], "code": code, "A": _values(case, (M, K), dtype, gen), "sizes": (M, N, K)}
+    A = _values(case, (M, K), dtype, gen)
     if case["kind"] == "simt":
-        s["B"] = _values(case, (N, K) if case["transposed"] else (K, N), dtype, gen)
-        s["D"] = torch.empty((M, N), dtype=TORCH[dtype], device="cuda")
+        return A, _values(case, (N, K) if case["transposed"] else (K, N), dtype, gen), None
+    B = _values(case, (N, K), dtype, gen)
+    return A, B, _values(case, (M, N), _result(case), gen) if case["beta"] != 0.0 else None
+
+
+def _result(case):
+    return case["dtype"] if case["kind"] == "simt" or case["out"] == "same" else "f32"
+
+
+def prepare(case, seed):
+    ck = package()
+    M, N, K, dtype = case["M"], case["N"], case["K"], case["dtype"]
+    code = {"f16": ck.DT_F16, "bf16": ck.DT_BF16, "f32": ck.DT_F32, "i32": ck.DT_I32}[dtype]
+    s = {"kind": case["kind"], "code": code, "sizes": (M, N, K)}
+    s["A"], s["B"], s["C"] = _operands(case, seed)
+    s["D"] = torch.empty((M, N), dtype=TORCH[_result(case)], device="cuda")
+    if case["kind"] == "simt":
         s["tuning"] = (case["tile"], case["block_rows"], case["transposed"])
         return s
-    s["B"] = _values(case, (N, K), dtype, gen)
-    result = "f32" if case["out"] == "f32" else dtype
-    s["C"] = _values(case, (M, N), result, gen) if case["beta"] != 0.0 else None
-    s["D"] = torch.empty((M, N), dtype=TORCH[result], device="cuda")
     s["beta"] = case["beta"]
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     if case["kind"] == "gemm":
@@ -173,6 +183,15 @@ def work(case):
     result = 4 if case.get("out") == "f32" else e
     c = 1 if case.get("beta", 0.0) else 0
     return {"bytes": (M * K + N * K) * e + M * N * result * (1 + c), "flops": 2.0 * M * N * K}
+
+
+def exact(case, seed):
+    A, B, C = _operands(case, seed)
+    A, B = A.double(), B.double()
+    D = A @ (B if case["kind"] == "simt" and not case["transposed"] else B.t())
+    if C is not None:
+        D += case["beta"] * C.double()
+    return D.to(torch.int32) if case["dtype"] == "i32" else D   # (sums of whole numbers far below 2^53)
 
 
 def tolerance(case):
