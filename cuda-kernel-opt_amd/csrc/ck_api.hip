@@ -912,8 +912,9 @@ int ckopt_matmul_shmem(int dtype, const void* A, const void* B, void* C, int M, 
     if (((uintptr_t)A & 15) || ((uintptr_t)B & 15) || ((uintptr_t)C & 3)) return CK_ERR_ALIGNMENT;
     if (N / tile_dim > 65535) return CK_ERR_TOO_LARGE;
     SimtArgs a{A, B, C, M, N, K};
-    const hipError_t e = launch_matmul_shmem(dtype, tile_dim, tile_dim / block_rows, b_transposed != 0,
-                                             dim3(M / tile_dim, N / tile_dim), static_cast<hipStream_t>(stream), a);
+    const SimtInstance inst = simt_instance(dtype, tile_dim, block_rows, M, N, device_cus());
+    const hipError_t e = launch_matmul_shmem(dtype, inst.tile, inst.accs, b_transposed != 0, dim3(M / inst.tile, N / inst.tile),
+                                             static_cast<hipStream_t>(stream), a);
     if (e == hipErrorInvalidValue) return CK_ERR_NO_INSTANCE;
     return e == hipSuccess ? CK_OK : CK_ERR_HIP;
 }

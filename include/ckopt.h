@@ -234,7 +234,8 @@ int ckopt_suggest_gemm_tuning(int M, int N, int K, int num_cus, int* tuning_out)
  * the reference; b_transposed != 0: B is given as N x K row-major.
  * tile_dim in {32,64,128}, tile_dim % block_rows == 0, accumulators per thread
  * tile_dim/block_rows in {1,2,4,8,16,32,64}, 64 <= tile_dim*block_rows <= 1024.
- * M, N must be multiples of tile_dim and K a multiple of 16. */
+ * M, N must be multiples of tile_dim and K a multiple of 16. Where few tiles would leave the device idle the launch runs
+ * smaller ones, or fewer accumulators per thread (simt_instance in csrc/ck_common.h); results are the same bit for bit. */
 int ckopt_matmul_shmem(int dtype, const void* A, const void* B, void* C, int M, int N, int K, int tile_dim,
                        int block_rows, int b_transposed, void* stream);
 

@@ -109,3 +109,33 @@ def test_cpp_driver_through_the_matmul_shmem_template(ck):
     passed = [l for l in r.stdout.splitlines() if l.endswith(": passed")]
     rates = [l for l in r.stdout.splitlines() if l.startswith("(") and "): " in l and not l.endswith("ed")]
     assert len(passed) >= 3 * 2 * 10 and len(rates) >= 3 * 10 and all(float(l.split("): ")[1]) > 0.1 for l in rates)
+
+
+@pytest.mark.parametrize("name", ["f32", "f16", "i32"])
+def test_every_instance_where_the_grid_keeps_it_and_where_it_is_replaced(ck, oracle, name):
+    # The launcher runs 32 tiles in the place of 64 and 128 ones up to 8192 outputs per CU, and 16 or 32 accumulators in the
+    # place of more where 128 tiles are at most one per CU; neither may change a bit. Outputs per CU (256 CUs): 64; 1280 and 1408, 4608 and
+    # 4736 (either side of the lines between 4, 8 and 16 accumulators); 8192 and 8704; 9216 (144 tiles of 128) and 17408 (272
+    # tiles: every tuple on its own instance). K: one slice, and three.
+    dtype = {"f32": ck.DT_F32, "f16": ck.DT_F16, "i32": ck.DT_I32}[name]
+    odt = {"f32": oracle.DT_F32, "f16": oracle.DT_F16, "i32": oracle.DT_I32}[name]
+    big = name == "i32"
+    for M, N, K in ((128, 128, 16), (640, 512, 48), (704, 512, 48), (2304, 512, 48), (2368, 512, 16), (2048, 1024, 48), (2176, 1024, 48),
+                    (1536, 1536, 16), (2176, 2048, 48)):
+        for bt in (False, True):
+            shape_b = (N, K) if bt else (K, N)
+            if big:
+                rng = np.random.default_rng(23)
+                a, b = (rng.integers(-2 ** 31, 2 ** 31, s, dtype=np.int32) for s in ((M, K), shape_b))
+            else:
+                a, b = ck.fill_uniform(dtype, (M, K), 23, 0), ck.fill_uniform(dtype, shape_b, 23, 1)
+            if big:   # sums and products wrap modulo 2^32
+                want = (a.astype(np.int64) @ (b.T if bt else b).astype(np.int64)).astype(np.int32)
+            else:
+                want = oracle.matmul(odt, a, b, bt, fused=True)
+                want = want.astype(np.float16) if name == "f16" else want
+            for tile, br in LEGAL:
+                if tile < 64 or M % tile or N % tile:
+                    continue
+                got = run(ck, dtype, a, b, M, N, K, tile, br, bt)
+                assert np.array_equal(got.view(np.uint8), want.view(np.uint8)), (M, N, K, bt, tile, br)
