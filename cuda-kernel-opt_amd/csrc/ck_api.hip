@@ -26,6 +26,7 @@ bool gemm_stream_applies(const GemmArgs& a, int tile_dim, int segment_dim_k, int
 constexpr int STREAM_K_MULTIPLE_HOST = 64;  // K extent of one loop body of the straight-line kernel
 hipError_t launch_gemm_fused_f16(int tile, int segk, int cw, dim3 grid, size_t lds, hipStream_t stream, const GemmArgs& a);
 hipError_t launch_gemm_fused_bf16(int tile, int segk, int cw, dim3 grid, size_t lds, hipStream_t stream, const GemmArgs& a);
+hipError_t launch_gemm_direct(bool bf16, int tile, bool aligned, hipStream_t stream, const GemmArgs& a);
 hipError_t launch_gemm_sync_f16(int tile, int segk, int cw, dim3 grid, size_t lds, hipStream_t stream, const GemmArgs& a);
 hipError_t launch_gemm_sync_bf16(int tile, int segk, int cw, dim3 grid, size_t lds, hipStream_t stream, const GemmArgs& a);
 hipError_t launch_matmul_shmem(int dtype, int tile, int accs, bool bt, dim3 grid, hipStream_t s, const SimtArgs& a);
@@ -472,11 +473,47 @@ int launch_k(int K, bool operands_aligned, const ck::GemmTuning& t, const Option
     return needs_copies(K, operands_aligned) ? padded_k(K, t, opt) : K;
 }
 
+// ---- tiles of at most 64: the ring kernel (gemm_fused_kernel) or the small-product kernel (gemm_direct_kernel) --------------------
+// Estimated microseconds, measured on 256 CUs with fp16 operands and fp32 results. The ring kernel on square tiles: one
+// workgroup per CU, per 128 of K 1.4 us for a 128 x 128 tile, 0.65 us for a 64 x 64 tile, about 4 us per round besides. The
+// small-product kernel: per round of one workgroup per CU 1.7 us for 32 x 32 and 3.0 us for 64 x 64 tiles, and per 512 of K (a
+// unit of 64 for each of the eight waves) 0.55 and 1.2 us while the device is nearly empty, 0.8 and 1.6 us when it is full
+// (L2); rows on 2-byte boundaries cost half as much again. Zero-padded operand copies: two allocations and a launch more.
+constexpr double COPIES_US = 16.0;
+double ring_us(int tile, int64_t tiles, int K, int num_cus) { return std::ceil((double)tiles / num_cus) * ((double)K / 128.0 * (tile == 128 ? 1.4 : 0.65) + 4.0); }
+double direct_us(int tile, int64_t tiles, int K, bool even, int num_cus) {
+    const double rounds = std::ceil((double)tiles / num_cus), units = std::ceil((double)K / 512.0), full = std::min(1.0, (double)tiles / num_cus);
+    const double unit_us = (tile == 32 ? 0.55 + 0.25 * full : 1.2 + 0.4 * full) * (even ? 1.0 : 1.5);
+    return 1.5 + rounds * ((tile == 32 ? 1.7 : 3.0) + units * unit_us);
+}
+struct SmallPlan { int direct; double us; };   // direct: tile of the small-product kernel, 0: the ring kernel on 64 x 64 tiles
+SmallPlan small_plan(int M, int N, int K, bool operands_aligned, int num_cus) {
+    auto tiles = [&](int t) { return (int64_t)((M + t - 1) / t) * ((N + t - 1) / t); };
+    SmallPlan best{0, ring_us(64, tiles(64), K, num_cus) + (needs_copies(K, operands_aligned) ? COPIES_US : 0.0)};
+    if (K < ck::CHUNK_ELEMS) return best;   // the kernel reads whole chunks of a row
+    for (int t : {32, 64}) {
+        const double us = direct_us(t, tiles(t), K, operands_aligned && K % 2 == 0, num_cus);
+        if (us < best.us) best = {t, us};
+    }
+    return best;
+}
+// The tuple the library suggests for few tiles leaves the kernel to that estimate (512^3: 6.4 us on the ring, 5.1 on 32 x 32
+// tiles; 256 x 256 x 8192 45.8 -> 13.1; 1024^2 x 4096 25.3 -> 18.0 on 64 x 64; 200 x 136 x 1001 24 -> 6.0; 2048^2 x 128 stays on
+// the ring, 9.3 against 12.3). Only where it may use the whole device: one workgroup per tile, num_cus does not bound them.
+int direct_tile(int M, int N, int K, bool operands_aligned, const ck::GemmTuning& t, const Options& opt) {
+    if (!(opt[OPT_STRAIGHT_LINE] && opt[OPT_SWIZZLE] && t.num_producer_waves == 0 && t.num_consumer_waves == 8 && t.tile_dim == 64 &&
+          t.segment_dim_k == 128 && t.num_stages == 4 && t.num_cus >= device_cus()))
+        return 0;
+    return small_plan(M, N, K, operands_aligned, t.num_cus).direct;
+}
+
 // Scratch bytes a launch takes from a provided buffer whose start is on a 256-byte boundary (the launcher's own
 // rules, evaluated without launching): the zero-padded operand copies, then what the K slices need.
 size_t scratch_need(int M, int N, int K, bool operands_aligned, const ck::GemmTuning& t, const Options& opt) {
     using namespace ck;
     size_t need = 0;
+    // (For the tuple that the small-product kernel serves the answer stays what the ring kernel's copies take, which is more than
+    // that kernel's nothing: programs size one buffer for many calls by it.)
     const int k = launch_k(K, operands_aligned, t, opt);
     if (needs_copies(K, operands_aligned)) need += scratch_round(((size_t)M + (size_t)N) * k * 2);
     if (straight_line_tuple(t, opt)) {
@@ -522,20 +559,23 @@ int gemm_launch(int dtype, const void* A, const void* Bt, const void* C, void* D
     if (((uintptr_t)A & 1) || ((uintptr_t)Bt & 1)) return CK_ERR_ALIGNMENT;
     const uintptr_t elem_mask = out16 ? 1 : 3;
     if (((uintptr_t)D & elem_mask) || ((uintptr_t)C & elem_mask)) return CK_ERR_ALIGNMENT;
-    // the kernels want every operand row on a 16-byte boundary
-    if (needs_copies(K, !(((uintptr_t)A | (uintptr_t)Bt) & 15)))
+    // the ring kernels want every operand row on a 16-byte boundary
+    const bool aligned = !(((uintptr_t)A | (uintptr_t)Bt) & 15);
+    const int direct = direct_tile(M, N, K, aligned, t, opt);
+    if (!direct && needs_copies(K, aligned))
         return gemm_launch_repacked(dtype, A, Bt, C, D, alpha, beta, M, N, K, t, opt, stream, out16, sc);
     // one tile's rows are addressed through a 32-bit buffer offset
     if ((int64_t)t.tile_dim * K * 2 >= (int64_t)1 << 31) return CK_ERR_TOO_LARGE;
 
     const int mode = sync_mode_of(t.tile_dim, t.num_consumer_waves, t.bar_step_rows_a, t.bar_step_rows_b);
+    const int tile_rows = direct ? direct : t.tile_dim;
     GemmArgs a{};
     a.A = A; a.Bt = Bt; a.C = static_cast<const float*>(C); a.D = static_cast<float*>(D);
     a.out16 = out16 ? 1 : 0;
     a.alpha = alpha; a.beta = beta;
     a.M = M; a.N = N; a.K = K;
-    a.tiles_m = (M + t.tile_dim - 1) / t.tile_dim;
-    a.tiles_n = (N + t.tile_dim - 1) / t.tile_dim;
+    a.tiles_m = (M + tile_rows - 1) / tile_rows;
+    a.tiles_n = (N + tile_rows - 1) / tile_rows;
     a.nseg = (K + t.segment_dim_k - 1) / t.segment_dim_k;
     a.tile_group_m = t.tile_group_m;
     a.num_stages = t.num_stages;
@@ -573,7 +613,9 @@ int gemm_launch(int dtype, const void* A, const void* Bt, const void* C, void* D
     a.whole_tiles = (int)tiles;
     a.fix_partials = nullptr;
     a.fix_state = nullptr;
-    if (straight_line_tuple(t, opt) && gemm_stream_applies(a, t.tile_dim, t.segment_dim_k, t.num_stages, t.num_producer_waves, t.num_consumer_waves)) {
+    if (direct) {
+        e = launch_gemm_direct(dtype == CK_DT_BF16, direct, K % 2 == 0 && !(((uintptr_t)A | (uintptr_t)Bt) & 3), s, a);
+    } else if (straight_line_tuple(t, opt) && gemm_stream_applies(a, t.tile_dim, t.segment_dim_k, t.num_stages, t.num_producer_waves, t.num_consumer_waves)) {
         // Tile width, K slices and grid from the cost model: few tiles and a deep K are cut into slices so that every CU
         // has an item; the partly filled last round of many tiles likewise; tile counts that leave much of the device idle
         // take 256 x 128 tiles.
@@ -747,8 +789,9 @@ int ckopt_gemm_launch_plan_ex(int M, int N, int K, int operands_aligned, CK_TUNI
     if (M <= 0 || N <= 0 || K <= 0) return ck::CK_ERR_BAD_PARAM;
     const int rc = ck::check_gemm_tuning(t);
     if (rc != ck::CK_OK) return rc;
-    const bool copies = needs_copies(K, operands_aligned != 0);
-    plan_out[0] = 0; plan_out[1] = t.tile_dim; plan_out[2] = 1; plan_out[3] = copies ? 1 : 0;
+    const int direct = direct_tile(M, N, K, operands_aligned != 0, t, opt);
+    const bool copies = !direct && needs_copies(K, operands_aligned != 0);
+    plan_out[0] = 0; plan_out[1] = direct ? direct : t.tile_dim; plan_out[2] = 1; plan_out[3] = copies ? 1 : 0;
     plan_out[4] = 0; plan_out[5] = 0; plan_out[6] = 0;
     if (straight_line_tuple(t, opt)) {
         const StreamPlan plan = stream_plan(M, N, launch_k(K, operands_aligned != 0, t, opt), t.num_cus, opt);
@@ -886,14 +929,18 @@ int ckopt_suggest_gemm_tuning(int M, int N, int K, int num_cus, int* tuning_out)
         else if (tiles(128) * 2 >= num_cus) pick = fused_128;
     } else {
         // the shortest of three estimates: the straight-line kernel as the launcher would run it on aligned operands (its K,
-        // tile width and slice count: launch_k, stream_plan), and the general kernel on 128 and on 64 tiles - one
-        // workgroup per CU, measured per 128 of K: 1.4 us for a 128 x 128 tile, 0.65 us for a 64 x 64 tile, about 4 us
-        // per round besides
+        // tile width and slice count: launch_k, stream_plan), the ring kernel on 128 tiles, and what the tuple of 64
+        // tiles runs (small_plan). The straight-line estimate leaves out the launch itself, 1.5 us in the small-product one.
+        // Where the straight-line kernel would cut K, its tuple is weighed against the ring kernel alone: programs that own a
+        // workspace have sized it for those slices, and keep the tuple that uses it.
         const GemmTuning st{256, 32, 0, 0, 256, 256, 4, 5, 0, 8, num_cus, 0};
-        const double straight_us = stream_plan(M, N, launch_k(K, true, st, opt), num_cus, opt).us;
-        auto general_us = [&](int t, double seg_us) { return std::ceil((double)tiles(t) / num_cus) * ((double)K / 128.0 * seg_us + 4.0); };
-        const double us_128 = general_us(128, 1.4), us_64 = general_us(64, 0.65);
-        if (straight_us <= us_128 && straight_us <= us_64) pick = straight_line;
+        const StreamPlan straight = stream_plan(M, N, launch_k(K, true, st, opt), num_cus, opt);
+        const double us_128 = ring_us(128, tiles(128), K, num_cus), us_64 = ring_us(64, tiles(64), K, num_cus);
+        const SmallPlan small = small_plan(M, N, K, true, num_cus);
+        const double copies_us = needs_copies(K, true) ? COPIES_US : 0.0;
+        if (straight.slices > 1 && straight.us <= us_128 && straight.us <= us_64) pick = straight_line;
+        else if (small.direct && num_cus >= device_cus() && small.us < us_128 + copies_us && small.us < straight.us + 1.5 + copies_us) pick = fused_64;
+        else if (straight.us <= us_128 && straight.us <= us_64) pick = straight_line;
         else if (us_128 <= us_64) pick = fused_128;
     }
     for (int i = 0; i < 10; ++i) tuning_out[i] = pick[i];

@@ -1441,3 +1441,65 @@ def test_random_tunings_entry_points_and_options_exact(ck):
             for k, v in prev.items():
                 ck.set_option(k, v)
     assert ran >= 0.55 * cases
+
+
+SMALL_TUPLE = (64, 128, 0, 0, 64, 64, 4, 4, 0, 8, 256)   # what the library suggests for few tiles
+
+
+@pytest.mark.parametrize("shift", [0, 1, 2, 8])
+@pytest.mark.parametrize("bf16", [False, True])
+def test_small_product_kernel_exact_at_its_edges(ck, bf16, shift):
+    """The small-product kernel on rows and ends of every alignment, exact on small integers (sums below 2^24): tiles of 32 and 64,
+    ragged edges, K around one unit of 64, around eight (one per wave) and around the depth of the fetch; operands that start
+    `shift` elements behind a 16-byte boundary inside a buffer full of NaN, which no lane may multiply; C, alpha and 16-bit results."""
+    dtype, tdt = (ck.DT_BF16, torch.bfloat16) if bf16 else (ck.DT_F16, torch.float16)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(7)
+    seen = set()
+    sizes = [(1, 1, 8), (31, 33, 9), (32, 32, 15), (33, 65, 63), (64, 31, 64), (100, 7, 65), (65, 64, 72), (40, 100, 127), (32, 64, 512), (96, 33, 513),
+             (33, 40, 576), (64, 64, 1001), (31, 32, 2048), (32, 33, 2049), (50, 50, 2560), (20, 30, 5001), (700, 700, 512), (1000, 600, 130),
+             (690, 1030, 1001), (1024, 1024, 4097), (1024, 1024, 1026)]
+    for M, N, K in sizes:
+        def operand(rows):
+            buf = torch.full((rows * K + 16 + shift,), float("nan"), dtype=tdt, device="cuda")
+            view = buf[shift:shift + rows * K].view(rows, K)
+            view.copy_(torch.randint(-2, 3, (rows, K), device="cuda", generator=gen))
+            return buf, view
+        buf_a, a = operand(M)
+        buf_b, b = operand(N)
+        plan = ck.gemm_launch_plan(M, N, K, shift % 8 == 0, *SMALL_TUPLE)
+        assert not plan["operand_copies"] and plan["tile_cols"] in (32, 64)
+        seen.add(plan["tile_cols"])
+        exact = (a.cpu().double() @ b.cpu().double().t())
+        guard = 64
+        d = torch.full((M * N + guard,), float("nan"), dtype=torch.float32, device="cuda")
+        ck.gemm_shmem_tc_async_opt_port(dtype, a, b, None, d, 1.0, 0.0, M, N, K, *SMALL_TUPLE)
+        assert torch.equal(d[:M * N].view(M, N).cpu().double(), exact), (M, N, K)
+        assert torch.isnan(d[M * N:]).all()
+        # alpha and C: |2 x - 3 c| stays below 2^24 as well
+        c = torch.randint(-8, 9, (M, N), device="cuda", generator=gen).float()
+        ck.gemm_shmem_tc_async_opt_port(dtype, a, b, c, d, 2.0, -3.0, M, N, K, *SMALL_TUPLE)
+        assert torch.equal(d[:M * N].view(M, N).cpu().double(), 2 * exact - 3 * c.cpu().double()), (M, N, K)
+        # 16-bit C and D: one rounding of the exact value
+        d16 = torch.full((M * N + guard,), float("nan"), dtype=tdt, device="cuda")
+        ck.gemm_shmem_tc_async_opt_port_lp(dtype, a, b, c.to(tdt), d16, 1.0, 1.0, M, N, K, *SMALL_TUPLE)
+        assert torch.equal(d16[:M * N].view(M, N).cpu(), (exact + c.cpu().double()).to(tdt)), (M, N, K)
+        assert torch.isnan(d16[M * N:]).all()
+    assert seen == {32, 64}
+    assert ck.device_status() == 0
+
+
+def test_small_product_kernel_keeps_infinities_to_their_rows(ck):
+    """Rows and k past the edges are read as other rows or masked: an infinity or a NaN in the last row, column or k reaches the
+    outputs that it belongs to and no other."""
+    M, N, K = 40, 50, 77
+    a = torch.ones((M, K), dtype=torch.float16, device="cuda")
+    b = torch.ones((N, K), dtype=torch.float16, device="cuda")
+    a[M - 1, K - 1] = float("inf")
+    b[N - 1, 0] = float("nan")
+    d = torch.zeros((M, N), dtype=torch.float32, device="cuda")
+    ck.gemm_shmem_tc_async_opt_port(ck.DT_F16, a, b, None, d, 1.0, 0.0, M, N, K, *SMALL_TUPLE)
+    want = torch.full((M, N), float(K))
+    want[M - 1, :] = float("inf")
+    want[:, N - 1] = float("nan")
+    assert torch.equal(torch.nan_to_num(d.cpu(), nan=-1.0), torch.nan_to_num(want, nan=-1.0))

@@ -503,3 +503,25 @@ def test_query_and_plan_are_pure_functions_of_their_arguments(ck):
     with pytest.raises(ck.CkoptError) as e:
         ck.gemm_shmem_tc_async_opt_port_ex(ck.DT_F16, ck.DT_F32, None, None, None, None, 1.0, 0.0, 256, 256, 256, *straight, options=ck.launch_options())
     assert e.value.code == ck.ERR_NULL
+
+
+def test_small_tuple_leaves_the_kernel_to_the_estimate(ck):
+    # the tuple of 64 tiles that the library suggests: the small-product kernel where that is estimated shorter, without copies
+    small = (64, 128, 0, 0, 64, 64, 4, 4, 0, 8, 256)
+    tile = lambda *s, aligned=True, t=small, **kw: ck.gemm_launch_plan(*s, aligned, *t, **kw)["tile_cols"]
+    assert tile(512, 512, 512) == 32 and tile(256, 256, 8192) == 32 and tile(200, 136, 1001) == 32
+    p = ck.gemm_launch_plan(1000, 1000, 1001, True, *small)
+    assert p["tile_cols"] == 64 and not p["operand_copies"]
+    assert ck.gemm_launch_plan(512, 512, 512, False, *small)["operand_copies"] is False   # the query stays an upper bound here:
+    assert ck.gemm_workspace_bytes(512, 512, 512, False, *small) >= 2 * 512 * 512 * 2
+    # the ring kernel: where it is shorter, with its copies; K below one chunk; another tuple; the straight-line switch or the
+    # swizzle off; fewer CUs than the device has (one workgroup per tile would not keep to them)
+    ring = lambda *s, aligned=True, t=small, **kw: (ck.gemm_launch_plan(*s, aligned, *t, **kw)["operand_copies"], ck.gemm_workspace_bytes(*s, aligned, *t, **kw) > 0)
+    assert ring(6000, 6000, 67) == (True, True) and ring(40, 100, 7) == (True, True)
+    assert ring(512, 512, 513, t=(64, 64) + small[2:]) == (True, True) and ring(512, 512, 513, t=small[:-1] + (128,)) == (True, True)
+    for off in (dict(straight_line=0), dict(lds_swizzle=0)):
+        assert ring(512, 512, 513, options=ck.launch_options(**off)) == (True, True)
+    # suggested where it is the shortest of all; where the straight-line kernel would cut K, that tuple stays
+    assert ck.suggest_gemm_tuning(300, 520, 4090)["tile_dim"] == 256
+    for s in ((32, 32, 64), (65, 31, 9), (200, 136, 1001), (512, 512, 512), (100, 3000, 501), (300, 300, 30000), (1500, 1500, 301)):
+        assert ck.suggest_gemm_tuning(*s)["tile_dim"] == 64, s
