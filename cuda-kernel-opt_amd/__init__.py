@@ -136,19 +136,11 @@ def _check(code, where):
 
 
 def _dptr(x):
-    if x is None:
-        return None
-    if isinstance(x, int):
-        return ctypes.c_void_p(x)
-    return ctypes.c_void_p(x.data_ptr())  # torch tensor
+    return x if x is None or isinstance(x, int) else x.data_ptr()  # torch tensor (the argument types make it a pointer)
 
 
 def _stream(stream):
-    if stream is None:
-        return None
-    if isinstance(stream, int):
-        return ctypes.c_void_p(stream)
-    return ctypes.c_void_p(stream.cuda_stream)  # torch.cuda.Stream
+    return stream if stream is None or isinstance(stream, int) else stream.cuda_stream  # torch.cuda.Stream
 
 
 def get_num_acc(tile_dim, num_consumer_waves):
