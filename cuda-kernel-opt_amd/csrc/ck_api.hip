@@ -27,6 +27,7 @@ constexpr int STREAM_K_MULTIPLE_HOST = 64;  // K extent of one loop body of the 
 hipError_t launch_gemm_fused_f16(int tile, int segk, int cw, dim3 grid, size_t lds, hipStream_t stream, const GemmArgs& a);
 hipError_t launch_gemm_fused_bf16(int tile, int segk, int cw, dim3 grid, size_t lds, hipStream_t stream, const GemmArgs& a);
 hipError_t launch_gemm_direct(bool bf16, int tile, bool aligned, hipStream_t stream, const GemmArgs& a);
+hipError_t launch_gemm_mid(bool bf16, hipStream_t stream, const GemmArgs& a);
 hipError_t launch_gemm_sync_f16(int tile, int segk, int cw, dim3 grid, size_t lds, hipStream_t stream, const GemmArgs& a);
 hipError_t launch_gemm_sync_bf16(int tile, int segk, int cw, dim3 grid, size_t lds, hipStream_t stream, const GemmArgs& a);
 hipError_t launch_matmul_shmem(int dtype, int tile, int accs, bool bt, dim3 grid, hipStream_t s, const SimtArgs& a);
@@ -102,23 +103,22 @@ unsigned char* g_scratch_ptr[MAX_DEV] = {};
 
 // Compute units of the current device (what the cost model's measurements scale with), read once per device;
 // 256, the device the model was calibrated on, where no device can be asked.
-int g_device_cus[MAX_DEV] = {};
+std::atomic<int> g_device_cus[MAX_DEV] = {};   // (asked for by every launch: no lock)
 int device_cus() {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= MAX_DEV) {
         (void)hipGetLastError();
         return 256;
     }
-    std::lock_guard<std::mutex> lock(g_status_mutex);
-    if (!g_device_cus[dev]) {
-        int n = 0;
+    int n = g_device_cus[dev].load(std::memory_order_relaxed);
+    if (!n) {
         if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) {
             (void)hipGetLastError();
             n = 256;
         }
-        g_device_cus[dev] = n;
+        g_device_cus[dev].store(n, std::memory_order_relaxed);
     }
-    return g_device_cus[dev];
+    return n;
 }
 
 // Device address of this device's copy of `scratch`, looked up once per device with that device current.
@@ -507,6 +507,14 @@ int direct_tile(int M, int N, int K, bool operands_aligned, const ck::GemmTuning
     return small_plan(M, N, K, operands_aligned, t.num_cus).direct;
 }
 
+// The tuple the library suggests for 128 x 128 tiles runs the register-staged kernel (gemm_mid_kernel) where it may use the whole
+// device: one workgroup per tile, num_cus does not bound
+// them (ring against this, us: 2048^3 26.2 / 26.4, 2048^2 x 2176 27.2 / 25.9, 256 x 16384 x 4096 47.7 / 44.8, 8192^2 x 8128 1261 / 1237).
+bool mid_tuple(const ck::GemmTuning& t, const Options& opt) {
+    return opt[OPT_STRAIGHT_LINE] && opt[OPT_SWIZZLE] && t.num_producer_waves == 0 && t.num_consumer_waves == 8 && t.tile_dim == 128 &&
+           t.segment_dim_k == 128 && t.num_stages == 2 && t.num_cus >= device_cus();
+}
+
 // Scratch bytes a launch takes from a provided buffer whose start is on a 256-byte boundary (the launcher's own
 // rules, evaluated without launching): the zero-padded operand copies, then what the K slices need.
 size_t scratch_need(int M, int N, int K, bool operands_aligned, const ck::GemmTuning& t, const Options& opt) {
@@ -691,6 +699,8 @@ int gemm_launch(int dtype, const void* A, const void* Bt, const void* C, void* D
             }
             if (!scratch_release(sc, ws, s) && e == hipSuccess) e = hipErrorUnknown;
         }
+    } else if (mid_tuple(t, opt)) {
+        e = launch_gemm_mid(dtype == CK_DT_BF16, s, a);
     } else if (t.num_producer_waves == 0 && t.num_stages == 1) {
         // one stage, no producers: load, barrier, multiply, barrier (the synchronous A/B partner)
         e = dtype == CK_DT_F16 ? launch_gemm_sync_f16(t.tile_dim, t.segment_dim_k, t.num_consumer_waves, dim3(grid), lds, s, a)

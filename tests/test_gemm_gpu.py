@@ -1503,3 +1503,30 @@ def test_small_product_kernel_keeps_infinities_to_their_rows(ck):
     want[M - 1, :] = float("inf")
     want[:, N - 1] = float("nan")
     assert torch.equal(torch.nan_to_num(d.cpu(), nan=-1.0), torch.nan_to_num(want, nan=-1.0))
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+def test_register_staged_128_tiles_exact_at_their_edges(ck, bf16):
+    """The kernel behind the tuple suggested for 128 x 128 tiles, exact on small integers: ragged edges, one segment of 128 and less, the
+    two stages' parities, K that ends inside a segment's first and second line, more tiles than CUs; C, 16-bit results, a guard
+    behind D; fewer CUs (the persistent ring kernel) give the same."""
+    dtype, tdt = (ck.DT_BF16, torch.bfloat16) if bf16 else (ck.DT_F16, torch.float16)
+    tup = (128, 128, 0, 0, 128, 128, 4, 2, 0, 8, 256)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(11)
+    for M, N, K in [(1, 4, 8), (128, 128, 128), (130, 127, 56), (64, 200, 72), (256, 129, 120), (300, 300, 136), (257, 384, 256), (128, 640, 384),
+                    (200, 136, 512), (129, 1, 648), (384, 256, 1024), (2100, 2060, 200)]:
+        a = torch.randint(-2, 3, (M, K), device="cuda", generator=gen).to(tdt)
+        b = torch.randint(-2, 3, (N, K), device="cuda", generator=gen).to(tdt)
+        exact = a.cpu().double() @ b.cpu().double().t()
+        c = torch.randint(-8, 9, (M, N), device="cuda", generator=gen).float()
+        for t in (tup, tup[:-1] + (40,)):
+            d = torch.full((M * N + 64,), float("nan"), dtype=torch.float32, device="cuda")
+            ck.gemm_shmem_tc_async_opt_port(dtype, a, b, c, d, 2.0, -3.0, M, N, K, *t)
+            assert torch.equal(d[:M * N].view(M, N).cpu().double(), 2 * exact - 3 * c.cpu().double()), (M, N, K, t[-1])
+            assert torch.isnan(d[M * N:]).all()
+        d16 = torch.full((M * N + 64,), float("nan"), dtype=tdt, device="cuda")
+        ck.gemm_shmem_tc_async_opt_port_lp(dtype, a, b, None, d16, 1.0, 0.0, M, N, K, *tup)
+        assert torch.equal(d16[:M * N].view(M, N).cpu(), exact.to(tdt)), (M, N, K)
+        assert torch.isnan(d16[M * N:]).all()
+    assert ck.device_status() == 0
