@@ -223,9 +223,9 @@ int ckopt_check_gemm_tuning(int tile_dim, int segment_dim_k, int bar_steps_a, in
 /* A tuning tuple for a problem size, from the measurements on MI355X (no counterpart in the reference, whose
  * drivers sweep the tuples by hand, port_2.cu:1463-1480): tuning_out receives {tile_dim, segment_dim_k,
  * bar_steps_a, bar_steps_b, bar_step_rows_a, bar_step_rows_b, tile_group_m, num_stages, num_producer_warps,
- * num_consumer_warps} in the launcher's parameter order. Enough 256 x 256 tiles for half the CUs (or a K deep
- * enough to be cut into at least four slices): the straight-line kernel's tuple; else 128 x 128 tiles if those
- * occupy half the CUs; else 64 x 64 tiles. */
+ * num_consumer_warps} in the launcher's parameter order: the straight-line kernel's tuple (256), the one of 128 x 128 or
+ * the one of 64 x 64 tiles, whichever is estimated shortest on the size (where the straight-line kernel would cut K, its tuple
+ * is weighed against the ring kernels alone). */
 int ckopt_suggest_gemm_tuning(int M, int N, int K, int num_cus, int* tuning_out);
 
 /* Replaces matmul_shmem<DT,DT_ACC>() of matmul_shmem.cu:143-174: C = A * B without matrix cores.
