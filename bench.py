@@ -500,6 +500,10 @@ def main():
         elif args.producers == 0:
             kernel = "gemm_fused_kernel<%s, tile %d, seg_k %d, %d waves, workgroup barrier per segment>" % (
                 dtype, args.tile, args.segk, args.consumers)
+            plan = ck.gemm_launch_plan(M, N, K, True, args.tile, args.segk, args.bar_steps_a, args.bar_steps_b, rows_a, rows_b, args.group,
+                                       args.stages, args.producers, args.consumers, cus)
+            if plan["tile_cols"] != args.tile:
+                kernel = "gemm_direct_kernel<%s, %d x %d tiles, 8 waves on slices of K>" % (dtype, plan["tile_cols"], plan["tile_cols"])
         else:
             kernel = "gemm_pc_kernel<%s, tile %d, seg_k %d, %dC+%dP waves, %s sync>" % (
                 dtype, args.tile, args.segk, args.consumers, args.producers, args.mode)
