@@ -57,6 +57,8 @@ _lib.ckopt_gemm_shmem_tc_async_opt_port_2_ex.restype = _i
 _lib.ckopt_gemm_shmem_tc_async_opt_port_2_ex.argtypes = [_i, _i, _p, _p, _p, _p, _f, _f] + [_i] * 14 + [ctypes.POINTER(LaunchOptions), _p, ctypes.c_size_t, _p]
 _lib.ckopt_gemm_workspace_bytes_ex.restype = _i64
 _lib.ckopt_gemm_workspace_bytes_ex.argtypes = [_i] * 15 + [ctypes.POINTER(LaunchOptions)]
+_lib.ckopt_gemm_launch_kernel.restype = _i
+_lib.ckopt_gemm_launch_kernel.argtypes = [_i] * 15 + [ctypes.POINTER(LaunchOptions)]
 _lib.ckopt_gemm_launch_plan_ex.restype = _i
 _lib.ckopt_gemm_launch_plan_ex.argtypes = [_i] * 15 + [ctypes.POINTER(LaunchOptions), ctypes.POINTER(ctypes.c_int)]
 _lib.ckopt_gemm_shmem_tc_async_opt_port_1_lp.restype = _i
@@ -108,7 +110,7 @@ _lib.ckopt_error_string.argtypes = [_i]
 
 EXPORTED_SYMBOLS = [
     "ckopt_gemm_shmem_tc_async_opt_port_2", "ckopt_gemm_shmem_tc_async_opt_port_2_lp", "ckopt_gemm_shmem_tc_async_opt_port_2_noalloc",
-    "ckopt_gemm_workspace_bytes", "ckopt_gemm_launch_plan", "ckopt_gemm_shmem_tc_async_opt_port_2_ws",
+    "ckopt_gemm_workspace_bytes", "ckopt_gemm_launch_kernel", "ckopt_gemm_launch_plan", "ckopt_gemm_shmem_tc_async_opt_port_2_ws",
     "ckopt_launch_options_init", "ckopt_gemm_shmem_tc_async_opt_port_2_ex", "ckopt_gemm_workspace_bytes_ex", "ckopt_gemm_launch_plan_ex",
     "ckopt_gemm_shmem_tc_async_opt_port_1", "ckopt_gemm_shmem_tc_async_opt_port_1_lp",
     "ckopt_gemm_shmem_tc_async_opt_port_0", "ckopt_gemm_shmem_tc_async_opt_port_0_lp", "ckopt_get_lds_req", "ckopt_get_num_acc", "ckopt_get_warp_tile_rows",
@@ -236,6 +238,20 @@ def gemm_launch_plan(M, N, K, operands_aligned, tile_dim, segment_dim_k, bar_ste
                                           num_consumer_warps, num_sms, _optr(options), out), "gemm_launch_plan")
     return dict(straight_line=bool(out[0]), tile_cols=int(out[1]), k_slices=int(out[2]), operand_copies=bool(out[3]),
                 sliced_tiles=int(out[4]), reduced_in_kernel=bool(out[5]), grid=int(out[6]))
+
+
+KERNELS = ("gemm_fused_kernel", "gemm_stream_kernel", "gemm_direct_kernel", "gemm_mid_kernel", "gemm_sync_kernel", "gemm_pcb_kernel", "gemm_pc_kernel")
+
+
+def gemm_launch_kernel(M, N, K, operands_aligned, tile_dim, segment_dim_k, bar_steps_a, bar_steps_b, bar_step_rows_a,
+                       bar_step_rows_b, tile_group_m, num_stages, num_producer_warps, num_consumer_warps, num_sms, options=None):
+    """Name of the kernel the launch will run (one of KERNELS)."""
+    r = _lib.ckopt_gemm_launch_kernel(M, N, K, int(bool(operands_aligned)), tile_dim, segment_dim_k, bar_steps_a, bar_steps_b,
+                                      bar_step_rows_a, bar_step_rows_b, tile_group_m, num_stages, num_producer_warps,
+                                      num_consumer_warps, num_sms, _optr(options))
+    if r < 0:
+        raise CkoptError(int(r), "gemm_launch_kernel")
+    return KERNELS[r]
 
 
 def gemm_shmem_tc_async_opt_port_ex(dtype, cd_dtype, A, B, C, D, alpha, beta, M, N, K, tile_dim, segment_dim_k, bar_steps_a,

@@ -22,7 +22,6 @@ hipError_t launch_gemm_pcb_f16(int tile, int segk, int cw, dim3 grid, dim3 block
 hipError_t launch_gemm_pcb_bf16(int tile, int segk, int cw, dim3 grid, dim3 block, size_t lds, hipStream_t stream, const GemmArgs& a);
 hipError_t launch_gemm_stream_f16(dim3 grid, hipStream_t stream, const GemmArgs& a, bool barrier_every_kstep, int tile_n);
 hipError_t launch_gemm_stream_bf16(dim3 grid, hipStream_t stream, const GemmArgs& a, bool barrier_every_kstep, int tile_n);
-bool gemm_stream_applies(const GemmArgs& a, int tile_dim, int segment_dim_k, int num_stages, int producer_waves, int consumer_waves);
 constexpr int STREAM_K_MULTIPLE_HOST = 64;  // K extent of one loop body of the straight-line kernel
 hipError_t launch_gemm_fused_f16(int tile, int segk, int cw, dim3 grid, size_t lds, hipStream_t stream, const GemmArgs& a);
 hipError_t launch_gemm_fused_bf16(int tile, int segk, int cw, dim3 grid, size_t lds, hipStream_t stream, const GemmArgs& a);
@@ -486,25 +485,29 @@ double direct_us(int tile, int64_t tiles, int K, bool even, int num_cus) {
     const double unit_us = (tile == 32 ? 0.55 + 0.25 * full : 1.2 + 0.4 * full) * (even ? 1.0 : 1.5);
     return 1.5 + rounds * ((tile == 32 ? 1.7 : 3.0) + units * unit_us);
 }
-struct SmallPlan { int direct; double us; };   // direct: tile of the small-product kernel, 0: the ring kernel on 64 x 64 tiles
+// direct: tile of the small-product kernel, 0: the ring kernel on 64 x 64 tiles; copies: behind zero-padded operand copies
+struct SmallPlan { int direct; bool copies; double us; };
 SmallPlan small_plan(int M, int N, int K, bool operands_aligned, int num_cus) {
     auto tiles = [&](int t) { return (int64_t)((M + t - 1) / t) * ((N + t - 1) / t); };
-    SmallPlan best{0, ring_us(64, tiles(64), K, num_cus) + (needs_copies(K, operands_aligned) ? COPIES_US : 0.0)};
-    if (K < ck::CHUNK_ELEMS) return best;   // the kernel reads whole chunks of a row
+    SmallPlan best;
+    if (needs_copies(K, operands_aligned)) {   // what the launch on the copies, whose rows are padded to whole chunks, runs
+        best = small_plan(M, N, (K + ck::CHUNK_ELEMS - 1) / ck::CHUNK_ELEMS * ck::CHUNK_ELEMS, true, num_cus);
+        best.copies = true;
+        best.us += COPIES_US;
+    } else best = SmallPlan{0, false, ring_us(64, tiles(64), K, num_cus)};
+    if (K < ck::CHUNK_ELEMS) return best;   // the small-product kernel reads whole chunks of a row
     for (int t : {32, 64}) {
         const double us = direct_us(t, tiles(t), K, operands_aligned && K % 2 == 0, num_cus);
-        if (us < best.us) best = {t, us};
+        if (us < best.us) best = {t, false, us};
     }
     return best;
 }
 // The tuple the library suggests for few tiles leaves the kernel to that estimate (512^3: 6.4 us on the ring, 5.1 on 32 x 32
 // tiles; 256 x 256 x 8192 45.8 -> 13.1; 1024^2 x 4096 25.3 -> 18.0 on 64 x 64; 200 x 136 x 1001 24 -> 6.0; 2048^2 x 128 stays on
 // the ring, 9.3 against 12.3). Only where it may use the whole device: one workgroup per tile, num_cus does not bound them.
-int direct_tile(int M, int N, int K, bool operands_aligned, const ck::GemmTuning& t, const Options& opt) {
-    if (!(opt[OPT_STRAIGHT_LINE] && opt[OPT_SWIZZLE] && t.num_producer_waves == 0 && t.num_consumer_waves == 8 && t.tile_dim == 64 &&
-          t.segment_dim_k == 128 && t.num_stages == 4 && t.num_cus >= device_cus()))
-        return 0;
-    return small_plan(M, N, K, operands_aligned, t.num_cus).direct;
+bool small_tuple(const ck::GemmTuning& t, const Options& opt) {
+    return opt[OPT_STRAIGHT_LINE] && opt[OPT_SWIZZLE] && t.num_producer_waves == 0 && t.num_consumer_waves == 8 && t.tile_dim == 64 &&
+           t.segment_dim_k == 128 && t.num_stages == 4 && t.num_cus >= device_cus();
 }
 
 // The tuple the library suggests for 128 x 128 tiles runs the register-staged kernel (gemm_mid_kernel) where it may use the whole
@@ -513,6 +516,29 @@ int direct_tile(int M, int N, int K, bool operands_aligned, const ck::GemmTuning
 bool mid_tuple(const ck::GemmTuning& t, const Options& opt) {
     return opt[OPT_STRAIGHT_LINE] && opt[OPT_SWIZZLE] && t.num_producer_waves == 0 && t.num_consumer_waves == 8 && t.tile_dim == 128 &&
            t.segment_dim_k == 128 && t.num_stages == 2 && t.num_cus >= device_cus();
+}
+
+// What a launch runs: the one decision that the launcher and the queries share. A launch behind operand copies is decided
+// on the copies (K of launch_k, aligned), and the launch on them decides the same again.
+struct Route {
+    int kernel;    // CKOPT_KERNEL_*
+    int tile;      // rows of its tiles of D (and their columns, but for the straight-line kernel, whose width stream_plan chooses)
+    bool copies;   // A and Bt are first copied into zero-padded rows
+};
+Route route_of(int M, int N, int K, bool operands_aligned, const ck::GemmTuning& t, const Options& opt) {
+    using namespace ck;
+    if (small_tuple(t, opt)) {
+        const SmallPlan p = small_plan(M, N, K, operands_aligned, t.num_cus);
+        return {p.direct ? CKOPT_KERNEL_DIRECT : CKOPT_KERNEL_FUSED, p.direct ? p.direct : t.tile_dim, p.copies};
+    }
+    Route r{CKOPT_KERNEL_PC, t.tile_dim, needs_copies(K, operands_aligned)};
+    if (straight_line_tuple(t, opt)) r.kernel = CKOPT_KERNEL_STREAM;
+    else if (mid_tuple(t, opt)) r.kernel = CKOPT_KERNEL_MID;
+    else if (t.num_producer_waves == 0) r.kernel = t.num_stages == 1 ? CKOPT_KERNEL_SYNC : CKOPT_KERNEL_FUSED;
+    else if (sync_mode_of(t.tile_dim, t.num_consumer_waves, t.bar_step_rows_a, t.bar_step_rows_b) == CK_SYNC_TILE && t.num_stages >= 2 &&
+             opt[OPT_TILE_SYNC_BARRIER] && t.num_producer_waves != 1 && t.segment_dim_k <= 128)
+        r.kernel = CKOPT_KERNEL_PCB;
+    return r;
 }
 
 // Scratch bytes a launch takes from a provided buffer whose start is on a 256-byte boundary (the launcher's own
@@ -569,21 +595,20 @@ int gemm_launch(int dtype, const void* A, const void* Bt, const void* C, void* D
     if (((uintptr_t)D & elem_mask) || ((uintptr_t)C & elem_mask)) return CK_ERR_ALIGNMENT;
     // the ring kernels want every operand row on a 16-byte boundary
     const bool aligned = !(((uintptr_t)A | (uintptr_t)Bt) & 15);
-    const int direct = direct_tile(M, N, K, aligned, t, opt);
-    if (!direct && needs_copies(K, aligned))
+    const Route route = route_of(M, N, K, aligned, t, opt);
+    if (route.copies)
         return gemm_launch_repacked(dtype, A, Bt, C, D, alpha, beta, M, N, K, t, opt, stream, out16, sc);
     // one tile's rows are addressed through a 32-bit buffer offset
     if ((int64_t)t.tile_dim * K * 2 >= (int64_t)1 << 31) return CK_ERR_TOO_LARGE;
 
     const int mode = sync_mode_of(t.tile_dim, t.num_consumer_waves, t.bar_step_rows_a, t.bar_step_rows_b);
-    const int tile_rows = direct ? direct : t.tile_dim;
     GemmArgs a{};
     a.A = A; a.Bt = Bt; a.C = static_cast<const float*>(C); a.D = static_cast<float*>(D);
     a.out16 = out16 ? 1 : 0;
     a.alpha = alpha; a.beta = beta;
     a.M = M; a.N = N; a.K = K;
-    a.tiles_m = (M + tile_rows - 1) / tile_rows;
-    a.tiles_n = (N + tile_rows - 1) / tile_rows;
+    a.tiles_m = (M + route.tile - 1) / route.tile;
+    a.tiles_n = (N + route.tile - 1) / route.tile;
     a.nseg = (K + t.segment_dim_k - 1) / t.segment_dim_k;
     a.tile_group_m = t.tile_group_m;
     a.num_stages = t.num_stages;
@@ -621,9 +646,9 @@ int gemm_launch(int dtype, const void* A, const void* Bt, const void* C, void* D
     a.whole_tiles = (int)tiles;
     a.fix_partials = nullptr;
     a.fix_state = nullptr;
-    if (direct) {
-        e = launch_gemm_direct(dtype == CK_DT_BF16, direct, K % 2 == 0 && !(((uintptr_t)A | (uintptr_t)Bt) & 3), s, a);
-    } else if (straight_line_tuple(t, opt) && gemm_stream_applies(a, t.tile_dim, t.segment_dim_k, t.num_stages, t.num_producer_waves, t.num_consumer_waves)) {
+    if (route.kernel == CKOPT_KERNEL_DIRECT) {
+        e = launch_gemm_direct(dtype == CK_DT_BF16, route.tile, K % 2 == 0 && !(((uintptr_t)A | (uintptr_t)Bt) & 3), s, a);
+    } else if (route.kernel == CKOPT_KERNEL_STREAM) {
         // Tile width, K slices and grid from the cost model: few tiles and a deep K are cut into slices so that every CU
         // has an item; the partly filled last round of many tiles likewise; tile counts that leave much of the device idle
         // take 256 x 128 tiles.
@@ -699,16 +724,16 @@ int gemm_launch(int dtype, const void* A, const void* Bt, const void* C, void* D
             }
             if (!scratch_release(sc, ws, s) && e == hipSuccess) e = hipErrorUnknown;
         }
-    } else if (mid_tuple(t, opt)) {
+    } else if (route.kernel == CKOPT_KERNEL_MID) {
         e = launch_gemm_mid(dtype == CK_DT_BF16, s, a);
-    } else if (t.num_producer_waves == 0 && t.num_stages == 1) {
+    } else if (route.kernel == CKOPT_KERNEL_SYNC) {
         // one stage, no producers: load, barrier, multiply, barrier (the synchronous A/B partner)
         e = dtype == CK_DT_F16 ? launch_gemm_sync_f16(t.tile_dim, t.segment_dim_k, t.num_consumer_waves, dim3(grid), lds, s, a)
                                : launch_gemm_sync_bf16(t.tile_dim, t.segment_dim_k, t.num_consumer_waves, dim3(grid), lds, s, a);
-    } else if (t.num_producer_waves == 0) {
+    } else if (route.kernel == CKOPT_KERNEL_FUSED) {
         e = dtype == CK_DT_F16 ? launch_gemm_fused_f16(t.tile_dim, t.segment_dim_k, t.num_consumer_waves, dim3(grid), lds, s, a)
                                : launch_gemm_fused_bf16(t.tile_dim, t.segment_dim_k, t.num_consumer_waves, dim3(grid), lds, s, a);
-    } else if (mode == CK_SYNC_TILE && t.num_stages >= 2 && opt[OPT_TILE_SYNC_BARRIER] && !a.single_producer && t.segment_dim_k <= 128) {
+    } else if (route.kernel == CKOPT_KERNEL_PCB) {
         // tile granularity through the workgroup barrier: the ring is the whole LDS allocation
         const size_t ring = (size_t)t.num_stages * 2 * stage_bytes_one_operand(t.tile_dim, t.segment_dim_k);
         e = dtype == CK_DT_F16 ? launch_gemm_pcb_f16(t.tile_dim, t.segment_dim_k, t.num_consumer_waves, dim3(grid), block, ring, s, a)
@@ -799,11 +824,10 @@ int ckopt_gemm_launch_plan_ex(int M, int N, int K, int operands_aligned, CK_TUNI
     if (M <= 0 || N <= 0 || K <= 0) return ck::CK_ERR_BAD_PARAM;
     const int rc = ck::check_gemm_tuning(t);
     if (rc != ck::CK_OK) return rc;
-    const int direct = direct_tile(M, N, K, operands_aligned != 0, t, opt);
-    const bool copies = !direct && needs_copies(K, operands_aligned != 0);
-    plan_out[0] = 0; plan_out[1] = direct ? direct : t.tile_dim; plan_out[2] = 1; plan_out[3] = copies ? 1 : 0;
+    const Route route = route_of(M, N, K, operands_aligned != 0, t, opt);
+    plan_out[0] = 0; plan_out[1] = route.tile; plan_out[2] = 1; plan_out[3] = route.copies ? 1 : 0;
     plan_out[4] = 0; plan_out[5] = 0; plan_out[6] = 0;
-    if (straight_line_tuple(t, opt)) {
+    if (route.kernel == CKOPT_KERNEL_STREAM) {
         const StreamPlan plan = stream_plan(M, N, launch_k(K, operands_aligned != 0, t, opt), t.num_cus, opt);
         plan_out[0] = 1;
         plan_out[1] = plan.tile_n;
@@ -817,6 +841,17 @@ int ckopt_gemm_launch_plan_ex(int M, int N, int K, int operands_aligned, CK_TUNI
 int ckopt_gemm_launch_plan(int M, int N, int K, int operands_aligned, CK_TUNING_PARAMS, int* plan_out) {
     return ckopt_gemm_launch_plan_ex(M, N, K, operands_aligned, tile_dim, segment_dim_k, bar_steps_a, bar_steps_b, bar_step_rows_a,
                                      bar_step_rows_b, tile_group_m, num_stages, num_producer_waves, num_consumer_waves, num_cus, nullptr, plan_out);
+}
+
+int ckopt_gemm_launch_kernel(int M, int N, int K, int operands_aligned, CK_TUNING_PARAMS, const ckopt_launch_options* options) {
+    Options opt;
+    const int orc = options_from_public(options, &opt);
+    if (orc != ck::CK_OK) return orc;
+    const ck::GemmTuning t = CK_TUNING_VALUE;
+    if (M <= 0 || N <= 0 || K <= 0) return ck::CK_ERR_BAD_PARAM;
+    const int rc = ck::check_gemm_tuning(t);
+    if (rc != ck::CK_OK) return rc;
+    return route_of(M, N, K, operands_aligned != 0, t, opt).kernel;
 }
 
 int ckopt_gemm_shmem_tc_async_opt_port_2_ws(int dtype, int cd_dtype, const void* A, const void* Bt, const void* C, void* D, float alpha,

@@ -45,9 +45,5 @@ hipError_t launch_gemm_stream_bf16(dim3 grid, hipStream_t stream, const GemmArgs
 }
 
 // what the kernel assumes about a launch (the caller falls back to the general fused kernel otherwise)
-bool gemm_stream_applies(const GemmArgs& a, int tile_dim, int segment_dim_k, int num_stages, int producer_waves, int consumer_waves) {
-    return producer_waves == 0 && consumer_waves == 8 && tile_dim == STREAM_TILE && segment_dim_k == STREAM_SEGK &&
-           num_stages == STREAM_STAGES && a.K % CHUNK_ELEMS == 0 && a.swizzle;
-}
 
 }  // namespace ck

@@ -90,7 +90,8 @@ int64_t ckopt_gemm_workspace_bytes(int M, int N, int K, int operands_aligned, in
 
 /* What a launch with these sizes and this tuning will run under the process's current options, without launching:
  * plan_out[0] = 1 if it takes the straight-line kernel (gemm_stream_kernel), 0 for the other designs;
- * plan_out[1] = width of its tiles in columns of D (256 or 128 for the straight-line kernel, else tile_dim);
+ * plan_out[1] = width of its tiles in columns of D (256, 192 or 128 for the straight-line kernel, 32 or 64 for
+ * gemm_direct_kernel, else tile_dim);
  * plan_out[2] = number of K slices (1: no split-K); plan_out[3] = 1 if A and Bt are first copied into zero-padded rows;
  * plan_out[4] = number of tiles that are cut into those slices (all of them when there are fewer tiles than num_cus; the
  * tiles of the partly filled last round otherwise; 0 without slices); plan_out[5] = 1 if the slices are added inside the
@@ -174,6 +175,22 @@ int ckopt_gemm_launch_plan_ex(int M, int N, int K, int operands_aligned, int til
                               int bar_steps_b, int bar_step_rows_a, int bar_step_rows_b, int tile_group_m, int num_stages,
                               int num_producer_waves, int num_consumer_waves, int num_cus, const ckopt_launch_options* options,
                               int* plan_out);
+
+/* Which kernel a launch with these sizes, this tuning and these options (NULL: the process's current ones) runs, without
+ * launching: a CKOPT_KERNEL_* value or, negative, the error the launch would give. Behind operand copies it is the kernel that
+ * runs on the copies. No reference counterpart. */
+enum {
+    CKOPT_KERNEL_FUSED = 0,   /* gemm_fused_kernel: LDS ring, no producer waves */
+    CKOPT_KERNEL_STREAM = 1,  /* gemm_stream_kernel: the straight-line kernel */
+    CKOPT_KERNEL_DIRECT = 2,  /* gemm_direct_kernel: small products */
+    CKOPT_KERNEL_MID = 3,     /* gemm_mid_kernel: 128 x 128 tiles staged through registers */
+    CKOPT_KERNEL_SYNC = 4,    /* gemm_sync_kernel: one stage */
+    CKOPT_KERNEL_PCB = 5,     /* gemm_pcb_kernel: producer waves, workgroup barrier */
+    CKOPT_KERNEL_PC = 6       /* gemm_pc_kernel: producer waves, LDS counters */
+};
+int ckopt_gemm_launch_kernel(int M, int N, int K, int operands_aligned, int tile_dim, int segment_dim_k, int bar_steps_a, int bar_steps_b,
+                             int bar_step_rows_a, int bar_step_rows_b, int tile_group_m, int num_stages, int num_producer_waves,
+                             int num_consumer_waves, int num_cus, const ckopt_launch_options* options);
 
 /* Replaces gemm_shmem_tc_async_opt_port<DT,DT_ACC>() of matmul_shmem_tc_async_opt_port_1.cu:889-965:
  * every wave tile (or every 16-row block) has its own signal, i.e. port_2 with maximal bar_steps. */

@@ -514,7 +514,7 @@ def test_small_tuple_leaves_the_kernel_to_the_estimate(ck):
     assert p["tile_cols"] == 64 and not p["operand_copies"]
     assert ck.gemm_launch_plan(512, 512, 512, False, *small)["operand_copies"] is False   # the query stays an upper bound here:
     assert ck.gemm_workspace_bytes(512, 512, 512, False, *small) >= 2 * 512 * 512 * 2
-    # the ring kernel: where it is shorter, with its copies; K below one chunk; another tuple; the straight-line switch or the
+    # operand copies: where the ring kernel behind them is shorter; K below one chunk; another tuple; the straight-line switch or the
     # swizzle off; fewer CUs than the device has (one workgroup per tile would not keep to them)
     ring = lambda *s, aligned=True, t=small, **kw: (ck.gemm_launch_plan(*s, aligned, *t, **kw)["operand_copies"], ck.gemm_workspace_bytes(*s, aligned, *t, **kw) > 0)
     assert ring(6000, 6000, 67) == (True, True) and ring(40, 100, 7) == (True, True)
@@ -525,3 +525,34 @@ def test_small_tuple_leaves_the_kernel_to_the_estimate(ck):
     assert ck.suggest_gemm_tuning(300, 520, 4090)["tile_dim"] == 256
     for s in ((32, 32, 64), (65, 31, 9), (200, 136, 1001), (512, 512, 512), (100, 3000, 501), (300, 300, 30000), (1500, 1500, 301)):
         assert ck.suggest_gemm_tuning(*s)["tile_dim"] == 64, s
+
+
+def test_plan_and_kernel_query_name_what_runs_behind_operand_copies(ck):
+    """A launch behind operand copies is a launch on sizes with K padded and aligned rows: the queries answer for that one. K below one
+    chunk of 8, odd K and operands off 16 bytes, few tiles and many, on the tuples whose kernel depends on the sizes."""
+    small, mid, straight = (64, 128, 0, 0, 64, 64, 4, 4, 0, 8, 256), (128, 128, 0, 0, 128, 128, 4, 2, 0, 8, 256), (256, 32, 0, 0, 256, 256, 4, 5, 0, 8, 256)
+    kernel = lambda *a, **kw: ck.gemm_launch_kernel(*a, **kw)
+    seen = set()
+    for t in (small, mid, straight):
+        unit = 64 if t is straight else 8
+        for M, N, K in ((40, 100, 7), (40, 100, 1), (1000, 1000, 1001), (2000, 2000, 3), (2048, 2048, 2049), (6000, 6000, 67), (4096, 4096, 2049), (10240, 10240, 201),
+                        (512, 512, 8192), (2000, 2100, 5127)):
+            for aligned in (False, True):
+                p = ck.gemm_launch_plan(M, N, K, aligned, *t)
+                if p["operand_copies"]:
+                    Kp = (K + unit - 1) // unit * unit
+                    q = ck.gemm_launch_plan(M, N, Kp, True, *t)
+                    assert not q["operand_copies"] and q["tile_cols"] == p["tile_cols"], (M, N, K, aligned, t[0])
+                    assert kernel(M, N, K, aligned, *t) == kernel(M, N, Kp, True, *t)
+                    seen.add((t[0], kernel(M, N, K, aligned, *t)))
+                else:
+                    assert K % 8 == 0 and aligned or kernel(M, N, K, aligned, *t) == "gemm_direct_kernel" and K >= 8
+    assert {(64, "gemm_direct_kernel"), (64, "gemm_fused_kernel"), (128, "gemm_mid_kernel"), (256, "gemm_stream_kernel")} <= seen
+    # the kernels that the tuple and the options decide alone
+    assert kernel(512, 512, 512, True, *small[:-1], 128) == "gemm_fused_kernel" == kernel(512, 512, 512, True, *small, options=ck.launch_options(straight_line=0))
+    assert kernel(512, 512, 512, True, 128, 64, 0, 0, 128, 128, 4, 1, 0, 8, 256) == "gemm_sync_kernel"
+    pc = (128, 64, 0, 0, 128, 128, 4, 2, 2, 4, 256)
+    assert kernel(512, 512, 512, True, *pc) == "gemm_pc_kernel"
+    assert kernel(512, 512, 512, True, *pc, options=ck.launch_options(tile_sync_barrier=1)) == "gemm_pcb_kernel"
+    with pytest.raises(ck.CkoptError):
+        kernel(0, 1, 1, True, *small)
