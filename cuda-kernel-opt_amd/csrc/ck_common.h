@@ -96,6 +96,15 @@ CK_HD int xcd_slot(int block, int grid, int num_xcd) {
     return (block % num_xcd) * (grid / num_xcd) + block / num_xcd;
 }
 
+// The same for kernels that launch one workgroup per tile, whatever the tile count is: XCD x gets the workgroups x, x + num_xcd, ...
+// and with them one run of consecutive tile counts. (Without it a count that 8 does not divide lost the L2: gemm_direct_kernel on
+// 384 x 10310 x 2048, 972 tiles, 61.6 us where the ring kernel takes 47.4, and 38.4 with it; 96 x 15808 x 4096 61.1 -> 33.3.)
+CK_HD int xcd_tile(int block, int tiles, int num_xcd) {
+    if (num_xcd <= 1) return block;
+    const int x = block % num_xcd, longer = tiles % num_xcd;   // the first `longer` XCDs have one tile more
+    return x * (tiles / num_xcd) + (x < longer ? x : longer) + block / num_xcd;
+}
+
 // ---- LDS ring layout ----------------------------------------------------------------------------
 // One stage of one operand is tile_dim rows of segment_dim_k 16-bit elements, stored row-major with
 // NO padding (a direct-to-LDS wave load writes 64 lanes x 16 B linearly), and the 16-byte chunks of

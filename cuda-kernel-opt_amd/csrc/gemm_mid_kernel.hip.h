@@ -34,7 +34,7 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(const GemmArgs g) {
     const int lane = threadIdx.x & 63;
     const unsigned long long clk0 = clock64(), wall0 = wall_clock64();
 
-    const TileRC rc = tile_order(g.tiles_m, g.tiles_n, g.tile_group_m, xcd_slot(blockIdx.x, gridDim.x, g.num_xcd));
+    const TileRC rc = tile_order(g.tiles_m, g.tiles_n, g.tile_group_m, xcd_tile(blockIdx.x, gridDim.x, g.num_xcd));
     const int row_a = rc.row * MID_TILE, row_b = rc.col * MID_TILE;
     const int64_t pitch = (int64_t)g.K * 2;
     const char* base_a = (const char*)g.A + row_a * pitch;

@@ -556,3 +556,27 @@ def test_plan_and_kernel_query_name_what_runs_behind_operand_copies(ck):
     assert kernel(512, 512, 512, True, *pc, options=ck.launch_options(tile_sync_barrier=1)) == "gemm_pcb_kernel"
     with pytest.raises(ck.CkoptError):
         kernel(0, 1, 1, True, *small)
+
+
+def test_tiles_of_an_xcd_are_one_run_whatever_their_number(tmp_path):
+    # workgroups are dealt to the XCDs in turn; every tile has one workgroup, and the tiles of an XCD are consecutive
+    import subprocess
+    src = tmp_path / "xcd.cpp"
+    src.write_text('''#include "ck_common.h"
+#include <vector>
+int main() {
+    for (int xcds : {1, 2, 8})
+        for (int tiles = 1; tiles < 600; ++tiles) {
+            std::vector<int> owner(tiles, -1);
+            for (int b = 0; b < tiles; ++b) {
+                const int t = ck::xcd_tile(b, tiles, xcds);
+                if (t < 0 || t >= tiles || owner[t] >= 0) return 1;
+                owner[t] = xcds > 1 ? b % xcds : 0;
+            }
+            for (int t = 1; t < tiles; ++t) if (owner[t] < owner[t - 1]) return 2;
+        }
+    return 0;
+}''')
+    exe = tmp_path / "xcd"
+    subprocess.run(["g++", "-std=c++17", "-I", os.path.join(ROOT, "cuda-kernel-opt_amd", "csrc"), str(src), "-o", str(exe)], check=True, timeout=120)
+    assert subprocess.run([str(exe)], timeout=60).returncode == 0
