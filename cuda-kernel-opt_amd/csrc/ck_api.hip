@@ -473,41 +473,49 @@ int launch_k(int K, bool operands_aligned, const ck::GemmTuning& t, const Option
 }
 
 // ---- tiles of at most 64: the ring kernel (gemm_fused_kernel) or the small-product kernel (gemm_direct_kernel) --------------------
-// Estimated microseconds, measured on 256 CUs with fp16 operands and fp32 results. The ring kernel on square tiles: one
-// workgroup per CU, per 128 of K 1.4 us for a 128 x 128 tile, 0.65 us for a 64 x 64 tile, about 4 us per round besides. The
-// small-product kernel: per round of one workgroup per CU 1.7 us for 32 x 32 and 3.0 us for 64 x 64 tiles, and per 512 of K (a
-// unit of 64 for each of the eight waves) 0.55 and 1.2 us while the device is nearly empty, 0.8 and 1.6 us when it is full
-// (L2); rows on 2-byte boundaries cost half as much again. Zero-padded operand copies: two allocations and a launch more.
-constexpr double COPIES_US = 16.0;
-double ring_us(int tile, int64_t tiles, int K, int num_cus) { return std::ceil((double)tiles / num_cus) * ((double)K / 128.0 * (tile == 128 ? 1.4 : 0.65) + 4.0); }
-double direct_us(int tile, int64_t tiles, int K, bool even, int num_cus) {
-    const double rounds = std::ceil((double)tiles / num_cus), units = std::ceil((double)K / 512.0), full = std::min(1.0, (double)tiles / num_cus);
-    const double unit_us = (tile == 32 ? 0.55 + 0.25 * full : 1.2 + 0.4 * full) * (even ? 1.0 : 1.5);
-    return 1.5 + rounds * ((tile == 32 ? 1.7 : 3.0) + units * unit_us);
+// Estimated microseconds of a call among others, fitted to calls on 1 to 64 rounds of tiles and K from 8 to 8192 (256 CUs). The ring
+// kernel on 64 tiles: per round 0.8 us and 0.655 per segment of 128 k (4096^2, 16 rounds: K 128 27 us, 1024 100, 4096 357); it is
+// persistent, so a round costs no launch and no empty device. The small-product kernel pays a fixed cost per round, one workgroup
+// per tile and one per CU, and per 512 of K (64 for each of the eight waves): least where every row starts on a line, more on
+// 4-byte boundaries and most on 2-byte ones (64 tiles, 4096^2: K 512 73 / 78 / 108 us, 1024 101 / 117 / 156, about 4096 243 / 317 /
+// 412), and less while the device is nearly empty (L2). Zero-padded operand copies: two allocations and a launch more, in all no less
+// than the 20 us and more that the host takes for them, and the copies' bytes.
+double ring_us(int64_t tiles, int K, int cus) { return 3.5 + std::ceil((double)tiles / cus) * (0.8 + 0.655 * std::ceil((double)K / 128.0)); }
+double direct_us(int tile, int64_t tiles, int K, int rows_aligned, int cus) {
+    struct Cost { double fixed, unit; };
+    constexpr Cost cost[2][3] = {{{1.7, 1.0}, {1.7, 1.35}, {2.2, 1.75}}, {{3.1, 0.95}, {2.5, 1.34}, {4.0, 1.69}}};   // 32, 64 tiles; lines, 4 bytes, 2 bytes
+    const Cost c = cost[tile == 64][rows_aligned >= LINE_BYTES ? 0 : rows_aligned >= 4 ? 1 : 2];
+    const double rounds = std::ceil((double)tiles / cus), full = std::min(1.0, (double)tiles / cus);
+    const double unit_us = (tile == 32 ? 0.55 + 0.25 * full : 1.2 + 0.4 * full) * c.unit;
+    return 1.5 + rounds * (c.fixed + unit_us * (double)std::max(K, 128) / 512.0);
 }
+double behind_copies_us(double us, int M, int N, int K) { return std::max(21.5, us + 7.5 + 4.0 * ((double)M + N) * K / 6e6); }
 // direct: tile of the small-product kernel, 0: the ring kernel on 64 x 64 tiles; copies: behind zero-padded operand copies
 struct SmallPlan { int direct; bool copies; double us; };
-SmallPlan small_plan(int M, int N, int K, bool operands_aligned, int num_cus) {
+SmallPlan small_plan(int M, int N, int K, int operand_alignment, int cus) {
     auto tiles = [&](int t) { return (int64_t)((M + t - 1) / t) * ((N + t - 1) / t); };
     SmallPlan best;
-    if (needs_copies(K, operands_aligned)) {   // what the launch on the copies, whose rows are padded to whole chunks, runs
-        best = small_plan(M, N, (K + ck::CHUNK_ELEMS - 1) / ck::CHUNK_ELEMS * ck::CHUNK_ELEMS, true, num_cus);
+    if (needs_copies(K, operand_alignment >= 16)) {   // what the launch on the copies, whose rows are padded to whole chunks, runs
+        const int Kp = (K + ck::CHUNK_ELEMS - 1) / ck::CHUNK_ELEMS * ck::CHUNK_ELEMS;
+        best = small_plan(M, N, Kp, 16, cus);
         best.copies = true;
-        best.us += COPIES_US;
-    } else best = SmallPlan{0, false, ring_us(64, tiles(64), K, num_cus)};
+        best.us = behind_copies_us(best.us, M, N, Kp);
+    } else best = SmallPlan{0, false, ring_us(tiles(64), K, cus)};
     if (K < ck::CHUNK_ELEMS) return best;   // the small-product kernel reads whole chunks of a row
+    const int rows_aligned = K % 2 ? 2 : operand_alignment < 16 || K % 64 ? std::min(operand_alignment, 4) : LINE_BYTES;
     for (int t : {32, 64}) {
-        const double us = direct_us(t, tiles(t), K, operands_aligned && K % 2 == 0, num_cus);
-        if (us < best.us) best = {t, false, us};
+        const double us = direct_us(t, tiles(t), K, rows_aligned, cus);
+        if (us < 0.95 * best.us) best = {t, false, us};   // (the ring where the two are level: 16-bit results favour it, 4096^2 x 1024 100 / 105)
     }
     return best;
 }
-// The tuple the library suggests for few tiles leaves the kernel to that estimate (512^3: 6.4 us on the ring, 5.1 on 32 x 32
-// tiles; 256 x 256 x 8192 45.8 -> 13.1; 1024^2 x 4096 25.3 -> 18.0 on 64 x 64; 200 x 136 x 1001 24 -> 6.0; 2048^2 x 128 stays on
-// the ring, 9.3 against 12.3). Only where it may use the whole device: one workgroup per tile, num_cus does not bound them.
+// The tuple the library suggests for few tiles leaves the kernel to that estimate (ring against this, us: 512^3 6.4 / 4.4;
+// 256 x 256 x 8192 45.8 / 13.1; 1024^2 x 4096 25.0 / 17.6; 200 x 136 x 1001 24 / 6.0. On several rounds the ring up to K about
+// 1100 - 2048^2 x 256 12.2 / 14.5, 8192^2 x 128 97 / 168 -, then this: 4096^2 x 2048 185 / 147). Only where it may use the
+// whole device: one workgroup per tile, num_cus does not bound them.
 bool small_tuple(const ck::GemmTuning& t, const Options& opt) {
     return opt[OPT_STRAIGHT_LINE] && opt[OPT_SWIZZLE] && t.num_producer_waves == 0 && t.num_consumer_waves == 8 && t.tile_dim == 64 &&
-           t.segment_dim_k == 128 && t.num_stages == 4 && t.num_cus >= device_cus();
+           t.segment_dim_k == 128 && t.num_stages == 4;
 }
 
 // The tuple the library suggests for 128 x 128 tiles runs the register-staged kernel (gemm_mid_kernel) where it may use the whole
@@ -518,20 +526,21 @@ bool mid_tuple(const ck::GemmTuning& t, const Options& opt) {
            t.segment_dim_k == 128 && t.num_stages == 2 && t.num_cus >= device_cus();
 }
 
-// What a launch runs: the one decision that the launcher and the queries share. A launch behind operand copies is decided
+// What a launch runs: the one decision that the launcher and the queries share. operand_alignment: bytes that A and Bt both lie on,
+// 16, 4 or 2 (the queries are promised 16 or nothing). A launch behind operand copies is decided
 // on the copies (K of launch_k, aligned), and the launch on them decides the same again.
 struct Route {
     int kernel;    // CKOPT_KERNEL_*
     int tile;      // rows of its tiles of D (and their columns, but for the straight-line kernel, whose width stream_plan chooses)
     bool copies;   // A and Bt are first copied into zero-padded rows
 };
-Route route_of(int M, int N, int K, bool operands_aligned, const ck::GemmTuning& t, const Options& opt) {
+Route route_of(int M, int N, int K, int operand_alignment, const ck::GemmTuning& t, const Options& opt) {
     using namespace ck;
-    if (small_tuple(t, opt)) {
-        const SmallPlan p = small_plan(M, N, K, operands_aligned, t.num_cus);
+    if (const int cus = small_tuple(t, opt) ? device_cus() : 0; cus && t.num_cus >= cus) {
+        const SmallPlan p = small_plan(M, N, K, operand_alignment, cus);
         return {p.direct ? CKOPT_KERNEL_DIRECT : CKOPT_KERNEL_FUSED, p.direct ? p.direct : t.tile_dim, p.copies};
     }
-    Route r{CKOPT_KERNEL_PC, t.tile_dim, needs_copies(K, operands_aligned)};
+    Route r{CKOPT_KERNEL_PC, t.tile_dim, needs_copies(K, operand_alignment >= 16)};
     if (straight_line_tuple(t, opt)) r.kernel = CKOPT_KERNEL_STREAM;
     else if (mid_tuple(t, opt)) r.kernel = CKOPT_KERNEL_MID;
     else if (t.num_producer_waves == 0) r.kernel = t.num_stages == 1 ? CKOPT_KERNEL_SYNC : CKOPT_KERNEL_FUSED;
@@ -594,8 +603,8 @@ int gemm_launch(int dtype, const void* A, const void* Bt, const void* C, void* D
     const uintptr_t elem_mask = out16 ? 1 : 3;
     if (((uintptr_t)D & elem_mask) || ((uintptr_t)C & elem_mask)) return CK_ERR_ALIGNMENT;
     // the ring kernels want every operand row on a 16-byte boundary
-    const bool aligned = !(((uintptr_t)A | (uintptr_t)Bt) & 15);
-    const Route route = route_of(M, N, K, aligned, t, opt);
+    const uintptr_t both = (uintptr_t)A | (uintptr_t)Bt;
+    const Route route = route_of(M, N, K, both & 15 ? both & 3 ? 2 : 4 : 16, t, opt);
     if (route.copies)
         return gemm_launch_repacked(dtype, A, Bt, C, D, alpha, beta, M, N, K, t, opt, stream, out16, sc);
     // one tile's rows are addressed through a 32-bit buffer offset
@@ -647,7 +656,7 @@ int gemm_launch(int dtype, const void* A, const void* Bt, const void* C, void* D
     a.fix_partials = nullptr;
     a.fix_state = nullptr;
     if (route.kernel == CKOPT_KERNEL_DIRECT) {
-        e = launch_gemm_direct(dtype == CK_DT_BF16, route.tile, K % 2 == 0 && !(((uintptr_t)A | (uintptr_t)Bt) & 3), s, a);
+        e = launch_gemm_direct(dtype == CK_DT_BF16, route.tile, K % 2 == 0 && !(both & 3), s, a);
     } else if (route.kernel == CKOPT_KERNEL_STREAM) {
         // Tile width, K slices and grid from the cost model: few tiles and a deep K are cut into slices so that every CU
         // has an item; the partly filled last round of many tiles likewise; tile counts that leave much of the device idle
@@ -824,7 +833,7 @@ int ckopt_gemm_launch_plan_ex(int M, int N, int K, int operands_aligned, CK_TUNI
     if (M <= 0 || N <= 0 || K <= 0) return ck::CK_ERR_BAD_PARAM;
     const int rc = ck::check_gemm_tuning(t);
     if (rc != ck::CK_OK) return rc;
-    const Route route = route_of(M, N, K, operands_aligned != 0, t, opt);
+    const Route route = route_of(M, N, K, operands_aligned ? 16 : 2, t, opt);
     plan_out[0] = 0; plan_out[1] = route.tile; plan_out[2] = 1; plan_out[3] = route.copies ? 1 : 0;
     plan_out[4] = 0; plan_out[5] = 0; plan_out[6] = 0;
     if (route.kernel == CKOPT_KERNEL_STREAM) {
@@ -851,7 +860,7 @@ int ckopt_gemm_launch_kernel(int M, int N, int K, int operands_aligned, CK_TUNIN
     if (M <= 0 || N <= 0 || K <= 0) return ck::CK_ERR_BAD_PARAM;
     const int rc = ck::check_gemm_tuning(t);
     if (rc != ck::CK_OK) return rc;
-    return route_of(M, N, K, operands_aligned != 0, t, opt).kernel;
+    return route_of(M, N, K, operands_aligned ? 16 : 2, t, opt).kernel;
 }
 
 int ckopt_gemm_shmem_tc_async_opt_port_2_ws(int dtype, int cd_dtype, const void* A, const void* Bt, const void* C, void* D, float alpha,
@@ -980,11 +989,14 @@ int ckopt_suggest_gemm_tuning(int M, int N, int K, int num_cus, int* tuning_out)
         // workspace have sized it for those slices, and keep the tuple that uses it.
         const GemmTuning st{256, 32, 0, 0, 256, 256, 4, 5, 0, 8, num_cus, 0};
         const StreamPlan straight = stream_plan(M, N, launch_k(K, true, st, opt), num_cus, opt);
-        const double us_128 = ring_us(128, tiles(128), K, num_cus), us_64 = ring_us(64, tiles(64), K, num_cus);
-        const SmallPlan small = small_plan(M, N, K, true, num_cus);
-        const double copies_us = needs_copies(K, true) ? COPIES_US : 0.0;
+        // (Measured per 128 of K: 1.4 us for a 128 x 128 tile, 0.65 us for a 64 x 64 tile, about 4 us per round besides.)
+        auto general_us = [&](int t, double seg_us) { return std::ceil((double)tiles(t) / num_cus) * ((double)K / 128.0 * seg_us + 4.0); };
+        const double us_128 = general_us(128, 1.4), us_64 = general_us(64, 0.65);
+        const int dev_cus = device_cus();
+        const SmallPlan small = small_plan(M, N, K, 16, dev_cus);
+        auto launched_us = [&](double us) { return needs_copies(K, true) ? behind_copies_us(us, M, N, K) : us; };
         if (straight.slices > 1 && straight.us <= us_128 && straight.us <= us_64) pick = straight_line;
-        else if (small.direct && num_cus >= device_cus() && small.us < us_128 + copies_us && small.us < straight.us + 1.5 + copies_us) pick = fused_64;
+        else if (small.direct && num_cus >= dev_cus && small.us < launched_us(us_128) && small.us < launched_us(straight.us + 1.5)) pick = fused_64;
         else if (straight.us <= us_128 && straight.us <= us_64) pick = straight_line;
         else if (us_128 <= us_64) pick = fused_128;
     }

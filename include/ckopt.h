@@ -178,7 +178,8 @@ int ckopt_gemm_launch_plan_ex(int M, int N, int K, int operands_aligned, int til
 
 /* Which kernel a launch with these sizes, this tuning and these options (NULL: the process's current ones) runs, without
  * launching: a CKOPT_KERNEL_* value or, negative, the error the launch would give. Behind operand copies it is the kernel that
- * runs on the copies. No reference counterpart. */
+ * runs on the copies. operands_aligned == 0 is answered, as by the plan query, for operands on 2-byte boundaries; a launch whose operands lie
+ * on 4-byte boundaries may run gemm_direct_kernel without the copies that are named here. No reference counterpart. */
 enum {
     CKOPT_KERNEL_FUSED = 0,   /* gemm_fused_kernel: LDS ring, no producer waves */
     CKOPT_KERNEL_STREAM = 1,  /* gemm_stream_kernel: the straight-line kernel */

@@ -580,3 +580,28 @@ int main() {
     exe = tmp_path / "xcd"
     subprocess.run(["g++", "-std=c++17", "-I", os.path.join(ROOT, "cuda-kernel-opt_amd", "csrc"), str(src), "-o", str(exe)], check=True, timeout=120)
     assert subprocess.run([str(exe)], timeout=60).returncode == 0
+
+
+def test_small_tuple_on_many_tiles_keeps_the_ring_kernel_where_it_is_the_faster(ck):
+    # The tuple of 64 tiles on several rounds of tiles; us per call of the ring kernel / the small-product kernel, measured on 256 CUs
+    small = (64, 128, 0, 0, 64, 64, 4, 4, 0, 8, 256)
+    kernel = lambda *s, aligned=True, cus=256: ck.gemm_launch_kernel(*s, aligned, *small[:-1], cus)
+    for s in ((2048, 2048, 256),    # 12.2 / 14.5
+              (3072, 3072, 512),    # 34.6 / 41.1
+              (4096, 4096, 256),    # 37.2 / 51.6
+              (4096, 4096, 768),    # 79.5 / 90.5
+              (8192, 8192, 128),    # 97 / 168
+              (8192, 8192, 513),    # 285 (behind copies) / 353
+              (6144, 6144, 201)):   # 94 (behind copies) / 184
+        assert kernel(*s) == "gemm_fused_kernel" == kernel(*s, cus=100000), s
+    for s in ((4096, 4096, 128), (4096, 4096, 512)):   # operands off a 16-byte boundary: 35 / 64, 69 / 108
+        assert kernel(*s, aligned=False) == "gemm_fused_kernel", s
+    for s in ((1024, 1024, 512),    # 6.9 / 6.2
+              (1536, 1536, 1024),   # 21.5 / 18.8
+              (2048, 2048, 2048),   # 48.5 / 38.7
+              (4096, 4096, 2048),   # 185 / 147
+              (8192, 8192, 4096)):  # 1420 / 970
+        assert kernel(*s) == "gemm_direct_kernel" == kernel(*s, cus=100000), s
+    # a long odd K on many tiles: 3072^2 x 2049 125 us (ring behind copies), 141 (rows where they are), 105 on aligned rows: copies and the small-product kernel
+    for s in ((3072, 3072, 2049), (4096, 4096, 4097)):
+        assert kernel(*s) == "gemm_direct_kernel" and ck.gemm_launch_plan(*s, True, *small)["operand_copies"], s
