@@ -289,8 +289,9 @@ bool scratch_release(const Scratch& sc, void* piece, hipStream_t s) {
     return sc.mode != Scratch::ALLOCATE || hipFreeAsync(piece, s) == hipSuccess;
 }
 
+struct Route;
 int gemm_launch(int dtype, const void* A, const void* Bt, const void* C, void* D, float alpha, float beta, int M,
-                int N, int K, const ck::GemmTuning& t, const Options& opt, void* stream, int out16, Scratch sc);
+                int N, int K, const ck::GemmTuning& t, const Options& opt, void* stream, int out16, Scratch sc, const Route* on_copies = nullptr);
 
 // Estimated duration (microseconds) of the straight-line kernel on `tiles` tiles of 256 x tile_n (256, 192 or 128) of an
 // M x N product with K cut into S slices, plus what adding the slices costs when S > 1. The constants
@@ -518,17 +519,27 @@ bool small_tuple(const ck::GemmTuning& t, const Options& opt) {
            t.segment_dim_k == 128 && t.num_stages == 4;
 }
 
-// The tuple the library suggests for 128 x 128 tiles runs the register-staged kernel (gemm_mid_kernel) where it may use the whole
-// device: one workgroup per tile, num_cus does not bound
-// them (ring against this, us: 2048^3 26.2 / 26.4, 2048^2 x 2176 27.2 / 25.9, 256 x 16384 x 4096 47.7 / 44.8, 8192^2 x 8128 1261 / 1237).
+// The tuple the library suggests for 128 x 128 tiles, where it may use the whole device, runs the register-staged kernel (gemm_mid_kernel)
+// or the ring kernel. The former has one workgroup per tile and CU and pays its prologue (three segments of 128 k) and epilogue on
+// every tile; the persistent ring kernel overlaps them with the next tile's loads, and on a full device loses less where the
+// rows of the operands do not start on lines. Ring / register-staged, us:
+//   fewer tiles than CUs, 1024^2 x 256 7.8 / 8.4, x 512 10.0 / 10.3, x 4096 41.8 / 39.0; 60 drawn shapes of 24 to 255 tiles, fp32 results: K 256 1.04 to
+//     1.09, 576 0.92 to 1.01, 1024 0.88 to 0.97, 3000 0.80 to 1.01 (16-bit results 0.82 to 1.07)
+//   as many tiles as CUs, 2048^2 x 512 11.6 / 12.1, x 1536 21 / 21, x 4096 44.1 / 42.0, 256 x 16384 x 1024 16.9 / 17.7, x 4096 47.6 / 43.5, x 3000 1.04
+//     (behind operand copies the ring everywhere: 12096 x 104 x 688 27.9 / 33.8, 4096 x 768 x 2692 46.4 / 48.2)
+//   several rounds, 4096^2 x 512 35.4 / 42.4, x 2048 91.5 / 97.5, x 4096 167 / 163, x 4104 1.09; 6144^2 (9 rounds) x 4096 372 / 368;
+//     8192^2 (16) with 16-bit results x 512 135 / 239, x 6144 958 / 985
 bool mid_tuple(const ck::GemmTuning& t, const Options& opt) {
     return opt[OPT_STRAIGHT_LINE] && opt[OPT_SWIZZLE] && t.num_producer_waves == 0 && t.num_consumer_waves == 8 && t.tile_dim == 128 &&
-           t.segment_dim_k == 128 && t.num_stages == 2 && t.num_cus >= device_cus();
+           t.segment_dim_k == 128 && t.num_stages == 2;
+}
+bool mid_is_shorter(int64_t tiles, int K, int cus) {
+    if (tiles < cus) return K > 512;
+    return K % 64 == 0 && (tiles == cus ? K >= 1536 : tiles <= 9 * (int64_t)cus && K >= 4096);
 }
 
 // What a launch runs: the one decision that the launcher and the queries share. operand_alignment: bytes that A and Bt both lie on,
-// 16, 4 or 2 (the queries are promised 16 or nothing). A launch behind operand copies is decided
-// on the copies (K of launch_k, aligned), and the launch on them decides the same again.
+// 16, 4 or 2 (the queries are promised 16 or nothing). Behind operand copies it is what runs on them.
 struct Route {
     int kernel;    // CKOPT_KERNEL_*
     int tile;      // rows of its tiles of D (and their columns, but for the straight-line kernel, whose width stream_plan chooses)
@@ -536,13 +547,17 @@ struct Route {
 };
 Route route_of(int M, int N, int K, int operand_alignment, const ck::GemmTuning& t, const Options& opt) {
     using namespace ck;
-    if (const int cus = small_tuple(t, opt) ? device_cus() : 0; cus && t.num_cus >= cus) {
+    Route r{CKOPT_KERNEL_PC, t.tile_dim, needs_copies(K, operand_alignment >= 16)};
+    // (the two kernels with one workgroup per tile, which num_cus does not bound, only where the launch may use the whole device)
+    const bool small = small_tuple(t, opt), mid = mid_tuple(t, opt);
+    const int cus = small || mid ? device_cus() : 0;
+    if (small && t.num_cus >= cus) {
         const SmallPlan p = small_plan(M, N, K, operand_alignment, cus);
         return {p.direct ? CKOPT_KERNEL_DIRECT : CKOPT_KERNEL_FUSED, p.direct ? p.direct : t.tile_dim, p.copies};
     }
-    Route r{CKOPT_KERNEL_PC, t.tile_dim, needs_copies(K, operand_alignment >= 16)};
     if (straight_line_tuple(t, opt)) r.kernel = CKOPT_KERNEL_STREAM;
-    else if (mid_tuple(t, opt)) r.kernel = CKOPT_KERNEL_MID;
+    else if (mid && t.num_cus >= cus && !r.copies && mid_is_shorter((int64_t)((M + 127) / 128) * ((N + 127) / 128), K, cus))
+        r.kernel = CKOPT_KERNEL_MID;
     else if (t.num_producer_waves == 0) r.kernel = t.num_stages == 1 ? CKOPT_KERNEL_SYNC : CKOPT_KERNEL_FUSED;
     else if (sync_mode_of(t.tile_dim, t.num_consumer_waves, t.bar_step_rows_a, t.bar_step_rows_b) == CK_SYNC_TILE && t.num_stages >= 2 &&
              opt[OPT_TILE_SYNC_BARRIER] && t.num_producer_waves != 1 && t.segment_dim_k <= 128)
@@ -570,7 +585,7 @@ size_t scratch_need(int M, int N, int K, bool operands_aligned, const ck::GemmTu
 // K % 8 != 0 or operands off a 16-byte boundary: the product is computed from zero-padded,
 // aligned copies of A and Bt in a stream-ordered temporary (zeros in the K tail add nothing).
 int gemm_launch_repacked(int dtype, const void* A, const void* Bt, const void* C, void* D, float alpha, float beta,
-                         int M, int N, int K, const ck::GemmTuning& t, const Options& opt, void* stream, int out16, Scratch sc) {
+                         int M, int N, int K, const ck::GemmTuning& t, const Options& opt, void* stream, int out16, Scratch sc, Route route) {
     using namespace ck;
     const int Kp = padded_k(K, t, opt);
     const size_t bytes_a = (size_t)M * Kp * 2, bytes_b = (size_t)N * Kp * 2;
@@ -585,13 +600,14 @@ int gemm_launch_repacked(int dtype, const void* A, const void* Bt, const void* C
     hipLaunchKernelGGL(pad_rows_kernel, dim3(blocks(((long long)M + N) * (Kp / 8))), dim3(threads), 0, s, static_cast<const unsigned short*>(A), pa, M,
                        static_cast<const unsigned short*>(Bt), pb, N, K, Kp);
     int rc = hipGetLastError() == hipSuccess ? CK_OK : CK_ERR_HIP;
-    if (rc == CK_OK) rc = gemm_launch(dtype, pa, pb, C, D, alpha, beta, M, N, Kp, t, opt, stream, out16, sc);
+    route.copies = false;
+    if (rc == CK_OK) rc = gemm_launch(dtype, pa, pb, C, D, alpha, beta, M, N, Kp, t, opt, stream, out16, sc, &route);
     if (!scratch_release(sc, ws, s) && rc == CK_OK) rc = CK_ERR_HIP;
     return rc;
 }
 
 int gemm_launch(int dtype, const void* A, const void* Bt, const void* C, void* D, float alpha, float beta, int M,
-                int N, int K, const ck::GemmTuning& t, const Options& opt, void* stream, int out16, Scratch sc) {
+                int N, int K, const ck::GemmTuning& t, const Options& opt, void* stream, int out16, Scratch sc, const Route* on_copies) {
     using namespace ck;
     if (!(dtype == CK_DT_F16 || dtype == CK_DT_BF16)) return CK_ERR_BAD_PARAM;
     if (M <= 0 || N <= 0 || K <= 0) return CK_ERR_BAD_PARAM;
@@ -604,9 +620,9 @@ int gemm_launch(int dtype, const void* A, const void* Bt, const void* C, void* D
     if (((uintptr_t)D & elem_mask) || ((uintptr_t)C & elem_mask)) return CK_ERR_ALIGNMENT;
     // the ring kernels want every operand row on a 16-byte boundary
     const uintptr_t both = (uintptr_t)A | (uintptr_t)Bt;
-    const Route route = route_of(M, N, K, both & 15 ? both & 3 ? 2 : 4 : 16, t, opt);
+    const Route route = on_copies ? *on_copies : route_of(M, N, K, both & 15 ? both & 3 ? 2 : 4 : 16, t, opt);
     if (route.copies)
-        return gemm_launch_repacked(dtype, A, Bt, C, D, alpha, beta, M, N, K, t, opt, stream, out16, sc);
+        return gemm_launch_repacked(dtype, A, Bt, C, D, alpha, beta, M, N, K, t, opt, stream, out16, sc, route);
     // one tile's rows are addressed through a 32-bit buffer offset
     if ((int64_t)t.tile_dim * K * 2 >= (int64_t)1 << 31) return CK_ERR_TOO_LARGE;
 

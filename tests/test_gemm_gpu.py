@@ -1469,6 +1469,7 @@ def test_small_product_kernel_exact_at_its_edges(ck, bf16, shift):
         buf_b, b = operand(N)
         plan = ck.gemm_launch_plan(M, N, K, shift % 8 == 0, *SMALL_TUPLE)
         assert not plan["operand_copies"] and plan["tile_cols"] in (32, 64)
+        assert ck.gemm_launch_kernel(M, N, K, shift % 8 == 0, *SMALL_TUPLE) == "gemm_direct_kernel"
         seen.add(plan["tile_cols"])
         exact = (a.cpu().double() @ b.cpu().double().t())
         guard = 64
@@ -1507,7 +1508,7 @@ def test_small_product_kernel_keeps_infinities_to_their_rows(ck):
 
 @pytest.mark.parametrize("bf16", [False, True])
 def test_register_staged_128_tiles_exact_at_their_edges(ck, bf16):
-    """The kernel behind the tuple suggested for 128 x 128 tiles, exact on small integers: ragged edges, one segment of 128 and less, the
+    """The tuple suggested for 128 x 128 tiles (sizes on the ring kernel and on the register-staged one), exact on small integers: ragged edges, one segment of 128 and less, the
     two stages' parities, K that ends inside a segment's first and second line, more tiles than CUs; C, 16-bit results, a guard
     behind D; fewer CUs (the persistent ring kernel) give the same."""
     dtype, tdt = (ck.DT_BF16, torch.bfloat16) if bf16 else (ck.DT_F16, torch.float16)
@@ -1529,4 +1530,75 @@ def test_register_staged_128_tiles_exact_at_their_edges(ck, bf16):
         ck.gemm_shmem_tc_async_opt_port_lp(dtype, a, b, None, d16, 1.0, 0.0, M, N, K, *tup)
         assert torch.equal(d16[:M * N].view(M, N).cpu(), exact.to(tdt)), (M, N, K)
         assert torch.isnan(d16[M * N:]).all()
+    assert ck.device_status() == 0
+
+
+MID_TUPLE = (128, 128, 0, 0, 128, 128, 4, 2, 0, 8, 256)   # what the library suggests for 128 x 128 tiles
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+def test_register_staged_kernel_on_its_own_sizes(ck, bf16):
+    """gemm_mid_kernel where the launcher takes it, exact on small integers (sums below 2^24; 16-bit results round the exact value once): K
+    that ends in the first and second line of a segment of 128 and on its edge, an odd and an even number of segments, ragged edges, tile
+    counts that 8 does not divide, two rounds of tiles. The operands lie in buffers full of NaN, which no lane may multiply; fp32 and
+    16-bit C; a guard behind D."""
+    dtype, tdt = (ck.DT_BF16, torch.bfloat16) if bf16 else (ck.DT_F16, torch.float16)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(17)
+    for M, N, K in [(1, 4, 520), (130, 127, 568), (64, 200, 584), (256, 129, 632), (300, 300, 640), (257, 384, 648), (129, 1, 768), (200, 136, 896),
+                    (384, 250, 1024), (1300, 1100, 1000), (2048, 2048, 1536), (2100, 2060, 4096)]:
+        def operand(rows):
+            buf = torch.full((rows * K + 16,), float("nan"), dtype=tdt, device="cuda")
+            view = buf[:rows * K].view(rows, K)
+            view.copy_(torch.randint(-2, 3, (rows, K), device="cuda", generator=gen))
+            return buf, view
+        buf_a, a = operand(M)
+        buf_b, b = operand(N)
+        assert ck.gemm_launch_kernel(M, N, K, True, *MID_TUPLE) == "gemm_mid_kernel"
+        exact = a.cpu().double() @ b.cpu().double().t()
+        c = torch.randint(-8, 9, (M, N), device="cuda", generator=gen).float()
+        d = torch.full((M * N + 64,), float("nan"), dtype=torch.float32, device="cuda")
+        ck.gemm_shmem_tc_async_opt_port(dtype, a, b, c, d, 2.0, -3.0, M, N, K, *MID_TUPLE)
+        assert torch.equal(d[:M * N].view(M, N).cpu().double(), 2 * exact - 3 * c.cpu().double()), (M, N, K)
+        assert torch.isnan(d[M * N:]).all()
+        d16 = torch.full((M * N + 64,), float("nan"), dtype=tdt, device="cuda")
+        ck.gemm_shmem_tc_async_opt_port_lp(dtype, a, b, c.to(tdt), d16, 1.0, 1.0, M, N, K, *MID_TUPLE)
+        assert torch.equal(d16[:M * N].view(M, N).cpu(), (exact + c.cpu().double()).to(tdt)), (M, N, K)
+        assert torch.isnan(d16[M * N:]).all()
+    assert ck.device_status() == 0
+
+
+def test_register_staged_kernel_keeps_infinities_to_their_rows(ck):
+    """Rows past the edge are read as the last row and k past the end as zeros: an infinity or a NaN in the last row, column or k
+    reaches the outputs that it belongs to and no other."""
+    M, N, K = 140, 150, 584
+    assert ck.gemm_launch_kernel(M, N, K, True, *MID_TUPLE) == "gemm_mid_kernel"
+    a = torch.ones((M, K), dtype=torch.float16, device="cuda")
+    b = torch.ones((N, K), dtype=torch.float16, device="cuda")
+    a[M - 1, K - 1] = float("inf")
+    b[N - 1, 0] = float("nan")
+    d = torch.zeros((M, N), dtype=torch.float32, device="cuda")
+    ck.gemm_shmem_tc_async_opt_port(ck.DT_F16, a, b, None, d, 1.0, 0.0, M, N, K, *MID_TUPLE)
+    want = torch.full((M, N), float(K))
+    want[M - 1, :] = float("inf")
+    want[:, N - 1] = float("nan")
+    assert torch.equal(torch.nan_to_num(d.cpu(), nan=-1.0), torch.nan_to_num(want, nan=-1.0))
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+def test_small_tuple_on_many_tiles_and_behind_copies(ck, bf16):
+    """The tuple of 64 tiles on the other sides of its rule, exact on small integers: the ring kernel on several rounds of tiles, on aligned
+    rows and behind copies, and the small-product kernel behind copies (K below one chunk of 8, a long odd K on many tiles)."""
+    dtype, tdt = (ck.DT_BF16, torch.bfloat16) if bf16 else (ck.DT_F16, torch.float16)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(19)
+    for M, N, K, kernel, copies in [(1600, 1500, 256, "gemm_fused_kernel", False), (3000, 2900, 201, "gemm_fused_kernel", True),
+                                    (40, 100, 7, "gemm_direct_kernel", True), (33, 31, 1, "gemm_direct_kernel", True), (3000, 3100, 2049, "gemm_direct_kernel", True)]:
+        assert ck.gemm_launch_kernel(M, N, K, True, *SMALL_TUPLE) == kernel and ck.gemm_launch_plan(M, N, K, True, *SMALL_TUPLE)["operand_copies"] == copies
+        a = torch.randint(-2, 3, (M, K), device="cuda", generator=gen).to(tdt)
+        b = torch.randint(-2, 3, (N, K), device="cuda", generator=gen).to(tdt)
+        d = torch.full((M * N + 64,), float("nan"), dtype=torch.float32, device="cuda")
+        ck.gemm_shmem_tc_async_opt_port(dtype, a, b, None, d, 1.0, 0.0, M, N, K, *SMALL_TUPLE)
+        assert torch.equal(d[:M * N].view(M, N).cpu(), a.cpu().float() @ b.cpu().float().t()), (M, N, K)   # (fp32 sums of whole numbers below 2^24 are exact)
+        assert torch.isnan(d[M * N:]).all()
     assert ck.device_status() == 0

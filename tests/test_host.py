@@ -543,11 +543,12 @@ def test_plan_and_kernel_query_name_what_runs_behind_operand_copies(ck):
                     Kp = (K + unit - 1) // unit * unit
                     q = ck.gemm_launch_plan(M, N, Kp, True, *t)
                     assert not q["operand_copies"] and q["tile_cols"] == p["tile_cols"], (M, N, K, aligned, t[0])
-                    assert kernel(M, N, K, aligned, *t) == kernel(M, N, Kp, True, *t)
+                    # (the tuple of 128 tiles: always the ring kernel behind copies)
+                    assert kernel(M, N, K, aligned, *t) == ("gemm_fused_kernel" if t is mid else kernel(M, N, Kp, True, *t))
                     seen.add((t[0], kernel(M, N, K, aligned, *t)))
                 else:
-                    assert K % 8 == 0 and aligned or kernel(M, N, K, aligned, *t) == "gemm_direct_kernel" and K >= 8
-    assert {(64, "gemm_direct_kernel"), (64, "gemm_fused_kernel"), (128, "gemm_mid_kernel"), (256, "gemm_stream_kernel")} <= seen
+                    assert K % 8 == 0 and aligned or t is small and kernel(M, N, K, aligned, *t) == "gemm_direct_kernel" and K >= 8
+    assert {(64, "gemm_direct_kernel"), (64, "gemm_fused_kernel"), (128, "gemm_fused_kernel"), (256, "gemm_stream_kernel")} == seen
     # the kernels that the tuple and the options decide alone
     assert kernel(512, 512, 512, True, *small[:-1], 128) == "gemm_fused_kernel" == kernel(512, 512, 512, True, *small, options=ck.launch_options(straight_line=0))
     assert kernel(512, 512, 512, True, 128, 64, 0, 0, 128, 128, 4, 1, 0, 8, 256) == "gemm_sync_kernel"
@@ -605,3 +606,33 @@ def test_small_tuple_on_many_tiles_keeps_the_ring_kernel_where_it_is_the_faster(
     # a long odd K on many tiles: 3072^2 x 2049 125 us (ring behind copies), 141 (rows where they are), 105 on aligned rows: copies and the small-product kernel
     for s in ((3072, 3072, 2049), (4096, 4096, 4097)):
         assert kernel(*s) == "gemm_direct_kernel" and ck.gemm_launch_plan(*s, True, *small)["operand_copies"], s
+
+
+def test_tuple_of_128_tiles_keeps_the_ring_kernel_where_it_is_the_faster(ck):
+    # us per call of the ring kernel / the register-staged kernel, measured on 256 CUs
+    mid = (128, 128, 0, 0, 128, 128, 4, 2, 0, 8, 256)
+    kernel = lambda *s, aligned=True, cus=256: ck.gemm_launch_kernel(*s, aligned, *mid[:-1], cus)
+    for s in ((2048, 2048, 256),     # 9.3 / 10.0
+              (256, 16384, 512),     # 11.6 / 12.6
+              (1024, 1024, 256),     # 7.8 / 8.4
+              (256, 16384, 3000),    # 1.04 times: rows off a line
+              (4096, 4096, 4104),    # 1.09 times: the same
+              (2048, 2176, 128),     # 9.6 / 13.6
+              (4096, 4096, 512),     # 35.4 / 42.4
+              (6144, 6144, 256),     # 48 / 71
+              (8192, 8192, 256),     # 80 / 119, with 16-bit results 105 / 194
+              (8192, 8192, 6144),    # with 16-bit results 958 / 985
+              (1, 1100000000, 8)):   # 8.6 million tiles: one workgroup each is more than a launch can have
+        for aligned in (True, False):
+            assert kernel(*s, aligned=aligned) == "gemm_fused_kernel", s
+    for s in ((2048, 2048, 2048),    # 25.5 / 25.3
+              (256, 16384, 4096),    # 47.6 / 43.5
+              (1024, 1024, 4096),    # 41.8 / 39.0
+              (4096, 192, 1024),     # 17.6 / 16.1
+              (128, 32768, 1536),    # 26 / 24
+              (2048, 2176, 4096),    # 83.9 / 77.8
+              (4096, 4096, 5120)):   # 208 / 205
+        assert kernel(*s) == "gemm_mid_kernel" == kernel(*s, cus=512), s
+        assert kernel(*s, cus=255) == "gemm_fused_kernel" == kernel(*s, aligned=False)   # (behind copies: 12096 x 104 x 688 27.9 / 33.8)
+    assert kernel(2048, 2048, 2041) == "gemm_fused_kernel"
+    assert ck.gemm_launch_kernel(1, 600000000, 200, True, 64, 128, 0, 0, 64, 64, 4, 4, 0, 8, 256) == "gemm_fused_kernel"   # (as above, 64 tiles)
