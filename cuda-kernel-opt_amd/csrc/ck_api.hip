@@ -285,6 +285,11 @@ int scratch_take(Scratch& sc, size_t need, hipStream_t s, void** out) {
     sc.bytes -= used < sc.bytes ? used : sc.bytes;
     return ck::CK_OK;
 }
+// Would scratch_take find `need` bytes? (An allocation is not tried.)
+bool scratch_holds(Scratch sc, size_t need) {
+    void* at = nullptr;
+    return sc.mode == Scratch::ALLOCATE || scratch_take(sc, need, nullptr, &at) == ck::CK_OK;
+}
 bool scratch_release(const Scratch& sc, void* piece, hipStream_t s) {
     return sc.mode != Scratch::ALLOCATE || hipFreeAsync(piece, s) == hipSuccess;
 }
@@ -570,8 +575,8 @@ Route route_of(int M, int N, int K, int operand_alignment, const ck::GemmTuning&
 size_t scratch_need(int M, int N, int K, bool operands_aligned, const ck::GemmTuning& t, const Options& opt) {
     using namespace ck;
     size_t need = 0;
-    // (For the tuple that the small-product kernel serves the answer stays what the ring kernel's copies take, which is more than
-    // that kernel's nothing: programs size one buffer for many calls by it.)
+    // (For the tuple that the small-product kernel serves the answer is what the copies take, whether that kernel runs without
+    // them or not: programs size one buffer for many calls by it, and the launch asks for no less.)
     const int k = launch_k(K, operands_aligned, t, opt);
     if (needs_copies(K, operands_aligned)) need += scratch_round(((size_t)M + (size_t)N) * k * 2);
     if (straight_line_tuple(t, opt)) {
@@ -623,6 +628,9 @@ int gemm_launch(int dtype, const void* A, const void* Bt, const void* C, void* D
     const Route route = on_copies ? *on_copies : route_of(M, N, K, both & 15 ? both & 3 ? 2 : 4 : 16, t, opt);
     if (route.copies)
         return gemm_launch_repacked(dtype, A, Bt, C, D, alpha, beta, M, N, K, t, opt, stream, out16, sc, route);
+    // A provided buffer has to hold what the workspace query names, also where the small-product kernel makes no copies in it: whether a
+    // call is accepted does not hang on the kernel that an estimate picks.
+    if (!on_copies && needs_copies(K, !(both & 15)) && !scratch_holds(sc, ((size_t)M + (size_t)N) * padded_k(K, t, opt) * 2)) return CK_ERR_TOO_LARGE;
     // one tile's rows are addressed through a 32-bit buffer offset
     if ((int64_t)t.tile_dim * K * 2 >= (int64_t)1 << 31) return CK_ERR_TOO_LARGE;
 

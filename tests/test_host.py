@@ -636,3 +636,22 @@ def test_tuple_of_128_tiles_keeps_the_ring_kernel_where_it_is_the_faster(ck):
         assert kernel(*s, cus=255) == "gemm_fused_kernel" == kernel(*s, aligned=False)   # (behind copies: 12096 x 104 x 688 27.9 / 33.8)
     assert kernel(2048, 2048, 2041) == "gemm_fused_kernel"
     assert ck.gemm_launch_kernel(1, 600000000, 200, True, 64, 128, 0, 0, 64, 64, 4, 4, 0, 8, 256) == "gemm_fused_kernel"   # (as above, 64 tiles)
+
+
+def test_a_provided_buffer_must_hold_what_the_query_names_whatever_kernel_runs(ck):
+    # the tuple of 64 tiles on an odd K: the small-product kernel reads the rows where they are, and a buffer too small for the copies that
+    # the query names is refused all the same, before anything is launched (the pointers below are never used)
+    small = (64, 128, 0, 0, 64, 64, 4, 4, 0, 8, 256)
+    M, N, K = 200, 136, 1001
+    assert ck.gemm_launch_kernel(M, N, K, True, *small) == "gemm_direct_kernel" and not ck.gemm_launch_plan(M, N, K, True, *small)["operand_copies"]
+    need = ck.gemm_workspace_bytes(M, N, K, True, *small)
+    assert need >= (M + N) * 1008 * 2
+    base = 1 << 40
+    for dtype, cd in ((ck.DT_F16, ck.DT_F32), (ck.DT_BF16, ck.DT_BF16)):
+        for ws, nbytes in ((None, 0), (base, (M + N) * 1008 * 2 - 1), (base + 1, (M + N) * 1008 * 2)):
+            with pytest.raises(ck.CkoptError) as e:
+                ck.gemm_shmem_tc_async_opt_port_ws(dtype, cd, base, base, None, base, 1.0, 0.0, M, N, K, *small, workspace=ws, workspace_bytes=nbytes)
+            assert e.value.code == ck.ERR_TOO_LARGE, (dtype, nbytes)
+    with pytest.raises(ck.CkoptError) as e:   # operands off a 16-byte boundary: the same
+        ck.gemm_shmem_tc_async_opt_port_ws(ck.DT_F16, ck.DT_F32, base + 2, base, None, base, 1.0, 0.0, 512, 512, 512, *small, workspace=base, workspace_bytes=1000)
+    assert e.value.code == ck.ERR_TOO_LARGE
