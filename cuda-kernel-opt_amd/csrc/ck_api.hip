@@ -626,13 +626,13 @@ int gemm_launch(int dtype, const void* A, const void* Bt, const void* C, void* D
     // the ring kernels want every operand row on a 16-byte boundary
     const uintptr_t both = (uintptr_t)A | (uintptr_t)Bt;
     const Route route = on_copies ? *on_copies : route_of(M, N, K, both & 15 ? both & 3 ? 2 : 4 : 16, t, opt);
+    // one tile's rows are addressed through a 32-bit buffer offset (rows of the copies, also where a kernel does without them)
+    if ((int64_t)t.tile_dim * launch_k(K, !(both & 15), t, opt) * 2 >= (int64_t)1 << 31) return CK_ERR_TOO_LARGE;
     if (route.copies)
         return gemm_launch_repacked(dtype, A, Bt, C, D, alpha, beta, M, N, K, t, opt, stream, out16, sc, route);
     // A provided buffer has to hold what the workspace query names, also where the small-product kernel makes no copies in it: whether a
     // call is accepted does not hang on the kernel that an estimate picks.
     if (!on_copies && needs_copies(K, !(both & 15)) && !scratch_holds(sc, ((size_t)M + (size_t)N) * padded_k(K, t, opt) * 2)) return CK_ERR_TOO_LARGE;
-    // one tile's rows are addressed through a 32-bit buffer offset
-    if ((int64_t)t.tile_dim * K * 2 >= (int64_t)1 << 31) return CK_ERR_TOO_LARGE;
 
     const int mode = sync_mode_of(t.tile_dim, t.num_consumer_waves, t.bar_step_rows_a, t.bar_step_rows_b);
     GemmArgs a{};

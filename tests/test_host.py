@@ -655,3 +655,15 @@ def test_a_provided_buffer_must_hold_what_the_query_names_whatever_kernel_runs(c
     with pytest.raises(ck.CkoptError) as e:   # operands off a 16-byte boundary: the same
         ck.gemm_shmem_tc_async_opt_port_ws(ck.DT_F16, ck.DT_F32, base + 2, base, None, base, 1.0, 0.0, 512, 512, 512, *small, workspace=base, workspace_bytes=1000)
     assert e.value.code == ck.ERR_TOO_LARGE
+
+
+def test_the_largest_k_is_the_same_for_rows_in_place_and_rows_copied(ck):
+    # 64 rows of the padded copies have to lie within 2^31 bytes; the small-product kernel, which reads the rows in place, refuses the same K
+    # (nothing is launched: the pointers are never used)
+    small = (64, 128, 0, 0, 64, 64, 4, 4, 0, 8, 256)
+    assert ck.gemm_launch_kernel(1, 1, 16777209, True, *small) == "gemm_direct_kernel"
+    base = 1 << 40
+    for K in (16777209, 16777215, 16777216):
+        with pytest.raises(ck.CkoptError) as e:
+            ck.gemm_shmem_tc_async_opt_port(ck.DT_F16, base, base, None, base, 1.0, 0.0, 1, 1, K, *small)
+        assert e.value.code == ck.ERR_TOO_LARGE, K
