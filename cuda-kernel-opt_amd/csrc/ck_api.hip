@@ -484,34 +484,36 @@ int launch_k(int K, bool operands_aligned, const ck::GemmTuning& t, const Option
 // persistent, so a round costs no launch and no empty device. The small-product kernel pays a fixed cost per round, one workgroup
 // per tile and one per CU, and per 512 of K (64 for each of the eight waves): least where every row starts on a line, more on
 // 4-byte boundaries and most on 2-byte ones (64 tiles, 4096^2: K 512 73 / 78 / 108 us, 1024 101 / 117 / 156, about 4096 243 / 317 /
-// 412), and less while the device is nearly empty (L2). Zero-padded operand copies: two allocations and a launch more, in all no less
+// 412), less while the device is nearly empty (L2), and on rows off a line more where the operands, with their copies, leave the last-level cache of
+// 256 MB (128 x 9244 x 12808 116, x 17048 227, ring 143 and 189; 2048^2 x 48008 914, ring 996). Zero-padded operand copies: two allocations and a launch more, in all no less
 // than the 20 us and more that the host takes for them, and the copies' bytes.
 double ring_us(int64_t tiles, int K, int cus) { return 3.5 + std::ceil((double)tiles / cus) * (0.8 + 0.655 * std::ceil((double)K / 128.0)); }
-double direct_us(int tile, int64_t tiles, int K, int rows_aligned, int cus) {
+double direct_us(int tile, int64_t tiles, int K, int rows_aligned, double bytes, int cus) {
     struct Cost { double fixed, unit; };
     constexpr Cost cost[2][3] = {{{1.7, 1.0}, {1.7, 1.35}, {2.2, 1.75}}, {{3.1, 0.95}, {2.5, 1.34}, {4.0, 1.69}}};   // 32, 64 tiles; lines, 4 bytes, 2 bytes
     const Cost c = cost[tile == 64][rows_aligned >= LINE_BYTES ? 0 : rows_aligned >= 4 ? 1 : 2];
     const double rounds = std::ceil((double)tiles / cus), full = std::min(1.0, (double)tiles / cus);
-    const double unit_us = (tile == 32 ? 0.55 + 0.25 * full : 1.2 + 0.4 * full) * c.unit;
+    const double unit_us = (tile == 32 ? 0.55 + 0.25 * full : 1.2 + 0.4 * full) * c.unit * (rows_aligned < LINE_BYTES && bytes > 270e6 ? 1.2 : 1.0);
     return 1.5 + rounds * (c.fixed + unit_us * (double)std::max(K, 128) / 512.0);
 }
 double behind_copies_us(double us, int M, int N, int K) { return std::max(21.5, us + 7.5 + 4.0 * ((double)M + N) * K / 6e6); }
 // direct: tile of the small-product kernel, 0: the ring kernel on 64 x 64 tiles; copies: behind zero-padded operand copies
 struct SmallPlan { int direct; bool copies; double us; };
-SmallPlan small_plan(int M, int N, int K, int operand_alignment, int cus) {
+SmallPlan small_plan(int M, int N, int K, int operand_alignment, int cus, bool on_copies = false) {
     auto tiles = [&](int t) { return (int64_t)((M + t - 1) / t) * ((N + t - 1) / t); };
     SmallPlan best;
     if (needs_copies(K, operand_alignment >= 16)) {   // what the launch on the copies, whose rows are padded to whole chunks, runs
         const int Kp = (K + ck::CHUNK_ELEMS - 1) / ck::CHUNK_ELEMS * ck::CHUNK_ELEMS;
-        best = small_plan(M, N, Kp, 16, cus);
+        best = small_plan(M, N, Kp, 16, cus, true);
         best.copies = true;
         best.us = behind_copies_us(best.us, M, N, Kp);
     } else best = SmallPlan{0, false, ring_us(tiles(64), K, cus)};
     if (K < ck::CHUNK_ELEMS) return best;   // the small-product kernel reads whole chunks of a row
     const int rows_aligned = K % 2 ? 2 : operand_alignment < 16 || K % 64 ? std::min(operand_alignment, 4) : LINE_BYTES;
     for (int t : {32, 64}) {
-        const double us = direct_us(t, tiles(t), K, rows_aligned, cus);
-        if (us < 0.95 * best.us) best = {t, false, us};   // (the ring where the two are level: 16-bit results favour it, 4096^2 x 1024 100 / 105)
+        const double us = direct_us(t, tiles(t), K, rows_aligned, ((double)M + N) * K * (on_copies ? 4.0 : 2.0), cus);
+        // (the ring where the two are level: 16-bit results favour it, 4096^2 x 1024 100 / 105; but no copies where those are level)
+        if (us < (best.copies ? 1.0 : 0.95) * best.us) best = {t, false, us};
     }
     return best;
 }
@@ -1021,10 +1023,13 @@ int ckopt_suggest_gemm_tuning(int M, int N, int K, int num_cus, int* tuning_out)
         const double us_128 = general_us(128, 1.4), us_64 = general_us(64, 0.65);
         const int dev_cus = device_cus();
         const SmallPlan small = small_plan(M, N, K, 16, dev_cus);
+        // Rows off a line, which the estimate leaves out: 1.3 to 2.2 times on 256 x 128 tiles (2048^2 x 4104 67.6 us against 49.0 on the tuple of 128
+        // tiles and 79.1 on the one of 64; 8896 x 253 x 12808 219 / 141 / 172), 1.1 on wider ones and on a short K.
+        const double straight_us = straight.us * (K >= 2048 && K % 8 == 0 && K % 64 != 0 && straight.tile_n == 128 ? 1.4 : 1.0);
         auto launched_us = [&](double us) { return needs_copies(K, true) ? behind_copies_us(us, M, N, K) : us; };
-        if (straight.slices > 1 && straight.us <= us_128 && straight.us <= us_64) pick = straight_line;
-        else if (small.direct && num_cus >= dev_cus && small.us < launched_us(us_128) && small.us < launched_us(straight.us + 1.5)) pick = fused_64;
-        else if (straight.us <= us_128 && straight.us <= us_64) pick = straight_line;
+        if (straight.slices > 1 && straight_us <= us_128 && straight_us <= us_64) pick = straight_line;
+        else if (small.direct && num_cus >= dev_cus && small.us < launched_us(us_128) && small.us < launched_us(straight_us + 1.5)) pick = fused_64;
+        else if (straight_us <= us_128 && straight_us <= us_64) pick = straight_line;
         else if (us_128 <= us_64) pick = fused_128;
     }
     for (int i = 0; i < 10; ++i) tuning_out[i] = pick[i];

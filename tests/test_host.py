@@ -603,6 +603,8 @@ def test_small_tuple_on_many_tiles_keeps_the_ring_kernel_where_it_is_the_faster(
               (4096, 4096, 2048),   # 185 / 147
               (8192, 8192, 4096)):  # 1420 / 970
         assert kernel(*s) == "gemm_direct_kernel" == kernel(*s, cus=100000), s
+    # rows off a line and operands beyond the last-level cache (256 MB): 128 x 9244 x 24008 263 us (ring) against 319, x 12808 143 against 116
+    assert kernel(128, 9244, 24008) == "gemm_fused_kernel" and kernel(128, 9244, 12808) == "gemm_direct_kernel" == kernel(128, 9244, 24000)
     # a long odd K on many tiles: 3072^2 x 2049 125 us (ring behind copies), 141 (rows where they are), 105 on aligned rows: copies and the small-product kernel
     for s in ((3072, 3072, 2049), (4096, 4096, 4097)):
         assert kernel(*s) == "gemm_direct_kernel" and ck.gemm_launch_plan(*s, True, *small)["operand_copies"], s
@@ -667,3 +669,13 @@ def test_the_largest_k_is_the_same_for_rows_in_place_and_rows_copied(ck):
         with pytest.raises(ck.CkoptError) as e:
             ck.gemm_shmem_tc_async_opt_port(ck.DT_F16, base, base, None, base, 1.0, 0.0, 1, 1, K, *small)
         assert e.value.code == ck.ERR_TOO_LARGE, K
+
+
+def test_suggestion_where_rows_lie_off_a_line(ck):
+    # K a multiple of 8 and not of 64: the straight-line kernel on 256 x 128 tiles loses up to half of its rate there (us: it, 128 tiles, 64 tiles)
+    for s, tile in (((2048, 2048, 4104), 128),      # 67.6, 49.0, 79.1
+                    ((8896, 253, 12808), 128),      # 219, 141, 172
+                    ((3000, 700, 21656), 128),      # 353, 225, 285
+                    ((4096, 4096, 4104), 256),      # 124, 182, 310: 256 x 256 tiles lose a tenth
+                    ((1000, 1000, 8200), 64)):      # 116, 84, 40
+        assert ck.suggest_gemm_tuning(*s)["tile_dim"] == tile, s
