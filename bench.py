@@ -294,6 +294,28 @@ GRID_SHAPES = [(512, 512, 512), (1024, 1024, 1024), (1536, 1536, 1536), (2048, 2
                (2048, 8192, 8192)]
 
 
+def gemm_kernel_name(ck, dtype, M, N, K, tup, mode):
+    """The kernel that a launch on aligned operands runs, as the library names it, with its tiles."""
+    plan, name = ck.gemm_launch_plan(M, N, K, True, *tup), ck.gemm_launch_kernel(M, N, K, True, *tup)
+    tile, segk, producers, consumers, cols = tup[0], tup[1], tup[8], tup[9], plan["tile_cols"]
+    if name == "gemm_stream_kernel":
+        what = "tile %s, five 32-deep quarters, 8 waves, pair fetch" % ("256" if cols == 256 else "256 x %d" % cols)
+    elif name == "gemm_direct_kernel":
+        what = "%d x %d tiles, 8 waves on slices of K" % (cols, cols)
+    elif name == "gemm_mid_kernel":
+        what = "128 x 128 tiles staged through registers, 8 waves"
+    elif producers == 0:
+        what = "tile %d, seg_k %d, %d waves, workgroup barrier per segment" % (tile, segk, consumers)
+    else:
+        what = "tile %d, seg_k %d, %dC+%dP waves, %s sync" % (tile, segk, consumers, producers, mode)
+    text = "%s<%s, %s>" % (name, dtype, what)
+    if plan["k_slices"] > 1:
+        text += " with K in %d slices and a reduction pass" % plan["k_slices"]
+    if plan["operand_copies"]:
+        text += " behind zero-padded operand copies"
+    return text
+
+
 def grid(ck, torch, cus, stream):
     """fp16 products of many shapes, each on the tuple the library suggests for it, with the vendor library's GEMM
     (torch.mm, fp32 output) on the same operands beside it: one text line per shape, then one JSON line."""
@@ -487,26 +509,8 @@ def main():
                                             args.bar_steps_a, args.bar_steps_b, rows_a, rows_b, args.group, args.stages,
                                             args.producers, args.consumers, cus, stream)
         peak, bound_name, arith = PEAK_TFLOPS["mfma_f16"], "mfma", dtype
-        if (args.producers == 0 and args.tile == 256 and args.segk == 32 and args.stages == 5 and args.consumers == 8
-                and options.get(6, 1) and options.get(0, 1)):
-            plan = ck.gemm_launch_plan(M, N, K, True, args.tile, args.segk, args.bar_steps_a, args.bar_steps_b, rows_a, rows_b, args.group,
-                                       args.stages, args.producers, args.consumers, cus)
-            kernel = "gemm_stream_kernel<%s, tile %s, five 32-deep quarters, 8 waves, pair fetch>" % (
-                dtype, "256" if plan["tile_cols"] == 256 else "256 x 128")
-            if plan["k_slices"] > 1:
-                kernel += " with K in %d slices and a reduction pass" % plan["k_slices"]
-            if plan["operand_copies"]:
-                kernel += " behind zero-padded operand copies"
-        elif args.producers == 0:
-            kernel = "gemm_fused_kernel<%s, tile %d, seg_k %d, %d waves, workgroup barrier per segment>" % (
-                dtype, args.tile, args.segk, args.consumers)
-            plan = ck.gemm_launch_plan(M, N, K, True, args.tile, args.segk, args.bar_steps_a, args.bar_steps_b, rows_a, rows_b, args.group,
-                                       args.stages, args.producers, args.consumers, cus)
-            if plan["tile_cols"] != args.tile:
-                kernel = "gemm_direct_kernel<%s, %d x %d tiles, 8 waves on slices of K>" % (dtype, plan["tile_cols"], plan["tile_cols"])
-        else:
-            kernel = "gemm_pc_kernel<%s, tile %d, seg_k %d, %dC+%dP waves, %s sync>" % (
-                dtype, args.tile, args.segk, args.consumers, args.producers, args.mode)
+        kernel = gemm_kernel_name(ck, dtype, M, N, K, (args.tile, args.segk, args.bar_steps_a, args.bar_steps_b, rows_a, rows_b, args.group, args.stages,
+                                                       args.producers, args.consumers, cus), args.mode)
     else:
         def step():
             ck.matmul_shmem(ck.DT_F32, da, db, dd, M, N, K, args.simt_tile, args.block_rows, True, stream)

@@ -679,3 +679,20 @@ def test_suggestion_where_rows_lie_off_a_line(ck):
                     ((4096, 4096, 4104), 256),      # 124, 182, 310: 256 x 256 tiles lose a tenth
                     ((1000, 1000, 8200), 64)):      # 116, 84, 40
         assert ck.suggest_gemm_tuning(*s)["tile_dim"] == tile, s
+
+
+def test_bench_names_the_kernel_that_runs(ck):
+    import importlib.util
+    spec = importlib.util.spec_from_file_location("bench_names", os.path.join(ROOT, "bench.py"))
+    bench = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(bench)
+    small, mid, straight = (64, 128, 0, 0, 64, 64, 4, 4, 0, 8, 256), (128, 128, 0, 0, 128, 128, 4, 2, 0, 8, 256), (256, 32, 0, 0, 256, 256, 4, 5, 0, 8, 256)
+    name = lambda *a, mode="tile": bench.gemm_kernel_name(ck, "f16", *a, mode)
+    assert name(8192, 8192, 8192, straight) == "gemm_stream_kernel<f16, tile 256, five 32-deep quarters, 8 waves, pair fetch>"
+    assert name(3072, 3072, 3072, straight).startswith("gemm_stream_kernel<f16, tile 256 x 192,")
+    assert name(2048, 2048, 32768, straight).endswith(" with K in 4 slices and a reduction pass")
+    assert name(6143, 4097, 3071, straight).endswith(" behind zero-padded operand copies")
+    assert name(512, 512, 512, small).startswith("gemm_direct_kernel<f16, 32 x 32 tiles") and name(1000, 1000, 1001, small).startswith("gemm_direct_kernel<f16, 64 x 64 tiles")
+    assert name(4096, 4096, 256, small).startswith("gemm_fused_kernel<f16, tile 64, seg_k 128, 8 waves")
+    assert name(2048, 2048, 2048, mid).startswith("gemm_mid_kernel<") and name(2048, 2048, 256, mid).startswith("gemm_fused_kernel<f16, tile 128,")
+    assert name(512, 512, 512, (256, 64, 4, 2, 64, 128, 4, 2, 2, 8, 256), mode="wave") == "gemm_pc_kernel<f16, tile 256, seg_k 64, 8C+2P waves, wave sync>"
