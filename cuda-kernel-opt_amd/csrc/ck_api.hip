@@ -488,13 +488,16 @@ int launch_k(int K, bool operands_aligned, const ck::GemmTuning& t, const Option
 // 256 MB (128 x 9244 x 12808 116, x 17048 227, ring 143 and 189; 2048^2 x 48008 914, ring 996). Zero-padded operand copies: two allocations and a launch more, in all no less
 // than the 20 us and more that the host takes for them, and the copies' bytes.
 double ring_us(int64_t tiles, int K, int cus) { return 3.5 + std::ceil((double)tiles / cus) * (0.8 + 0.655 * std::ceil((double)K / 128.0)); }
-double direct_us(int tile, int64_t tiles, int K, int rows_aligned, double bytes, int cus) {
+double direct_us(int tile, int64_t tiles, int K, int rows_aligned, double operand_bytes, bool on_copies, int cus) {
     struct Cost { double fixed, unit; };
     constexpr Cost cost[2][3] = {{{1.7, 1.0}, {1.7, 1.35}, {2.2, 1.75}}, {{3.1, 0.95}, {2.5, 1.34}, {4.0, 1.69}}};   // 32, 64 tiles; lines, 4 bytes, 2 bytes
     const Cost c = cost[tile == 64][rows_aligned >= LINE_BYTES ? 0 : rows_aligned >= 4 ? 1 : 2];
-    const double rounds = std::ceil((double)tiles / cus), full = std::min(1.0, (double)tiles / cus);
-    const double unit_us = (tile == 32 ? 0.55 + 0.25 * full : 1.2 + 0.4 * full) * c.unit * (rows_aligned < LINE_BYTES && bytes > 270e6 ? 1.2 : 1.0);
-    return 1.5 + rounds * (c.fixed + unit_us * (double)std::max(K, 128) / 512.0);
+    const bool off_lines = rows_aligned < LINE_BYTES;
+    const double slow = c.unit * (off_lines && operand_bytes * (on_copies ? 2.0 : 1.0) > 270e6 ? 1.5 : 1.0), units = (double)std::max(K, 128) / 512.0;
+    auto round = [&](double full) { return c.fixed + (tile == 32 ? 0.55 + 0.25 * full : 1.2 + 0.4 * full) * slow * units; };   // full: share of the CUs with a tile
+    const int64_t rest = tiles % cus;
+    const double us = 1.5 + (double)(tiles / cus) * round(1.0) + (rest ? round((double)rest / cus) : 0.0);
+    return off_lines ? std::max(us, 1.5 + operand_bytes / 2.2e6) : us;   // (from memory: 64 x 8768 x 10600 87.6, ring 68.6)
 }
 double behind_copies_us(double us, int M, int N, int K) { return std::max(21.5, us + 7.5 + 4.0 * ((double)M + N) * K / 6e6); }
 // direct: tile of the small-product kernel, 0: the ring kernel on 64 x 64 tiles; copies: behind zero-padded operand copies
@@ -511,9 +514,10 @@ SmallPlan small_plan(int M, int N, int K, int operand_alignment, int cus, bool o
     if (K < ck::CHUNK_ELEMS) return best;   // the small-product kernel reads whole chunks of a row
     const int rows_aligned = K % 2 ? 2 : operand_alignment < 16 || K % 64 ? std::min(operand_alignment, 4) : LINE_BYTES;
     for (int t : {32, 64}) {
-        const double us = direct_us(t, tiles(t), K, rows_aligned, ((double)M + N) * K * (on_copies ? 4.0 : 2.0), cus);
-        // (the ring where the two are level: 16-bit results favour it, 4096^2 x 1024 100 / 105; but no copies where those are level)
-        if (us < (best.copies ? 1.0 : 0.95) * best.us) best = {t, false, us};
+        const double us = direct_us(t, tiles(t), K, rows_aligned, ((double)M + N) * K * 2.0, on_copies, cus);
+        // (the ring where the two are level: 16-bit results and operands from memory favour it, 2048^2 x 1024 29.3 / 32.8; but no copies
+        // where those are level)
+        if (us < (best.copies ? 1.0 : 0.93) * best.us) best = {t, false, us};
     }
     return best;
 }
@@ -682,9 +686,10 @@ int gemm_launch(int dtype, const void* A, const void* Bt, const void* C, void* D
     a.fix_partials = nullptr;
     a.fix_state = nullptr;
     if (route.kernel == CKOPT_KERNEL_DIRECT) {
-        // (short K and a tile count that the XCDs do not divide: the workgroups as they come, the L2 has little to give and runs of tiles
-        // put an XCD's first loads on few memory channels: 118 x 2176 x 124 4.8 us against 5.2)
-        if (K < 512 && tiles % a.num_xcd != 0) a.num_xcd = 1;
+        // (A tile count that the XCDs do not divide: the workgroups as they come where runs of tiles per XCD lose. With a short K they put an
+        // XCD's first loads on few memory channels, 118 x 2176 x 124 4.8 us against 5.2; with few columns of tiles and a deep K every XCD
+        // streams a stretch of A of its own, 6528 x 396 x 33344 360 against 390, while 12864 x 192 x 4096 takes 51.3 as they come, 46.2 in runs.)
+        if (tiles % a.num_xcd != 0 && (K < 512 || (a.tiles_n < 8 && K > 8192))) a.num_xcd = 1;
         e = launch_gemm_direct(dtype == CK_DT_BF16, route.tile, K % 2 == 0 && !(both & 3), s, a);
     } else if (route.kernel == CKOPT_KERNEL_STREAM) {
         // Tile width, K slices and grid from the cost model: few tiles and a deep K are cut into slices so that every CU
@@ -1028,7 +1033,7 @@ int ckopt_suggest_gemm_tuning(int M, int N, int K, int num_cus, int* tuning_out)
         const double straight_us = straight.us * (K >= 2048 && K % 8 == 0 && K % 64 != 0 && straight.tile_n == 128 ? 1.4 : 1.0);
         auto launched_us = [&](double us) { return needs_copies(K, true) ? behind_copies_us(us, M, N, K) : us; };
         if (straight.slices > 1 && straight_us <= us_128 && straight_us <= us_64) pick = straight_line;
-        else if (small.direct && num_cus >= dev_cus && small.us < launched_us(us_128) && small.us < launched_us(straight_us + 1.5)) pick = fused_64;
+        else if (small.direct && num_cus >= dev_cus && small.us < 0.93 * launched_us(us_128) && small.us < 0.93 * launched_us(straight_us + 1.5)) pick = fused_64;
         else if (straight_us <= us_128 && straight_us <= us_64) pick = straight_line;
         else if (us_128 <= us_64) pick = fused_128;
     }

@@ -1,16 +1,21 @@
 // 128 x 128 tiles with the operands staged through registers: one workgroup of eight waves per tile of D, two LDS stages of 128 k.
 //
 // What bounds it: a segment (64 KiB of operands) takes about 1.2 us, on one CU as on all of them, where its MFMAs take 0.43: the
-// waves of the one workgroup on a CU go through the segment in step - fragment reads, MFMAs, writes of the next segment -
-// and the phases of the eight add up. (The ring kernels on the same tile take 1.3 us with two stages as with five, with
-// direct-to-LDS loads and fragments read one k-step ahead; neither the rate of the loads nor L2 is the limit.) A wave
-// fetches its share of a segment into registers two segments ahead, whole 128-byte lines, and writes it to LDS between the
-// MFMAs of its two k-steps.
+// phases of a wave - fragment reads, MFMAs, writes of the next segment - add up instead of covering each other. The compiled loop
+// shows where: the wait in front of the barrier orders memory accesses only, so the compiler moves the MFMAs of the second k-step
+// behind it, and the eight writes drain with no MFMA of their own wave beside them; at the head of every other segment all 16
+// fragment reads are waited for before the first MFMA; the test for the end of K splits the loop into blocks that the scheduler
+// does not cross. The kernel takes all 256 registers of a wave and keeps four more values in scratch memory (stored in front of the
+// loop, loaded behind it). (The ring kernels on the same tile take 1.3 us with two stages as with five, with direct-to-LDS loads
+// and fragments read one k-step ahead; neither the rate of the loads nor L2 is the limit.) A wave fetches its share of a segment
+// into registers two segments ahead, whole 128-byte lines, and writes it to LDS behind the MFMAs of the first k-step.
 //
 // The waves form two groups of four; each covers the tile with wave tiles of 64 x 64 and takes two of a segment's four k-steps
 // (16 MFMAs on 8 fragments: a third less LDS traffic than eight tiles of 32 x 64). The partial tiles of the two
 // groups meet in LDS at the end, first + second.
-// bf16 256 x 16384 x 4096 with 16-bit results 59.2 -> 53.8 us (638 TFLOP/s), fp16 1024^2 x 4096 41.9 -> 38.9, 2048^3 25.7 as before.
+// Against the ring kernel: bf16 256 x 16384 x 4096 with 16-bit results 59.4 -> 53.5 us (642 TFLOP/s; 49.9 -> 44.8 on operands that lie in the last-level cache
+// from call to call), fp16 1024^2 x 4096 41.8 -> 39.0, 2048^3 25.5 -> 24.9. One workgroup per tile and CU: the launcher takes it where
+// a deep K or fewer tiles than CUs make up for the prologue and epilogue of every tile.
 #ifndef CK_GEMM_MID_KERNEL_HIP_H
 #define CK_GEMM_MID_KERNEL_HIP_H
 
