@@ -13,9 +13,9 @@
 // The waves form two groups of four; each covers the tile with wave tiles of 64 x 64 and takes two of a segment's four k-steps
 // (16 MFMAs on 8 fragments: a third less LDS traffic than eight tiles of 32 x 64). The partial tiles of the two
 // groups meet in LDS at the end, first + second.
-// Against the ring kernel: bf16 256 x 16384 x 4096 with 16-bit results 59.4 -> 53.5 us (642 TFLOP/s; 49.9 -> 44.8 on operands that lie in the last-level cache
-// from call to call), fp16 1024^2 x 4096 41.8 -> 39.0, 2048^3 25.5 -> 24.9. One workgroup per tile and CU: the launcher takes it where
-// a deep K or fewer tiles than CUs make up for the prologue and epilogue of every tile.
+// Against the ring kernel: bf16 256 x 16384 x 4096 with 16-bit results 59.3 -> 54.2 us (634 TFLOP/s; 49.9 -> 44.8 where
+// the operands stay in the last-level cache from call to call), fp16 1024^2 x 4096 41.8 -> 39.0, 2048^3 level (25.8 and 25.7). One workgroup
+// per tile and CU: the launcher takes it where a deep K or fewer tiles than CUs make up for the prologue and epilogue of every tile.
 #ifndef CK_GEMM_MID_KERNEL_HIP_H
 #define CK_GEMM_MID_KERNEL_HIP_H
 

@@ -59,7 +59,11 @@ enum {
  * not a multiple of 8, or A / Bt is not 16-byte aligned (2-byte alignment is required), the call first copies both
  * operands into zero-padded rows in a stream-ordered temporary (hipMallocAsync / hipFreeAsync on `stream`,
  * (M + N) * Kp * 2 bytes with Kp = round_up(K, 8), or round_up(K, 64) for the tuple tile_dim 256, segment_dim_k 32,
- * num_stages 5, no producer waves, whose straight-line kernel works in loop bodies of 64). */
+ * num_stages 5, no producer waves, whose straight-line kernel works in loop bodies of 64). One kernel reads rows on any
+ * 2-byte boundary: the tuple tile_dim 64, segment_dim_k 128, num_stages 4, no producer waves, 8 consumer waves and num_cus at least the
+ * device's leaves the choice between the ring kernel and gemm_direct_kernel, with or without the copies, to an estimate;
+ * tile_dim 128, segment_dim_k 128, num_stages 2 likewise runs the ring kernel or gemm_mid_kernel (ckopt_gemm_launch_kernel names
+ * it). */
 int ckopt_gemm_shmem_tc_async_opt_port_2(int dtype, const void* A, const void* Bt, const float* C, float* D,
                                          float alpha, float beta, int M, int N, int K, int tile_dim,
                                          int segment_dim_k, int bar_steps_a, int bar_steps_b, int bar_step_rows_a,
@@ -83,7 +87,8 @@ int ckopt_gemm_shmem_tc_async_opt_port_2_lp(int dtype, const void* A, const void
  * the launch needs none. ckopt_gemm_workspace_bytes returns how much the launch with these sizes and this tuning
  * needs under the process's current options (0: none; negative: the error the launch would give);
  * operands_aligned != 0 promises A and Bt on 16-byte boundaries. A workspace that is too small gives
- * CKOPT_ERR_TOO_LARGE and D is not written; nothing is allocated in any case. */
+ * CKOPT_ERR_TOO_LARGE and D is not written, also where the kernel that runs makes no use of it (gemm_direct_kernel on rows off a 16-byte
+ * boundary); nothing is allocated in any case. */
 int64_t ckopt_gemm_workspace_bytes(int M, int N, int K, int operands_aligned, int tile_dim, int segment_dim_k, int bar_steps_a,
                                    int bar_steps_b, int bar_step_rows_a, int bar_step_rows_b, int tile_group_m, int num_stages,
                                    int num_producer_waves, int num_consumer_waves, int num_cus);
@@ -118,7 +123,7 @@ int ckopt_gemm_shmem_tc_async_opt_port_2_ws(int dtype, int cd_dtype, const void*
  * device (different streams, different threads) race on it. Nothing in it needs to start at zero (the counters of
  * a reduction inside the kernel are cleared by a small kernel of the same launch, not by a memset).
  * Before a launch is recorded into a HIP graph, one eager call with the same element type, shape class (K a
- * multiple of 64 or not, the tile width the plan query reports) and options must have run on the device: the first
+ * multiple of 64 or not, even or odd, the kernel and the tile width that the queries report) and options must have run on the device: the first
  * call on a device resolves the array's address and the first use of each kernel instance sets its LDS-size
  * attribute, neither of which may happen under capture. The array is resident on every device the process uses the
  * library on, whether or not this entry point is ever called. */
@@ -290,7 +295,7 @@ int ckopt_last_launch_clocks(void* stream, uint64_t* shader_cycles, uint64_t* re
  *        (gemm_pcb_kernel, needs num_stages >= 2) instead of LDS counters (default 0).
  * key 6: launches with num_producer_warps 0, tile_dim 256, segment_dim_k 32, num_stages 5, 8 consumer warps (any M, N, K)
  *        take the straight-line kernel written for exactly that shape (gemm_stream_kernel; default 1); 0 sends them
- *        through the general fused kernel.
+ *        through the general fused kernel. It also sends the suggested tuples of 64 and 128 tiles through the ring kernel.
  * key 7: split-K of the straight-line kernel. 1 (default): with fewer tiles than num_sms, K is cut into the number of
  *        slices (at most 16, each a multiple of 64 and at least 1024 deep) for which a cost model of the device gives
  *        the shortest time - loop bodies at the rate the active CUs sustain, the store burst of every round, the
