@@ -5,16 +5,15 @@
 // shows where: the wait in front of the barrier orders memory accesses only, so the compiler moves the MFMAs of the second k-step
 // behind it, and the eight writes drain with no MFMA of their own wave beside them; at the head of every other segment all 16
 // fragment reads are waited for before the first MFMA; the test for the end of K splits the loop into blocks that the scheduler
-// does not cross. The kernel takes all 256 registers of a wave and keeps four more values in scratch memory (stored in front of the
-// loop, loaded behind it). (The ring kernels on the same tile take 1.3 us with two stages as with five, with direct-to-LDS loads
+// does not cross. The kernel takes all 256 registers of a wave. (The ring kernels on the same tile take 1.3 us with two stages as with five, with direct-to-LDS loads
 // and fragments read one k-step ahead; neither the rate of the loads nor L2 is the limit.) A wave fetches its share of a segment
 // into registers two segments ahead, whole 128-byte lines, and writes it to LDS behind the MFMAs of the first k-step.
 //
 // The waves form two groups of four; each covers the tile with wave tiles of 64 x 64 and takes two of a segment's four k-steps
 // (16 MFMAs on 8 fragments: a third less LDS traffic than eight tiles of 32 x 64). The partial tiles of the two
 // groups meet in LDS at the end, first + second.
-// Against the ring kernel: bf16 256 x 16384 x 4096 with 16-bit results 59.3 -> 54.2 us (634 TFLOP/s; 49.9 -> 44.8 where
-// the operands stay in the last-level cache from call to call), fp16 1024^2 x 4096 41.8 -> 39.0, 2048^3 level (25.8 and 25.7). One workgroup
+// Against the ring kernel: bf16 256 x 16384 x 4096 with 16-bit results 59.3 -> 53.5 us (642 TFLOP/s; 49.9 -> 44.8 where
+// the operands stay in the last-level cache from call to call), fp16 1024^2 x 4096 41.8 -> 39.0, 2048^3 25.8 -> 25.5. One workgroup
 // per tile and CU: the launcher takes it where a deep K or fewer tiles than CUs make up for the prologue and epilogue of every tile.
 #ifndef CK_GEMM_MID_KERNEL_HIP_H
 #define CK_GEMM_MID_KERNEL_HIP_H
@@ -151,11 +150,13 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(const GemmArgs g) {
     }
     if (s < segs) segment(s, std::integral_constant<int, 0>{}, odd);
 
+    // (the lane's number once more: carried through the loop it and what comes of it went to scratch memory)
+    const int out_lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), out_lr = out_lane & 15, out_lg = out_lane >> 4;
     // The two partial sums of a wave tile: the first group keeps the upper half of the block rows, the second the lower one, and
     // each hands the other half over.
     const bool lower = group != 0;
-    CK_LDS char* mine = lds + wave * (WT / 2 * WT * 1024) + lane * 16;
-    const CK_LDS char* theirs = lds + (wave ^ 4) * (WT / 2 * WT * 1024) + lane * 16;
+    CK_LDS char* mine = lds + wave * (WT / 2 * WT * 1024) + out_lane * 16;
+    const CK_LDS char* theirs = lds + (wave ^ 4) * (WT / 2 * WT * 1024) + out_lane * 16;
 #pragma unroll
     for (int i = 0; i < WT / 2; ++i)
 #pragma unroll
@@ -167,10 +168,10 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(const GemmArgs g) {
 #pragma unroll
         for (int j = 0; j < WT; ++j) {
             const f32x4 sum = (lower ? acc[WT / 2 + i][j] : acc[i][j]) + *(const CK_LDS f32x4*)(theirs + (i * WT + j) * 1024);
-            epilogue_block<DT>(g, row_a + R * 64 + ((lower ? WT / 2 : 0) + i) * 16 + lr, row_b + Cc * 64 + j * 16 + lg * 4, sum, vec_cols);
+            epilogue_block<DT>(g, row_a + R * 64 + ((lower ? WT / 2 : 0) + i) * 16 + out_lr, row_b + Cc * 64 + j * 16 + out_lg * 4, sum, vec_cols);
         }
 
-    if (blockIdx.x == 0 && threadIdx.x == blockDim.x - 1) {
+    if (blockIdx.x == 0 && wave == 7 && out_lane == 63) {
         const unsigned long long dc = clock64() - clk0, dw = wall_clock64() - wall0;
         g.status[2] = (unsigned)dc; g.status[3] = (unsigned)(dc >> 32);
         g.status[4] = (unsigned)dw; g.status[5] = (unsigned)(dw >> 32);

@@ -696,3 +696,23 @@ def test_bench_names_the_kernel_that_runs(ck):
     assert name(4096, 4096, 256, small).startswith("gemm_fused_kernel<f16, tile 64, seg_k 128, 8 waves")
     assert name(2048, 2048, 2048, mid).startswith("gemm_mid_kernel<") and name(2048, 2048, 256, mid).startswith("gemm_fused_kernel<f16, tile 128,")
     assert name(512, 512, 512, (256, 64, 4, 2, 64, 128, 4, 2, 2, 8, 256), mode="wave") == "gemm_pc_kernel<f16, tile 256, seg_k 64, 8C+2P waves, wave sync>"
+
+
+def test_kernels_of_the_smaller_tuples_keep_every_value_in_registers(tmp_path):
+    # the small-product and the register-staged kernel are written to the 256 registers of a wave at two waves per SIMD: no scratch memory
+    import importlib.util
+    import subprocess
+    spec = importlib.util.spec_from_file_location("ckopt_build", os.path.join(ROOT, "cuda-kernel-opt_amd", "build.py"))
+    b = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(b)
+    seen = 0
+    for name in ("gemm_direct_inst", "gemm_mid_inst"):
+        out = str(tmp_path / (name + ".s"))
+        src = os.path.join(ROOT, "cuda-kernel-opt_amd", "csrc", name + ".hip")
+        r = subprocess.run([b.HIPCC] + [f for f in b.DEVICE_FLAGS if f != "-fPIC"] + ["-S", "--cuda-device-only", src, "-o", out], capture_output=True, text=True)
+        assert r.returncode == 0, r.stderr[-2000:]
+        text = open(out).read()
+        sizes, registers = re.findall(r"; ScratchSize: (\d+)", text), re.findall(r"; TotalNumVgprs: (\d+)", text)
+        assert sizes and set(sizes) == {"0"} and all(int(v) <= 256 for v in registers), (name, sizes, registers)
+        seen += len(sizes)
+    assert seen >= 10   # four instances of the small-product kernel per element type, one of the other
