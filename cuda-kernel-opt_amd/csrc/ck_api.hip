@@ -530,23 +530,28 @@ bool small_tuple(const ck::GemmTuning& t, const Options& opt) {
            t.segment_dim_k == 128 && t.num_stages == 4;
 }
 
-// The tuple the library suggests for 128 x 128 tiles, where it may use the whole device, runs the register-staged kernel (gemm_mid_kernel)
-// or the ring kernel. The former has one workgroup per tile and CU and pays its prologue (three segments of 128 k) and epilogue on
-// every tile; the persistent ring kernel overlaps them with the next tile's loads, and on a full device loses less where the
-// rows of the operands do not start on lines. Ring / register-staged, us:
-//   fewer tiles than CUs, 1024^2 x 256 7.8 / 8.4, x 512 10.0 / 10.3, x 4096 41.8 / 39.0; 60 drawn shapes of 24 to 255 tiles, fp32 results: K 256 1.04 to
-//     1.09, 576 0.92 to 1.01, 1024 0.88 to 0.97, 3000 0.80 to 1.01 (16-bit results 0.82 to 1.07)
-//   as many tiles as CUs, 2048^2 x 512 11.6 / 12.1, x 1536 21 / 21, x 4096 44.1 / 42.0, 256 x 16384 x 1024 16.9 / 17.7, x 4096 47.6 / 43.5, x 3000 1.04
-//     (behind operand copies the ring everywhere: 12096 x 104 x 688 27.9 / 33.8, 4096 x 768 x 2692 46.4 / 48.2)
-//   several rounds, 4096^2 x 512 35.4 / 42.4, x 2048 91.5 / 97.5, x 4096 167 / 163, x 4104 1.09; 6144^2 (9 rounds) x 4096 372 / 368;
-//     8192^2 (16) with 16-bit results x 512 135 / 239, x 6144 958 / 985
+// The tuple the library suggests for 128 x 128 tiles, where it may use the whole device, runs the kernel with a ring of 64-deep slabs
+// (gemm_mid_kernel) or the general ring kernel. The former has one workgroup per tile and CU and pays its prologue (five slabs) and
+// epilogue on every tile; the latter is persistent and overlaps them with the next tile's loads. 16-bit results cost
+// the latter more, rows that do not start on lines the former. General ring / slabs, us (fp32 results; 16-bit ones in brackets):
+//   fewer tiles than CUs, 1024^2 x 256 7.8 / 8.1, x 384 8.9 / 8.7, x 512 9.9 / 9.5; more than half as many, 2048 x 1920 x 128 7.6 / 7.6,
+//     x 256 9.1 / 8.1 (10.9 / 8.8)
+//   as many tiles as CUs, 2048^2 x 768 13.9 / 12.3, x 1024 16.2 / 14.0 (18.1 / 14.3), 256 x 16384 x 1024 16.8 / 14.1; off a line
+//     2048^2 x 1000 16.8 / 16.2, x 3000 36.3 / 34.6, but from memory 256 x 16384 x 3000 46.5 / 48.8
+//     (behind operand copies the general ring everywhere)
+//   several rounds, 4096^2 x 512 35.2 / 36.8 (42.2 / 39.0), x 1024 53.8 / 51.4 (60.1 / 52.9), x 2048 92.4 / 83.2; 6144^2 (9 rounds) x 768 93.7 / 95.4,
+//     x 1024 115.5 / 111.9, x 2048 204 / 184; off a line 4096^2 x 1000 55.3 / 57.8, x 3000 136 / 132. (More rounds than nine: left on the
+//     general ring, as many such tiles are suggested 256 x 256.)
 bool mid_tuple(const ck::GemmTuning& t, const Options& opt) {
     return opt[OPT_STRAIGHT_LINE] && opt[OPT_SWIZZLE] && t.num_producer_waves == 0 && t.num_consumer_waves == 8 && t.tile_dim == 128 &&
            t.segment_dim_k == 128 && t.num_stages == 2;
 }
-bool mid_is_shorter(int64_t tiles, int K, int cus) {
-    if (tiles < cus) return K > 512;
-    return K % 64 == 0 && (tiles == cus ? K >= 1536 : tiles <= 9 * (int64_t)cus && K >= 4096);
+bool mid_is_shorter(int M, int N, int K, int cus) {
+    const int64_t tiles = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
+    const bool lines = K % 64 == 0;
+    if (tiles < cus) return K >= (2 * tiles > cus ? 256 : 512);
+    if (tiles == cus) return K > 512 && (lines || ((double)M + N) * K * 2.0 < 64e6);
+    return lines && tiles <= 9 * (int64_t)cus && K >= 1024;
 }
 
 // What a launch runs: the one decision that the launcher and the queries share. operand_alignment: bytes that A and Bt both lie on,
@@ -567,7 +572,7 @@ Route route_of(int M, int N, int K, int operand_alignment, const ck::GemmTuning&
         return {p.direct ? CKOPT_KERNEL_DIRECT : CKOPT_KERNEL_FUSED, p.direct ? p.direct : t.tile_dim, p.copies};
     }
     if (straight_line_tuple(t, opt)) r.kernel = CKOPT_KERNEL_STREAM;
-    else if (mid && t.num_cus >= cus && !r.copies && mid_is_shorter((int64_t)((M + 127) / 128) * ((N + 127) / 128), K, cus))
+    else if (mid && t.num_cus >= cus && !r.copies && mid_is_shorter(M, N, K, cus))
         r.kernel = CKOPT_KERNEL_MID;
     else if (t.num_producer_waves == 0) r.kernel = t.num_stages == 1 ? CKOPT_KERNEL_SYNC : CKOPT_KERNEL_FUSED;
     else if (sync_mode_of(t.tile_dim, t.num_consumer_waves, t.bar_step_rows_a, t.bar_step_rows_b) == CK_SYNC_TILE && t.num_stages >= 2 &&

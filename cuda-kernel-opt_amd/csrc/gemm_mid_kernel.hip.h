@@ -1,20 +1,20 @@
-// 128 x 128 tiles with the operands staged through registers: one workgroup of eight waves per tile of D, two LDS stages of 128 k.
+// 128 x 128 tiles on a ring of five 64-deep slabs: one workgroup of eight waves per tile of D (and K slice), all of the CU's LDS.
 //
-// What bounds it: a segment (64 KiB of operands) takes about 1.2 us, on one CU as on all of them, where its MFMAs take 0.43: the
-// phases of a wave - fragment reads, MFMAs, writes of the next segment - add up instead of covering each other. The compiled loop
-// shows where: the wait in front of the barrier orders memory accesses only, so the compiler moves the MFMAs of the second k-step
-// behind it, and the eight writes drain with no MFMA of their own wave beside them; at the head of every other segment all 16
-// fragment reads are waited for before the first MFMA; the test for the end of K splits the loop into blocks that the scheduler
-// does not cross. The kernel takes all 256 registers of a wave. (The ring kernels on the same tile take 1.3 us with two stages as with five, with direct-to-LDS loads
-// and fragments read one k-step ahead; neither the rate of the loads nor L2 is the limit.) A wave fetches its share of a segment
-// into registers two segments ahead, whole 128-byte lines, and writes it to LDS behind the MFMAs of the first k-step.
+// What bounds it: on a full device the L2s, which give 26 TB/s to loads of whole lines (5.2 ns per k of 256 tiles; the loads of this
+// kernel alone reach that), and on random operands the power limit (2048^2 x 8192: 64 us at 1.85 GHz, 53 us at 2.4 GHz on constant
+// ones). On few tiles the loads of one CU take 4.0 ns per k, the MFMAs 3.5 and MFMAs with fragment reads 4.2; all together 5.4.
 //
-// The waves form two groups of four; each covers the tile with wave tiles of 64 x 64 and takes two of a segment's four k-steps
-// (16 MFMAs on 8 fragments: a third less LDS traffic than eight tiles of 32 x 64). The partial tiles of the two
-// groups meet in LDS at the end, first + second.
-// Against the ring kernel: bf16 256 x 16384 x 4096 with 16-bit results 59.3 -> 53.5 us (642 TFLOP/s; 49.9 -> 44.8 where
-// the operands stay in the last-level cache from call to call), fp16 1024^2 x 4096 41.8 -> 39.0, 2048^3 25.8 -> 25.5. One workgroup
-// per tile and CU: the launcher takes it where a deep K or fewer tiles than CUs make up for the prologue and epilogue of every tile.
+// A slab is one 128-byte line of every row. A wave brings 16 rows of each operand straight into LDS, four loads of 1 KiB, four to
+// five slabs ahead of the MFMAs. The waves form two groups of four; each covers the tile with wave tiles of 64 x 64 and takes one of a
+// slab's two k-steps: 16 MFMAs on 8 fragments per slab and wave, a third less LDS traffic than eight tiles of 32 x 64. The fragments
+// of slab s + 1 are read under the MFMAs of slab s, and the barrier of body s stands for slab s + 2, so that no read waits behind it.
+// The partial tiles of the two groups meet in LDS at the end, in rows: first + second, and whole lines of D.
+//
+// The eight XCDs begin at eight different slabs. With rows of a power of two in bytes all tiles would otherwise ask the same few
+// memory channels at a time: bf16 256 x 16384 x 4096 from memory 52.0 -> 46.4 us, loads alone on 4096^2 x 8192 228 -> 192.
+//
+// Against the kernel before (two 128-deep stages written through registers; a wave's reads, MFMAs and writes added up): fp16 2048^3
+// 25.5 -> 21.8 us, bf16 256 x 16384 x 4096 with 16-bit results 53.5 -> 45.0.
 #ifndef CK_GEMM_MID_KERNEL_HIP_H
 #define CK_GEMM_MID_KERNEL_HIP_H
 
@@ -23,155 +23,190 @@
 namespace ck {
 
 constexpr int MID_TILE = 128;
-constexpr int MID_SEGK = 128;
-constexpr int MID_ROW_BYTES = MID_SEGK * 2;
-constexpr int MID_OPERAND = MID_TILE * MID_ROW_BYTES;
-constexpr int MID_LDS_BYTES = 2 * 2 * MID_OPERAND;
+constexpr int MID_SLAB_K = 64;                                 // one 128-byte line of an operand row
+constexpr int MID_OPERAND = MID_TILE * MID_SLAB_K * 2;
+constexpr int MID_STAGE = 2 * MID_OPERAND;
+constexpr int MID_STAGES = 5;
+constexpr int MID_OUT_ROW = 64 * 4 + 16;                       // a row of a wave's partial tile: 64 sums, and 16 bytes against bank conflicts
+constexpr int MID_OUT_WAVE = 64 * MID_OUT_ROW;
+constexpr int MID_LDS_BYTES = MID_STAGES * MID_STAGE;
+static_assert(8 * MID_OUT_WAVE <= MID_LDS_BYTES && MID_LDS_BYTES <= LDS_BYTES_PER_CU, "the partial tiles take the ring's place");
 
-// Rows start on 16-byte boundaries and K % 8 == 0 (a 16-byte chunk of a row is inside it or past it).
+// Four neighbouring results of a row, the first in column n: D = alpha * sum + beta * C. C is what row_c() fetched.
+typedef uint32_t u32x2_a2 __attribute__((ext_vector_type(2), aligned(2)));
 template <typename DT>
+__device__ __forceinline__ f32x4 row_c(const GemmArgs& g, int m, int n) {
+    f32x4 c = {0.f, 0.f, 0.f, 0.f};
+    if (g.beta == 0.f || m >= g.M || n >= g.N) return c;
+    const int64_t off = (int64_t)m * g.N + n;
+    const unsigned short* c16 = (const unsigned short*)g.C;
+    if (n + 4 <= g.N) {
+        if (!g.out16) return *(const f32x4_u*)(g.C + off);
+        const u32x2_a2 x = *(const u32x2_a2*)(c16 + off);
+        return f32x4{Out16<DT>::load((unsigned short)(x[0] & 0xffffu)), Out16<DT>::load((unsigned short)(x[0] >> 16)),
+                     Out16<DT>::load((unsigned short)(x[1] & 0xffffu)), Out16<DT>::load((unsigned short)(x[1] >> 16))};
+    }
+#pragma unroll
+    for (int e = 0; e < 3; ++e)
+        if (n + e < g.N) c[e] = g.out16 ? Out16<DT>::load(c16[off + e]) : g.C[off + e];
+    return c;
+}
+template <typename DT>
+__device__ __forceinline__ void store_row(const GemmArgs& g, int m, int n, f32x4 sum, f32x4 c) {
+    if (m >= g.M || n >= g.N) return;
+    const int64_t off = (int64_t)m * g.N + n;
+    f32x4 v = sum * g.alpha;
+    if (g.beta != 0.f) v += c * g.beta;
+    unsigned short* d16 = (unsigned short*)g.D;
+    if (n + 4 <= g.N) {
+        if (!g.out16) {
+            if (g.nt_store) store_b128_nt(g.D + off, __builtin_bit_cast(u32x4, v));
+            else *(f32x4_u*)(g.D + off) = v;
+        } else {
+            const u32x2 o = {(uint32_t)Out16<DT>::store(v[0]) | (uint32_t)Out16<DT>::store(v[1]) << 16, (uint32_t)Out16<DT>::store(v[2]) | (uint32_t)Out16<DT>::store(v[3]) << 16};
+            if (g.nt_store) store_b64_nt(d16 + off, o);
+            else *(u32x2_a2*)(d16 + off) = o;
+        }
+        return;
+    }
+#pragma unroll
+    for (int e = 0; e < 3; ++e)
+        if (n + e < g.N) {
+            if (g.out16) d16[off + e] = Out16<DT>::store(v[e]);
+            else g.D[off + e] = v[e];
+        }
+}
+
+// Rows start on 16-byte boundaries and K % 8 == 0 (a 16-byte chunk of a row is inside it or past it); KTAIL: K % 64 != 0.
+template <typename DT, bool KTAIL>
 __global__ __launch_bounds__(512) void gemm_mid_kernel(const GemmArgs g) {
     constexpr int WT = 4;   // 16 x 16 blocks per edge of a wave tile
     extern __shared__ __attribute__((aligned(1024))) char ck_smem[];
-    CK_LDS char* const lds = (CK_LDS char*)ck_smem;
+    const uint32_t ring = (uint32_t)(uintptr_t)(CK_LDS char*)ck_smem;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     const unsigned long long clk0 = clock64(), wall0 = wall_clock64();
 
     const TileRC rc = tile_order(g.tiles_m, g.tiles_n, g.tile_group_m, xcd_tile(blockIdx.x, gridDim.x, g.num_xcd));
-    const int row_a = rc.row * MID_TILE, row_b = rc.col * MID_TILE;
-    const int64_t pitch = (int64_t)g.K * 2;
-    const char* base_a = (const char*)g.A + row_a * pitch;
-    const char* base_b = (const char*)g.Bt + row_b * pitch;
+    const int row_a = __builtin_amdgcn_readfirstlane(rc.row * MID_TILE), row_b = __builtin_amdgcn_readfirstlane(rc.col * MID_TILE);
+    const uint32_t pitch = (uint32_t)g.K * 2u;
+    const int rows_a = g.M - row_a < MID_TILE ? g.M - row_a : MID_TILE, rows_b = g.N - row_b < MID_TILE ? g.N - row_b : MID_TILE;
+    i32x4 rsrc_a = make_rsrc((const char*)g.A + (int64_t)row_a * pitch, (uint32_t)rows_a * pitch);
+    i32x4 rsrc_b = make_rsrc((const char*)g.Bt + (int64_t)row_b * pitch, (uint32_t)rows_b * pitch);
 
-    // Loader: wave w brings rows 16w .. 16w + 15 of both operands, a load is 8 rows of one 128-byte line. Rows past the edge
-    // of a ragged tile read the last row instead: what they give is never stored.
-    const int lane_row = lane / 8, lane_chunk = lane % 8;
-    uint32_t off_a[2], off_b[2];
-    CK_LDS char* put[2][2];   // [rows 0 .. 7, 8 .. 15][first, second line of the segment]
+    // Loader: wave w brings rows 16w .. 16w + 15 of both operands, a load is 8 rows of one line. The offset inside the tile is range
+    // checked: rows past the edge of a ragged tile, chunks past the end of K and slabs past the last one are zeros in LDS.
+    uint32_t off[2];
+    int chunk_k[2];
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-        const int row = wave * 16 + j * 8 + lane_row, ra = g.M - 1 - row_a, rb = g.N - 1 - row_b;
-        off_a[j] = (uint32_t)(row < ra ? row : ra) * (uint32_t)pitch;
-        off_b[j] = (uint32_t)(row < rb ? row : rb) * (uint32_t)pitch;
-#pragma unroll
-        for (int h = 0; h < 2; ++h) put[j][h] = lds + row * MID_ROW_BYTES + swizzle_slot(row, h * 8 + lane_chunk, 16, 1) * CHUNK_BYTES;
+        const int row = wave * 16 + j * 8 + lane / 8, chunk = swizzle_slot(row, lane % 8, 8, 1);
+        off[j] = (uint32_t)row * pitch + (uint32_t)chunk * CHUNK_BYTES;
+        chunk_k[j] = chunk * CHUNK_ELEMS;
     }
-    struct Part { u32x4 a[2][2], b[2][2]; };
-    // (a segment past the end of K reads the row's last chunks over again: its part is never multiplied, and a fetch under no
-    // condition lets the compiler count the loads in flight)
-    auto fetch = [&](Part& p, int seg) __attribute__((always_inline)) {
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int k = seg * MID_SEGK + h * 64 + lane_chunk * 8;
-            const uint32_t at = (uint32_t)(k < g.K - 8 ? k : g.K - 8) * 2;
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                p.a[j][h] = *(const u32x4*)(base_a + (off_a[j] + at));
-                p.b[j][h] = *(const u32x4*)(base_b + (off_b[j] + at));
-            }
-        }
+    const int slabs = (g.K + MID_SLAB_K - 1) / MID_SLAB_K;
+    int ld_slab = (int)(blockIdx.x % (unsigned)g.num_xcd) % slabs, ld_left = slabs, ld_stage = 0;
+    auto load = [&](int i) __attribute__((always_inline)) {   // 0, 1: A; 2, 3: Bt
+        uint32_t voff = off[i % 2];
+        // (beyond every descriptor's range, which is below 2^31)
+        if (KTAIL && ld_slab * MID_SLAB_K + chunk_k[i % 2] >= g.K) voff = 0x80000000u;
+        dma_load_b128(i < 2 ? rsrc_a : rsrc_b, ring + (uint32_t)(ld_stage * MID_STAGE + (i < 2 ? 0 : MID_OPERAND) + wave * 2048 + i % 2 * 1024), voff,
+                      (uint32_t)ld_slab * (MID_SLAB_K * 2));
     };
-    auto stash = [&](Part& p, int seg, int stage) __attribute__((always_inline)) {
-        if ((seg + 1) * MID_SEGK > g.K) {   // zeros from K on
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
-                if (seg * MID_SEGK + h * 64 + lane_chunk * 8 >= g.K)
-#pragma unroll
-                    for (int j = 0; j < 2; ++j) p.a[j][h] = p.b[j][h] = u32x4{0, 0, 0, 0};
-        }
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                *(CK_LDS u32x4*)(put[j][h] + stage * 2 * MID_OPERAND) = p.a[j][h];
-                *(CK_LDS u32x4*)(put[j][h] + stage * 2 * MID_OPERAND + MID_OPERAND) = p.b[j][h];
-            }
-    };
-    auto meet = []() __attribute__((always_inline)) {   // every wave's LDS accesses are done
-        wait_lgkmcnt0();
-        wg_barrier();
+    // (behind the last slab the loads go on, for the count of those in flight, with descriptors of no bytes)
+    auto next_slab = [&]() __attribute__((always_inline)) {
+        ld_slab = ld_slab + 1 == slabs ? 0 : ld_slab + 1;
+        if (--ld_left <= 0) { rsrc_a[2] = rsrc_b[2] = 0; ld_slab = 0; }
+        ld_stage = ld_stage + 1 == MID_STAGES ? 0 : ld_stage + 1;
     };
 
     const int group = wave / 4, R = wave % 4 / 2, Cc = wave % 2;
     const int lr = lane & 15, lg = lane >> 4;
-    const CK_LDS char* get_a[2];
-    const CK_LDS char* get_b[2];
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-        const int chunk = (group * 2 + s) * 4 + lg;
-        get_a[s] = lds + (R * 64 + lr) * MID_ROW_BYTES + swizzle_slot(lr, chunk, 16, 1) * CHUNK_BYTES;
-        get_b[s] = lds + MID_OPERAND + (Cc * 64 + lr) * MID_ROW_BYTES + swizzle_slot(lr, chunk, 16, 1) * CHUNK_BYTES;
-    }
+    const uint32_t slot = (uint32_t)(swizzle_slot(lr, group * 4 + lg, 8, 1) * CHUNK_BYTES);
+    const uint32_t get_a = ring + (uint32_t)(R * 64 + lr) * (MID_SLAB_K * 2) + slot, get_b = ring + MID_OPERAND + (uint32_t)(Cc * 64 + lr) * (MID_SLAB_K * 2) + slot;
+    u32x4 fa[2][WT], fb[2][WT];   // fragments of the slab being multiplied and of the next one
     f32x4 acc[WT][WT];
 #pragma unroll
     for (int i = 0; i < WT; ++i)
 #pragma unroll
         for (int j = 0; j < WT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    const int segs = (g.K + MID_SEGK - 1) / MID_SEGK;
-    // Segment s lies in stage STAGE, segment s + 1 in p on its way: the fragments of s first, then p goes to the other stage
-    // (whose readers met at the barrier before) and the loads of s + 3 take its registers, then the MFMAs.
-    auto segment = [&](int s, auto stage_index, Part& p) __attribute__((always_inline)) {
-        constexpr int STAGE = decltype(stage_index)::value;
-        u32x4 a[2][WT], b[2][WT];
+#pragma unroll 1
+    for (int p = 0; p < MID_STAGES; ++p) {
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int i = 0; i < WT; ++i) {
-                a[t][i] = *(const CK_LDS u32x4*)(get_a[t] + STAGE * 2 * MID_OPERAND + i * 16 * MID_ROW_BYTES);
-                b[t][i] = *(const CK_LDS u32x4*)(get_b[t] + STAGE * 2 * MID_OPERAND + i * 16 * MID_ROW_BYTES);
-            }
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int i = 0; i < WT; ++i)
-#pragma unroll
-            for (int j = 0; j < WT; ++j) acc[i][j] = MfmaOp<DT>::run(b[0][j], a[0][i], acc[i][j]);
-        __builtin_amdgcn_sched_barrier(0);
-        stash(p, s + 1, 1 - STAGE);
-        fetch(p, s + 3);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int i = 0; i < WT; ++i)
-#pragma unroll
-            for (int j = 0; j < WT; ++j) acc[i][j] = MfmaOp<DT>::run(b[1][j], a[1][i], acc[i][j]);
-        meet();
-    };
-    Part odd, even;
-    fetch(even, 0);
-    fetch(odd, 1);
-    stash(even, 0, 0);
-    fetch(even, 2);
-    meet();
-    int s = 0;
-    for (; s + 1 < segs; s += 2) {
-        segment(s, std::integral_constant<int, 0>{}, odd);
-        segment(s + 1, std::integral_constant<int, 1>{}, even);
+        for (int i = 0; i < 4; ++i) load(i);
+        next_slab();
     }
-    if (s < segs) segment(s, std::integral_constant<int, 0>{}, odd);
-
-    // (the lane's number once more: carried through the loop it and what comes of it went to scratch memory)
-    const int out_lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), out_lr = out_lane & 15, out_lg = out_lane >> 4;
-    // The two partial sums of a wave tile: the first group keeps the upper half of the block rows, the second the lower one, and
-    // each hands the other half over.
-    const bool lower = group != 0;
-    CK_LDS char* mine = lds + wave * (WT / 2 * WT * 1024) + out_lane * 16;
-    const CK_LDS char* theirs = lds + (wave ^ 4) * (WT / 2 * WT * 1024) + out_lane * 16;
+    wait_vmcnt_imm<12>();   // slabs 0 and 1
+    wg_barrier();
 #pragma unroll
-    for (int i = 0; i < WT / 2; ++i)
-#pragma unroll
-        for (int j = 0; j < WT; ++j) *(CK_LDS f32x4*)(mine + (i * WT + j) * 1024) = lower ? acc[i][j] : acc[WT / 2 + i][j];
-    meet();
-    const bool vec_cols = g.vec_store && (rc.col + 1) * MID_TILE <= g.N;
-#pragma unroll
-    for (int i = 0; i < WT / 2; ++i)
+    for (int i = 0; i < WT; ++i) {
+        fa[0][i] = *(const CK_LDS u32x4*)(uintptr_t)(get_a + i * 16 * MID_SLAB_K * 2);
+        fb[0][i] = *(const CK_LDS u32x4*)(uintptr_t)(get_b + i * 16 * MID_SLAB_K * 2);
+    }
+    uint32_t stage = 0;
+    // Body s: its fragments are in f[P]. Behind its barrier slab s + 2 is complete (this wave's loads of s + 3 and s + 4 may fly), and every
+    // wave holds the fragments of s: slab s + 5 takes their stage. (After the last slab the fragments of a stage that nothing needs are read.)
+    auto body = [&](auto parity) __attribute__((always_inline)) {
+        constexpr int P = decltype(parity)::value;
+        stage = stage + 1 == MID_STAGES ? 0 : stage + 1;
+        const uint32_t at_a = get_a + stage * MID_STAGE, at_b = get_b + stage * MID_STAGE;
+        use_fragments(fa[P], fb[P]);
+        wait_vmcnt_imm<8>();
+        wg_barrier();
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int j = 0; j < WT; ++j) {
-            const f32x4 sum = (lower ? acc[WT / 2 + i][j] : acc[i][j]) + *(const CK_LDS f32x4*)(theirs + (i * WT + j) * 1024);
-            epilogue_block<DT>(g, row_a + R * 64 + ((lower ? WT / 2 : 0) + i) * 16 + out_lr, row_b + Cc * 64 + j * 16 + out_lg * 4, sum, vec_cols);
+            load(j);
+            if (j == WT - 1) next_slab();
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int f = j * 2 + i;
+                if (f < WT) fa[1 - P][f] = *(const CK_LDS u32x4*)(uintptr_t)(at_a + f * 16 * MID_SLAB_K * 2);
+                else fb[1 - P][f - WT] = *(const CK_LDS u32x4*)(uintptr_t)(at_b + (f - WT) * 16 * MID_SLAB_K * 2);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+            for (int i = 0; i < WT; ++i) acc[i][j] = MfmaOp<DT>::run(fb[P][j], fa[P][i], acc[i][j]);
+            __builtin_amdgcn_s_setprio(0);
+            __builtin_amdgcn_sched_barrier(0);
         }
+    };
+    int s = 0;
+#pragma unroll 1
+    for (; s + 1 < slabs; s += 2) {
+        body(std::integral_constant<int, 0>{});
+        body(std::integral_constant<int, 1>{});
+    }
+    if (s < slabs) body(std::integral_constant<int, 0>{});
 
-    if (blockIdx.x == 0 && wave == 7 && out_lane == 63) {
+    // The partial sums in rows: every wave writes its wave tile, and of the two waves of one place each finishes 32 rows, 16 lanes to
+    // a row. (No load, of nothing, is on its way into LDS any more.)
+    wait_vmcnt_imm<0>();
+    wait_lgkmcnt0();
+    wg_barrier();
+    CK_LDS char* const out = (CK_LDS char*)ck_smem;
+#pragma unroll
+    for (int i = 0; i < WT; ++i)
+#pragma unroll
+        for (int j = 0; j < WT; ++j)
+            *(CK_LDS f32x4*)(out + wave * MID_OUT_WAVE + (i * 16 + lr) * MID_OUT_ROW + (j * 16 + lg * 4) * 4) = acc[i][j];
+    const int m0 = row_a + R * 64 + group * 32 + lg, n0 = row_b + Cc * 64 + lr * 4;
+    f32x4 c[8];
+#pragma unroll
+    for (int t = 0; t < 8; ++t) c[t] = row_c<DT>(g, m0 + t * 4, n0);
+    wait_lgkmcnt0();
+    wg_barrier();
+    const CK_LDS char* first = out + wave % 4 * MID_OUT_WAVE + (group * 32 + lg) * MID_OUT_ROW + lr * 16;
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+        const CK_LDS char* at = first + t * 4 * MID_OUT_ROW;
+        store_row<DT>(g, m0 + t * 4, n0, *(const CK_LDS f32x4*)at + *(const CK_LDS f32x4*)(at + 4 * MID_OUT_WAVE), c[t]);
+    }
+
+    if (blockIdx.x == 0 && threadIdx.x == blockDim.x - 1) {
         const unsigned long long dc = clock64() - clk0, dw = wall_clock64() - wall0;
         g.status[2] = (unsigned)dc; g.status[3] = (unsigned)(dc >> 32);
         g.status[4] = (unsigned)dw; g.status[5] = (unsigned)(dw >> 32);

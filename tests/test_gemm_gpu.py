@@ -1602,3 +1602,32 @@ def test_small_tuple_on_many_tiles_and_behind_copies(ck, bf16):
         assert torch.equal(d[:M * N].view(M, N).cpu(), a.cpu().float() @ b.cpu().float().t()), (M, N, K)   # (fp32 sums of whole numbers below 2^24 are exact)
         assert torch.isnan(d[M * N:]).all()
     assert ck.device_status() == 0
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+def test_ring_of_slabs_at_its_shortest_and_past_a_row_end(ck, bf16):
+    """gemm_mid_kernel on K of four to twelve slabs of 64 (the ring holds five, loaded before the first is used), K that ends inside the
+    first and the last slab of a ring's round, N that no store of four values divides, in fp32 and 16-bit C and D. Small integers: exact. NaN
+    around the operands (rows past the edge, k past the end and slabs past the last read zeros), a guard behind D."""
+    dtype, tdt = (ck.DT_BF16, torch.bfloat16) if bf16 else (ck.DT_F16, torch.float16)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(23)
+    for M, N, K in [(1500, 1401, 256), (1500, 1402, 264), (1537, 1403, 320), (1500, 1400, 328), (1440, 1601, 376), (1500, 1405, 384), (200, 130, 512), (131, 259, 704), (2048, 2045, 776)]:
+        def operand(rows):
+            buf = torch.full((rows * K + 4096,), float("nan"), dtype=tdt, device="cuda")
+            view = buf[2048:2048 + rows * K].view(rows, K)
+            view.copy_(torch.randint(-2, 3, (rows, K), device="cuda", generator=gen))
+            return view
+        a, b = operand(M), operand(N)
+        assert ck.gemm_launch_kernel(M, N, K, True, *MID_TUPLE) == "gemm_mid_kernel"
+        exact = a.cpu().float() @ b.cpu().float().t()
+        c = torch.randint(-8, 9, (M, N), device="cuda", generator=gen).float()
+        d = torch.full((M * N + 64,), float("nan"), dtype=torch.float32, device="cuda")
+        ck.gemm_shmem_tc_async_opt_port(dtype, a, b, c, d, 2.0, -3.0, M, N, K, *MID_TUPLE)
+        assert torch.equal(d[:M * N].view(M, N).cpu(), 2 * exact - 3 * c.cpu()), (M, N, K)
+        assert torch.isnan(d[M * N:]).all()
+        d16 = torch.full((M * N + 64,), float("nan"), dtype=tdt, device="cuda")
+        ck.gemm_shmem_tc_async_opt_port_lp(dtype, a, b, c.to(tdt), d16, 1.0, 1.0, M, N, K, *MID_TUPLE)
+        assert torch.equal(d16[:M * N].view(M, N).cpu(), (exact + c.cpu()).to(tdt)), (M, N, K)
+        assert torch.isnan(d16[M * N:]).all()
+    assert ck.device_status() == 0
