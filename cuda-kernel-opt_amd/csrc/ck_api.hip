@@ -263,12 +263,58 @@ hipMemPool_t scratch_pool_for_current_device() {
     return g_scratch_pool[dev];
 }
 
+// Blocks of that pool kept for the launches on a device's default stream, which is in order and never destroyed: a launch that
+// finds one free uses it behind the launches before it, without the 9 to 11 us of host time that an allocation and its release take (two
+// launches take 6). A block is held by one call at a time; a call that finds none free or needs more than KEPT_MOST, and every call on another stream (whose
+// handle may pass to a new stream while work is still under way), allocates. ckopt_trim_scratch_pool gives the blocks back.
+constexpr int KEPT_BLOCKS = 2;                            // operand copies and K planes of one call
+constexpr size_t KEPT_MOST = (size_t)256 << 20;
+struct KeptBlock { void* ptr; size_t bytes; bool held; };
+KeptBlock g_kept[MAX_DEV][KEPT_BLOCKS] = {};
+int kept_device() {
+    int dev = 0;
+    return hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < MAX_DEV ? dev : -1;
+}
+void* kept_take(size_t need, hipMemPool_t pool) {
+    const int dev = kept_device();
+    if (!pool || dev < 0 || need > KEPT_MOST) return nullptr;
+    std::lock_guard<std::mutex> lock(g_status_mutex);
+    KeptBlock* pick = nullptr;   // the smallest free block that is large enough, else the largest free one, which grows
+    for (KeptBlock& b : g_kept[dev])
+        if (!b.held && (!pick || (b.bytes >= need ? pick->bytes < need || b.bytes < pick->bytes : pick->bytes < need && b.bytes > pick->bytes))) pick = &b;
+    if (!pick) return nullptr;
+    if (pick->bytes < need) {
+        if (pick->ptr) (void)hipFreeAsync(pick->ptr, nullptr);
+        *pick = KeptBlock{nullptr, 0, false};
+        void* p = nullptr;
+        if (hipMallocFromPoolAsync(&p, need, pool, nullptr) != hipSuccess || !p) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        *pick = KeptBlock{p, need, false};
+    }
+    pick->held = true;
+    return pick->ptr;
+}
+bool kept_release(void* piece) {
+    const int dev = kept_device();
+    if (dev < 0) return false;
+    std::lock_guard<std::mutex> lock(g_status_mutex);
+    for (KeptBlock& b : g_kept[dev])
+        if (b.held && b.ptr == piece) {
+            b.held = false;
+            return true;
+        }
+    return false;
+}
+
 // Takes `need` bytes: CK_OK with *out set, CK_ERR_HIP if the allocation failed, CK_ERR_TOO_LARGE if a provided buffer
 // is too small. A piece of an ALLOCATE scratch is handed back with scratch_release().
 int scratch_take(Scratch& sc, size_t need, hipStream_t s, void** out) {
     if (sc.mode == Scratch::ALLOCATE) {
         *out = nullptr;
         hipMemPool_t pool = scratch_pool_for_current_device();
+        if (!s && (*out = kept_take(need, pool))) return ck::CK_OK;
         if ((pool ? hipMallocFromPoolAsync(out, need, pool, s) : hipMallocAsync(out, need, s)) != hipSuccess || !*out) {
             (void)hipGetLastError();  // the failure is reported through the return value, not left for the next HIP call
             return ck::CK_ERR_HIP;
@@ -291,7 +337,7 @@ bool scratch_holds(Scratch sc, size_t need) {
     return sc.mode == Scratch::ALLOCATE || scratch_take(sc, need, nullptr, &at) == ck::CK_OK;
 }
 bool scratch_release(const Scratch& sc, void* piece, hipStream_t s) {
-    return sc.mode != Scratch::ALLOCATE || hipFreeAsync(piece, s) == hipSuccess;
+    return sc.mode != Scratch::ALLOCATE || (!s && kept_release(piece)) || hipFreeAsync(piece, s) == hipSuccess;
 }
 
 struct Route;
@@ -1109,11 +1155,19 @@ int ckopt_trim_scratch_pool(size_t keep_bytes) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= MAX_DEV) return ck::CK_ERR_HIP;
     hipMemPool_t pool = nullptr;
+    bool freed = false;
     {
         std::lock_guard<std::mutex> lock(g_status_mutex);
         pool = g_scratch_pool[dev];
+        for (KeptBlock& b : g_kept[dev])
+            if (b.ptr && !b.held) {
+                if (hipFreeAsync(b.ptr, nullptr) != hipSuccess) return ck::CK_ERR_HIP;
+                b = KeptBlock{nullptr, 0, false};
+                freed = true;
+            }
     }
     if (!pool) return ck::CK_OK;
+    if (freed && hipStreamSynchronize(nullptr) != hipSuccess) return ck::CK_ERR_HIP;   // (the pool lets go of what is free)
     return hipMemPoolTrimTo(pool, keep_bytes) == hipSuccess ? ck::CK_OK : ck::CK_ERR_HIP;
 }
 

@@ -13,7 +13,8 @@
  * operand is off a 16-byte boundary; partial planes when the straight-line kernel cuts K into slices). The reference's
  * launcher needs none and allocates nothing (port_2.cu:1088-1168; its drivers own all memory, :1200-1203). Here the
  * plain entry points take it from stream-ordered allocations on `stream`, out of a memory pool the library keeps per
- * device (freed blocks stay in the pool for the next launch; ckopt_trim_scratch_pool hands them back);
+ * device (freed blocks stay in the pool for the next launch, and two of up to 256 MiB are kept for the launches on the device's default
+ * stream; ckopt_trim_scratch_pool hands them back);
  * ckopt_gemm_shmem_tc_async_opt_port_2_ws takes it from a workspace the caller owns and allocates nothing;
  * ckopt_gemm_shmem_tc_async_opt_port_2_noalloc takes it from a static array inside the library.
  */
@@ -268,7 +269,8 @@ int ckopt_check_matmul_shmem_tuning(int tile_dim, int block_rows);
 
 /* Releases what the library's stream-ordered scratch pool of the current device holds beyond keep_bytes (0: everything
  * that is not in use). The pool keeps the largest scratch a launch of the allocating entry points has used on the device,
- * so that the next launch does not pay for a fresh allocation. No reference counterpart. */
+ * so that the next launch does not pay for a fresh allocation. Where blocks were kept for the default stream it waits for that stream.
+ * No reference counterpart. */
 int ckopt_trim_scratch_pool(size_t keep_bytes);
 
 /* Waits for `stream`, then returns the device status word of the current device and clears it:

@@ -1631,3 +1631,44 @@ def test_ring_of_slabs_at_its_shortest_and_past_a_row_end(ck, bf16):
         assert torch.equal(d16[:M * N].view(M, N).cpu(), (exact + c.cpu()).to(tdt)), (M, N, K)
         assert torch.isnan(d16[M * N:]).all()
     assert ck.device_status() == 0
+
+
+def test_kept_scratch_blocks_with_threads_and_given_back(ck):
+    """Launches of several host threads on the default stream, with scratch memory of different sizes (K planes; operand copies and planes): each
+    call has a block to itself, and every product is exact. Afterwards the blocks are given back, and the next call takes new ones."""
+    import threading
+    cases = [(MID_TUPLE, 213, 320, 36672), (SMALL_TUPLE, 64, 192, 14080), ((256, 32, 0, 0, 256, 256, 4, 5, 0, 8, 256), 300, 200, 4090), (MID_TUPLE, 512, 512, 28608)]
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(37)
+    work = []
+    for t, M, N, K in cases:
+        a = torch.randint(-2, 3, (M, K), device="cuda", generator=gen).half()
+        b = torch.randint(-2, 3, (N, K), device="cuda", generator=gen).half()
+        outs = [torch.full((M, N), float("nan"), dtype=torch.float32, device="cuda") for _ in range(10)]
+        work.append((t, M, N, K, a, b, outs, (a.cpu().float() @ b.cpu().float().t()).cuda()))
+    torch.cuda.synchronize()
+    errors = []
+
+    def launch(w):
+        t, M, N, K, a, b, outs, _ = w
+        try:
+            for d in outs:
+                ck.gemm_shmem_tc_async_opt_port(ck.DT_F16, a, b, None, d, 1.0, 0.0, M, N, K, *t)
+        except Exception as e:
+            errors.append(e)
+    for _ in range(2):
+        threads = [threading.Thread(target=launch, args=(w,)) for w in work]
+        for th in threads:
+            th.start()
+        for th in threads:
+            th.join()
+        torch.cuda.synchronize()
+        assert not errors
+        for w in work:
+            for d in w[6]:
+                assert torch.equal(d, w[7]), w[:4]
+                d.fill_(float("nan"))
+        before = torch.cuda.mem_get_info()[0]
+        ck.trim_scratch_pool()
+        assert torch.cuda.mem_get_info()[0] >= before
+    assert ck.device_status() == 0
