@@ -303,7 +303,7 @@ def gemm_kernel_name(ck, dtype, M, N, K, tup, mode):
     elif name == "gemm_direct_kernel":
         what = "%d x %d tiles, 8 waves on slices of K" % (cols, cols)
     elif name == "gemm_mid_kernel":
-        what = "128 x 128 tiles staged through registers, 8 waves"
+        what = "128 x 128 tiles, five 64-deep slabs, 8 waves"
     elif producers == 0:
         what = "tile %d, seg_k %d, %d waves, workgroup barrier per segment" % (tile, segk, consumers)
     else:

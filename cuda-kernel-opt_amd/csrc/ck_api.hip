@@ -185,36 +185,60 @@ __global__ void pad_rows_kernel(const unsigned short* __restrict__ src_a, unsign
     }
 }
 
-// Second pass of a split-K product: D = alpha * (plane 0 + plane 1 + ...) + beta * C, the planes added in
-// slice order (the result does not depend on how the first pass was scheduled). One thread per element;
-// DT16 selects the 16-bit C/D forms.
+// Second pass of a split-K product: D = alpha * (plane 0 + plane 1 + ...) + beta * C, the planes added in slice order (the result does not
+// depend on how the first pass was scheduled). OUT16 selects the 16-bit C/D forms. Four outputs per thread, rows of planes, C and D on
+// any boundary of their own elements. Bound by memory for few planes of a large product (5.3 TB/s), by round trips to it for many of a small one: the loads of
+// eight planes are in flight at a time (one plane at a time: calls of 256 x 64 x 57856 in 60 slices 28.7 us, 17.5 now; 360 x 190 x 34304 in 36 28.1, 20.2).
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 template <int OUT16, bool BF16>
 __global__ void splitk_reduce_kernel(const float* __restrict__ ws, int slices, long long count, const void* C, void* D, float alpha, float beta) {
-    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < count; i += (long long)gridDim.x * blockDim.x) {
-        float sum = ws[i];
-        for (int s = 1; s < slices; ++s) sum += ws[(long long)s * count + i];
-        float v = alpha * sum;
-        if (OUT16) {
-            using O = ck::Out16<typename std::conditional<BF16, ck::bf16_tag, ck::f16_tag>::type>;
-            if (beta != 0.f) v += O::load(static_cast<const unsigned short*>(C)[i]) * beta;
-            static_cast<unsigned short*>(D)[i] = O::store(v);
-        } else {
-            if (beta != 0.f) v += static_cast<const float*>(C)[i] * beta;
-            static_cast<float*>(D)[i] = v;
+    using O = ck::Out16<typename std::conditional<BF16, ck::bf16_tag, ck::f16_tag>::type>;
+    typedef unsigned short u16x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
+    const long long groups = (count + 3) / 4;
+    for (long long g = (long long)blockIdx.x * blockDim.x + threadIdx.x; g < groups; g += (long long)gridDim.x * blockDim.x) {
+        const long long i = g * 4;
+        if (i + 4 > count) {   // the end of the last plane
+            for (long long e = i; e < count; ++e) {
+                float sum = ws[e];
+                for (int s = 1; s < slices; ++s) sum += ws[(long long)s * count + e];
+                float v = alpha * sum;
+                if (OUT16) {
+                    if (beta != 0.f) v += O::load(static_cast<const unsigned short*>(C)[e]) * beta;
+                    static_cast<unsigned short*>(D)[e] = O::store(v);
+                } else {
+                    if (beta != 0.f) v += static_cast<const float*>(C)[e] * beta;
+                    static_cast<float*>(D)[e] = v;
+                }
+            }
+            continue;
         }
-    }
-}
-
-// The fp32 form of the same pass with four elements per thread (16-byte loads and stores): same additions in
-// the same order per element. For count % 4 == 0 and C, D on 16-byte boundaries.
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-__global__ void splitk_reduce4_kernel(const f32x4* __restrict__ ws, int slices, long long count4, const f32x4* C, f32x4* D, float alpha, float beta) {
-    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < count4; i += (long long)gridDim.x * blockDim.x) {
-        f32x4 sum = __builtin_nontemporal_load(ws + i);
-        for (int s = 1; s < slices; ++s) sum += __builtin_nontemporal_load(ws + (long long)s * count4 + i);
+        auto plane = [&](int s) { return (f32x4)__builtin_nontemporal_load((const ck::f32x4_u*)(ws + (long long)s * count + i)); };
+        f32x4 sum = {0.f, 0.f, 0.f, 0.f};   // (a plane's sums started from +0 and are never -0)
+        int s = 0;
+        auto batch = [&](auto planes) __attribute__((always_inline)) {
+            constexpr int B = decltype(planes)::value;
+            f32x4 x[B];
+#pragma unroll
+            for (int t = 0; t < B; ++t) x[t] = plane(s + t);
+#pragma unroll
+            for (int t = 0; t < B; ++t) sum += x[t];
+            s += B;
+        };
+        while (s + 8 <= slices) batch(std::integral_constant<int, 8>{});
+        if (slices & 4) batch(std::integral_constant<int, 4>{});
+        if (slices & 2) batch(std::integral_constant<int, 2>{});
+        if (slices & 1) batch(std::integral_constant<int, 1>{});
         f32x4 v = alpha * sum;
-        if (beta != 0.f) v += C[i] * beta;
-        D[i] = v;
+        if (OUT16) {
+            if (beta != 0.f) {
+                const u16x4_a2 c = *(const u16x4_a2*)(static_cast<const unsigned short*>(C) + i);
+                v += f32x4{O::load(c[0]), O::load(c[1]), O::load(c[2]), O::load(c[3])} * beta;
+            }
+            *(u16x4_a2*)(static_cast<unsigned short*>(D) + i) = u16x4_a2{O::store(v[0]), O::store(v[1]), O::store(v[2]), O::store(v[3])};
+        } else {
+            if (beta != 0.f) v += *(const ck::f32x4_u*)(static_cast<const float*>(C) + i) * beta;
+            *(ck::f32x4_u*)(static_cast<float*>(D) + i) = v;
+        }
     }
 }
 
@@ -231,6 +255,7 @@ struct Scratch {
     enum Mode { ALLOCATE, PROVIDED } mode;
     char* ptr;
     size_t bytes;
+    bool shared;   // the library's static array, which every call of the entry point that allocates nothing works in
 };
 constexpr size_t SCRATCH_ALIGN = 256;
 size_t scratch_round(size_t n) { return (n + SCRATCH_ALIGN - 1) / SCRATCH_ALIGN * SCRATCH_ALIGN; }
@@ -546,25 +571,41 @@ double direct_us(int tile, int64_t tiles, int K, int rows_aligned, double operan
     return off_lines ? std::max(us, 1.5 + operand_bytes / 2.2e6) : us;   // (from memory: 64 x 8768 x 10600 87.6, ring 68.6)
 }
 double behind_copies_us(double us, int M, int N, int K) { return std::max(21.5, us + 7.5 + 4.0 * ((double)M + N) * K / 6e6); }
+// K slices of the two kernels with one workgroup per tile: (tile, slice) items fill the device where the tiles do not, each slice writes an
+// fp32 plane of scratch memory, and the reduction pass adds the planes. call_us: what such a call takes the host, with a block kept for the default
+// stream or a provided workspace, and with an allocation; 0: no slices.
+constexpr int ITEM_MAX_SLICES = 64;
+constexpr int ITEM_MIN_SLICE = 512;
+constexpr double KEPT_CALL_US = 10.0, ALLOCATED_CALL_US = 23.0;
+double sliced_us(double us, int S, int64_t mn, double call_us) { return std::max(call_us, us + 3.5 + (double)(S + 1) * (double)mn * 4.0 / 5.3e6); }
 // direct: tile of the small-product kernel, 0: the ring kernel on 64 x 64 tiles; copies: behind zero-padded operand copies
-struct SmallPlan { int direct; bool copies; double us; };
-SmallPlan small_plan(int M, int N, int K, int operand_alignment, int cus, bool on_copies = false) {
+struct SmallPlan { int direct; bool copies; int slices; double us; };
+SmallPlan small_plan(int M, int N, int K, int operand_alignment, int cus, double call_us, bool on_copies = false) {
     auto tiles = [&](int t) { return (int64_t)((M + t - 1) / t) * ((N + t - 1) / t); };
     SmallPlan best;
     if (needs_copies(K, operand_alignment >= 16)) {   // what the launch on the copies, whose rows are padded to whole chunks, runs
         const int Kp = (K + ck::CHUNK_ELEMS - 1) / ck::CHUNK_ELEMS * ck::CHUNK_ELEMS;
-        best = small_plan(M, N, Kp, 16, cus, true);
+        best = small_plan(M, N, Kp, 16, cus, 0.0, true);
         best.copies = true;
         best.us = behind_copies_us(best.us, M, N, Kp);
-    } else best = SmallPlan{0, false, ring_us(tiles(64), K, cus)};
+    } else best = SmallPlan{0, false, 1, ring_us(tiles(64), K, cus)};
     if (K < ck::CHUNK_ELEMS) return best;   // the small-product kernel reads whole chunks of a row
     const int rows_aligned = K % 2 ? 2 : operand_alignment < 16 || K % 64 ? std::min(operand_alignment, 4) : LINE_BYTES;
+    const double bytes = ((double)M + N) * K * 2.0;
     for (int t : {32, 64}) {
-        const double us = direct_us(t, tiles(t), K, rows_aligned, ((double)M + N) * K * 2.0, on_copies, cus);
+        const double us = direct_us(t, tiles(t), K, rows_aligned, bytes, on_copies, cus);
         // (the ring where the two are level: 16-bit results and operands from memory favour it, 2048^2 x 1024 29.3 / 32.8; but no copies
         // where those are level)
-        if (us < (best.copies ? 1.0 : 0.93) * best.us) best = {t, false, us};
+        if (us < (best.copies ? 1.0 : 0.93) * best.us) best = {t, false, 1, us};
     }
+    if (call_us == 0.0 || K < 2 * ITEM_MIN_SLICE || 0.9 * best.us <= call_us) return best;
+    const SmallPlan whole = best;
+    for (int t : {32, 64})
+        for (int S = 2; S <= ITEM_MAX_SLICES && K / S >= ITEM_MIN_SLICE && tiles(t) * S <= 2 * cus; ++S) {
+            // (from seven slices on 4 to 9 us more than that: 360 x 190 x 34304 in 14 25.3, 213 x 320 x 36672 in 12 25.0, 1149 x 128 x 11520 in 7 17.7; 512^2 x 12288 in 4 17.8)
+            const double us = sliced_us(direct_us(t, tiles(t) * S, (K + S - 1) / S, rows_aligned, bytes, on_copies, cus), S, (int64_t)M * N, call_us) + (S > 6 ? 6.0 : 0.0);
+            if (us < 0.9 * whole.us && us < 0.98 * best.us) best = {t, false, S, us};
+        }
     return best;
 }
 // The tuple the library suggests for few tiles leaves the kernel to that estimate (ring against this, us: 512^3 6.4 / 4.4;
@@ -600,27 +641,54 @@ bool mid_is_shorter(int M, int N, int K, int cus) {
     return lines && tiles <= 9 * (int64_t)cus && K >= 1024;
 }
 
+// Estimated microseconds of gemm_mid_kernel on S slices of every tile, fitted to calls on aligned operands: a launch, per round 5.8 us of prologue
+// and epilogue, per slab of 64 k 0.355 us on up to 64 CUs to 0.46 on all 256 (1024^2: K 768 11.1, 1024 12.6, 2048 18.4, 4096 29.8;
+// 2048^2: K 1536 18.7, 2048 22.2, 4096 37.2; 4096^2 x 4096 145), rows off a line 1.2 to 1.4 times that (1024^2 x 1000 15.2, 2048^2 x 4104 44.7);
+// operands from memory at 3.4 TB/s where they leave the last-level cache (bf16 256 x 16384 x 4096 46.6).
+double mid_us(int64_t tiles, int K, int S, double operand_bytes, int cus) {
+    const double items = (double)tiles * S, rounds = std::ceil(items / cus), share = items / rounds / cus;
+    const double slab = (0.355 + 0.14 * std::max(0.0, share - 0.25)) * (K % 64 ? 1.3 : 1.0);
+    const double us = 1.5 + rounds * (5.8 + std::ceil((double)K / 64.0 / S) * slab);
+    return std::max(us, operand_bytes > 80e6 ? 6.0 + operand_bytes / 3.4e6 : 0.0);
+}
+struct MidPlan { int slices; double us; };
+MidPlan mid_plan(int M, int N, int K, int cus, double call_us) {
+    const int64_t tiles = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
+    const double bytes = ((double)M + N) * K * 2.0;
+    const MidPlan whole = {1, mid_us(tiles, K, 1, bytes, cus)};
+    MidPlan best = whole;
+    if (call_us > 0.0 && 0.9 * whole.us > call_us)
+        for (int S = 2; S <= ITEM_MAX_SLICES && K / S >= ITEM_MIN_SLICE && tiles * S <= 2 * cus; ++S) {
+            const double us = sliced_us(mid_us(tiles, K, S, bytes, cus), S, (int64_t)M * N, call_us);
+            if (us < 0.9 * whole.us && us < 0.98 * best.us) best = {S, us};
+        }
+    return best;
+}
+
 // What a launch runs: the one decision that the launcher and the queries share. operand_alignment: bytes that A and Bt both lie on,
 // 16, 4 or 2 (the queries are promised 16 or nothing). Behind operand copies it is what runs on them.
 struct Route {
     int kernel;    // CKOPT_KERNEL_*
     int tile;      // rows of its tiles of D (and their columns, but for the straight-line kernel, whose width stream_plan chooses)
     bool copies;   // A and Bt are first copied into zero-padded rows
+    int slices;    // K slices of a kernel with one workgroup per tile, where the launch finds scratch memory for their planes
 };
-Route route_of(int M, int N, int K, int operand_alignment, const ck::GemmTuning& t, const Options& opt) {
+Route route_of(int M, int N, int K, int operand_alignment, const ck::GemmTuning& t, const Options& opt, double sliced_call_us = KEPT_CALL_US) {
     using namespace ck;
-    Route r{CKOPT_KERNEL_PC, t.tile_dim, needs_copies(K, operand_alignment >= 16)};
+    Route r{CKOPT_KERNEL_PC, t.tile_dim, needs_copies(K, operand_alignment >= 16), 1};
     // (the two kernels with one workgroup per tile, which num_cus does not bound, only where the launch may use the whole device)
     const bool small = small_tuple(t, opt), mid = mid_tuple(t, opt);
+    const double call_us = opt[OPT_SPLIT_K] == 1 ? sliced_call_us : 0.0;
     const int cus = small || mid ? device_cus() : 0;
     if (small && t.num_cus >= cus) {
-        const SmallPlan p = small_plan(M, N, K, operand_alignment, cus);
-        return {p.direct ? CKOPT_KERNEL_DIRECT : CKOPT_KERNEL_FUSED, p.direct ? p.direct : t.tile_dim, p.copies};
+        const SmallPlan p = small_plan(M, N, K, operand_alignment, cus, call_us);
+        return {p.direct ? CKOPT_KERNEL_DIRECT : CKOPT_KERNEL_FUSED, p.direct ? p.direct : t.tile_dim, p.copies, p.slices};
     }
     if (straight_line_tuple(t, opt)) r.kernel = CKOPT_KERNEL_STREAM;
-    else if (mid && t.num_cus >= cus && !r.copies && mid_is_shorter(M, N, K, cus))
+    else if (mid && t.num_cus >= cus && !r.copies && mid_is_shorter(M, N, K, cus)) {
         r.kernel = CKOPT_KERNEL_MID;
-    else if (t.num_producer_waves == 0) r.kernel = t.num_stages == 1 ? CKOPT_KERNEL_SYNC : CKOPT_KERNEL_FUSED;
+        r.slices = mid_plan(M, N, K, cus, call_us).slices;
+    } else if (t.num_producer_waves == 0) r.kernel = t.num_stages == 1 ? CKOPT_KERNEL_SYNC : CKOPT_KERNEL_FUSED;
     else if (sync_mode_of(t.tile_dim, t.num_consumer_waves, t.bar_step_rows_a, t.bar_step_rows_b) == CK_SYNC_TILE && t.num_stages >= 2 &&
              opt[OPT_TILE_SYNC_BARRIER] && t.num_producer_waves != 1 && t.segment_dim_k <= 128)
         r.kernel = CKOPT_KERNEL_PCB;
@@ -640,6 +708,10 @@ size_t scratch_need(int M, int N, int K, bool operands_aligned, const ck::GemmTu
         const StreamPlan p = stream_plan(M, N, k, t.num_cus, opt);
         if (p.slices > 1 && p.fused) need += scratch_round(fix_state_bytes(p)) + scratch_round(fix_partial_bytes(p));
         else if (p.slices > 1) need += scratch_round((size_t)p.slices * M * N * sizeof(float));
+    } else {
+        // (the slices of the other two kernels are made of rows where they are: the planes or the copies, never both)
+        const Route r = route_of(M, N, K, operands_aligned ? 16 : 2, t, opt);
+        if (r.slices > 1) need = std::max(need, scratch_round((size_t)r.slices * M * N * sizeof(float)));
     }
     return need;
 }
@@ -668,6 +740,39 @@ int gemm_launch_repacked(int dtype, const void* A, const void* Bt, const void* C
     return rc;
 }
 
+// D = alpha * (plane 0 + plane 1 + ...) + beta * C
+hipError_t add_planes(int dtype, const float* ws, int slices, int64_t count, const void* C, void* D, float alpha, float beta, int out16, hipStream_t s) {
+    const dim3 blocks((unsigned)std::min<int64_t>(((count + 3) / 4 + 255) / 256, 65535 * 8));
+    if (!out16) hipLaunchKernelGGL((splitk_reduce_kernel<0, false>), blocks, dim3(256), 0, s, ws, slices, (long long)count, C, D, alpha, beta);
+    else if (dtype == ck::CK_DT_F16) hipLaunchKernelGGL((splitk_reduce_kernel<1, false>), blocks, dim3(256), 0, s, ws, slices, (long long)count, C, D, alpha, beta);
+    else hipLaunchKernelGGL((splitk_reduce_kernel<1, true>), blocks, dim3(256), 0, s, ws, slices, (long long)count, C, D, alpha, beta);
+    return hipGetLastError();
+}
+
+// One workgroup per (tile, K slice): `launch` on fp32 planes of scratch memory and the pass that adds them, or on D itself without slices. Slices are
+// only taken where there is room for their planes without a new condition on the caller: not in the static array, whose calls without
+// copies may overlap; not while the stream records a graph, which then holds one kernel and no allocation; and a provided buffer that
+// is too small or a failed allocation leaves one pass over all of K.
+template <typename F>
+hipError_t launch_items(const ck::GemmArgs& a, int slices, int dtype, Scratch sc, hipStream_t s, F launch) {
+    const int64_t count = (int64_t)a.M * a.N;
+    void* ws = nullptr;
+    if (slices > 1) {
+        hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+        if (sc.mode == Scratch::ALLOCATE && s && (hipStreamIsCapturing(s, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone))
+            slices = 1;
+        else if (scratch_take(sc, (size_t)slices * count * sizeof(float), s, &ws) != ck::CK_OK) slices = 1;
+    }
+    if (slices <= 1) return launch(a);
+    ck::GemmArgs p = a;
+    p.split_k = slices;
+    p.D = static_cast<float*>(ws); p.C = nullptr; p.alpha = 1.f; p.beta = 0.f; p.out16 = 0; p.vec_store = 1; p.nt_store = 0;
+    hipError_t e = launch(p);
+    if (e == hipSuccess) e = add_planes(dtype, p.D, slices, count, a.C, a.D, a.alpha, a.beta, a.out16, s);
+    if (!scratch_release(sc, ws, s) && e == hipSuccess) e = hipErrorUnknown;
+    return e;
+}
+
 int gemm_launch(int dtype, const void* A, const void* Bt, const void* C, void* D, float alpha, float beta, int M,
                 int N, int K, const ck::GemmTuning& t, const Options& opt, void* stream, int out16, Scratch sc, const Route* on_copies) {
     using namespace ck;
@@ -682,7 +787,8 @@ int gemm_launch(int dtype, const void* A, const void* Bt, const void* C, void* D
     if (((uintptr_t)D & elem_mask) || ((uintptr_t)C & elem_mask)) return CK_ERR_ALIGNMENT;
     // the ring kernels want every operand row on a 16-byte boundary
     const uintptr_t both = (uintptr_t)A | (uintptr_t)Bt;
-    const Route route = on_copies ? *on_copies : route_of(M, N, K, both & 15 ? both & 3 ? 2 : 4 : 16, t, opt);
+    const Route route = on_copies ? *on_copies : route_of(M, N, K, both & 15 ? both & 3 ? 2 : 4 : 16, t, opt,
+                                                      sc.shared ? 0.0 : sc.mode == Scratch::ALLOCATE && stream ? ALLOCATED_CALL_US : KEPT_CALL_US);
     // one tile's rows are addressed through a 32-bit buffer offset (rows of the copies, also where a kernel does without them)
     if ((int64_t)t.tile_dim * launch_k(K, !(both & 15), t, opt) * 2 >= (int64_t)1 << 31) return CK_ERR_TOO_LARGE;
     if (route.copies)
@@ -741,7 +847,8 @@ int gemm_launch(int dtype, const void* A, const void* Bt, const void* C, void* D
         // XCD's first loads on few memory channels, 118 x 2176 x 124 4.8 us against 5.2; with few columns of tiles and a deep K every XCD
         // streams a stretch of A of its own, 6528 x 396 x 33344 360 against 390, while 12864 x 192 x 4096 takes 51.3 as they come, 46.2 in runs.)
         if (tiles % a.num_xcd != 0 && (K < 512 || (a.tiles_n < 8 && K > 8192))) a.num_xcd = 1;
-        e = launch_gemm_direct(dtype == CK_DT_BF16, route.tile, K % 2 == 0 && !(both & 3), s, a);
+        e = launch_items(a, route.slices, dtype, sc, s,
+                         [&](const GemmArgs& args) { return launch_gemm_direct(dtype == CK_DT_BF16, route.tile, K % 2 == 0 && !(both & 3), s, args); });
     } else if (route.kernel == CKOPT_KERNEL_STREAM) {
         // Tile width, K slices and grid from the cost model: few tiles and a deep K are cut into slices so that every CU
         // has an item; the partly filled last round of many tiles likewise; tile counts that leave much of the device idle
@@ -802,24 +909,11 @@ int gemm_launch(int dtype, const void* A, const void* Bt, const void* C, void* D
             p.D = ws; p.C = nullptr; p.alpha = 1.f; p.beta = 0.f; p.out16 = 0; p.vec_store = 1;
             p.nt_store = store_policy == 1 || (store_policy == 0 && whole_lines(ws, (int64_t)N * 4) && count * 4 % LINE_BYTES == 0);
             e = launch(p, plan.grid);
-            if (e == hipSuccess) {
-                const unsigned blocks = (unsigned)((count + 255) / 256 < 65535 * 8 ? (count + 255) / 256 : 65535 * 8);
-                const bool vec4 = !out16 && count % 4 == 0 && ((uintptr_t)D | (uintptr_t)(beta != 0.f ? C : nullptr)) % 16 == 0;
-                const int slices = plan.slices;
-                if (vec4) {
-                    const long long count4 = count / 4;
-                    const unsigned b4 = (unsigned)((count4 + 255) / 256 < 65535 * 8 ? (count4 + 255) / 256 : 65535 * 8);
-                    hipLaunchKernelGGL(splitk_reduce4_kernel, dim3(b4), dim3(256), 0, s, reinterpret_cast<const f32x4*>(ws), slices, count4,
-                                       static_cast<const f32x4*>(C), static_cast<f32x4*>(D), alpha, beta);
-                } else if (!out16) hipLaunchKernelGGL((splitk_reduce_kernel<0, false>), dim3(blocks), dim3(256), 0, s, ws, slices, count, C, D, alpha, beta);
-                else if (dtype == CK_DT_F16) hipLaunchKernelGGL((splitk_reduce_kernel<1, false>), dim3(blocks), dim3(256), 0, s, ws, slices, count, C, D, alpha, beta);
-                else hipLaunchKernelGGL((splitk_reduce_kernel<1, true>), dim3(blocks), dim3(256), 0, s, ws, slices, count, C, D, alpha, beta);
-                e = hipGetLastError();
-            }
+            if (e == hipSuccess) e = add_planes(dtype, ws, plan.slices, count, C, D, alpha, beta, out16, s);
             if (!scratch_release(sc, ws, s) && e == hipSuccess) e = hipErrorUnknown;
         }
     } else if (route.kernel == CKOPT_KERNEL_MID) {
-        e = launch_gemm_mid(dtype == CK_DT_BF16, s, a);
+        e = launch_items(a, route.slices, dtype, sc, s, [&](const GemmArgs& args) { return launch_gemm_mid(dtype == CK_DT_BF16, s, args); });
     } else if (route.kernel == CKOPT_KERNEL_SYNC) {
         // one stage, no producers: load, barrier, multiply, barrier (the synchronous A/B partner)
         e = dtype == CK_DT_F16 ? launch_gemm_sync_f16(t.tile_dim, t.segment_dim_k, t.num_consumer_waves, dim3(grid), lds, s, a)
@@ -865,12 +959,12 @@ int ckopt_launch_options_init(ckopt_launch_options* options) {
 
 int ckopt_gemm_shmem_tc_async_opt_port_2(int dtype, const void* A, const void* Bt, const float* C, float* D, float alpha, float beta,
                                          int M, int N, int K, CK_TUNING_PARAMS, void* stream) {
-    return gemm_launch(dtype, A, Bt, C, D, alpha, beta, M, N, K, CK_TUNING_VALUE, default_options(), stream, 0, Scratch{Scratch::ALLOCATE, nullptr, 0});
+    return gemm_launch(dtype, A, Bt, C, D, alpha, beta, M, N, K, CK_TUNING_VALUE, default_options(), stream, 0, Scratch{Scratch::ALLOCATE, nullptr, 0, false});
 }
 
 int ckopt_gemm_shmem_tc_async_opt_port_2_lp(int dtype, const void* A, const void* Bt, const void* C, void* D, float alpha, float beta,
                                             int M, int N, int K, CK_TUNING_PARAMS, void* stream) {
-    return gemm_launch(dtype, A, Bt, C, D, alpha, beta, M, N, K, CK_TUNING_VALUE, default_options(), stream, 1, Scratch{Scratch::ALLOCATE, nullptr, 0});
+    return gemm_launch(dtype, A, Bt, C, D, alpha, beta, M, N, K, CK_TUNING_VALUE, default_options(), stream, 1, Scratch{Scratch::ALLOCATE, nullptr, 0, false});
 }
 
 int ckopt_gemm_shmem_tc_async_opt_port_2_noalloc(int dtype, const void* A, const void* Bt, const float* C, float* D, float alpha, float beta,
@@ -879,7 +973,7 @@ int ckopt_gemm_shmem_tc_async_opt_port_2_noalloc(int dtype, const void* A, const
     const int rc = static_scratch_for_current_device(&ptr);
     if (rc != ck::CK_OK) return rc;
     return gemm_launch(dtype, A, Bt, C, D, alpha, beta, M, N, K, CK_TUNING_VALUE, default_options(), stream, 0,
-                       Scratch{Scratch::PROVIDED, reinterpret_cast<char*>(ptr), (size_t)CKOPT_NOALLOC_SCRATCH_BYTES});
+                       Scratch{Scratch::PROVIDED, reinterpret_cast<char*>(ptr), (size_t)CKOPT_NOALLOC_SCRATCH_BYTES, true});
 }
 
 int ckopt_gemm_shmem_tc_async_opt_port_2_ex(int dtype, int cd_dtype, const void* A, const void* Bt, const void* C, void* D, float alpha,
@@ -889,7 +983,7 @@ int ckopt_gemm_shmem_tc_async_opt_port_2_ex(int dtype, int cd_dtype, const void*
     const int orc = options_from_public(options, &opt);
     if (orc != ck::CK_OK) return orc;
     if (!(cd_dtype == ck::CK_DT_F32 || cd_dtype == dtype)) return ck::CK_ERR_BAD_PARAM;
-    const Scratch sc = workspace ? Scratch{Scratch::PROVIDED, static_cast<char*>(workspace), workspace_bytes} : Scratch{Scratch::ALLOCATE, nullptr, 0};
+    const Scratch sc = workspace ? Scratch{Scratch::PROVIDED, static_cast<char*>(workspace), workspace_bytes, false} : Scratch{Scratch::ALLOCATE, nullptr, 0, false};
     return gemm_launch(dtype, A, Bt, C, D, alpha, beta, M, N, K, CK_TUNING_VALUE, opt, stream, cd_dtype == ck::CK_DT_F32 ? 0 : 1, sc);
 }
 
@@ -921,6 +1015,8 @@ int ckopt_gemm_launch_plan_ex(int M, int N, int K, int operands_aligned, CK_TUNI
     const Route route = route_of(M, N, K, operands_aligned ? 16 : 2, t, opt);
     plan_out[0] = 0; plan_out[1] = route.tile; plan_out[2] = 1; plan_out[3] = route.copies ? 1 : 0;
     plan_out[4] = 0; plan_out[5] = 0; plan_out[6] = 0;
+    plan_out[2] = route.slices;
+    if (route.slices > 1) plan_out[4] = ((M + route.tile - 1) / route.tile) * ((N + route.tile - 1) / route.tile);
     if (route.kernel == CKOPT_KERNEL_STREAM) {
         const StreamPlan plan = stream_plan(M, N, launch_k(K, operands_aligned != 0, t, opt), t.num_cus, opt);
         plan_out[0] = 1;
@@ -953,7 +1049,7 @@ int ckopt_gemm_shmem_tc_async_opt_port_2_ws(int dtype, int cd_dtype, const void*
                                             void* stream) {
     if (!(cd_dtype == ck::CK_DT_F32 || cd_dtype == dtype)) return ck::CK_ERR_BAD_PARAM;
     return gemm_launch(dtype, A, Bt, C, D, alpha, beta, M, N, K, CK_TUNING_VALUE, default_options(), stream, cd_dtype == ck::CK_DT_F32 ? 0 : 1,
-                       Scratch{Scratch::PROVIDED, static_cast<char*>(workspace), workspace ? workspace_bytes : 0});
+                       Scratch{Scratch::PROVIDED, static_cast<char*>(workspace), workspace ? workspace_bytes : 0, false});
 }
 
 // port_1: every wave tile (or every 16-row block) has its own signal = port_2 with maximal bar_steps
@@ -971,7 +1067,7 @@ static int launch_port_1(int dtype, const void* A, const void* Bt, const void* C
     }
     const ck::GemmTuning t{tile_dim, segment_dim_k, sa, sb, bar_step_rows_a, bar_step_rows_b,
                            tile_group_m, num_stages, num_producer_waves, num_consumer_waves, num_cus, 0};
-    return gemm_launch(dtype, A, Bt, C, D, alpha, beta, M, N, K, t, default_options(), stream, out16, Scratch{Scratch::ALLOCATE, nullptr, 0});
+    return gemm_launch(dtype, A, Bt, C, D, alpha, beta, M, N, K, t, default_options(), stream, out16, Scratch{Scratch::ALLOCATE, nullptr, 0, false});
 }
 int ckopt_gemm_shmem_tc_async_opt_port_1(int dtype, const void* A, const void* Bt, const float* C, float* D,
                                          float alpha, float beta, int M, int N, int K, int tile_dim,
@@ -996,7 +1092,7 @@ static int launch_port_0(int dtype, const void* A, const void* Bt, const void* C
                          int num_cus, void* stream, int out16) {
     const ck::GemmTuning t{tile_dim, segment_dim_k, 0, 0, tile_dim, tile_dim, tile_group_m, num_stages, num_producer_waves, num_consumer_waves,
                            num_cus, 1};
-    return gemm_launch(dtype, A, Bt, C, D, alpha, beta, M, N, K, t, default_options(), stream, out16, Scratch{Scratch::ALLOCATE, nullptr, 0});
+    return gemm_launch(dtype, A, Bt, C, D, alpha, beta, M, N, K, t, default_options(), stream, out16, Scratch{Scratch::ALLOCATE, nullptr, 0, false});
 }
 int ckopt_gemm_shmem_tc_async_opt_port_0(int dtype, const void* A, const void* Bt, const float* C, float* D,
                                          float alpha, float beta, int M, int N, int K, int tile_dim,
@@ -1068,23 +1164,38 @@ int ckopt_suggest_gemm_tuning(int M, int N, int K, int num_cus, int* tuning_out)
         else if (tiles(128) * 2 >= num_cus) pick = fused_128;
     } else {
         // the shortest of three estimates: the straight-line kernel as the launcher would run it on aligned operands (its K,
-        // tile width and slice count: launch_k, stream_plan), the ring kernel on 128 tiles, and what the tuple of 64
-        // tiles runs (small_plan). The straight-line estimate leaves out the launch itself, 1.5 us in the small-product one.
-        // Where the straight-line kernel would cut K, its tuple is weighed against the ring kernels alone, as before there was a small-product
-        // kernel, though that is shorter on many such sizes (1000^2 x 4096: 18.5 us against 37).
+        // tile width and slice count: launch_k, stream_plan), what the tuple of 128 tiles runs, and what the tuple of 64
+        // tiles runs (small_plan). The straight-line estimate leaves out the launch itself, 1.5 us in the others.
         const GemmTuning st{256, 32, 0, 0, 256, 256, 4, 5, 0, 8, num_cus, 0};
         const StreamPlan straight = stream_plan(M, N, launch_k(K, true, st, opt), num_cus, opt);
         // (Measured per 128 of K: 1.4 us for a 128 x 128 tile, 0.65 us for a 64 x 64 tile, about 4 us per round besides.)
         auto general_us = [&](int t, double seg_us) { return std::ceil((double)tiles(t) / num_cus) * ((double)K / 128.0 * seg_us + 4.0); };
         const double us_128 = general_us(128, 1.4), us_64 = general_us(64, 0.65);
         const int dev_cus = device_cus();
-        const SmallPlan small = small_plan(M, N, K, 16, dev_cus);
+        const bool whole_device = num_cus >= dev_cus;
+        const double call_us = opt[OPT_SPLIT_K] == 1 ? KEPT_CALL_US : 0.0;
+        const SmallPlan small = small_plan(M, N, K, 16, dev_cus, call_us);
+        const bool mid_runs = whole_device && !needs_copies(K, true) && mid_is_shorter(M, N, K, dev_cus);
+        const MidPlan mid = mid_plan(M, N, K, dev_cus, call_us);
         // Rows off a line, which the estimate leaves out: 1.3 to 2.2 times on 256 x 128 tiles (2048^2 x 4104 67.6 us against 49.0 on the tuple of 128
         // tiles and 79.1 on the one of 64; 8896 x 253 x 12808 219 / 141 / 172), 1.1 on wider ones and on a short K.
         const double straight_us = straight.us * (K >= 2048 && K % 8 == 0 && K % 64 != 0 && straight.tile_n == 128 ? 1.4 : 1.0);
         auto launched_us = [&](double us) { return needs_copies(K, true) ? behind_copies_us(us, M, N, K) : us; };
-        if (straight.slices > 1 && straight_us <= us_128 && straight_us <= us_64) pick = straight_line;
-        else if (small.direct && num_cus >= dev_cus && small.us < 0.93 * launched_us(us_128) && small.us < 0.93 * launched_us(straight_us + 1.5)) pick = fused_64;
+        // a sliced straight-line launch allocates its planes
+        const double straight_call_us = launched_us(straight.slices > 1 ? std::max(KEPT_CALL_US, straight_us + 1.5) : straight_us + 1.5);
+        const double mid_call_us = mid_runs ? mid.us : launched_us(us_128), small_call_us = whole_device ? small.us : 1e30;
+        // 64 tiles against 128: less per tile, no scratch memory where the other needs some, and off a line in place of a kernel that reads every line twice
+        const double keep_64 = K % 64 ? 1.0 / 0.8 : mid.slices > 1 && small.slices == 1 ? 1.0 / 0.9 : 0.93;
+        const bool prefer_64 = small_call_us < (mid_runs ? keep_64 : 0.93) * mid_call_us;
+        // Where the straight-line kernel cuts K the others have to be clearly shorter, above all up to K 8192, where its launches are short: programs keep a
+        // workspace for that tuple, and the estimates are coarse there (1024^2 x 8192 31.0 on it, 28 and 29 on the others; 512^2 x 8192 21.6 and 15.2, 300 x 520 x 4090
+        // 27.7 and 11.8; but 213 x 320 x 36672 131 and 20, 233 x 128 x 53667 541 and 26).
+        const bool cut = straight.slices > 1 && straight_us <= us_128 && straight_us <= us_64;
+        const double clearly = K > 8192 ? 0.85 : needs_copies(K, true) ? 0.35 : 0.6;
+        const double bar = (cut ? clearly : 0.93) * straight_call_us;
+        if (prefer_64 && small_call_us < bar) pick = fused_64;
+        else if (mid_runs && mid_call_us < bar) pick = fused_128;
+        else if (cut) pick = straight_line;
         else if (straight_us <= us_128 && straight_us <= us_64) pick = straight_line;
         else if (us_128 <= us_64) pick = fused_128;
     }

@@ -105,6 +105,9 @@ CK_HD int xcd_tile(int block, int tiles, int num_xcd) {
     return x * (tiles / num_xcd) + (x < longer ? x : longer) + block / num_xcd;
 }
 
+// First of the `units` units of K that belong to slice s of S (slices differ by at most one unit; S <= units: none is empty).
+CK_HD int slice_begin(int units, int s, int S) { return (int)((int64_t)units * s / S); }
+
 // ---- LDS ring layout ----------------------------------------------------------------------------
 // One stage of one operand is tile_dim rows of segment_dim_k 16-bit elements, stored row-major with
 // NO padding (a direct-to-LDS wave load writes 64 lanes x 16 B linearly), and the 16-byte chunks of

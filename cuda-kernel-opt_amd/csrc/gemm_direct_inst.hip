@@ -1,12 +1,12 @@
-// Launcher of the small-product kernel (one instance per element type, tile and operand alignment).
+// Launcher of the small-product kernel (one instance per element type, tile, operand alignment, and with K slices or without).
 #include <atomic>
 #include "gemm_direct_kernel.hip.h"
 
 namespace ck {
 
-template <typename DT, int WT, int DEPTH, bool EVEN>
-static hipError_t direct_launch_one(hipStream_t stream, const GemmArgs& a) {
-    auto kern = gemm_direct_kernel<DT, WT, DEPTH, EVEN>;
+template <typename DT, int WT, int DEPTH, bool EVEN, bool SLICED>
+static hipError_t direct_launch_as(hipStream_t stream, const GemmArgs& a) {
+    auto kern = gemm_direct_kernel<DT, WT, DEPTH, EVEN, SLICED>;
     constexpr int lds = direct_lds_bytes(WT * 16);
     if (lds > 64 * 1024) {
         static std::atomic<bool> opted[64] = {};   // (threads may launch at once; setting the attribute twice is harmless)
@@ -19,8 +19,12 @@ static hipError_t direct_launch_one(hipStream_t stream, const GemmArgs& a) {
             if (dev >= 0 && dev < 64) opted[dev].store(true, std::memory_order_release);
         }
     }
-    hipLaunchKernelGGL(kern, dim3((unsigned)(a.tiles_m * a.tiles_n)), dim3(DIRECT_WAVES * WAVE), lds, stream, a);
+    hipLaunchKernelGGL(kern, dim3((unsigned)(a.tiles_m * a.tiles_n * a.split_k)), dim3(DIRECT_WAVES * WAVE), lds, stream, a);
     return hipGetLastError();
+}
+template <typename DT, int WT, int DEPTH, bool EVEN>
+static hipError_t direct_launch_one(hipStream_t stream, const GemmArgs& a) {
+    return a.split_k > 1 ? direct_launch_as<DT, WT, DEPTH, EVEN, true>(stream, a) : direct_launch_as<DT, WT, DEPTH, EVEN, false>(stream, a);
 }
 template <typename DT>
 static hipError_t direct_launch(int tile, bool even, hipStream_t stream, const GemmArgs& a) {

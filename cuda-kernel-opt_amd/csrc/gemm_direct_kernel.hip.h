@@ -27,8 +27,9 @@ constexpr int DIRECT_ROW_BYTES = DIRECT_UNIT_K * 2;
 // dynamic LDS for tiles of T x T: per wave one unit of both operands; afterwards its partial tile
 constexpr int direct_lds_bytes(int T) { return DIRECT_WAVES * 2 * T * DIRECT_ROW_BYTES; }
 
-// WT: 16 x 16 blocks per tile edge (2: 32 x 32 tiles, 4: 64 x 64 tiles); DEPTH: units in flight per wave
-template <typename DT, int WT, int DEPTH, bool EVEN>
+// WT: 16 x 16 blocks per tile edge (2: 32 x 32 tiles, 4: 64 x 64 tiles); DEPTH: units in flight per wave; SLICED: work items are (tile, K slice), an
+// instance of its own because its divisions and bounds cost a call of 6 to 10 us 0.1 to 0.25 us
+template <typename DT, int WT, int DEPTH, bool EVEN, bool SLICED>
 __global__ __launch_bounds__(DIRECT_WAVES * 64) void gemm_direct_kernel(const GemmArgs g) {
     constexpr int T = WT * 16;
     constexpr int BLOCKS = WT * WT;
@@ -40,7 +41,9 @@ __global__ __launch_bounds__(DIRECT_WAVES * 64) void gemm_direct_kernel(const Ge
     const int lane = threadIdx.x & 63;
     const unsigned long long clk0 = clock64(), wall0 = wall_clock64();
 
-    const TileRC rc = tile_order(g.tiles_m, g.tiles_n, g.tile_group_m, xcd_tile(blockIdx.x, gridDim.x, g.num_xcd));
+    // work items: the tiles of the first K slice, then those of the second ...
+    const int item = xcd_tile(blockIdx.x, gridDim.x, g.num_xcd), tiles = g.tiles_m * g.tiles_n, slice = SLICED ? item / tiles : 0;
+    const TileRC rc = tile_order(g.tiles_m, g.tiles_n, g.tile_group_m, item - slice * tiles);
     const int row_a = rc.row * T, row_b = rc.col * T;
     const int64_t pitch = (int64_t)g.K * 2;
     const char* base_a = (const char*)g.A + row_a * pitch;
@@ -89,10 +92,16 @@ __global__ __launch_bounds__(DIRECT_WAVES * 64) void gemm_direct_kernel(const Ge
             fetch_chunk(base_b, off_b[l] + k, sel_b[l], f.b[l], f.head_b[l]);
         }
     };
-    // Whole units w, w + 8, ... belong to wave w; the one with the end of K comes first in the wave that it falls to. (EVEN
+    // Of a slice's whole units, the w-th, w + 8-th, ... belong to wave w; the one with the end of K comes first in the wave that it falls to. (EVEN
     // false: also a K that is a multiple of 64 ends in such a unit, since the element behind a chunk is read as well.)
     const int whole = EVEN ? g.K / DIRECT_UNIT_K : (g.K - 1) / DIRECT_UNIT_K;
-    const bool has_end = whole * DIRECT_UNIT_K != g.K && whole % DIRECT_WAVES == wave;
+    const int units = whole + (whole * DIRECT_UNIT_K != g.K);
+    int begin = 0, end = units;
+    if constexpr (SLICED) {
+        begin = slice_begin(units, slice, g.split_k);
+        end = slice_begin(units, slice + 1, g.split_k);
+    }
+    const bool has_end = end > whole && (whole - begin) % DIRECT_WAVES == wave;
     // In the unit with the end of K, chunks that reach past a row's end are read so that they end with the row (K >= 8), and
     // mask_end drops what lies in front of them and fills up with zeros. Two steps, so that nothing waits for the loads
     // between them.
@@ -169,8 +178,8 @@ __global__ __launch_bounds__(DIRECT_WAVES * 64) void gemm_direct_kernel(const Ge
         wave_order();
     };
 
-    const int first = has_end ? wave - DIRECT_WAVES : wave;
-    const int mine = first < whole ? (whole - first + DIRECT_WAVES - 1) / DIRECT_WAVES : 0;   // units of this wave
+    const int first = begin + (has_end ? wave - DIRECT_WAVES : wave), stop = end < whole ? end : whole;
+    const int mine = first < stop ? (stop - first + DIRECT_WAVES - 1) / DIRECT_WAVES : 0;   // units of this wave
     Unit f[DEPTH];
     auto fetch_first = [&]() __attribute__((always_inline)) {
         if (has_end) fetch_end(f[0]);
@@ -214,7 +223,9 @@ __global__ __launch_bounds__(DIRECT_WAVES * 64) void gemm_direct_kernel(const Ge
 
     // The partial tiles, each in its wave's buffer (a wave writes it behind its own last fragment reads), added in the waves'
     // order by the waves that had a share of K.
-    const int units = (g.K + DIRECT_UNIT_K - 1) / DIRECT_UNIT_K, waves = units < DIRECT_WAVES ? units : DIRECT_WAVES;
+    const int waves = end - begin < DIRECT_WAVES ? end - begin : DIRECT_WAVES;
+    GemmArgs go = g;
+    if constexpr (SLICED) go.D = g.D + (int64_t)slice * g.M * g.N;   // fp32 planes of a workspace
     const bool vec_cols = g.vec_store && (rc.col + 1) * T <= g.N;
 #pragma unroll
     for (int b = 0; b < BLOCKS; ++b) *(CK_LDS f32x4*)(buffer + b * 1024 + lane * 16) = acc[b / WT][b % WT];
@@ -223,7 +234,7 @@ __global__ __launch_bounds__(DIRECT_WAVES * 64) void gemm_direct_kernel(const Ge
         const CK_LDS char* at = (const CK_LDS char*)ck_smem + b * 1024 + lane * 16;
         f32x4 sum = *(const CK_LDS f32x4*)at;
         for (int w = 1; w < waves; ++w) sum += *(const CK_LDS f32x4*)(at + w * 2 * OPERAND);
-        epilogue_block<DT>(g, row_a + b / WT * 16 + lr, row_b + b % WT * 16 + lg * 4, sum, vec_cols);
+        epilogue_block<DT>(go, row_a + b / WT * 16 + lr, row_b + b % WT * 16 + lg * 4, sum, vec_cols);
     }
 
     if (blockIdx.x == 0 && threadIdx.x == blockDim.x - 1) {

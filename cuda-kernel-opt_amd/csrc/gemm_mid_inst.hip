@@ -16,7 +16,7 @@ static hipError_t mid_launch(hipStream_t stream, const GemmArgs& a) {
         if (e != hipSuccess) return e;
         if (dev >= 0 && dev < 64) opted[dev].store(true, std::memory_order_release);
     }
-    hipLaunchKernelGGL(kern, dim3((unsigned)(a.tiles_m * a.tiles_n)), dim3(512), MID_LDS_BYTES, stream, a);
+    hipLaunchKernelGGL(kern, dim3((unsigned)(a.tiles_m * a.tiles_n * a.split_k)), dim3(512), MID_LDS_BYTES, stream, a);
     return hipGetLastError();
 }
 template <typename DT>

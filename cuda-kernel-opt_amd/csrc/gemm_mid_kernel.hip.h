@@ -52,16 +52,16 @@ __device__ __forceinline__ f32x4 row_c(const GemmArgs& g, int m, int n) {
     return c;
 }
 template <typename DT>
-__device__ __forceinline__ void store_row(const GemmArgs& g, int m, int n, f32x4 sum, f32x4 c) {
+__device__ __forceinline__ void store_row(const GemmArgs& g, float* D, int m, int n, f32x4 sum, f32x4 c) {
     if (m >= g.M || n >= g.N) return;
     const int64_t off = (int64_t)m * g.N + n;
     f32x4 v = sum * g.alpha;
     if (g.beta != 0.f) v += c * g.beta;
-    unsigned short* d16 = (unsigned short*)g.D;
+    unsigned short* d16 = (unsigned short*)D;
     if (n + 4 <= g.N) {
         if (!g.out16) {
-            if (g.nt_store) store_b128_nt(g.D + off, __builtin_bit_cast(u32x4, v));
-            else *(f32x4_u*)(g.D + off) = v;
+            if (g.nt_store) store_b128_nt(D + off, __builtin_bit_cast(u32x4, v));
+            else *(f32x4_u*)(D + off) = v;
         } else {
             const u32x2 o = {(uint32_t)Out16<DT>::store(v[0]) | (uint32_t)Out16<DT>::store(v[1]) << 16, (uint32_t)Out16<DT>::store(v[2]) | (uint32_t)Out16<DT>::store(v[3]) << 16};
             if (g.nt_store) store_b64_nt(d16 + off, o);
@@ -73,7 +73,7 @@ __device__ __forceinline__ void store_row(const GemmArgs& g, int m, int n, f32x4
     for (int e = 0; e < 3; ++e)
         if (n + e < g.N) {
             if (g.out16) d16[off + e] = Out16<DT>::store(v[e]);
-            else g.D[off + e] = v[e];
+            else D[off + e] = v[e];
         }
 }
 
@@ -87,7 +87,9 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(const GemmArgs g) {
     const int lane = threadIdx.x & 63;
     const unsigned long long clk0 = clock64(), wall0 = wall_clock64();
 
-    const TileRC rc = tile_order(g.tiles_m, g.tiles_n, g.tile_group_m, xcd_tile(blockIdx.x, gridDim.x, g.num_xcd));
+    // work items: the tiles of the first K slice, then those of the second ...; an XCD's run of items shares operand panels
+    const int item = xcd_tile(blockIdx.x, gridDim.x, g.num_xcd), tiles = g.tiles_m * g.tiles_n, slice = g.split_k > 1 ? __builtin_amdgcn_readfirstlane(item / tiles) : 0;
+    const TileRC rc = tile_order(g.tiles_m, g.tiles_n, g.tile_group_m, item - slice * tiles);
     const int row_a = __builtin_amdgcn_readfirstlane(rc.row * MID_TILE), row_b = __builtin_amdgcn_readfirstlane(rc.col * MID_TILE);
     const uint32_t pitch = (uint32_t)g.K * 2u;
     const int rows_a = g.M - row_a < MID_TILE ? g.M - row_a : MID_TILE, rows_b = g.N - row_b < MID_TILE ? g.N - row_b : MID_TILE;
@@ -104,8 +106,14 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(const GemmArgs g) {
         off[j] = (uint32_t)row * pitch + (uint32_t)chunk * CHUNK_BYTES;
         chunk_k[j] = chunk * CHUNK_ELEMS;
     }
-    const int slabs = (g.K + MID_SLAB_K - 1) / MID_SLAB_K;
-    int ld_slab = (int)(blockIdx.x % (unsigned)g.num_xcd) % slabs, ld_left = slabs, ld_stage = 0;
+    const int all = (g.K + MID_SLAB_K - 1) / MID_SLAB_K;
+    int begin = 0, end = all;
+    if (g.split_k > 1) {
+        begin = __builtin_amdgcn_readfirstlane(slice_begin(all, slice, g.split_k));
+        end = __builtin_amdgcn_readfirstlane(slice_begin(all, slice + 1, g.split_k));
+    }
+    const int slabs = end - begin;
+    int ld_slab = begin + (int)(blockIdx.x % (unsigned)g.num_xcd) % slabs, ld_left = slabs, ld_stage = 0;
     auto load = [&](int i) __attribute__((always_inline)) {   // 0, 1: A; 2, 3: Bt
         uint32_t voff = off[i % 2];
         // (beyond every descriptor's range, which is below 2^31)
@@ -115,7 +123,7 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(const GemmArgs g) {
     };
     // (behind the last slab the loads go on, for the count of those in flight, with descriptors of no bytes)
     auto next_slab = [&]() __attribute__((always_inline)) {
-        ld_slab = ld_slab + 1 == slabs ? 0 : ld_slab + 1;
+        ld_slab = ld_slab + 1 == end ? begin : ld_slab + 1;
         if (--ld_left <= 0) { rsrc_a[2] = rsrc_b[2] = 0; ld_slab = 0; }
         ld_stage = ld_stage + 1 == MID_STAGES ? 0 : ld_stage + 1;
     };
@@ -199,11 +207,12 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(const GemmArgs g) {
     for (int t = 0; t < 8; ++t) c[t] = row_c<DT>(g, m0 + t * 4, n0);
     wait_lgkmcnt0();
     wg_barrier();
+    float* const plane = g.D + (int64_t)slice * g.M * g.N;   // (more than one slice: fp32 planes of a workspace)
     const CK_LDS char* first = out + wave % 4 * MID_OUT_WAVE + (group * 32 + lg) * MID_OUT_ROW + lr * 16;
 #pragma unroll
     for (int t = 0; t < 8; ++t) {
         const CK_LDS char* at = first + t * 4 * MID_OUT_ROW;
-        store_row<DT>(g, m0 + t * 4, n0, *(const CK_LDS f32x4*)at + *(const CK_LDS f32x4*)(at + 4 * MID_OUT_WAVE), c[t]);
+        store_row<DT>(g, plane, m0 + t * 4, n0, *(const CK_LDS f32x4*)at + *(const CK_LDS f32x4*)(at + 4 * MID_OUT_WAVE), c[t]);
     }
 
     if (blockIdx.x == 0 && threadIdx.x == blockDim.x - 1) {

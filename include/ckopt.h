@@ -89,7 +89,8 @@ int ckopt_gemm_shmem_tc_async_opt_port_2_lp(int dtype, const void* A, const void
  * needs under the process's current options (0: none; negative: the error the launch would give);
  * operands_aligned != 0 promises A and Bt on 16-byte boundaries. A workspace that is too small gives
  * CKOPT_ERR_TOO_LARGE and D is not written, also where the kernel that runs makes no use of it (gemm_direct_kernel on rows off a 16-byte
- * boundary); nothing is allocated in any case. */
+ * boundary); nothing is allocated in any case. Except for the K slices of gemm_mid_kernel and gemm_direct_kernel (few tiles, a deep K): the query
+ * names their planes, and a workspace without room for them, NULL included, leaves one pass over all of K. */
 int64_t ckopt_gemm_workspace_bytes(int M, int N, int K, int operands_aligned, int tile_dim, int segment_dim_k, int bar_steps_a,
                                    int bar_steps_b, int bar_step_rows_a, int bar_step_rows_b, int tile_group_m, int num_stages,
                                    int num_producer_waves, int num_consumer_waves, int num_cus);
@@ -101,7 +102,8 @@ int64_t ckopt_gemm_workspace_bytes(int M, int N, int K, int operands_aligned, in
  * plan_out[2] = number of K slices (1: no split-K); plan_out[3] = 1 if A and Bt are first copied into zero-padded rows;
  * plan_out[4] = number of tiles that are cut into those slices (all of them when there are fewer tiles than num_cus; the
  * tiles of the partly filled last round otherwise; 0 without slices); plan_out[5] = 1 if the slices are added inside the
- * kernel, 0 if by a second kernel; plan_out[6] = workgroups of the straight-line kernel's grid. plan_out points at 7 ints.
+ * kernel, 0 if by a second kernel (gemm_mid_kernel and gemm_direct_kernel: all of their tiles, where a launch finds room for the planes without an
+ * allocation); plan_out[6] = workgroups of the straight-line kernel's grid. plan_out points at 7 ints.
  * Returns CKOPT_OK or the error the launch would give. No reference counterpart (its launcher has one kernel form). */
 int ckopt_gemm_launch_plan(int M, int N, int K, int operands_aligned, int tile_dim, int segment_dim_k, int bar_steps_a, int bar_steps_b,
                            int bar_step_rows_a, int bar_step_rows_b, int tile_group_m, int num_stages, int num_producer_waves,
@@ -190,7 +192,7 @@ enum {
     CKOPT_KERNEL_FUSED = 0,   /* gemm_fused_kernel: LDS ring, no producer waves */
     CKOPT_KERNEL_STREAM = 1,  /* gemm_stream_kernel: the straight-line kernel */
     CKOPT_KERNEL_DIRECT = 2,  /* gemm_direct_kernel: small products */
-    CKOPT_KERNEL_MID = 3,     /* gemm_mid_kernel: 128 x 128 tiles staged through registers */
+    CKOPT_KERNEL_MID = 3,     /* gemm_mid_kernel: 128 x 128 tiles, a ring of five 64-deep slabs */
     CKOPT_KERNEL_SYNC = 4,    /* gemm_sync_kernel: one stage */
     CKOPT_KERNEL_PCB = 5,     /* gemm_pcb_kernel: producer waves, workgroup barrier */
     CKOPT_KERNEL_PC = 6       /* gemm_pc_kernel: producer waves, LDS counters */
@@ -303,7 +305,9 @@ int ckopt_last_launch_clocks(void* stream, uint64_t* shader_cycles, uint64_t* re
  *        the shortest time - loop bodies at the rate the active CUs sustain, the store burst of every round, the
  *        reduction pass (e.g. 64 tiles, K 32768: 4 slices; 128 tiles, K 16384: 2; 128 tiles, K 4096: none); the
  *        slices' partial products go to scratch memory (slices * M * N * 4 bytes) and a second kernel adds them in
- *        slice order and applies alpha, beta and the output type. 0: never. 2..16: that many slices whenever legal.
+ *        slice order and applies alpha, beta and the output type. 0: never. 2..16: that many slices whenever legal. With 1 the suggested
+ *        tuples of 64 and 128 tiles cut K too, into up to 64 slices of at least 512, where few tiles leave the device idle; not on a stream that
+ *        records a graph, not in the entry point that allocates nothing, and on other streams than the default one only in longer calls.
  * key 8: schedule of the straight-line kernel. 1 (default): a workgroup barrier in every k-step, the loads of a loop
  *        body spread over both (three k-steps to land); 0: one barrier per two k-steps, all loads behind it (two
  *        k-steps to land) - at 8192^3 on random operand values 1.5 % faster on one device and 0.7 % slower on another,

@@ -1633,6 +1633,77 @@ def test_ring_of_slabs_at_its_shortest_and_past_a_row_end(ck, bf16):
     assert ck.device_status() == 0
 
 
+@pytest.mark.parametrize("bf16", [False, True])
+def test_k_slices_of_the_smaller_tuples_exact(ck, bf16):
+    """(tile, K slice) items of gemm_mid_kernel and gemm_direct_kernel and the pass that adds their planes, exact on small integers (sums below
+    2^24): K that ends inside a slab and inside a unit of 64, odd K read in place, M x N that four does not divide, fp32 and 16-bit C and D,
+    a guard behind D; and the same bits from a provided workspace of the queried size, rows of NaN in it."""
+    dtype, tdt = (ck.DT_BF16, torch.bfloat16) if bf16 else (ck.DT_F16, torch.float16)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(29)
+    for t, M, N, K in [(MID_TUPLE, 213, 320, 36672), (MID_TUPLE, 131, 257, 20008), (MID_TUPLE, 512, 512, 28608), (MID_TUPLE, 960, 1424, 7808), (MID_TUPLE, 77, 85, 30000),
+                       (SMALL_TUPLE, 64, 192, 14080), (SMALL_TUPLE, 61, 187, 14081), (SMALL_TUPLE, 233, 128, 25667), (SMALL_TUPLE, 35, 33, 16390), (SMALL_TUPLE, 512, 512, 16448)]:
+        assert ck.gemm_launch_plan(M, N, K, True, *t)["k_slices"] > 1, (M, N, K)
+        a = torch.randint(-2, 3, (M, K), device="cuda", generator=gen).to(tdt)
+        b = torch.randint(-2, 3, (N, K), device="cuda", generator=gen).to(tdt)
+        exact = a.cpu().float() @ b.cpu().float().t()
+        c = torch.randint(-8, 9, (M, N), device="cuda", generator=gen).float()
+        d = torch.full((M * N + 64,), float("nan"), dtype=torch.float32, device="cuda")
+        ck.gemm_shmem_tc_async_opt_port(dtype, a, b, c, d, 2.0, -3.0, M, N, K, *t)
+        assert torch.equal(d[:M * N].view(M, N).cpu(), 2 * exact - 3 * c.cpu()), (M, N, K)
+        assert torch.isnan(d[M * N:]).all()
+        d16 = torch.full((M * N + 64,), float("nan"), dtype=tdt, device="cuda")
+        ck.gemm_shmem_tc_async_opt_port_lp(dtype, a, b, c.to(tdt), d16, 1.0, 1.0, M, N, K, *t)
+        assert torch.equal(d16[:M * N].view(M, N).cpu(), (exact + c.cpu()).to(tdt)), (M, N, K)
+        assert torch.isnan(d16[M * N:]).all()
+        need = ck.gemm_workspace_bytes(M, N, K, True, *t)
+        ws = torch.full((need + 512,), 255, dtype=torch.uint8, device="cuda")
+        x, y = (torch.randn((r, K), device="cuda", generator=gen).to(tdt) for r in (M, N))
+        want, got = (torch.empty((M, N), dtype=torch.float32, device="cuda") for _ in range(2))
+        ck.gemm_shmem_tc_async_opt_port(dtype, x, y, None, want, 1.0, 0.0, M, N, K, *t)
+        ck.gemm_shmem_tc_async_opt_port_ws(dtype, ck.DT_F32, x, y, None, got, 1.0, 0.0, M, N, K, *t, workspace=ws, workspace_bytes=need)
+        assert torch.equal(want, got) and (ws[need:] == 255).all(), (M, N, K)
+    assert ck.device_status() == 0
+
+
+def test_k_slices_only_where_there_is_room_for_their_planes(ck):
+    """What was accepted without scratch memory stays accepted: no workspace or one too small, the entry point that allocates nothing, a stream that
+    records a graph and a stream of one's own all compute the same product (small integers: exact), whether K is cut or not."""
+    M, N, K = 213, 320, 36672
+    assert ck.gemm_launch_plan(M, N, K, True, *MID_TUPLE)["k_slices"] > 1
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(31)
+    a = torch.randint(-2, 3, (M, K), device="cuda", generator=gen).half()
+    b = torch.randint(-2, 3, (N, K), device="cuda", generator=gen).half()
+    exact = (a.cpu().float() @ b.cpu().float().t()).cuda()
+    d = torch.empty((M, N), dtype=torch.float32, device="cuda")
+    ws = torch.empty(4096, dtype=torch.uint8, device="cuda")
+    for kw in (dict(workspace=None, workspace_bytes=0), dict(workspace=ws, workspace_bytes=4096)):
+        d.fill_(float("nan"))
+        ck.gemm_shmem_tc_async_opt_port_ws(ck.DT_F16, ck.DT_F32, a, b, None, d, 1.0, 0.0, M, N, K, *MID_TUPLE, **kw)
+        assert torch.equal(d, exact)
+    d.fill_(float("nan"))
+    ck.gemm_shmem_tc_async_opt_port_noalloc(ck.DT_F16, a, b, None, d, 1.0, 0.0, M, N, K, *MID_TUPLE)
+    assert torch.equal(d, exact)
+    side = torch.cuda.Stream()
+    d.fill_(float("nan"))
+    side.wait_stream(torch.cuda.current_stream())
+    ck.gemm_shmem_tc_async_opt_port(ck.DT_F16, a, b, None, d, 1.0, 0.0, M, N, K, *MID_TUPLE, side)
+    side.synchronize()
+    assert torch.equal(d, exact)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        ck.gemm_shmem_tc_async_opt_port(ck.DT_F16, a, b, None, d, 1.0, 0.0, M, N, K, *MID_TUPLE, torch.cuda.current_stream())
+    for _ in range(3):
+        d.fill_(float("nan"))
+        ck.gemm_shmem_tc_async_opt_port(ck.DT_F16, b, a, None, torch.empty((N, M), device="cuda"), 1.0, 0.0, N, M, K, *MID_TUPLE)   # eager, with slices
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(d, exact)
+    assert ck.device_status() == 0
+
+
 def test_kept_scratch_blocks_with_threads_and_given_back(ck):
     """Launches of several host threads on the default stream, with scratch memory of different sizes (K planes; operand copies and planes): each
     call has a block to itself, and every product is exact. Afterwards the blocks are given back, and the next call takes new ones."""

@@ -716,3 +716,43 @@ def test_kernels_of_the_smaller_tuples_keep_every_value_in_registers(tmp_path):
         assert sizes and set(sizes) == {"0"} and all(int(v) <= 256 for v in registers), (name, sizes, registers)
         seen += len(sizes)
     assert seen >= 10   # four instances of the small-product kernel per element type, one of the other
+
+
+def test_k_slices_of_the_smaller_tuples(ck, tmp_path):
+    # few tiles and a deep K: (tile, slice) items; the query names the planes, and no more than the copies for an odd K that is read in place
+    small, mid = (64, 128, 0, 0, 64, 64, 4, 4, 0, 8, 256), (128, 128, 0, 0, 128, 128, 4, 2, 0, 8, 256)
+    up = lambda n: (n + 255) // 256 * 256
+    for t, kernel, (M, N, K) in ((mid, "gemm_mid_kernel", (213, 320, 36672)), (mid, "gemm_mid_kernel", (512, 512, 28608)), (mid, "gemm_mid_kernel", (300, 300, 30000)),
+                                 (small, "gemm_direct_kernel", (64, 192, 14080)), (small, "gemm_direct_kernel", (233, 128, 53667))):
+        p = ck.gemm_launch_plan(M, N, K, True, *t)
+        assert ck.gemm_launch_kernel(M, N, K, True, *t) == kernel and p["k_slices"] > 1 and not p["operand_copies"], (M, N, K, p)
+        planes = up(p["k_slices"] * M * N * 4)
+        assert ck.gemm_workspace_bytes(M, N, K, True, *t) == 256 + (max(planes, up((M + N) * ((K + 7) // 8 * 8) * 2)) if K % 8 else planes)
+        for n in (0, 2, 4):   # the switch: never, and only the straight-line kernel's count
+            assert ck.gemm_launch_plan(M, N, K, True, *t, options=ck.launch_options(split_k=n))["k_slices"] == 1
+        assert ck.gemm_launch_plan(M, N, K, True, *t[:-1], 40)["k_slices"] == 1   # (fewer CUs than the device: the ring kernel)
+    # suggested where the straight-line kernel would take clearly longer
+    for s, tile in (((213, 320, 36672), 128), ((233, 128, 53667), 64), ((64, 192, 14080), 64), ((512, 512, 8192), 256), ((2048, 2048, 32768), 256)):
+        assert ck.suggest_gemm_tuning(*s)["tile_dim"] == tile, s
+    # short calls, many tiles: none
+    for t in (small, mid):
+        for s in ((200, 136, 1001), (512, 512, 512), (1024, 1024, 1024), (2048, 2048, 2048), (4096, 4096, 8192)):
+            assert ck.gemm_launch_plan(*s, True, *t)["k_slices"] == 1, s
+    # the units of K fall to the slices without a gap, and to every one of them
+    import subprocess
+    src = tmp_path / "slices.cpp"
+    src.write_text('''#include "ck_common.h"
+int main() {
+    for (int units = 1; units < 700; ++units)
+        for (int S = 1; S <= 64 && S <= units; ++S) {
+            if (ck::slice_begin(units, 0, S) != 0 || ck::slice_begin(units, S, S) != units) return 1;
+            for (int s = 0; s < S; ++s) {
+                const int n = ck::slice_begin(units, s + 1, S) - ck::slice_begin(units, s, S);
+                if (n < units / S || n > units / S + 1) return 2;
+            }
+        }
+    return ck::slice_begin(1 << 25, 63, 64) == (int)((int64_t)(1 << 25) * 63 / 64) ? 0 : 3;
+}''')
+    exe = tmp_path / "slices"
+    subprocess.run(["g++", "-std=c++17", "-I", os.path.join(ROOT, "cuda-kernel-opt_amd", "csrc"), str(src), "-o", str(exe)], check=True, timeout=120)
+    assert subprocess.run([str(exe)], timeout=60).returncode == 0
