@@ -766,7 +766,7 @@ hipError_t launch_items(const ck::GemmArgs& a, int slices, int dtype, Scratch sc
     if (slices <= 1) return launch(a);
     ck::GemmArgs p = a;
     p.split_k = slices;
-    p.D = static_cast<float*>(ws); p.C = nullptr; p.alpha = 1.f; p.beta = 0.f; p.out16 = 0; p.vec_store = 1; p.nt_store = 0;
+    p.D = static_cast<float*>(ws); p.C = nullptr; p.alpha = 1.f; p.beta = 0.f; p.out16 = 0; p.nt_store = 0;
     hipError_t e = launch(p);
     if (e == hipSuccess) e = add_planes(dtype, p.D, slices, count, a.C, a.D, a.alpha, a.beta, a.out16, s);
     if (!scratch_release(sc, ws, s) && e == hipSuccess) e = hipErrorUnknown;
@@ -816,14 +816,11 @@ int gemm_launch(int dtype, const void* A, const void* Bt, const void* C, void* D
     a.bar_steps_b = mode == CK_SYNC_TILE ? 0 : t.bar_steps_b;
     a.swizzle = opt[OPT_SWIZZLE];
     a.num_xcd = opt[OPT_NUM_XCD];
-    // one vector access per accumulator block: 16 bytes of fp32 need only the 4-byte alignment checked above
-    // (any N); 8 bytes of 16-bit results need their own alignment
-    a.vec_store = !out16 || ((N % 4 == 0) && !((uintptr_t)D & 7) && (beta == 0.f || !((uintptr_t)C & 7)));
     // Non-temporal stores of D pay where the stores of a row fill whole 128-byte lines; rows that start anywhere make
     // every 128-byte run straddle two lines, and only ordinary stores let the two parts meet in L2.
     const int store_policy = opt[OPT_D_STORE_POLICY];
     auto whole_lines = [](const void* base, int64_t row_bytes) { return (uintptr_t)base % LINE_BYTES == 0 && row_bytes % LINE_BYTES == 0; };
-    a.nt_store = store_policy == 1 || (store_policy == 0 && whole_lines(D, (int64_t)N * (out16 ? 2 : 4)));
+    a.nt_store = (store_policy == 1 && (!out16 || (N % 4 == 0 && !((uintptr_t)D & 7)))) || (store_policy == 0 && whole_lines(D, (int64_t)N * (out16 ? 2 : 4)));
     a.spin_limit = (uint32_t)opt[OPT_SPIN_LIMIT];
     a.prio_mode = opt[OPT_PRIO_MODE];
     a.producer_nap = opt[OPT_PRODUCER_NAP];
@@ -906,7 +903,7 @@ int gemm_launch(int dtype, const void* A, const void* Bt, const void* C, void* D
             p.split_k = plan.slices;
             p.whole_tiles = 0;
             p.split_chunk = plan.tiles % 32 == 0 ? 32 : (int)plan.tiles;
-            p.D = ws; p.C = nullptr; p.alpha = 1.f; p.beta = 0.f; p.out16 = 0; p.vec_store = 1;
+            p.D = ws; p.C = nullptr; p.alpha = 1.f; p.beta = 0.f; p.out16 = 0;
             p.nt_store = store_policy == 1 || (store_policy == 0 && whole_lines(ws, (int64_t)N * 4) && count * 4 % LINE_BYTES == 0);
             e = launch(p, plan.grid);
             if (e == hipSuccess) e = add_planes(dtype, ws, plan.slices, count, C, D, alpha, beta, out16, s);

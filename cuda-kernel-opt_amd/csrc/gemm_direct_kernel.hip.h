@@ -226,7 +226,6 @@ __global__ __launch_bounds__(DIRECT_WAVES * 64) void gemm_direct_kernel(const Ge
     const int waves = end - begin < DIRECT_WAVES ? end - begin : DIRECT_WAVES;
     GemmArgs go = g;
     if constexpr (SLICED) go.D = g.D + (int64_t)slice * g.M * g.N;   // fp32 planes of a workspace
-    const bool vec_cols = g.vec_store && (rc.col + 1) * T <= g.N;
 #pragma unroll
     for (int b = 0; b < BLOCKS; ++b) *(CK_LDS f32x4*)(buffer + b * 1024 + lane * 16) = acc[b / WT][b % WT];
     __syncthreads();
@@ -234,7 +233,7 @@ __global__ __launch_bounds__(DIRECT_WAVES * 64) void gemm_direct_kernel(const Ge
         const CK_LDS char* at = (const CK_LDS char*)ck_smem + b * 1024 + lane * 16;
         f32x4 sum = *(const CK_LDS f32x4*)at;
         for (int w = 1; w < waves; ++w) sum += *(const CK_LDS f32x4*)(at + w * 2 * OPERAND);
-        epilogue_block<DT>(go, row_a + b / WT * 16 + lr, row_b + b % WT * 16 + lg * 4, sum, vec_cols);
+        epilogue_block<DT>(go, row_a + b / WT * 16 + lr, row_b + b % WT * 16 + lg * 4, sum);
     }
 
     if (blockIdx.x == 0 && threadIdx.x == blockDim.x - 1) {

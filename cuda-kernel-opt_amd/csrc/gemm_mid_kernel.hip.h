@@ -33,7 +33,6 @@ constexpr int MID_LDS_BYTES = MID_STAGES * MID_STAGE;
 static_assert(8 * MID_OUT_WAVE <= MID_LDS_BYTES && MID_LDS_BYTES <= LDS_BYTES_PER_CU, "the partial tiles take the ring's place");
 
 // Four neighbouring results of a row, the first in column n: D = alpha * sum + beta * C. C is what row_c() fetched.
-typedef uint32_t u32x2_a2 __attribute__((ext_vector_type(2), aligned(2)));
 template <typename DT>
 __device__ __forceinline__ f32x4 row_c(const GemmArgs& g, int m, int n) {
     f32x4 c = {0.f, 0.f, 0.f, 0.f};

@@ -452,7 +452,7 @@ __global__ __launch_bounds__(512) void gemm_stream_kernel(const GemmArgs g) {
             // vec_cols: every column of the tile is inside the matrix, one vector access per block (rows past M are
             // skipped lane by lane); interior: every row as well, so every wave issues exactly the stores that the next
             // body's landing wait counts
-            const bool vec_cols = g.vec_store && (rc.col + 1) * TILE_N <= g.N;
+            const bool vec_cols = (rc.col + 1) * TILE_N <= g.N;
             const bool interior = vec_cols && (rc.row + 1) * TILE <= g.M;
             // rows of D on 128-byte lines: the stores below fill whole lines and bypass L2 retention; otherwise every
             // 128-byte run of a row straddles two lines, and ordinary stores let the halves meet in L2 (N = 4097,
@@ -541,11 +541,11 @@ __global__ __launch_bounds__(512) void gemm_stream_kernel(const GemmArgs g) {
                 const bool with_c = beta != 0.f;
                 const unsigned short* c16 = (const unsigned short*)go.C;
                 const int64_t c_lane = (int64_t)(rc.row * TILE + R * WTR * 16 + lr) * g.N + (rc.col * TILE_N + Cc * WTC * 16 + lg * 4);
-                typedef uint32_t pair_u32 __attribute__((ext_vector_type(2)));
+                typedef uint32_t pair_u32 __attribute__((ext_vector_type(2)));   // (C itself may lie on any 2-byte boundary)
                 auto fetch_c = [&](int i, int j, pair_u32 (&c)[H16_GROUP]) __attribute__((always_inline)) {
 #pragma unroll
                     for (int b = 0; b < H16_GROUP; ++b)
-                        c[b] = with_c ? *(const pair_u32*)(c16 + c_lane + (int64_t)(i * 16) * g.N + (j + b) * 16) : pair_u32{0u, 0u};
+                        c[b] = with_c ? (pair_u32)*(const u32x2_a2*)(c16 + c_lane + (int64_t)(i * 16) * g.N + (j + b) * 16) : pair_u32{0u, 0u};
                 };
                 auto scaled = [&](f32x4 x, pair_u32 c) __attribute__((always_inline)) {
                     f32x4 v = x * alpha;
@@ -600,7 +600,7 @@ __global__ __launch_bounds__(512) void gemm_stream_kernel(const GemmArgs g) {
                 for (int i = 0; i < WTR; ++i)
 #pragma unroll
                     for (int j = 0; j < WTC; ++j)
-                        epilogue_block<DT>(go, m_base + i * 16, n_base + j * 16, acc[i][j], vec_cols);
+                        epilogue_block<DT>(go, m_base + i * 16, n_base + j * 16, acc[i][j]);
             }
             return interior;
         };

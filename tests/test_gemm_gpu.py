@@ -1743,3 +1743,33 @@ def test_kept_scratch_blocks_with_threads_and_given_back(ck):
         ck.trim_scratch_pool()
         assert torch.cuda.mem_get_info()[0] >= before
     assert ck.device_status() == 0
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+def test_16_bit_c_and_d_on_any_two_byte_boundary(ck, bf16):
+    """Four 16-bit results go in one access wherever they start: every kernel, N with every remainder by four, C and D one element off each
+    other's and the operands' alignment, edge tiles. Small integers, the exact value rounded once; guards in front of D and behind it."""
+    dtype, tdt = (ck.DT_BF16, torch.bfloat16) if bf16 else (ck.DT_F16, torch.float16)
+    tuples = [(256, 32, 0, 0, 256, 256, 4, 5, 0, 8, 256), MID_TUPLE, SMALL_TUPLE, (128, 128, 0, 0, 128, 128, 4, 2, 0, 8, 40), (128, 64, 0, 0, 128, 128, 4, 1, 0, 8, 256),
+              (128, 64, 0, 0, 128, 128, 4, 3, 2, 8, 256), (256, 64, 4, 2, 64, 128, 4, 2, 2, 8, 256), (64, 64, 0, 0, 64, 64, 4, 2, 0, 4, 256)]
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(41)
+    seen = set()
+    for M, N, K in [(520, 1030, 128), (300, 517, 576), (256, 1283, 192), (33, 70, 64), (700, 512, 512), (64, 64, 8)]:
+        a = torch.randint(-2, 3, (M, K), device="cuda", generator=gen).to(tdt)
+        b = torch.randint(-2, 3, (N, K), device="cuda", generator=gen).to(tdt)
+        exact = a.cpu().float() @ b.cpu().float().t()
+        for d_off, c_off in ((0, 0), (1, 0), (0, 1), (3, 2)):
+            buf_c = torch.randint(-8, 9, (M * N + 16,), device="cuda", generator=gen).to(tdt)
+            c = buf_c[c_off:c_off + M * N].view(M, N)
+            for t in tuples:
+                for width in (0, 2, 3) if t[1] == 32 else (1,):
+                    seen.add(ck.gemm_launch_kernel(M, N, K, True, *t))
+                    buf = torch.full((M * N + 64,), float("nan"), dtype=tdt, device="cuda")
+                    d = buf[16 + d_off:16 + d_off + M * N]
+                    for beta in (0.0, -3.0):
+                        ck.gemm_shmem_tc_async_opt_port_ex(dtype, dtype, a, b, c if beta else None, d, 2.0, beta, M, N, K, *t, options=ck.launch_options(half_width=width))
+                        assert torch.equal(d.view(M, N).cpu(), (2 * exact + beta * c.cpu().float()).to(tdt)), (M, N, K, d_off, c_off, t, width, beta)
+                    assert torch.isnan(buf[:16 + d_off]).all() and torch.isnan(buf[16 + d_off + M * N:]).all()
+    assert seen >= {"gemm_stream_kernel", "gemm_mid_kernel", "gemm_direct_kernel", "gemm_fused_kernel", "gemm_sync_kernel", "gemm_pc_kernel"}
+    assert ck.device_status() == 0
