@@ -31,6 +31,7 @@
 #define CK_GEMM_PC_KERNEL_HIP_H
 
 #include <hip/hip_runtime.h>
+#include <type_traits>
 #include "ck_common.h"
 
 namespace ck {
@@ -80,7 +81,7 @@ struct GemmArgs {
     uint32_t spin_limit;
     int prio_mode;      // 0: producers at raised priority; 1: also asymmetric consumer burst priorities per SIMD pair; 2: none
     int producer_nap;   // s_sleep argument class of the producers' flag polling: 0 -> 1, 1 -> 4, 2 -> 16
-    int batched_empty_reads;  // wave-tile granularity: a producer wave reads all "empty" counters of its operand and stage once per segment
+    int batched_empty_reads;  // finer granularities: a producer wave looks at all "empty" counters of its operand and stage at once
     unsigned int* status;  // device words: [0] OR of CK_STATUS_* bits, [2..3] shader cycles and [4..5] 100 MHz
                            // ticks workgroup 0 spent in the last launch (actual-clock evidence)
 };
@@ -203,21 +204,6 @@ __device__ __forceinline__ void flag_add(uint32_t lds_addr) {
     asm volatile("s_mov_b64 exec, 1\n\tds_add_u32 %0, %1\n\ts_mov_b64 exec, -1" ::"v"(lds_addr), "v"(one) : "memory");
 }
 
-// Up to five adjacent counters in one round trip to the LDS (the reads are issued back to back and waited for once):
-// what a producer wave of the wave-tile granularity looks at once per segment instead of polling every row block's
-// counter on its own.
-__device__ __forceinline__ void flag_load5(uint32_t lds_addr, int n, uint32_t (&out)[5]) {
-    uint32_t v0, v1, v2, v3, v4;
-    const uint32_t a1 = lds_addr + (n > 1 ? 4u : 0u), a2 = lds_addr + (n > 2 ? 8u : 0u), a3 = lds_addr + (n > 3 ? 12u : 0u),
-                   a4 = lds_addr + (n > 4 ? 16u : 0u);
-    asm volatile("ds_read_b32 %0, %5\n\tds_read_b32 %1, %6\n\tds_read_b32 %2, %7\n\tds_read_b32 %3, %8\n\tds_read_b32 %4, %9\n\ts_waitcnt lgkmcnt(0)"
-                 : "=&v"(v0), "=&v"(v1), "=&v"(v2), "=&v"(v3), "=&v"(v4)
-                 : "v"(lds_addr), "v"(a1), "v"(a2), "v"(a3), "v"(a4)
-                 : "memory");
-    out[0] = __builtin_amdgcn_readfirstlane(v0); out[1] = __builtin_amdgcn_readfirstlane(v1); out[2] = __builtin_amdgcn_readfirstlane(v2);
-    out[3] = __builtin_amdgcn_readfirstlane(v3); out[4] = __builtin_amdgcn_readfirstlane(v4);
-}
-
 // Counter read whose answer is needed later: a relaxed workgroup-scope atomic load compiles to a
 // plain ds_read_b32 that the compiler's wait-count pass tracks, so the wave keeps issuing and the
 // (counted) wait lands at the first use of the value. The read must stay visible to the compiler:
@@ -337,62 +323,108 @@ __device__ __forceinline__ void producer_wait(uint32_t addr, uint32_t target, Si
 // IS_A selects the operand: A producers walk wave-tile rows, Bt producers wave-tile columns.
 // PX = producer waves on this operand; wave q issues the wave loads E with E % PX == q.
 //
-// Address generation is kept off the vector ALU. A wave load E covers rows [E*RPI, (E+1)*RPI) of
-// the operand stage; lane (lane_row, lane_slot) fetches the 16-byte chunk that belongs at its
-// linear LDS slot under the XOR swizzle. The swizzle key of a lane repeats with period VAR in E,
-// so VAR per-lane byte offsets (row-in-load * pitch + chunk * 16) are computed once per kernel and
-// everything that changes from load to load (E * RPI * pitch), from segment to segment (k0 * 2)
-// and from tile to tile (the buffer base) is scalar: the load's soffset, M0 and the descriptor.
-// The scalar offset is not range-checked by the buffer unit, so that fast path is taken only when
-// all rows of the tile and all k of the segment exist; edge tiles and the K tail put the whole
-// offset in the range-checked vector offset and push absent k out of range (zero fill).
+// A wave load E covers rows [E*RPI, (E+1)*RPI) of the operand stage; lane (lane_row, lane_slot) fetches the 16-byte chunk that
+// belongs at its linear LDS slot under the XOR swizzle. The swizzle key of a lane repeats with period VAR in E, so VAR per-lane
+// byte offsets (row-in-load * pitch + chunk * 16) are computed once per kernel, one vector add makes a load's of them, and what changes from
+// segment to segment (k0 * 2) and from tile to tile (the buffer base) is scalar: the load's soffset, M0 and the descriptor.
+// The vector offset is range checked, the scalar one is not: rows past the edge read as zeros, and in the segment with the end of K the k
+// part goes through the vector offset too, absent k out of range.
+//
+// Block by block (a stage, a wave tile's rows, or 16 rows), with counters of their own for a segment's blocks. What bounds a producer is the wave's own
+// instructions: a queue of signals and a poll per block took about 1100 cycles per block. So a segment is one straight line: one look at its stage's
+// "empty" counters until all of them are there, then the loads of block b and the "landed" signals of block b of the segment before, behind a wait
+// whose immediate is the loads of one segment (a wave's loads complete in issue order). While the consumers have not released the
+// stage the wave retires its own signals, oldest first, so that it never holds back what they need to make progress.
+// us, polls and queue / this, two producer waves: 2048^3, 128 tiles, 4 stages, tile granularity 26.3 / 24.5, wave tiles with steps 2 and 1 50.6 / 24.4, with
+// 4 and 2 62.2 / 24.4; 3 stages 29.1 / 25.2, 50.7 / 28.5, 62.4 / 28.2; 4096^3, 256 tiles, 2 stages 124 / 122, 173 / 133, 150 / 130.
 template <int TILE, int SEGK, int CW, int MODE, bool IS_A, int PX>
 __device__ __forceinline__ void produce(const GemmArgs& g, uint32_t flags_base, uint32_t ring_base, int q, int lane) {
     constexpr int WTR = TILE / (CW / 2) / MFMA_M, WTC = TILE / 2 / MFMA_N;
-    constexpr int CPR = SEGK / CHUNK_ELEMS;      // 16-byte chunks per row
-    constexpr int RB = SEGK * 2;                 // row bytes in LDS
-    constexpr int RPI = WAVE / CPR;              // rows one wave load covers
-    constexpr int OPB = TILE * RB;               // bytes of one operand stage
-    constexpr int BLK_ROWS = MODE == CK_SYNC_TILE ? TILE : MODE == CK_SYNC_WAVE ? (IS_A ? WTR : WTC) * 16 : 16;
+    constexpr int CPR = SEGK / CHUNK_ELEMS, RB = SEGK * 2, RPI = WAVE / CPR, OPB = TILE * RB;
+    constexpr int WT = IS_A ? WTR : WTC;                      // 16-row blocks per wave tile
+    constexpr int BLK_ROWS = MODE == CK_SYNC_TILE ? TILE : MODE == CK_SYNC_WAVE ? WT * 16 : 16;
     constexpr int NBLK = TILE / BLK_ROWS;
-    constexpr int NIB = BLK_ROWS / RPI;          // wave loads per row block
-    constexpr int VAR = CPR == 4 ? 1 : CPR == 8 ? 2 : CPR == 16 ? 4 : 8;  // period of the swizzle key in E
-    static_assert(BLK_ROWS % RPI == 0, "row block must be whole wave loads");
+    constexpr int NIB = BLK_ROWS / RPI;                       // wave loads per block
+    constexpr int VAR = CPR == 4 ? 1 : CPR == 8 ? 2 : CPR == 16 ? 4 : 8;
+    static_assert(BLK_ROWS % RPI == 0 && NIB % VAR == 0, "a block is whole wave loads and whole periods of the swizzle key");
 
-    const int sa = g.bar_steps_a, sb = g.bar_steps_b;
-    const int S = g.num_stages;
-    const int ua = units_a(MODE, CW, sa), ub = units_b(MODE, CW, sb);
-    const int fps = 2 * ua + 2 * ub;
-    // counters of this operand inside one stage's flag set
-    const uint32_t full_off = IS_A ? 0 : 2 * ua;
-    const uint32_t empty_off = IS_A ? ua : 2 * ua + ub;
-    const int nres = CW - sa * sb;  // WAVE mode: consumer waves on the residual counters
+    const int sa = g.bar_steps_a, sb = g.bar_steps_b, S = g.num_stages;
+    const int ua = units_a(MODE, CW, sa), ub = units_b(MODE, CW, sb), fps = 2 * ua + 2 * ub;
+    const int s_own = MODE == CK_SYNC_TILE ? 0 : IS_A ? sa : sb, s_oth = MODE == CK_SYNC_TILE ? 0 : IS_A ? sb : sa, units = IS_A ? ua : ub;
+    const uint32_t full_off = IS_A ? 0 : 2 * ua, empty_off = IS_A ? ua : 2 * ua + ub;
+    // WAVE: consumer waves on the residual counters, and the block in front of which their release is waited for
+    const int nres = MODE == CK_SYNC_TILE ? CW : CW - sa * sb;
+    const int res_blk = nres > 0 ? (s_own == 0 || s_oth < (IS_A ? 2 : CW / 2) ? 0 : s_own) : -1;
 
     const char* base = (const char*)(IS_A ? g.A : g.Bt);
     const int rows_total = IS_A ? g.M : g.N;
     const int64_t pitch = (int64_t)g.K * 2;
     const uint32_t pitch32 = (uint32_t)pitch;
-
     const int lane_row = lane / CPR, lane_slot = lane % CPR;
-    uint32_t lane_off[VAR];  // row-in-load * pitch + logical chunk * 16, per swizzle-key variant
+    uint32_t lane_off[VAR];
     int lane_chunk[VAR];
 #pragma unroll
     for (int v = 0; v < VAR; ++v) {
         lane_chunk[v] = swizzle_slot(v * RPI + lane_row, lane_slot, CPR, g.swizzle);
         lane_off[v] = (uint32_t)lane_row * pitch32 + (uint32_t)lane_chunk[v] * CHUNK_BYTES;
     }
-    const uint32_t load_step = (uint32_t)RPI * pitch32;  // bytes between consecutive wave loads
-
+    const uint32_t load_step = (uint32_t)RPI * pitch32;
     const int grid = gridDim.x;
     const int slot = xcd_slot(blockIdx.x, grid, g.num_xcd);
     const int64_t total_tiles = (int64_t)g.tiles_m * g.tiles_n;
 
     Spin sp{g.spin_limit, g.status, CK_STATUS_PRODUCER_TIMEOUT, false};
-    SignalQueue<MODE == CK_SYNC_TILE ? 3 : MODE == CK_SYNC_WAVE ? 4 : 8> sq;
-    sq.init();
+    // lane i looks at the stage's "empty" counter i; `readers` consumer waves add to it per fill.
+    const uint32_t empty_lane = flags_base + (empty_off + (uint32_t)(lane < units ? lane : units - 1)) * 4;
+    const uint32_t readers = lane >= units ? 0u : MODE == CK_SYNC_ACC ? (IS_A ? 2u : CW / 2) : lane < s_own ? (uint32_t)s_oth : (uint32_t)nres;
+    uint64_t released = ~0ull;   // bit i: counter i was there at the last look
+    auto look = [&](int stage, uint32_t fill) __attribute__((always_inline)) {
+        uint32_t v;
+        asm volatile("ds_read_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=v"(v) : "v"(empty_lane + (uint32_t)(stage * fps * 4)) : "memory");
+        released = __ballot((int32_t)(v - readers * fill) >= 0);
+    };
+    // the counters that have to be there in front of a block
+    auto needs = [&](int blk) __attribute__((always_inline)) -> uint64_t {
+        if (MODE != CK_SYNC_ACC) return (blk < s_own ? 1ull << blk : 0ull) | (blk == res_blk ? 1ull << s_own : 0ull);
+        return blk % WT <= s_own ? 1ull << (blk / WT * (s_own + 1) + blk % WT) : 0ull;
+    };
+    // moves the "landed" counters that block blk of a stage completes, once at most LATER loads are in flight
+    auto signal = [&](uint32_t full, int blk, auto later) __attribute__((always_inline)) {
+        constexpr int LATER = decltype(later)::value < 63 ? decltype(later)::value : 63;
+        int own, residual;   // (-1: none)
+        if (MODE != CK_SYNC_ACC) {
+            own = blk < s_own ? blk : -1;
+            residual = blk == NBLK - 1 ? s_own : -1;
+        } else {
+            own = blk % WT < s_own ? blk / WT * (s_own + 1) + blk % WT : -1;
+            residual = blk % WT == WT - 1 ? blk / WT * (s_own + 1) + s_own : -1;
+            if (own >= 0) residual = -1;
+        }
+        if (own < 0 && residual < 0) return;
+        wait_vmcnt_imm<LATER>();
+        if (own >= 0) flag_add(full + (uint32_t)own * 4);
+        if (residual >= 0) flag_add(full + (uint32_t)residual * 4);
+    };
+    auto full_of = [&](int stage) { return flags_base + (uint32_t)(stage * fps + (int)full_off) * 4; };
+    int lag = 0, r_stage = 0, r_blk = 0;   // blocks issued and not signalled; the oldest of them
+    auto retire = [&]() __attribute__((always_inline)) {
+        const uint32_t full = full_of(r_stage);
+        if (lag >= 8) signal(full, r_blk, std::integral_constant<int, 7 * NIB / PX>{});
+        else if (lag >= 6) signal(full, r_blk, std::integral_constant<int, 5 * NIB / PX>{});
+        else if (lag >= 4) signal(full, r_blk, std::integral_constant<int, 3 * NIB / PX>{});
+        else if (lag == 3) signal(full, r_blk, std::integral_constant<int, 2 * NIB / PX>{});
+        else if (lag == 2) signal(full, r_blk, std::integral_constant<int, NIB / PX>{});
+        else signal(full, r_blk, std::integral_constant<int, 0>{});
+        --lag;
+        if (++r_blk == NBLK) {
+            r_blk = 0;
+            if (++r_stage == S) r_stage = 0;
+        }
+    };
 
     int stage = 0;
     uint32_t fill = 0;
+#pragma unroll 1
     for (int64_t tc = slot; tc < total_tiles; tc += grid) {
         const TileRC rc = tile_order(g.tiles_m, g.tiles_n, g.tile_group_m, tc);
         const int row0 = __builtin_amdgcn_readfirstlane((IS_A ? rc.row : rc.col) * TILE);
@@ -401,59 +433,47 @@ __device__ __forceinline__ void produce(const GemmArgs& g, uint32_t flags_base, 
         const uint32_t num_records = (uint32_t)((int64_t)rows_here * pitch);
         __amdgpu_buffer_rsrc_t rsrc =
             __builtin_amdgcn_make_buffer_rsrc((void*)(base + (int64_t)row0 * pitch), 0, (int)num_records, 0x00020000);
-        const bool all_rows = rows_here == TILE;
-
+#pragma unroll 1
         for (int seg = 0; seg < g.nseg; ++seg) {
-            // loop-carried scalars are pinned to SGPRs so that address and flag arithmetic stays scalar
+            // (loop-carried scalars pinned to SGPRs, so that address and flag arithmetic stays scalar)
             stage = __builtin_amdgcn_readfirstlane(stage);
             fill = __builtin_amdgcn_readfirstlane(fill);
-            const uint32_t fl = flags_base + (uint32_t)stage * fps * 4;
-            const uint32_t st_base = ring_base + (uint32_t)stage * (2 * OPB) + (IS_A ? 0 : OPB);
-            const int k0 = seg * SEGK;
-            const bool fast = all_rows && k0 + SEGK <= g.K;
-            // wave-tile granularity: all "empty" counters of this operand and stage in one look (g.batched_empty_reads);
-            // a row block whose counter was already there is not polled again
-            uint32_t seen[5] = {0, 0, 0, 0, 0};
-            const bool batched = MODE == CK_SYNC_WAVE && g.batched_empty_reads && fill > 0;
-            if (MODE == CK_SYNC_WAVE) {
-                if (batched) flag_load5(fl + empty_off * 4, (IS_A ? sa : sb) + 1, seen);
+            lag = __builtin_amdgcn_readfirstlane(lag);
+            r_stage = __builtin_amdgcn_readfirstlane(r_stage);
+            r_blk = __builtin_amdgcn_readfirstlane(r_blk);
+            // all counters of the stage in one look (g.batched_empty_reads), or those of one block after the other
+            const int rounds = fill == 0 ? 0 : g.batched_empty_reads ? 1 : NBLK;
+#pragma unroll 1
+            for (int r = 0; r < rounds; ++r) {
+                const uint64_t need = rounds == 1 ? ~0ull : needs(r);
+                look(stage, fill);
+                uint32_t polls = 0;
+#pragma unroll 1
+                while (!sp.dead && (released & need) != need) {
+                    if (lag > 0) retire();
+                    else if (++polls > sp.limit) {
+                        sp.dead = true;
+                        if ((threadIdx.x & 63) == 0) atomicOr(sp.status, sp.bit);
+                    } else if (g.producer_nap == 0) __builtin_amdgcn_s_sleep(1);
+                    else if (g.producer_nap == 1) __builtin_amdgcn_s_sleep(4);
+                    else __builtin_amdgcn_s_sleep(16);
+                    look(stage, fill);
+                }
             }
-            auto wave_wait = [&](int idx, uint32_t target) __attribute__((always_inline)) {
-                if (batched && (int32_t)(seen[idx] - target) >= 0) return;
-                producer_wait(fl + (empty_off + idx) * 4, target, sq, sp, g.producer_nap);
-            };
+            const int k0 = seg * SEGK;
+            const uint32_t st_base = ring_base + (uint32_t)(stage * 2 * OPB + (IS_A ? 0 : OPB)), full = full_of(r_stage);
+            const int first = NBLK - lag;   // the blocks of the segment before from here on are unsignalled
+            const bool k_tail = k0 + SEGK > g.K;
 #pragma unroll
             for (int blk = 0; blk < NBLK; ++blk) {
-                // ---- wait until the consumers of the previous fill have released these rows
-                if (MODE == CK_SYNC_TILE) {
-                    producer_wait(fl + (empty_off + 0) * 4, CW * fill, sq, sp, g.producer_nap);
-                } else if (MODE == CK_SYNC_WAVE) {
-                    const int s_own = IS_A ? sa : sb, s_oth = IS_A ? sb : sa;
-                    const int oth_max = IS_A ? 2 : CW / 2;
-                    const bool first_has_res = (s_own == 0 || s_oth < oth_max);
-                    if (blk == 0 && first_has_res && nres > 0) wave_wait(s_own, nres * fill);
-                    if (blk < s_own && s_oth > 0) {
-                        wave_wait(blk, s_oth * fill);
-                    } else if (blk == s_own && !first_has_res && nres > 0) {
-                        wave_wait(s_own, nres * fill);
-                    }
-                } else {
-                    constexpr int WT = IS_A ? WTR : WTC;
-                    const int s_own = IS_A ? sa : sb;
-                    const int unit = blk / WT, sub = blk % WT;
-                    const int readers = IS_A ? 2 : CW / 2;
-                    if (sub <= s_own) producer_wait(fl + (empty_off + unit * (s_own + 1) + sub) * 4, readers * fill, sq, sp, g.producer_nap);
-                }
-                // ---- this wave's share of the row block, straight into LDS
-                if (fast) {
-                    const uint32_t soff0 = (uint32_t)k0 * 2u;
+                // (the row part of the offset is range checked: rows past the edge read as zeros; at the end of K the k part is as well)
+                if (!k_tail) {
 #pragma unroll
                     for (int e = 0; e < NIB; ++e) {
                         const int E = blk * NIB + e;
                         if (PX > 1 && E % PX != q) continue;
                         __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (CK_LDS void*)(uintptr_t)(st_base + (uint32_t)E * 1024u), 16,
-                                                                 lane_off[E % VAR], soff0 + (uint32_t)E * load_step, 0, 0);
-                        sq.issued++;
+                                                                 lane_off[E % VAR] + (uint32_t)E * load_step, (uint32_t)k0 * 2u, 0, 0);
                     }
                 } else {
 #pragma unroll
@@ -463,28 +483,18 @@ __device__ __forceinline__ void produce(const GemmArgs& g, uint32_t flags_base, 
                         uint32_t voff = lane_off[E % VAR] + (uint32_t)E * load_step + (uint32_t)k0 * 2u;
                         if (k0 + lane_chunk[E % VAR] * CHUNK_ELEMS >= g.K) voff = num_records;  // absent k: zero fill
                         __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (CK_LDS void*)(uintptr_t)(st_base + (uint32_t)E * 1024u), 16, voff, 0, 0, 0);
-                        sq.issued++;
                     }
                 }
-                // ---- queue the "landed" signals this block completes
-                if (MODE == CK_SYNC_TILE) {
-                    sq.push(fl + (full_off + 0) * 4);
-                } else if (MODE == CK_SYNC_WAVE) {
-                    const int s_own = IS_A ? sa : sb;
-                    if (blk < s_own) sq.push(fl + (full_off + blk) * 4);
-                    if (blk == NBLK - 1) sq.push(fl + (full_off + s_own) * 4);
-                } else {
-                    constexpr int WT = IS_A ? WTR : WTC;
-                    const int s_own = IS_A ? sa : sb;
-                    const int unit = blk / WT, sub = blk % WT;
-                    if (sub < s_own) sq.push(fl + (full_off + unit * (s_own + 1) + sub) * 4);
-                    else if (sub == WT - 1) sq.push(fl + (full_off + unit * (s_own + 1) + s_own) * 4);
-                }
+                // (the loads behind block blk of the segment before: its own other blocks' and this one's up to here)
+                if (blk >= first) signal(full, blk, std::integral_constant<int, NBLK * NIB / PX>{});
             }
+            if (lag > 0 && ++r_stage == S) r_stage = 0;
+            lag = NBLK;
+            r_blk = 0;
             if (++stage == S) { stage = 0; ++fill; }
         }
     }
-    sq.drain();
+    while (lag > 0) retire();
 }
 
 // The single producer wave of the port_0 launcher (port_0.cu:106-147 with one producer warp): tile granularity, the one

@@ -340,10 +340,9 @@ int ckopt_last_launch_clocks(void* stream, uint64_t* shader_cycles, uint64_t* re
  *        less time (measured: two slices of 128 tiles 27 us against 22 for the second kernel, four of 64 tiles 47
  *        against 19 - the last wave's chain of memory round trips - so on a 256-CU device the second kernel is what
  *        runs); 2: always inside the kernel; 0: never.
- * key 14: wave-tile granularity of the counter-synchronised kernel (default 1). 1: a producer wave reads all "released"
- *        counters of its operand and stage in one look per segment and polls a row block's counter only if that look
- *        found it short; 0: it polls every row block's counter on its own, as the reference's producers wait on every
- *        barrier in turn (port_2.cu:212-232).
+ * key 14: the finer granularities of the counter-synchronised kernel (default 1). 1: a producer wave looks at all "released"
+ *        counters of its operand and stage at once until all are there; 0: at those of one row block after the other, as the reference's
+ *        producers wait on every barrier in turn (port_2.cu:212-232).
  * Returns the previous value or CKOPT_ERR_BAD_PARAM. */
 int ckopt_set_option(int key, int value);
 
