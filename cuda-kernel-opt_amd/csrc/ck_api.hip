@@ -603,7 +603,9 @@ SmallPlan small_plan(int M, int N, int K, int operand_alignment, int cus, double
     for (int t : {32, 64})
         for (int S = 2; S <= ITEM_MAX_SLICES && K / S >= ITEM_MIN_SLICE && tiles(t) * S <= 2 * cus; ++S) {
             // (from seven slices on 4 to 9 us more than that: 360 x 190 x 34304 in 14 25.3, 213 x 320 x 36672 in 12 25.0, 1149 x 128 x 11520 in 7 17.7; 512^2 x 12288 in 4 17.8)
-            const double us = sliced_us(direct_us(t, tiles(t) * S, (K + S - 1) / S, rows_aligned, bytes, on_copies, cus), S, (int64_t)M * N, call_us) + (S > 6 ? 6.0 : 0.0);
+            // (operands beyond 80 MB 2.6 TB/s: 128 x 2852 x 22464 in 5 53.8)
+            const double items_us = direct_us(t, tiles(t) * S, (K + S - 1) / S, rows_aligned, bytes, on_copies, cus) + (S > 6 ? 6.0 : 0.0);
+            const double us = sliced_us(std::max(items_us, bytes > 80e6 ? 3.0 + bytes / 2.6e6 : 0.0), S, (int64_t)M * N, call_us);
             if (us < 0.9 * whole.us && us < 0.98 * best.us) best = {t, false, S, us};
         }
     return best;
@@ -636,6 +638,9 @@ bool mid_tuple(const ck::GemmTuning& t, const Options& opt) {
 bool mid_is_shorter(int M, int N, int K, int cus) {
     const int64_t tiles = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
     const bool lines = K % 64 == 0;
+    // an even K that 8 does not divide, against the general ring behind operand copies: 384 x 10310 x 2692 33.5 / 60.4, 914 x 3264 x 916 16.9 / 31.0, but 1375 x 7872 x 418
+    // (three rounds) 41.6 / 43.7 and 35.3 on the straight-line kernel
+    if (needs_copies(K, true)) return tiles <= cus ? K >= 256 : tiles <= 9 * (int64_t)cus && K >= 1024;
     if (tiles < cus) return K >= (2 * tiles > cus ? 256 : 512);
     if (tiles == cus) return K > 512 && (lines || ((double)M + N) * K * 2.0 < 64e6);
     return lines && tiles <= 9 * (int64_t)cus && K >= 1024;
@@ -644,12 +649,14 @@ bool mid_is_shorter(int M, int N, int K, int cus) {
 // Estimated microseconds of gemm_mid_kernel on S slices of every tile, fitted to calls on aligned operands: a launch, per round 5.8 us of prologue
 // and epilogue, per slab of 64 k 0.355 us on up to 64 CUs to 0.46 on all 256 (1024^2: K 768 11.1, 1024 12.6, 2048 18.4, 4096 29.8;
 // 2048^2: K 1536 18.7, 2048 22.2, 4096 37.2; 4096^2 x 4096 145), rows off a line 1.2 to 1.4 times that (1024^2 x 1000 15.2, 2048^2 x 4104 44.7);
-// operands from memory at 3.4 TB/s where they leave the last-level cache (bf16 256 x 16384 x 4096 46.6).
+// operands from memory at 3.4 TB/s where they leave the last-level cache (bf16 256 x 16384 x 4096 46.6); beyond it every XCD's twelve panels of
+// a block of 32 tiles come over the fabric at 2.6 TB/s (2048^2 x 32768 292, 557 x 12077 x 54592 1003, 5120 x 601 x 21568 183).
 double mid_us(int64_t tiles, int K, int S, double operand_bytes, int cus) {
     const double items = (double)tiles * S, rounds = std::ceil(items / cus), share = items / rounds / cus;
     const double slab = (0.355 + 0.14 * std::max(0.0, share - 0.25)) * (K % 64 ? 1.3 : 1.0);
     const double us = 1.5 + rounds * (5.8 + std::ceil((double)K / 64.0 / S) * slab);
-    return std::max(us, operand_bytes > 80e6 ? 6.0 + operand_bytes / 3.4e6 : 0.0);
+    const double fabric = operand_bytes > 200e6 ? 6.0 + (double)tiles * K * 96.0 / 2.6e6 : 0.0;
+    return std::max({us, fabric, operand_bytes > 80e6 ? 6.0 + operand_bytes / 3.4e6 : 0.0});
 }
 struct MidPlan { int slices; double us; };
 MidPlan mid_plan(int M, int N, int K, int cus, double call_us) {
@@ -685,8 +692,9 @@ Route route_of(int M, int N, int K, int operand_alignment, const ck::GemmTuning&
         return {p.direct ? CKOPT_KERNEL_DIRECT : CKOPT_KERNEL_FUSED, p.direct ? p.direct : t.tile_dim, p.copies, p.slices};
     }
     if (straight_line_tuple(t, opt)) r.kernel = CKOPT_KERNEL_STREAM;
-    else if (mid && t.num_cus >= cus && !r.copies && mid_is_shorter(M, N, K, cus)) {
+    else if (mid && t.num_cus >= cus && (!r.copies || (K % 2 == 0 && K % CHUNK_ELEMS != 0 && operand_alignment >= 4)) && mid_is_shorter(M, N, K, cus)) {
         r.kernel = CKOPT_KERNEL_MID;
+        r.copies = false;
         r.slices = mid_plan(M, N, K, cus, call_us).slices;
     } else if (t.num_producer_waves == 0) r.kernel = t.num_stages == 1 ? CKOPT_KERNEL_SYNC : CKOPT_KERNEL_FUSED;
     else if (sync_mode_of(t.tile_dim, t.num_consumer_waves, t.bar_step_rows_a, t.bar_step_rows_b) == CK_SYNC_TILE && t.num_stages >= 2 &&
@@ -1172,7 +1180,7 @@ int ckopt_suggest_gemm_tuning(int M, int N, int K, int num_cus, int* tuning_out)
         const bool whole_device = num_cus >= dev_cus;
         const double call_us = opt[OPT_SPLIT_K] == 1 ? KEPT_CALL_US : 0.0;
         const SmallPlan small = small_plan(M, N, K, 16, dev_cus, call_us);
-        const bool mid_runs = whole_device && !needs_copies(K, true) && mid_is_shorter(M, N, K, dev_cus);
+        const bool mid_runs = whole_device && K % 2 == 0 && mid_is_shorter(M, N, K, dev_cus);
         const MidPlan mid = mid_plan(M, N, K, dev_cus, call_us);
         // Rows off a line, which the estimate leaves out: 1.3 to 2.2 times on 256 x 128 tiles (2048^2 x 4104 67.6 us against 49.0 on the tuple of 128
         // tiles and 79.1 on the one of 64; 8896 x 253 x 12808 219 / 141 / 172), 1.1 on wider ones and on a short K.

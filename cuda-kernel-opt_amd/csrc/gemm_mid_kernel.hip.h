@@ -76,7 +76,9 @@ __device__ __forceinline__ void store_row(const GemmArgs& g, float* D, int m, in
         }
 }
 
-// Rows start on 16-byte boundaries and K % 8 == 0 (a 16-byte chunk of a row is inside it or past it); KTAIL: K % 64 != 0.
+// Rows start on 16-byte boundaries and K % 8 == 0 (a 16-byte chunk of a row is inside it or past it), or with KTAIL (K % 64 != 0) on 4-byte
+// boundaries and K is even: direct-to-LDS loads take such rows as they are, and the last K % 8 values of the rows, which no whole chunk holds, are one
+// more k-step on fragments straight from memory (no zero-padded copies: bf16 384 x 10310 x 2692 60.4 -> 33.5 us, 914 x 3264 x 916 with 16-bit results 31.0 -> 16.9).
 template <typename DT, bool KTAIL>
 __global__ __launch_bounds__(512) void gemm_mid_kernel(const GemmArgs g) {
     constexpr int WT = 4;   // 16 x 16 blocks per edge of a wave tile
@@ -105,7 +107,7 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(const GemmArgs g) {
         off[j] = (uint32_t)row * pitch + (uint32_t)chunk * CHUNK_BYTES;
         chunk_k[j] = chunk * CHUNK_ELEMS;
     }
-    const int all = (g.K + MID_SLAB_K - 1) / MID_SLAB_K;
+    const int whole_k = KTAIL ? g.K & ~7 : g.K, all = (whole_k + MID_SLAB_K - 1) / MID_SLAB_K;
     int begin = 0, end = all;
     if (g.split_k > 1) {
         begin = __builtin_amdgcn_readfirstlane(slice_begin(all, slice, g.split_k));
@@ -116,7 +118,7 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(const GemmArgs g) {
     auto load = [&](int i) __attribute__((always_inline)) {   // 0, 1: A; 2, 3: Bt
         uint32_t voff = off[i % 2];
         // (beyond every descriptor's range, which is below 2^31)
-        if (KTAIL && ld_slab * MID_SLAB_K + chunk_k[i % 2] >= g.K) voff = 0x80000000u;
+        if (KTAIL && ld_slab * MID_SLAB_K + chunk_k[i % 2] >= whole_k) voff = 0x80000000u;
         dma_load_b128(i < 2 ? rsrc_a : rsrc_b, ring + (uint32_t)(ld_stage * MID_STAGE + (i < 2 ? 0 : MID_OPERAND) + wave * 2048 + i % 2 * 1024), voff,
                       (uint32_t)ld_slab * (MID_SLAB_K * 2));
     };
@@ -137,12 +139,34 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(const GemmArgs g) {
     for (int i = 0; i < WT; ++i)
 #pragma unroll
         for (int j = 0; j < WT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // the values behind the last whole chunk: k 0 .. 7 of one k-step, lanes of chunk 0 (rows past the edge: the last row, never stored)
+    const bool has_rest = KTAIL && whole_k != g.K && end == all && group == 0;
+    uint32_t ta[WT][3] = {}, tb[WT][3] = {};
+    if (KTAIL && has_rest && lg == 0) {
+        const int row0_a = R * 64 + lr, row0_b = Cc * 64 + lr;
+#pragma unroll
+        for (int i = 0; i < WT; ++i) {
+            const int ra = row0_a + i * 16 < rows_a ? row0_a + i * 16 : rows_a - 1, rb = row0_b + i * 16 < rows_b ? row0_b + i * 16 : rows_b - 1;
+            const uint32_t* at_a = (const uint32_t*)((const char*)g.A + (int64_t)(row_a + ra) * pitch + whole_k * 2);
+            const uint32_t* at_b = (const uint32_t*)((const char*)g.Bt + (int64_t)(row_b + rb) * pitch + whole_k * 2);
+#pragma unroll
+            for (int d = 0; d < 3; ++d)
+                if (whole_k + 2 * d < g.K) { ta[i][d] = at_a[d]; tb[i][d] = at_b[d]; }
+        }
+    }
 
 #pragma unroll 1
     for (int p = 0; p < MID_STAGES; ++p) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) load(i);
         next_slab();
+    }
+    if (KTAIL && has_rest) {
+#pragma unroll
+        for (int i = 0; i < WT; ++i)
+#pragma unroll
+            for (int j = 0; j < WT; ++j)
+                acc[i][j] = MfmaOp<DT>::run(u32x4{tb[j][0], tb[j][1], tb[j][2], 0}, u32x4{ta[i][0], ta[i][1], ta[i][2], 0}, acc[i][j]);
     }
     wait_vmcnt_imm<12>();   // slabs 0 and 1
     wg_barrier();

@@ -1773,3 +1773,36 @@ def test_16_bit_c_and_d_on_any_two_byte_boundary(ck, bf16):
                     assert torch.isnan(buf[:16 + d_off]).all() and torch.isnan(buf[16 + d_off + M * N:]).all()
     assert seen >= {"gemm_stream_kernel", "gemm_mid_kernel", "gemm_direct_kernel", "gemm_fused_kernel", "gemm_sync_kernel", "gemm_pc_kernel"}
     assert ck.device_status() == 0
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+def test_even_k_on_four_byte_rows_without_copies(ck, bf16):
+    """gemm_mid_kernel on an even K that 8 does not divide: rows on 4-byte boundaries straight into LDS, and the last 2, 4 or 6 values of every row as
+    a k-step of their own - behind whole slabs, inside a slab, in the last of several K slices. Small integers: exact; NaN around the
+    operands, a guard behind D; operands on a 4-byte boundary themselves; the provided buffer still has to hold the copies that the query names."""
+    dtype, tdt = (ck.DT_BF16, torch.bfloat16) if bf16 else (ck.DT_F16, torch.float16)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(43)
+    for M, N, K in [(300, 270, 258), (300, 270, 260), (300, 270, 262), (129, 131, 322), (257, 384, 514), (1000, 900, 1002), (200, 333, 4090), (77, 85, 30002), (213, 320, 36678), (2100, 2060, 1028)]:
+        assert ck.gemm_launch_kernel(M, N, K, True, *MID_TUPLE) == "gemm_mid_kernel" and not ck.gemm_launch_plan(M, N, K, True, *MID_TUPLE)["operand_copies"]
+        for shift in (0, 2):
+            def operand(rows):
+                buf = torch.full((rows * K + 4096,), float("nan"), dtype=tdt, device="cuda")
+                view = buf[2048 + shift:2048 + shift + rows * K].view(rows, K)
+                view.copy_(torch.randint(-2, 3, (rows, K), device="cuda", generator=gen))
+                return view
+            a, b = operand(M), operand(N)
+            exact = a.cpu().float() @ b.cpu().float().t()
+            c = torch.randint(-8, 9, (M, N), device="cuda", generator=gen).float()
+            d = torch.full((M * N + 64,), float("nan"), dtype=torch.float32, device="cuda")
+            ck.gemm_shmem_tc_async_opt_port(dtype, a, b, c, d, 2.0, -3.0, M, N, K, *MID_TUPLE)
+            assert torch.equal(d[:M * N].view(M, N).cpu(), 2 * exact - 3 * c.cpu()), (M, N, K, shift)
+            assert torch.isnan(d[M * N:]).all()
+    need = ck.gemm_workspace_bytes(300, 270, 258, True, *MID_TUPLE)
+    assert need >= (300 + 270) * 264 * 2
+    a = torch.zeros((300, 258), dtype=tdt, device="cuda")
+    d = torch.full((300, 270), 7.0, device="cuda")
+    with pytest.raises(ck.CkoptError) as e:
+        ck.gemm_shmem_tc_async_opt_port_ws(dtype, ck.DT_F32, a, a[:270], None, d, 1.0, 0.0, 300, 270, 258, *MID_TUPLE, workspace=torch.empty(1024, dtype=torch.uint8, device="cuda"), workspace_bytes=1024)
+    assert e.value.code == ck.ERR_TOO_LARGE and (d == 7.0).all()
+    assert ck.device_status() == 0
