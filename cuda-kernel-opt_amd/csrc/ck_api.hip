@@ -30,6 +30,7 @@ hipError_t launch_gemm_mid(bool bf16, hipStream_t stream, const GemmArgs& a);
 hipError_t launch_gemm_sync_f16(int tile, int segk, int cw, dim3 grid, size_t lds, hipStream_t stream, const GemmArgs& a);
 hipError_t launch_gemm_sync_bf16(int tile, int segk, int cw, dim3 grid, size_t lds, hipStream_t stream, const GemmArgs& a);
 hipError_t launch_matmul_shmem(int dtype, int tile, int accs, bool bt, dim3 grid, hipStream_t s, const SimtArgs& a);
+hipError_t launch_matmul_shmem_small(int dtype, const SimtSmallInstance& i, bool bt, hipStream_t s, const SimtArgs& a);
 }  // namespace ck
 
 // One status word per device; the kernels OR a bit into it when a bounded flag wait gives up.
@@ -1220,9 +1221,12 @@ int ckopt_matmul_shmem(int dtype, const void* A, const void* B, void* C, int M, 
     if (((uintptr_t)A & 15) || ((uintptr_t)B & 15) || ((uintptr_t)C & 3)) return CK_ERR_ALIGNMENT;
     if (N / tile_dim > 65535) return CK_ERR_TOO_LARGE;
     SimtArgs a{A, B, C, M, N, K};
-    const SimtInstance inst = simt_instance(dtype, tile_dim, block_rows, M, N, device_cus());
-    const hipError_t e = launch_matmul_shmem(dtype, inst.tile, inst.accs, b_transposed != 0, dim3(M / inst.tile, N / inst.tile),
-                                             static_cast<hipStream_t>(stream), a);
+    const int cus = device_cus();
+    const SimtSmallInstance small = simt_small_instance(dtype, tile_dim, b_transposed != 0, M, N, cus);
+    const SimtInstance inst = simt_instance(dtype, tile_dim, block_rows, M, N, cus);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const hipError_t e = small.tile ? launch_matmul_shmem_small(dtype, small, b_transposed != 0, s, a)
+                                    : launch_matmul_shmem(dtype, inst.tile, inst.accs, b_transposed != 0, dim3(M / inst.tile, N / inst.tile), s, a);
     if (e == hipErrorInvalidValue) return CK_ERR_NO_INSTANCE;
     return e == hipSuccess ? CK_OK : CK_ERR_HIP;
 }

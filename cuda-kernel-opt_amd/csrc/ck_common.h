@@ -269,6 +269,19 @@ CK_HD SimtInstance simt_instance(int dtype, int tile_dim, int block_rows, int M,
     }
     return s;
 }
+// The kernel for few outputs per CU (simt_small_kernel.hip.h) in the place of those instances of the tuples of 64 and 128 tiles, with rm x rn accumulators
+// per thread; tile 0: not taken. Bounds by measurement (256 CUs, us, K 1024 where none is named, the instance above / this, B transposed; K x N differs by
+// a tenth): 512 x 128 x 1248 f32 / f16 / i32 35 / 41 / 38 -> 13 / 15 / 15, 512^2 30 / 35 / 33 -> 19 / 19 / 21, 768^2 43 / 42 / 49 -> 35 / 35 / 42, 1024^2 52 / 52 / 62 -> 39 / 40 / 51.
+// Above the bounds level or behind: f32 1152^2 x 512 27.5 / 31.1; f16 2048 x 1024 66 / 68, K x N 1152^2 x 512 31.7 / 33.0; int32 1280^2 87 / 92, K x N 1152 x 1024 69 / 72.
+struct SimtSmallInstance { int tile, rm, rn; };
+CK_HD SimtSmallInstance simt_small_instance(int dtype, int tile_dim, bool b_transposed, int M, int N, int num_cus) {
+    const int64_t outputs_per_cu = (int64_t)M * N / num_cus;
+    const int most = dtype == CK_DT_I32 ? (b_transposed ? 5632 : 3072) : dtype == CK_DT_F16 && b_transposed ? 7168 : 4608;
+    if (tile_dim == 32 || outputs_per_cu > most) return {0, 0, 0};
+    if (outputs_per_cu <= 768) return {16, 1, 1};
+    if (outputs_per_cu <= 1408) return {32, 2, 1};
+    return outputs_per_cu <= 3072 ? SimtSmallInstance{32, 2, 2} : SimtSmallInstance{32, 4, 2};
+}
 CK_HD int check_simt_tuning(int tile_dim, int block_rows) {
     if (!(tile_dim == 32 || tile_dim == 64 || tile_dim == 128)) return CK_ERR_BAD_PARAM;
     if (block_rows < 1 || tile_dim % block_rows) return CK_ERR_BAD_PARAM;

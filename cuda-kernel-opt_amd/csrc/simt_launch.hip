@@ -1,5 +1,6 @@
-// Instance table and dispatch of the matmul_shmem (SIMT) kernel.
+// Instance tables and dispatch of the matmul_shmem (SIMT) kernels.
 #include "simt_kernel.hip.h"
+#include "simt_small_kernel.hip.h"
 
 namespace ck {
 
@@ -27,6 +28,29 @@ hipError_t launch_matmul_shmem(int dtype, int tile, int accs, bool bt, dim3 grid
         case CK_DT_F32: return simt_dispatch<float>(tile, accs, bt, grid, s, a);
         case CK_DT_I32: return simt_dispatch<int>(tile, accs, bt, grid, s, a);
         case CK_DT_F16: return simt_dispatch<_Float16>(tile, accs, bt, grid, s, a);
+        default: return hipErrorInvalidValue;
+    }
+}
+
+template <typename DT, int TILE, int RM, int RN>
+static hipError_t simt_small_launch_one(bool bt, hipStream_t stream, const SimtArgs& a) {
+    const dim3 grid((unsigned)(a.M / TILE), (unsigned)(a.N / TILE)), block(TILE * TILE / (RM * RN));
+    if (bt) hipLaunchKernelGGL((matmul_shmem_small_kernel<DT, TILE, RM, RN, true>), grid, block, simt_small_lds_bytes(TILE), stream, a);
+    else hipLaunchKernelGGL((matmul_shmem_small_kernel<DT, TILE, RM, RN, false>), grid, block, simt_small_lds_bytes(TILE), stream, a);
+    return hipGetLastError();
+}
+template <typename DT>
+static hipError_t simt_small_dispatch(const SimtSmallInstance& i, bool bt, hipStream_t s, const SimtArgs& a) {
+    if (i.tile == 16) return simt_small_launch_one<DT, 16, 1, 1>(bt, s, a);
+    if (i.rm == 2 && i.rn == 1) return simt_small_launch_one<DT, 32, 2, 1>(bt, s, a);
+    if (i.rm == 2) return simt_small_launch_one<DT, 32, 2, 2>(bt, s, a);
+    return simt_small_launch_one<DT, 32, 4, 2>(bt, s, a);
+}
+hipError_t launch_matmul_shmem_small(int dtype, const SimtSmallInstance& i, bool bt, hipStream_t s, const SimtArgs& a) {
+    switch (dtype) {
+        case CK_DT_F32: return simt_small_dispatch<float>(i, bt, s, a);
+        case CK_DT_I32: return simt_small_dispatch<int>(i, bt, s, a);
+        case CK_DT_F16: return simt_small_dispatch<_Float16>(i, bt, s, a);
         default: return hipErrorInvalidValue;
     }
 }

@@ -139,3 +139,33 @@ def test_every_instance_where_the_grid_keeps_it_and_where_it_is_replaced(ck, ora
                     continue
                 got = run(ck, dtype, a, b, M, N, K, tile, br, bt)
                 assert np.array_equal(got.view(np.uint8), want.view(np.uint8)), (M, N, K, bt, tile, br)
+
+
+@pytest.mark.parametrize("name", ["f32", "f16", "i32"])
+def test_few_outputs_per_cu_on_either_side_of_every_bound(ck, oracle, name):
+    # The kernel with rows of 32 k in LDS, its four instances and the bounds between and above them (outputs per CU, 256 CUs: 768 / 896, 1408 / 1536, 3072 / 3328,
+    # 4608 / 4736, 5632 / 5888, 7168 / 7424), and the smallest sizes; K of half a slice, an odd and an even number of halves, and none may change a bit.
+    dtype = {"f32": ck.DT_F32, "f16": ck.DT_F16, "i32": ck.DT_I32}[name]
+    odt = {"f32": oracle.DT_F32, "f16": oracle.DT_F16, "i32": oracle.DT_I32}[name]
+    rng = np.random.default_rng(29)
+    for M, N, K, tile, br in ((64, 64, 16, 64, 4), (128, 128, 32, 128, 4), (512, 384, 112, 128, 8), (512, 448, 48, 64, 1), (512, 704, 80, 64, 4), (512, 768, 16, 128, 2),
+                              (1024, 768, 64, 128, 4), (1024, 832, 48, 64, 16), (1152, 1024, 80, 128, 4), (1152, 1024, 96, 64, 2), (512, 2368, 48, 64, 4), (512, 2816, 80, 128, 8),
+                              (512, 2944, 32, 128, 8), (1024, 1792, 48, 128, 4), (1024, 1856, 16, 64, 4), (64, 3072, 144, 64, 8)):
+        for bt in (False, True):
+            shape_b = (N, K) if bt else (K, N)
+            if name == "i32":   # sums and products wrap modulo 2^32
+                a, b = (rng.integers(-2 ** 31, 2 ** 31, s, dtype=np.int32) for s in ((M, K), shape_b))
+                want = (a.astype(np.int64) @ (b.T if bt else b).astype(np.int64)).astype(np.int32)
+            else:
+                a, b = ck.fill_uniform(dtype, (M, K), 31, 0), ck.fill_uniform(dtype, shape_b, 31, 1)
+                want = oracle.matmul(odt, a, b, bt, fused=True)
+                want = want.astype(np.float16) if name == "f16" else want
+            got = run(ck, dtype, a, b, M, N, K, tile, br, bt)
+            assert np.array_equal(got.view(np.uint8), want.view(np.uint8)), (M, N, K, bt, tile, br)
+    # an infinity and a NaN in the last k reach the outputs of their row and column alone (nothing is read past the end of K)
+    if name != "i32":
+        a, b = ck.fill_uniform(dtype, (128, 48), 37, 0), ck.fill_uniform(dtype, (48, 128), 37, 1)
+        a[5, 47], b[47, 9] = np.inf, np.nan
+        got = run(ck, dtype, a, b, 128, 128, 48, 64, 4, False)
+        bad = ~np.isfinite(got.astype(np.float32))
+        assert bad[5].all() and bad[:, 9].all() and bad.sum() == 255
