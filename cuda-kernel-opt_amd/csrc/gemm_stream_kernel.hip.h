@@ -94,6 +94,8 @@ __global__ __launch_bounds__(512) void gemm_stream_kernel(const GemmArgs g) {
     constexpr int EPILOGUE_STORES_16 = H16_WHOLE_LINES ? WTR * (WTC / H16_GROUP) * STORES_PER_GROUP : EPILOGUE_STORES / 2;     // 16-bit output
     static_assert(WTC % F32_GROUP == 0, "whole groups per wave-tile row");
     static_assert(EPILOGUE_STORES_16 * 2 == EPILOGUE_STORES, "count_stores selects between the two with a shift by one");
+    constexpr int WAVE_TILE_SPAN = 1 << 24;   // columns of C and D up to which a wave tile's rows lie within 32-bit offsets (wider: block by block)
+    static_assert((uint64_t)WTR * 16 * WAVE_TILE_SPAN * 4 <= 1ull << 32, "a wave tile's extent in a descriptor");
     constexpr int PRE = 1;               // columns of MFMAs in front of the barrier
     constexpr int LOAD_COL_0 = WTC == 8 ? 3 : WTC == 6 ? 2 : 1;  // columns behind which a k-step's two load pairs are issued
     constexpr int LOAD_COL_1 = WTC == 8 ? 6 : WTC == 6 ? 4 : 3;
@@ -247,19 +249,16 @@ __global__ __launch_bounds__(512) void gemm_stream_kernel(const GemmArgs g) {
 #pragma unroll
         for (int j = 0; j < WTC; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    // How many stores an interior tile's epilogue leaves in flight, as the code the landing wait takes:
-    // 0 = wait for everything (beta is not zero: the epilogue also loads C), 2 = 32 stores (beta is plus or
-    // minus zero), 1 = 16 stores (beta zero, 16-bit output through the 16-byte store path below, which
-    // needs D and its rows on 16-byte boundaries). Worked out on the scalar unit in asm: a flag the compiler
-    // derives from a compare ends up in a vector register, which the "s" operands of the asm statements
-    // below cannot take.
+    // How many stores an interior tile's epilogue leaves in flight, as the code the landing wait takes: 2 = 32 stores, 1 = 16
+    // (16-bit output through the 16-byte store path below, which needs D and its rows on 16-byte boundaries). Where the
+    // epilogue also loads C there are more operations behind the ring's loads than counted: the wait is only the
+    // stronger for it. Worked out on the scalar unit in asm: a flag the compiler derives from a compare ends up in a
+    // vector register, which the "s" operands of the asm statements below cannot take.
     const uint32_t d16_misaligned = H16_WHOLE_LINES ? ((uint32_t)(uintptr_t)g.D | ((uint32_t)g.N << 1)) & 15u : 1u;
     uint32_t count_stores, count_tmp;
-    asm volatile("s_lshl_b32 %0, %2, 1\n\ts_cmp_eq_u32 %0, 0\n\ts_cselect_b32 %0, 2, 0\n\t"
-                 "s_cmp_eq_u32 %4, 0\n\ts_cselect_b32 %1, %3, 0\n\ts_lshr_b32 %0, %0, %1"
-                 : "=&s"(count_stores), "=&s"(count_tmp)
-                 : "s"(__builtin_amdgcn_readfirstlane(__builtin_bit_cast(uint32_t, g.beta))),
-                   "s"(__builtin_amdgcn_readfirstlane((uint32_t)g.out16)), "s"(__builtin_amdgcn_readfirstlane(d16_misaligned))
+    asm volatile("s_cmp_eq_u32 %3, 0\n\ts_cselect_b32 %1, %2, 0\n\ts_lshr_b32 %0, 2, %1"
+                 : "=s"(count_stores), "=&s"(count_tmp)
+                 : "s"(__builtin_amdgcn_readfirstlane((uint32_t)g.out16)), "s"(__builtin_amdgcn_readfirstlane(d16_misaligned))
                  : "scc");
     uint32_t stores_in_flight;  // nonzero in the loop body that follows an epilogue whose stores count in the wait
     asm volatile("s_mov_b32 %0, 0" : "=s"(stores_in_flight));
@@ -458,17 +457,35 @@ __global__ __launch_bounds__(512) void gemm_stream_kernel(const GemmArgs g) {
             // 128-byte run of a row straddles two lines, and ordinary stores let the halves meet in L2 (N = 4097,
             // 408 tiles: 138 us against 164 with non-temporal stores)
             const bool nt_store = g.nt_store != 0;
-            if (vec_cols && !g.out16) {
+            if (vec_cols && !g.out16 && g.N < WAVE_TILE_SPAN) {
                 // Whole 128-byte lines per store: an accumulator block gives a row 64 bytes (4 lanes x 16),
                 // and the write path's cost is per request, not per byte. Two neighbouring blocks are
                 // exchanged between lanes so that 8 lanes hold the 32 consecutive floats of one row:
                 // store t (0, 1) of a pair writes rows 8t .. 8t+7, lane L the piece L % 8 of row L / 8,
                 // which sits in lane (8t + L / 8) + 16 * (piece % 4) of block piece / 4.
+                // C and D are reached through descriptors of the wave tile, whose extent ends behind its last row inside
+                // the matrix (later rows are not stored and read as zeros): one 32-bit offset per row step, the
+                // columns in the immediate. With 64-bit addresses and a predicate per row step the masks, beta and the
+                // store policy did not fit into the scalar registers and came back from vector lanes at every store;
+                // fp16 16384^3 with C read 6.81 to 6.89 ms, 6.73 to 6.76 now;
+                // 6100 x 6144 x 1024 with C 113.4 us, 111.0; without C 8192^3 797, 796.
                 const int piece = lane & 7;
                 const int src0 = ((lane >> 3) + 16 * (piece & 3)) * 4;  // byte address of the source lane, t = 0
                 const bool second = piece >= 4;
-                const int64_t row0 = (int64_t)(rc.row * TILE + R * WTR * 16 + (lane >> 3));
-                const int col0 = rc.col * TILE_N + Cc * WTC * 16 + piece * 4;
+                const int row0 = __builtin_amdgcn_readfirstlane(rc.row * TILE + R * WTR * 16), col0 = __builtin_amdgcn_readfirstlane(rc.col * TILE_N + Cc * WTC * 16);
+                const int rows = g.M - row0 < WTR * 16 ? g.M - row0 : WTR * 16;
+                const uint32_t extent = rows > 0 ? ((uint32_t)(rows - 1) * (uint32_t)g.N + WTC * 16) * 4u : 0u;
+                auto tile_rsrc = [&](const float* p) __attribute__((always_inline)) {
+                    const uint64_t at = (uint64_t)(uintptr_t)(p + ((int64_t)row0 * g.N + col0));
+                    // (the builtin returns a signed word: unsigned again before it is widened)
+                    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)at), hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(at >> 32));
+                    return __builtin_amdgcn_make_buffer_rsrc((void*)(uintptr_t)((uint64_t)hi << 32 | lo), 0, (int)extent, 0x00020000);
+                };
+                const __amdgpu_buffer_rsrc_t rsrc_d = tile_rsrc(go.D);
+                uint32_t lane_off = ((uint32_t)(lane >> 3) * (uint32_t)g.N + (uint32_t)piece * 4) * 4u;
+                const uint32_t step = (uint32_t)g.N * 32u;
+                // (the offsets do not depend on the tile: opaque, or all sixteen are kept in registers over the main loop)
+                asm volatile("" : "+v"(lane_off));
                 const float alpha = g.alpha, beta = g.beta;
                 // store s of the epilogue: block row i, group of two block columns j, half tt
                 constexpr int GROUPS = WTC / F32_GROUP;
@@ -483,44 +500,45 @@ __global__ __launch_bounds__(512) void gemm_stream_kernel(const GemmArgs g) {
                     }
                     return v;
                 };
-                auto put = [&](int64_t off, f32x4 v) __attribute__((always_inline)) {
-                    if (nt_store) store_b128_nt(go.D + off, __builtin_bit_cast(u32x4, v));
-                    else *(f32x4_u*)(go.D + off) = v;
-                };
-                if (beta == 0.f) {
+                auto row_off = [&](int st) { return lane_off + (uint32_t)(st / (GROUPS * STORES_PER_GROUP) * 2 + st % STORES_PER_GROUP) * step; };
+                auto col_off = [](int st) { return ((st / STORES_PER_GROUP) % GROUPS) * F32_GROUP * 64; };
+                auto value = [&](int st) __attribute__((always_inline)) { return exchanged(st / (GROUPS * STORES_PER_GROUP), ((st / STORES_PER_GROUP) % GROUPS) * F32_GROUP, st % STORES_PER_GROUP); };
+                auto put_all = [&](auto policy) __attribute__((always_inline)) {
+                    constexpr int POLICY = decltype(policy)::value;
+                    auto put = [&](int st, f32x4 v) __attribute__((always_inline)) {
+                        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), rsrc_d, (int)(row_off(st) + col_off(st)), 0, POLICY);
+                    };
+                    if (beta == 0.f) {
 #pragma unroll
-                    for (int i = 0; i < WTR; ++i) {
+                        for (int st = 0; st < EPILOGUE_STORES; ++st) put(st, value(st));
+                    } else {
+                        // C is read C_DEPTH stores ahead of its use: the loads of a wave would otherwise wait for memory one
+                        // by one between the stores (a load may not pass the store in front of it). Eight fit into the registers
+                        // (249 of 256); four to eight measure the same, twelve spill.
+                        constexpr int C_DEPTH = 8;
+                        const __amdgpu_buffer_rsrc_t rsrc_c = tile_rsrc(go.C);
+                        f32x4 cv[C_DEPTH];
+                        float factor = beta;   // (in a vector register: as a scalar it is kept four times over and spilled)
+                        asm volatile("" : "+v"(factor));
+                        auto fetch = [&](int st) __attribute__((always_inline)) {
+                            return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc_c, (int)(row_off(st) + col_off(st)), 0, 0));
+                        };
 #pragma unroll
-                        for (int j = 0; j < WTC; j += F32_GROUP) {
+                        for (int st = 0; st < C_DEPTH; ++st) cv[st] = fetch(st);
 #pragma unroll
-                            for (int tt = 0; tt < STORES_PER_GROUP; ++tt) {
-                                const f32x4 v = exchanged(i, j, tt);
-                                const int64_t row = row0 + i * 16 + tt * 8;
-                                if (row < g.M) put(row * g.N + (col0 + j * 16), v);
-                            }
+                        for (int st = 0; st < EPILOGUE_STORES; ++st) {
+                            f32x4 v = value(st);
+                            landed(cv[st % C_DEPTH]);
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) v[e] += cv[st % C_DEPTH][e] * factor;
+                            put(st, v);
+                            if (st + C_DEPTH < EPILOGUE_STORES) cv[st % C_DEPTH] = fetch(st + C_DEPTH);
                         }
                     }
-                } else {
-                    // C is read C_DEPTH stores ahead of its use: the loads of a wave would otherwise wait for memory one
-                    // by one between the stores (a load may not pass the store in front of it)
-                    constexpr int C_DEPTH = 4;
-                    f32x4 cv[C_DEPTH];
-                    auto row_of = [&](int st) { return row0 + (st / (GROUPS * STORES_PER_GROUP)) * 16 + (st % STORES_PER_GROUP) * 8; };
-                    auto off_of = [&](int st) { return row_of(st) * g.N + (col0 + ((st / STORES_PER_GROUP) % GROUPS) * F32_GROUP * 16); };
-                    auto fetch = [&](int st) __attribute__((always_inline)) {
-                        return row_of(st) < g.M ? (f32x4)*(const f32x4_u*)(go.C + off_of(st)) : f32x4{0.f, 0.f, 0.f, 0.f};
-                    };
-#pragma unroll
-                    for (int st = 0; st < C_DEPTH; ++st) cv[st] = fetch(st);
-#pragma unroll
-                    for (int st = 0; st < EPILOGUE_STORES; ++st) {
-                        f32x4 v = exchanged(st / (GROUPS * STORES_PER_GROUP), ((st / STORES_PER_GROUP) % GROUPS) * F32_GROUP, st % STORES_PER_GROUP);
-                        landed(cv[st % C_DEPTH]);
-                        v += cv[st % C_DEPTH] * beta;
-                        if (row_of(st) < g.M) put(off_of(st), v);
-                        if (st + C_DEPTH < EPILOGUE_STORES) cv[st % C_DEPTH] = fetch(st + C_DEPTH);
-                    }
-                }
+                };
+                constexpr int NON_TEMPORAL = 2;   // nt of a buffer access
+                if (nt_store) put_all(std::integral_constant<int, NON_TEMPORAL>{});
+                else put_all(std::integral_constant<int, 0>{});
             } else if (H16_WHOLE_LINES && interior && g.out16 && d16_misaligned == 0) {
                 if constexpr (H16_WHOLE_LINES) {
                 // 16-bit output in whole 128-byte lines, 16 bytes per lane. A lane's 4 results of a block are

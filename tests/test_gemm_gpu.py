@@ -1806,3 +1806,45 @@ def test_even_k_on_four_byte_rows_without_copies(ck, bf16):
         ck.gemm_shmem_tc_async_opt_port_ws(dtype, ck.DT_F32, a, a[:270], None, d, 1.0, 0.0, 300, 270, 258, *MID_TUPLE, workspace=torch.empty(1024, dtype=torch.uint8, device="cuda"), workspace_bytes=1024)
     assert e.value.code == ck.ERR_TOO_LARGE and (d == 7.0).all()
     assert ck.device_status() == 0
+
+
+@pytest.mark.parametrize("width", [0, 2, 3])
+def test_fp32_epilogue_of_the_straight_line_kernel(ck, width):
+    """C read and D written through descriptors of the wave tile: last rows on either side of the 64-row wave tiles and of the tile, C and D off each
+    other's alignment, several tiles per workgroup (the landing wait behind an epilogue that loads C), every store policy. Small integers:
+    exact; guards in front of D and behind it."""
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(47)
+    for M, N, K, sms in [(1, 256, 64, 256), (63, 768, 128, 256), (64, 512, 72, 8), (65, 1536, 192, 8), (257, 1283, 256, 8), (1090, 2304, 320, 8), (700, 1024, 64, 256)]:
+        a = torch.randint(-2, 3, (M, K), device="cuda", generator=gen).half()
+        b = torch.randint(-2, 3, (N, K), device="cuda", generator=gen).half()
+        exact = a.cpu().float() @ b.cpu().float().t()
+        for off in (0, 1, 2):
+            c = torch.randint(-8, 9, (M * N + 8,), device="cuda", generator=gen).float()[off:off + M * N]
+            buf = torch.full((M * N + 1024,), float("nan"), device="cuda")
+            d = buf[512 + 2 * off:512 + 2 * off + M * N]
+            for policy in (0, 1, 2):
+                for beta in (0.0, -3.0):
+                    ck.gemm_shmem_tc_async_opt_port_ex(ck.DT_F16, ck.DT_F32, a, b, c if beta else None, d, 2.0, beta, M, N, K, 256, 32, 0, 0, 256, 256, 4, 5, 0, 8, sms,
+                                                       options=ck.launch_options(half_width=width, d_store_policy=policy))
+                    assert torch.equal(d.view(M, N).cpu(), 2 * exact + beta * c.view(M, N).cpu()), (M, N, K, off, policy, beta)
+            assert torch.isnan(buf[:512 + 2 * off]).all() and torch.isnan(buf[512 + 2 * off + M * N:]).all()
+    assert ck.device_status() == 0
+
+
+@pytest.mark.parametrize("N", [(1 << 24) - 256, 1 << 24])
+def test_rows_on_either_side_of_a_wave_tiles_32_bit_extent(ck, N):
+    """From 2^24 columns on 64 rows of D no longer lie within 32-bit offsets: block by block. Small integers: exact."""
+    M, K = 66, 8
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(53)
+    a = torch.randint(-2, 3, (M, K), device="cuda", generator=gen).half()
+    b = torch.randint(-2, 3, (N, K), device="cuda", generator=gen).half()
+    d = torch.full((M, N), float("nan"), device="cuda")
+    d[:, ::2] = 1
+    c = d[:, :].nan_to_num(2.0)
+    ck.gemm_shmem_tc_async_opt_port(ck.DT_F16, a, b, c, d, 1.0, 2.0, M, N, K, 256, 32, 0, 0, 256, 256, 4, 5, 0, 8, 256)
+    for at in range(0, N, 1 << 21):
+        part = slice(at, min(N, at + (1 << 21)))
+        assert torch.equal(d[:, part], a.float() @ b[part].float().t() + 2 * c[:, part]), (N, at)
+    assert ck.device_status() == 0
