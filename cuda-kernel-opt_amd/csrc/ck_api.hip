@@ -758,28 +758,25 @@ hipError_t add_planes(int dtype, const float* ws, int slices, int64_t count, con
     return hipGetLastError();
 }
 
-// One workgroup per (tile, K slice): `launch` on fp32 planes of scratch memory and the pass that adds them, or on D itself without slices. Slices are
-// only taken where there is room for their planes without a new condition on the caller: not in the static array, whose calls without
-// copies may overlap; not while the stream records a graph, which then holds one kernel and no allocation; and a provided buffer that
-// is too small or a failed allocation leaves one pass over all of K.
-template <typename F>
-hipError_t launch_items(const ck::GemmArgs& a, int slices, int dtype, Scratch sc, hipStream_t s, F launch) {
-    const int64_t count = (int64_t)a.M * a.N;
+// Scratch memory for the fp32 planes of a call on `slices` K slices, NULL where there is no room for them without a new condition on the caller: not while the
+// stream records a graph, which then holds no allocation; not in a provided buffer that is too small; not where the allocation fails. (Nor in the static array, whose calls without
+// copies may overlap: those ask for no slices.)
+float* take_planes(Scratch& sc, int slices, int64_t count, hipStream_t s) {
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (sc.mode == Scratch::ALLOCATE && s && (hipStreamIsCapturing(s, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone)) return nullptr;
     void* ws = nullptr;
-    if (slices > 1) {
-        hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-        if (sc.mode == Scratch::ALLOCATE && s && (hipStreamIsCapturing(s, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone))
-            slices = 1;
-        else if (scratch_take(sc, (size_t)slices * count * sizeof(float), s, &ws) != ck::CK_OK) slices = 1;
-    }
-    if (slices <= 1) return launch(a);
+    return scratch_take(sc, (size_t)slices * count * sizeof(float), s, &ws) == ck::CK_OK ? static_cast<float*>(ws) : nullptr;
+}
+
+// One workgroup per (tile, K slice): `launch` on the planes and the pass that adds them, or on D itself without planes.
+template <typename F>
+hipError_t launch_items(const ck::GemmArgs& a, int slices, float* planes, int dtype, hipStream_t s, F launch) {
+    if (!planes) return launch(a);
     ck::GemmArgs p = a;
     p.split_k = slices;
-    p.D = static_cast<float*>(ws); p.C = nullptr; p.alpha = 1.f; p.beta = 0.f; p.out16 = 0; p.nt_store = 0;
-    hipError_t e = launch(p);
-    if (e == hipSuccess) e = add_planes(dtype, p.D, slices, count, a.C, a.D, a.alpha, a.beta, a.out16, s);
-    if (!scratch_release(sc, ws, s) && e == hipSuccess) e = hipErrorUnknown;
-    return e;
+    p.D = planes; p.C = nullptr; p.alpha = 1.f; p.beta = 0.f; p.out16 = 0; p.nt_store = 0;
+    const hipError_t e = launch(p);
+    return e == hipSuccess ? add_planes(dtype, planes, slices, (int64_t)a.M * a.N, a.C, a.D, a.alpha, a.beta, a.out16, s) : e;
 }
 
 int gemm_launch(int dtype, const void* A, const void* Bt, const void* C, void* D, float alpha, float beta, int M,
@@ -796,15 +793,21 @@ int gemm_launch(int dtype, const void* A, const void* Bt, const void* C, void* D
     if (((uintptr_t)D & elem_mask) || ((uintptr_t)C & elem_mask)) return CK_ERR_ALIGNMENT;
     // the ring kernels want every operand row on a 16-byte boundary
     const uintptr_t both = (uintptr_t)A | (uintptr_t)Bt;
-    const Route route = on_copies ? *on_copies : route_of(M, N, K, both & 15 ? both & 3 ? 2 : 4 : 16, t, opt,
-                                                      sc.shared ? 0.0 : sc.mode == Scratch::ALLOCATE && stream ? ALLOCATED_CALL_US : KEPT_CALL_US);
+    const int operand_alignment = both & 15 ? both & 3 ? 2 : 4 : 16;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    Route route = on_copies ? *on_copies : route_of(M, N, K, operand_alignment, t, opt,
+                                                sc.shared ? 0.0 : sc.mode == Scratch::ALLOCATE && s ? ALLOCATED_CALL_US : KEPT_CALL_US);
     // one tile's rows are addressed through a 32-bit buffer offset (rows of the copies, also where a kernel does without them)
     if ((int64_t)t.tile_dim * launch_k(K, !(both & 15), t, opt) * 2 >= (int64_t)1 << 31) return CK_ERR_TOO_LARGE;
-    if (route.copies)
-        return gemm_launch_repacked(dtype, A, Bt, C, D, alpha, beta, M, N, K, t, opt, stream, out16, sc, route);
-    // A provided buffer has to hold what the workspace query names, also where the small-product kernel makes no copies in it: whether a
+    // A provided buffer has to hold what the workspace query names for the copies, also where a kernel makes none in it: whether a
     // call is accepted does not hang on the kernel that an estimate picks.
     if (!on_copies && needs_copies(K, !(both & 15)) && !scratch_holds(sc, ((size_t)M + (size_t)N) * padded_k(K, t, opt) * 2)) return CK_ERR_TOO_LARGE;
+    // Kernel, tile and slices were chosen together: without room for the planes the call runs what it runs with slices switched off (64 tiles,
+    // 512 x 512 x 16448: 32 x 32 tiles over all of K, and not the 64 workgroups that four slices of 64 x 64 tiles leave).
+    float* planes = nullptr;
+    if (route.slices > 1 && !(planes = take_planes(sc, route.slices, (int64_t)M * N, s))) route = route_of(M, N, K, operand_alignment, t, opt, 0.0);
+    if (route.copies)
+        return gemm_launch_repacked(dtype, A, Bt, C, D, alpha, beta, M, N, K, t, opt, stream, out16, sc, route);
 
     const int mode = sync_mode_of(t.tile_dim, t.num_consumer_waves, t.bar_step_rows_a, t.bar_step_rows_b);
     GemmArgs a{};
@@ -835,13 +838,15 @@ int gemm_launch(int dtype, const void* A, const void* Bt, const void* C, void* D
     a.producer_nap = opt[OPT_PRODUCER_NAP];
     a.batched_empty_reads = opt[OPT_BATCHED_EMPTY_READS];
     const int src = status_ptr_for_current_device(&a.status);
-    if (src != CK_OK) return src;
+    if (src != CK_OK) {
+        if (planes) (void)scratch_release(sc, planes, s);
+        return src;
+    }
 
     const int64_t tiles = (int64_t)a.tiles_m * a.tiles_n;
     const int grid = persistent_grid(tiles, t.num_cus, a.num_xcd, opt[OPT_EVEN_ROUNDS] != 0);
     const dim3 block((t.num_producer_waves + t.num_consumer_waves) * WAVE);
     const size_t lds = (size_t)gemm_lds_bytes(t);
-    hipStream_t s = static_cast<hipStream_t>(stream);
     hipError_t e = hipErrorInvalidValue;
     a.split_k = 1;
     a.split_chunk = 32;
@@ -853,7 +858,7 @@ int gemm_launch(int dtype, const void* A, const void* Bt, const void* C, void* D
         // XCD's first loads on few memory channels, 118 x 2176 x 124 4.8 us against 5.2; with few columns of tiles and a deep K every XCD
         // streams a stretch of A of its own, 6528 x 396 x 33344 360 against 390, while 12864 x 192 x 4096 takes 51.3 as they come, 46.2 in runs.)
         if (tiles % a.num_xcd != 0 && (K < 512 || (a.tiles_n < 8 && K > 8192))) a.num_xcd = 1;
-        e = launch_items(a, route.slices, dtype, sc, s,
+        e = launch_items(a, route.slices, planes, dtype, s,
                          [&](const GemmArgs& args) { return launch_gemm_direct(dtype == CK_DT_BF16, route.tile, K % 2 == 0 && !(both & 3), s, args); });
     } else if (route.kernel == CKOPT_KERNEL_STREAM) {
         // Tile width, K slices and grid from the cost model: few tiles and a deep K are cut into slices so that every CU
@@ -919,7 +924,7 @@ int gemm_launch(int dtype, const void* A, const void* Bt, const void* C, void* D
             if (!scratch_release(sc, ws, s) && e == hipSuccess) e = hipErrorUnknown;
         }
     } else if (route.kernel == CKOPT_KERNEL_MID) {
-        e = launch_items(a, route.slices, dtype, sc, s, [&](const GemmArgs& args) { return launch_gemm_mid(dtype == CK_DT_BF16, s, args); });
+        e = launch_items(a, route.slices, planes, dtype, s, [&](const GemmArgs& args) { return launch_gemm_mid(dtype == CK_DT_BF16, s, args); });
     } else if (route.kernel == CKOPT_KERNEL_SYNC) {
         // one stage, no producers: load, barrier, multiply, barrier (the synchronous A/B partner)
         e = dtype == CK_DT_F16 ? launch_gemm_sync_f16(t.tile_dim, t.segment_dim_k, t.num_consumer_waves, dim3(grid), lds, s, a)
@@ -941,6 +946,7 @@ int gemm_launch(int dtype, const void* A, const void* Bt, const void* C, void* D
         if (mode == 1) e = launch_gemm_pc_bf16_m1(t.tile_dim, t.segment_dim_k, t.num_consumer_waves, dim3(grid), block, lds, s, a);
         if (mode == 2) e = launch_gemm_pc_bf16_m2(t.tile_dim, t.segment_dim_k, t.num_consumer_waves, dim3(grid), block, lds, s, a);
     }
+    if (planes && !scratch_release(sc, planes, s) && e == hipSuccess) e = hipErrorUnknown;
     if (e == hipErrorInvalidValue) return CK_ERR_NO_INSTANCE;
     return e == hipSuccess ? CK_OK : CK_ERR_HIP;
 }

@@ -90,7 +90,7 @@ int ckopt_gemm_shmem_tc_async_opt_port_2_lp(int dtype, const void* A, const void
  * operands_aligned != 0 promises A and Bt on 16-byte boundaries. A workspace that is too small gives
  * CKOPT_ERR_TOO_LARGE and D is not written, also where the kernel that runs makes no use of it (gemm_direct_kernel on rows off a 16-byte
  * boundary); nothing is allocated in any case. Except for the K slices of gemm_mid_kernel and gemm_direct_kernel (few tiles, a deep K): the query
- * names their planes, and a workspace without room for them, NULL included, leaves one pass over all of K. */
+ * names their planes, and with a workspace without room for them, NULL included, the launch runs what it runs with key 7 of ckopt_set_option at 0. */
 int64_t ckopt_gemm_workspace_bytes(int M, int N, int K, int operands_aligned, int tile_dim, int segment_dim_k, int bar_steps_a,
                                    int bar_steps_b, int bar_step_rows_a, int bar_step_rows_b, int tile_group_m, int num_stages,
                                    int num_producer_waves, int num_consumer_waves, int num_cus);
@@ -102,8 +102,8 @@ int64_t ckopt_gemm_workspace_bytes(int M, int N, int K, int operands_aligned, in
  * plan_out[2] = number of K slices (1: no split-K); plan_out[3] = 1 if A and Bt are first copied into zero-padded rows;
  * plan_out[4] = number of tiles that are cut into those slices (all of them when there are fewer tiles than num_cus; the
  * tiles of the partly filled last round otherwise; 0 without slices); plan_out[5] = 1 if the slices are added inside the
- * kernel, 0 if by a second kernel (gemm_mid_kernel and gemm_direct_kernel: all of their tiles, where a launch finds room for the planes without an
- * allocation); plan_out[6] = workgroups of the straight-line kernel's grid. plan_out points at 7 ints.
+ * kernel, 0 if by a second kernel (gemm_mid_kernel and gemm_direct_kernel: all of their tiles, where a launch finds room for the planes;
+ * the query with split_k 0 says what it runs otherwise); plan_out[6] = workgroups of the straight-line kernel's grid. plan_out points at 7 ints.
  * Returns CKOPT_OK or the error the launch would give. No reference counterpart (its launcher has one kernel form). */
 int ckopt_gemm_launch_plan(int M, int N, int K, int operands_aligned, int tile_dim, int segment_dim_k, int bar_steps_a, int bar_steps_b,
                            int bar_step_rows_a, int bar_step_rows_b, int tile_group_m, int num_stages, int num_producer_waves,

@@ -55,3 +55,42 @@ def f32_to_bf16_bits(x):
 
 def as_f64(dtype_is_bf16, x):
     return (bf16_bits_to_f32(x) if dtype_is_bf16 else x.astype(np.float32)).astype(np.float64)
+
+
+def captured_kernels(launch):
+    """Records launch(stream) into a HIP graph that is never run: (kernel, grid, block, LDS bytes) of its kernel nodes in order, and the
+    number of its other nodes."""
+    import ctypes
+
+    with open("/proc/self/maps") as f:
+        hip = ctypes.CDLL(next(line.split()[-1] for line in f if "/libamdhip64.so" in line))
+
+    class Dim3(ctypes.Structure):
+        _fields_ = [("x", ctypes.c_uint), ("y", ctypes.c_uint), ("z", ctypes.c_uint)]
+
+    class KernelNodeParams(ctypes.Structure):
+        _fields_ = [("blockDim", Dim3), ("extra", ctypes.c_void_p), ("func", ctypes.c_void_p), ("gridDim", Dim3), ("kernelParams", ctypes.c_void_p), ("sharedMemBytes", ctypes.c_uint)]
+
+    stream = torch.cuda.Stream()
+    s, graph = ctypes.c_void_p(stream.cuda_stream), ctypes.c_void_p()
+    torch.cuda.synchronize()
+    assert hip.hipStreamBeginCapture(s, 2) == 0   # relaxed: other work of the process is no part of it
+    try:
+        launch(stream)
+    finally:
+        assert hip.hipStreamEndCapture(s, ctypes.byref(graph)) == 0
+    n = ctypes.c_size_t()
+    assert hip.hipGraphGetNodes(graph, None, ctypes.byref(n)) == 0
+    nodes = (ctypes.c_void_p * n.value)()
+    assert hip.hipGraphGetNodes(graph, nodes, ctypes.byref(n)) == 0
+    kernels, others = [], 0
+    for node in nodes:
+        kind, p = ctypes.c_int(), KernelNodeParams()
+        assert hip.hipGraphNodeGetType(ctypes.c_void_p(node), ctypes.byref(kind)) == 0
+        if kind.value != 0:
+            others += 1
+            continue
+        assert hip.hipGraphKernelNodeGetParams(ctypes.c_void_p(node), ctypes.byref(p)) == 0
+        kernels.append((p.func, (p.gridDim.x, p.gridDim.y, p.gridDim.z), (p.blockDim.x, p.blockDim.y, p.blockDim.z), p.sharedMemBytes))
+    assert hip.hipGraphDestroy(graph) == 0
+    return kernels, others

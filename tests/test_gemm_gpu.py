@@ -1848,3 +1848,42 @@ def test_rows_on_either_side_of_a_wave_tiles_32_bit_extent(ck, N):
         part = slice(at, min(N, at + (1 << 21)))
         assert torch.equal(d[:, part], a.float() @ b[part].float().t() + 2 * c[:, part]), (N, at)
     assert ck.device_status() == 0
+
+
+def test_without_room_for_planes_a_call_runs_the_plan_without_slices(ck):
+    """Kernel, tile and K slices are chosen together: where the planes have no room (a stream that records a graph, no workspace or one too small)
+    a launch is kernel for kernel and workgroup for workgroup the one with slices switched off, and not one pass of the sliced plan's kernel. Shapes
+    whose two plans differ in the tile, in the operand copies, and in neither; a workspace of the queried size is sliced under capture as well."""
+    off = ck.launch_options(split_k=0)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(59)
+    tiles = set()
+    for t, M, N, K in [(SMALL_TUPLE, 512, 512, 16448), (SMALL_TUPLE, 639, 166, 10994), (SMALL_TUPLE, 619, 248, 15873), (SMALL_TUPLE, 233, 128, 25667), (SMALL_TUPLE, 243, 380, 19833),
+                       (SMALL_TUPLE, 64, 192, 14080), (MID_TUPLE, 213, 320, 36672), (MID_TUPLE, 131, 257, 20010)]:
+        whole, sliced = (ck.gemm_launch_plan(M, N, K, True, *t, **kw) for kw in (dict(options=off), {}))
+        assert sliced["k_slices"] > 1 and whole["k_slices"] == 1
+        tiles.add((sliced["tile_cols"], whole["tile_cols"], whole["operand_copies"]))
+        a = torch.randint(-2, 3, (M, K), device="cuda", generator=gen).half()
+        b = torch.randint(-2, 3, (N, K), device="cuda", generator=gen).half()
+        d = torch.empty((M, N), dtype=torch.float32, device="cuda")
+        need = ck.gemm_workspace_bytes(M, N, K, True, *t)
+        ws = torch.empty(max(need, 4096), dtype=torch.uint8, device="cuda")
+        copies = (M + N) * ((K + 7) // 8 * 8) * 2 + 512 if K % 8 else 0
+
+        def plain(stream, **kw):
+            ck.gemm_shmem_tc_async_opt_port_ex(ck.DT_F16, ck.DT_F32, a, b, None, d, 1.0, 0.0, M, N, K, *t, stream=stream, **kw)
+
+        def on_workspace(n):
+            return lambda stream: ck.gemm_shmem_tc_async_opt_port_ws(ck.DT_F16, ck.DT_F32, a, b, None, d, 1.0, 0.0, M, N, K, *t, workspace=ws if n else None, workspace_bytes=n, stream=stream)
+        for warm in ({}, dict(options=off)):   # the first use of every kernel outside a capture
+            plain(torch.cuda.current_stream(), **warm)
+        want = G.captured_kernels(lambda s: plain(s, options=off))
+        assert G.captured_kernels(plain) == want, (t[0], M, N, K)
+        wanted, room = G.captured_kernels(lambda s: plain(s, options=off, workspace=ws, workspace_bytes=need)), [copies] if copies else [0, 4096]
+        for n in room:
+            if need - 256 > n:   # (an odd K: room for the copies is asked for, and may be as much as the planes take)
+                assert G.captured_kernels(on_workspace(n)) == wanted, (t[0], M, N, K, n)
+        kernels, others = G.captured_kernels(on_workspace(need))
+        assert others == 0 and len(kernels) == 2 and kernels[0][1][0] == sliced["sliced_tiles"] * sliced["k_slices"]
+    assert {(64, 32, False), (64, 32, True), (32, 32, False), (128, 128, False)} <= tiles
+    assert ck.device_status() == 0
