@@ -696,7 +696,15 @@ Route route_of(int M, int N, int K, int operand_alignment, const ck::GemmTuning&
     else if (mid && t.num_cus >= cus && (!r.copies || (K % 2 == 0 && K % CHUNK_ELEMS != 0 && operand_alignment >= 4)) && mid_is_shorter(M, N, K, cus)) {
         r.kernel = CKOPT_KERNEL_MID;
         r.copies = false;
-        r.slices = mid_plan(M, N, K, cus, call_us).slices;
+        const MidPlan p = mid_plan(M, N, K, cus, call_us);
+        r.slices = p.slices;
+        // Few tiles and a deep K that would be cut into slices, but not in this call (no room, too short for an allocation, switched off): the tiles of the
+        // small-product kernel reach more CUs. One pass of this kernel / of that one, replayed from a
+        // graph, us: 213 x 320 x 36672 194 / 53, 576 x 640 x 8128 51 / 30, 64 x 1641 x 35560 246 / 83, 640 x 640 x 20480 120 / 63; 1088 x 972 x 33464 (72 tiles) 298 / 276: stays.
+        if (p.slices == 1 && mid_plan(M, N, K, cus, KEPT_CALL_US).slices > 1) {
+            const SmallPlan q = small_plan(M, N, K, operand_alignment, cus, 0.0);
+            if (q.direct && !q.copies && q.us < 0.8 * p.us) return {CKOPT_KERNEL_DIRECT, q.direct, false, 1};
+        }
     } else if (t.num_producer_waves == 0) r.kernel = t.num_stages == 1 ? CKOPT_KERNEL_SYNC : CKOPT_KERNEL_FUSED;
     else if (sync_mode_of(t.tile_dim, t.num_consumer_waves, t.bar_step_rows_a, t.bar_step_rows_b) == CK_SYNC_TILE && t.num_stages >= 2 &&
              opt[OPT_TILE_SYNC_BARRIER] && t.num_producer_waves != 1 && t.segment_dim_k <= 128)
