@@ -256,7 +256,6 @@ struct Scratch {
     enum Mode { ALLOCATE, PROVIDED } mode;
     char* ptr;
     size_t bytes;
-    bool shared;   // the library's static array, which every call of the entry point that allocates nothing works in
 };
 constexpr size_t SCRATCH_ALIGN = 256;
 size_t scratch_round(size_t n) { return (n + SCRATCH_ALIGN - 1) / SCRATCH_ALIGN * SCRATCH_ALIGN; }
@@ -767,8 +766,7 @@ hipError_t add_planes(int dtype, const float* ws, int slices, int64_t count, con
 }
 
 // Scratch memory for the fp32 planes of a call on `slices` K slices, NULL where there is no room for them without a new condition on the caller: not while the
-// stream records a graph, which then holds no allocation; not in a provided buffer that is too small; not where the allocation fails. (Nor in the static array, whose calls without
-// copies may overlap: those ask for no slices.)
+// stream records a graph, which then holds no allocation; not in a provided buffer that is too small; not where the allocation fails.
 float* take_planes(Scratch& sc, int slices, int64_t count, hipStream_t s) {
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
     if (sc.mode == Scratch::ALLOCATE && s && (hipStreamIsCapturing(s, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone)) return nullptr;
@@ -803,8 +801,7 @@ int gemm_launch(int dtype, const void* A, const void* Bt, const void* C, void* D
     const uintptr_t both = (uintptr_t)A | (uintptr_t)Bt;
     const int operand_alignment = both & 15 ? both & 3 ? 2 : 4 : 16;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    Route route = on_copies ? *on_copies : route_of(M, N, K, operand_alignment, t, opt,
-                                                sc.shared ? 0.0 : sc.mode == Scratch::ALLOCATE && s ? ALLOCATED_CALL_US : KEPT_CALL_US);
+    Route route = on_copies ? *on_copies : route_of(M, N, K, operand_alignment, t, opt, sc.mode == Scratch::ALLOCATE && s ? ALLOCATED_CALL_US : KEPT_CALL_US);
     // one tile's rows are addressed through a 32-bit buffer offset (rows of the copies, also where a kernel does without them)
     if ((int64_t)t.tile_dim * launch_k(K, !(both & 15), t, opt) * 2 >= (int64_t)1 << 31) return CK_ERR_TOO_LARGE;
     // A provided buffer has to hold what the workspace query names for the copies, also where a kernel makes none in it: whether a
@@ -979,12 +976,12 @@ int ckopt_launch_options_init(ckopt_launch_options* options) {
 
 int ckopt_gemm_shmem_tc_async_opt_port_2(int dtype, const void* A, const void* Bt, const float* C, float* D, float alpha, float beta,
                                          int M, int N, int K, CK_TUNING_PARAMS, void* stream) {
-    return gemm_launch(dtype, A, Bt, C, D, alpha, beta, M, N, K, CK_TUNING_VALUE, default_options(), stream, 0, Scratch{Scratch::ALLOCATE, nullptr, 0, false});
+    return gemm_launch(dtype, A, Bt, C, D, alpha, beta, M, N, K, CK_TUNING_VALUE, default_options(), stream, 0, Scratch{Scratch::ALLOCATE, nullptr, 0});
 }
 
 int ckopt_gemm_shmem_tc_async_opt_port_2_lp(int dtype, const void* A, const void* Bt, const void* C, void* D, float alpha, float beta,
                                             int M, int N, int K, CK_TUNING_PARAMS, void* stream) {
-    return gemm_launch(dtype, A, Bt, C, D, alpha, beta, M, N, K, CK_TUNING_VALUE, default_options(), stream, 1, Scratch{Scratch::ALLOCATE, nullptr, 0, false});
+    return gemm_launch(dtype, A, Bt, C, D, alpha, beta, M, N, K, CK_TUNING_VALUE, default_options(), stream, 1, Scratch{Scratch::ALLOCATE, nullptr, 0});
 }
 
 int ckopt_gemm_shmem_tc_async_opt_port_2_noalloc(int dtype, const void* A, const void* Bt, const float* C, float* D, float alpha, float beta,
@@ -993,7 +990,7 @@ int ckopt_gemm_shmem_tc_async_opt_port_2_noalloc(int dtype, const void* A, const
     const int rc = static_scratch_for_current_device(&ptr);
     if (rc != ck::CK_OK) return rc;
     return gemm_launch(dtype, A, Bt, C, D, alpha, beta, M, N, K, CK_TUNING_VALUE, default_options(), stream, 0,
-                       Scratch{Scratch::PROVIDED, reinterpret_cast<char*>(ptr), (size_t)CKOPT_NOALLOC_SCRATCH_BYTES, true});
+                       Scratch{Scratch::PROVIDED, reinterpret_cast<char*>(ptr), (size_t)CKOPT_NOALLOC_SCRATCH_BYTES});
 }
 
 int ckopt_gemm_shmem_tc_async_opt_port_2_ex(int dtype, int cd_dtype, const void* A, const void* Bt, const void* C, void* D, float alpha,
@@ -1003,7 +1000,7 @@ int ckopt_gemm_shmem_tc_async_opt_port_2_ex(int dtype, int cd_dtype, const void*
     const int orc = options_from_public(options, &opt);
     if (orc != ck::CK_OK) return orc;
     if (!(cd_dtype == ck::CK_DT_F32 || cd_dtype == dtype)) return ck::CK_ERR_BAD_PARAM;
-    const Scratch sc = workspace ? Scratch{Scratch::PROVIDED, static_cast<char*>(workspace), workspace_bytes, false} : Scratch{Scratch::ALLOCATE, nullptr, 0, false};
+    const Scratch sc = workspace ? Scratch{Scratch::PROVIDED, static_cast<char*>(workspace), workspace_bytes} : Scratch{Scratch::ALLOCATE, nullptr, 0};
     return gemm_launch(dtype, A, Bt, C, D, alpha, beta, M, N, K, CK_TUNING_VALUE, opt, stream, cd_dtype == ck::CK_DT_F32 ? 0 : 1, sc);
 }
 
@@ -1069,7 +1066,7 @@ int ckopt_gemm_shmem_tc_async_opt_port_2_ws(int dtype, int cd_dtype, const void*
                                             void* stream) {
     if (!(cd_dtype == ck::CK_DT_F32 || cd_dtype == dtype)) return ck::CK_ERR_BAD_PARAM;
     return gemm_launch(dtype, A, Bt, C, D, alpha, beta, M, N, K, CK_TUNING_VALUE, default_options(), stream, cd_dtype == ck::CK_DT_F32 ? 0 : 1,
-                       Scratch{Scratch::PROVIDED, static_cast<char*>(workspace), workspace ? workspace_bytes : 0, false});
+                       Scratch{Scratch::PROVIDED, static_cast<char*>(workspace), workspace ? workspace_bytes : 0});
 }
 
 // port_1: every wave tile (or every 16-row block) has its own signal = port_2 with maximal bar_steps
@@ -1087,7 +1084,7 @@ static int launch_port_1(int dtype, const void* A, const void* Bt, const void* C
     }
     const ck::GemmTuning t{tile_dim, segment_dim_k, sa, sb, bar_step_rows_a, bar_step_rows_b,
                            tile_group_m, num_stages, num_producer_waves, num_consumer_waves, num_cus, 0};
-    return gemm_launch(dtype, A, Bt, C, D, alpha, beta, M, N, K, t, default_options(), stream, out16, Scratch{Scratch::ALLOCATE, nullptr, 0, false});
+    return gemm_launch(dtype, A, Bt, C, D, alpha, beta, M, N, K, t, default_options(), stream, out16, Scratch{Scratch::ALLOCATE, nullptr, 0});
 }
 int ckopt_gemm_shmem_tc_async_opt_port_1(int dtype, const void* A, const void* Bt, const float* C, float* D,
                                          float alpha, float beta, int M, int N, int K, int tile_dim,
@@ -1112,7 +1109,7 @@ static int launch_port_0(int dtype, const void* A, const void* Bt, const void* C
                          int num_cus, void* stream, int out16) {
     const ck::GemmTuning t{tile_dim, segment_dim_k, 0, 0, tile_dim, tile_dim, tile_group_m, num_stages, num_producer_waves, num_consumer_waves,
                            num_cus, 1};
-    return gemm_launch(dtype, A, Bt, C, D, alpha, beta, M, N, K, t, default_options(), stream, out16, Scratch{Scratch::ALLOCATE, nullptr, 0, false});
+    return gemm_launch(dtype, A, Bt, C, D, alpha, beta, M, N, K, t, default_options(), stream, out16, Scratch{Scratch::ALLOCATE, nullptr, 0});
 }
 int ckopt_gemm_shmem_tc_async_opt_port_0(int dtype, const void* A, const void* Bt, const float* C, float* D,
                                          float alpha, float beta, int M, int N, int K, int tile_dim,

@@ -117,13 +117,13 @@ int ckopt_gemm_shmem_tc_async_opt_port_2_ws(int dtype, int cd_dtype, const void*
 /* The port_2 launcher above for callers that cannot allocate device memory (code under HIP graph capture, tight
  * serving loops, harnesses that forbid hipMalloc). It has no counterpart in the reference, whose launcher needs no
  * memory beyond its operands. Same parameters and results as ckopt_gemm_shmem_tc_async_opt_port_2 (the same kernels
- * in the same order), but the zero-padded operand copies (K % 8 != 0 or operands off a 16-byte boundary:
+ * in the same order wherever both or neither cut K), but the zero-padded operand copies (K % 8 != 0 or operands off a 16-byte boundary:
  * (M + N) * round_up(K, 8 or 64) * 2 bytes) and the split-K planes (slices * M * N * 4 bytes) live in a static device array
  * of CKOPT_NOALLOC_SCRATCH_BYTES inside the library instead of stream-ordered allocations: no hipMalloc, hipFree or
  * allocating library routine is called. A launch that needs more than the array holds (both pieces, each rounded up
  * to 256 bytes) returns CKOPT_ERR_TOO_LARGE and D is not written; ckopt_set_option(7, 0) makes such a launch
- * fit by not cutting K. Every device holds one array and every call on a device uses it: calls that overlap on one
- * device (different streams, different threads) race on it. Nothing in it needs to start at zero (the counters of
+ * fit by not cutting K. Every device holds one array and every call on a device may use it, for any of these purposes: calls that overlap on one
+ * device (different streams, different threads) race on it, also where a query answers that such a call needs no memory. Nothing in it needs to start at zero (the counters of
  * a reduction inside the kernel are cleared by a small kernel of the same launch, not by a memset).
  * Before a launch is recorded into a HIP graph, one eager call with the same element type, shape class (K a
  * multiple of 64 or not, even or odd, the kernel and the tile width that the queries report) and options must have run on the device: the first
@@ -307,7 +307,7 @@ int ckopt_last_launch_clocks(void* stream, uint64_t* shader_cycles, uint64_t* re
  *        slices' partial products go to scratch memory (slices * M * N * 4 bytes) and a second kernel adds them in
  *        slice order and applies alpha, beta and the output type. 0: never. 2..16: that many slices whenever legal. With 1 the suggested
  *        tuples of 64 and 128 tiles cut K too, into up to 64 slices of at least 512, where few tiles leave the device idle; not on a stream that
- *        records a graph, not in the entry point that allocates nothing, and on other streams than the default one only in longer calls.
+ *        records a graph where the planes would have to be allocated, and on other streams than the default one only in longer calls.
  * key 8: schedule of the straight-line kernel. 1 (default): a workgroup barrier in every k-step, the loads of a loop
  *        body spread over both (three k-steps to land); 0: one barrier per two k-steps, all loads behind it (two
  *        k-steps to land) - at 8192^3 on random operand values 1.5 % faster on one device and 0.7 % slower on another,

@@ -1885,5 +1885,40 @@ def test_without_room_for_planes_a_call_runs_the_plan_without_slices(ck):
                 assert G.captured_kernels(on_workspace(n)) == wanted, (t[0], M, N, K, n)
         kernels, others = G.captured_kernels(on_workspace(need))
         assert others == 0 and len(kernels) == 2 and kernels[0][1][0] == sliced["sliced_tiles"] * sliced["k_slices"]
+        # the entry point that allocates nothing has room for them in its array
+        assert G.captured_kernels(lambda s: ck.gemm_shmem_tc_async_opt_port_noalloc(ck.DT_F16, a, b, None, d, 1.0, 0.0, M, N, K, *t, s)) == (kernels, 0)
     assert {(64, 32, False), (64, 32, True), (32, 32, False), (128, 32, False), (128, 128, False)} <= tiles
+    assert ck.device_status() == 0
+
+
+def test_suggested_tuples_keep_their_slices_without_an_allocation(ck):
+    """What is suggested for few tiles and a deep K counts on K slices: the entry point that allocates nothing takes them too, their planes in its
+    array (with a stream that records a graph, its use), and replays give the product. Small integers: exact."""
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(61)
+    for M, N, K in [(128, 128, 65536), (640, 640, 20480), (213, 320, 36672), (512, 512, 12288), (301, 512, 23403)]:
+        s = ck.suggest_gemm_tuning(M, N, K, 256)
+        t = [s[k] for k in ("tile_dim", "segment_dim_k", "bar_steps_a", "bar_steps_b", "bar_step_rows_a", "bar_step_rows_b", "tile_group_m", "num_stages", "num_producer_warps", "num_consumer_warps", "num_sms")]
+        plan = ck.gemm_launch_plan(M, N, K, True, *t)
+        assert t[0] < 256 and plan["k_slices"] > 1 and plan["k_slices"] * M * N * 4 <= ck.NOALLOC_SCRATCH_BYTES
+        a = torch.randint(-2, 3, (M, K), device="cuda", generator=gen).half()
+        b = torch.randint(-2, 3, (N, K), device="cuda", generator=gen).half()
+        exact = (a.cpu().float() @ b.cpu().float().t()).cuda()
+        d = torch.full((M, N), float("nan"), device="cuda")
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        ck.gemm_shmem_tc_async_opt_port_noalloc(ck.DT_F16, a, b, None, d, 1.0, 0.0, M, N, K, *t, side)
+        side.synchronize()
+        assert torch.equal(d, exact)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            ck.gemm_shmem_tc_async_opt_port_noalloc(ck.DT_F16, a, b, None, d, 1.0, 0.0, M, N, K, *t, torch.cuda.current_stream())
+        kernels, others = G.captured_kernels(lambda st: ck.gemm_shmem_tc_async_opt_port_noalloc(ck.DT_F16, a, b, None, d, 1.0, 0.0, M, N, K, *t, st))
+        assert others == 0 and [k[1][0] for k in kernels][0] == plan["sliced_tiles"] * plan["k_slices"] and len(kernels) == 2
+        for _ in range(3):
+            d.fill_(float("nan"))
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(d, exact), (M, N, K)
     assert ck.device_status() == 0
