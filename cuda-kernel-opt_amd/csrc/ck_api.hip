@@ -26,6 +26,8 @@ constexpr int STREAM_K_MULTIPLE_HOST = 64;  // K extent of one loop body of the 
 hipError_t launch_gemm_fused_f16(int tile, int segk, int cw, dim3 grid, size_t lds, hipStream_t stream, const GemmArgs& a);
 hipError_t launch_gemm_fused_bf16(int tile, int segk, int cw, dim3 grid, size_t lds, hipStream_t stream, const GemmArgs& a);
 hipError_t launch_gemm_direct(bool bf16, int tile, bool aligned, hipStream_t stream, const GemmArgs& a);
+hipError_t prepare_gemm_direct(bool bf16);
+hipError_t prepare_gemm_mid(bool bf16);
 hipError_t launch_gemm_mid(bool bf16, hipStream_t stream, const GemmArgs& a);
 hipError_t launch_gemm_sync_f16(int tile, int segk, int cw, dim3 grid, size_t lds, hipStream_t stream, const GemmArgs& a);
 hipError_t launch_gemm_sync_bf16(int tile, int segk, int cw, dim3 grid, size_t lds, hipStream_t stream, const GemmArgs& a);
@@ -774,6 +776,23 @@ float* take_planes(Scratch& sc, int slices, int64_t count, hipStream_t s) {
     return scratch_take(sc, (size_t)slices * count * sizeof(float), s, &ws) == ck::CK_OK ? static_cast<float*>(ws) : nullptr;
 }
 
+// On a deep K the room that a call finds for the planes decides which kernel the tuples of 64 and 128 tiles run, and the first use of a kernel sets its LDS size,
+// which may not happen while a graph is recorded: the first call makes all of them ready, so that it stands for the later ones whatever their room.
+hipError_t prepare_items(int dtype) {
+    static std::atomic<bool> ready[MAX_DEV][2] = {};
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess || dev < 0 || dev >= MAX_DEV) return e;
+    std::atomic<bool>& done = ready[dev][dtype == ck::CK_DT_BF16];
+    if (done.load(std::memory_order_acquire)) return hipSuccess;
+    e = ck::prepare_gemm_direct(dtype == ck::CK_DT_BF16);
+    if (e == hipSuccess) e = ck::prepare_gemm_mid(dtype == ck::CK_DT_BF16);
+    const auto ring = dtype == ck::CK_DT_F16 ? ck::launch_gemm_fused_f16 : ck::launch_gemm_fused_bf16;
+    if (e == hipSuccess) e = ring(64, 128, 8, dim3(0), 0, nullptr, ck::GemmArgs{});
+    if (e == hipSuccess) done.store(true, std::memory_order_release);
+    return e;
+}
+
 // One workgroup per (tile, K slice): `launch` on the planes and the pass that adds them, or on D itself without planes.
 template <typename F>
 hipError_t launch_items(const ck::GemmArgs& a, int slices, float* planes, int dtype, hipStream_t s, F launch) {
@@ -842,7 +861,8 @@ int gemm_launch(int dtype, const void* A, const void* Bt, const void* C, void* D
     a.prio_mode = opt[OPT_PRIO_MODE];
     a.producer_nap = opt[OPT_PRODUCER_NAP];
     a.batched_empty_reads = opt[OPT_BATCHED_EMPTY_READS];
-    const int src = status_ptr_for_current_device(&a.status);
+    int src = status_ptr_for_current_device(&a.status);
+    if (src == CK_OK && K >= 2 * ITEM_MIN_SLICE && (small_tuple(t, opt) || mid_tuple(t, opt)) && prepare_items(dtype) != hipSuccess) src = CK_ERR_HIP;
     if (src != CK_OK) {
         if (planes) (void)scratch_release(sc, planes, s);
         return src;

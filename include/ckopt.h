@@ -128,7 +128,8 @@ int ckopt_gemm_shmem_tc_async_opt_port_2_ws(int dtype, int cd_dtype, const void*
  * Before a launch is recorded into a HIP graph, one eager call with the same element type, shape class (K a
  * multiple of 64 or not, even or odd, the kernel and the tile width that the queries report) and options must have run on the device: the first
  * call on a device resolves the array's address and the first use of each kernel instance sets its LDS-size
- * attribute, neither of which may happen under capture. The array is resident on every device the process uses the
+ * attribute, neither of which may happen under capture. (From K 1024 on, where the tuples of 64 and 128 tiles run other kernels with room for K
+ * planes than without, one call of either kind stands for both.) The array is resident on every device the process uses the
  * library on, whether or not this entry point is ever called. */
 #define CKOPT_NOALLOC_SCRATCH_BYTES (64u << 20)
 int ckopt_gemm_shmem_tc_async_opt_port_2_noalloc(int dtype, const void* A, const void* Bt, const float* C, float* D,

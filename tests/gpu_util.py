@@ -1,6 +1,10 @@
 """Helpers shared by the GPU parity tests: device buffers via torch, launches via the C ABI."""
+import os
+
 import numpy as np
 import torch
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
 def to_dev(x):

@@ -1922,3 +1922,56 @@ def test_suggested_tuples_keep_their_slices_without_an_allocation(ck):
             torch.cuda.synchronize()
             assert torch.equal(d, exact), (M, N, K)
     assert ck.device_status() == 0
+
+
+def test_one_eager_call_stands_for_a_captured_one_with_other_room(tmp_path):
+    """The first use of a kernel sets its LDS size, which may not happen while a graph is recorded. One eager call of the same shape, sliced or not, stands for a
+    captured one that finds more or less room for the K planes and so runs another kernel: in a process of its own, no call of
+    hipFuncSetAttribute between the two."""
+    import subprocess
+    import sys
+    src = tmp_path / "count.cpp"
+    src.write_text('''#include <dlfcn.h>
+static int calls = 0;
+static void* runtime = nullptr;
+extern "C" int count_begin(const char* path) { return (runtime = dlopen(path, RTLD_NOW)) ? 0 : 1; }
+extern "C" int count() { return calls; }
+extern "C" int hipFuncSetAttribute(const void* kernel, int attribute, int value) {   // (found before the runtime's own)
+    ++calls;
+    return reinterpret_cast<int (*)(const void*, int, int)>(dlsym(runtime, "hipFuncSetAttribute"))(kernel, attribute, value);
+}''')
+    subprocess.run(["g++", "-shared", "-fPIC", str(src), "-o", str(tmp_path / "count.so"), "-ldl"], check=True, timeout=60)
+    prog = tmp_path / "prog.py"
+    prog.write_text('''import ctypes, sys
+import torch
+sys.path.insert(0, %r)
+torch.cuda.init()
+with open("/proc/self/maps") as f:
+    runtime = next(line.split()[-1] for line in f if "/libamdhip64.so" in line)
+shim = ctypes.CDLL(%r, mode=ctypes.RTLD_GLOBAL)
+assert shim.count_begin(runtime.encode()) == 0
+from tests import gpu_util as G
+from tests.conftest import load_package
+ck = load_package()
+small, mid = (64, 128, 0, 0, 64, 64, 4, 4, 0, 8, 256), (128, 128, 0, 0, 128, 128, 4, 2, 0, 8, 256)
+dtype, tdt, t, sliced_first = [(ck.DT_F16, torch.float16, small, True), (ck.DT_BF16, torch.bfloat16, small, False), (ck.DT_F16, torch.float16, mid, False)][int(sys.argv[1])]
+M, N, K = (577, 571, 47053) if t is small else (213, 320, 36672)
+off = ck.launch_options(split_k=0)
+assert ck.gemm_launch_plan(M, N, K, True, *t)["k_slices"] > 1 and ck.gemm_launch_plan(M, N, K, True, *t)["tile_cols"] != 32
+a, b = torch.zeros((M, K), dtype=tdt, device="cuda"), torch.zeros((N, K), dtype=tdt, device="cuda")
+d = torch.empty((M, N), device="cuda")
+need = ck.gemm_workspace_bytes(M, N, K, True, *t)
+ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+ck.gemm_shmem_tc_async_opt_port_ex(dtype, ck.DT_F32, a, b, None, d, 1.0, 0.0, M, N, K, *t, options=None if sliced_first else off)
+torch.cuda.synchronize()
+before = shim.count()
+assert before > 0
+whole, _ = G.captured_kernels(lambda s: ck.gemm_shmem_tc_async_opt_port(dtype, a, b, None, d, 1.0, 0.0, M, N, K, *t, s))
+sliced, _ = G.captured_kernels(lambda s: ck.gemm_shmem_tc_async_opt_port_ws(dtype, ck.DT_F32, a, b, None, d, 1.0, 0.0, M, N, K, *t, workspace=ws, workspace_bytes=need, stream=s))
+assert whole != sliced
+assert shim.count() == before, (before, shim.count())
+print("ok")
+''' % (G.ROOT, str(tmp_path / "count.so")))
+    for which in range(3):
+        r = subprocess.run([sys.executable, str(prog), str(which)], capture_output=True, text=True, timeout=100)
+        assert r.returncode == 0 and r.stdout.strip().endswith("ok"), (which, r.stdout[-500:], r.stderr[-1500:])
