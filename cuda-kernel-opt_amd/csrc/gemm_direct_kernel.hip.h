@@ -224,6 +224,7 @@ __global__ __launch_bounds__(DIRECT_WAVES * 64) void gemm_direct_kernel(const Ge
     // The partial tiles, each in its wave's buffer (a wave writes it behind its own last fragment reads), added in the waves'
     // order by the waves that had a share of K.
     const int waves = end - begin < DIRECT_WAVES ? end - begin : DIRECT_WAVES;
+    const bool whole_cols = (rc.col + 1) * T <= g.N;
     GemmArgs go = g;
     if constexpr (SLICED) go.D = g.D + (int64_t)slice * g.M * g.N;   // fp32 planes of a workspace
 #pragma unroll
@@ -233,7 +234,8 @@ __global__ __launch_bounds__(DIRECT_WAVES * 64) void gemm_direct_kernel(const Ge
         const CK_LDS char* at = (const CK_LDS char*)ck_smem + b * 1024 + lane * 16;
         f32x4 sum = *(const CK_LDS f32x4*)at;
         for (int w = 1; w < waves; ++w) sum += *(const CK_LDS f32x4*)(at + w * 2 * OPERAND);
-        epilogue_block<DT>(go, row_a + b / WT * 16 + lr, row_b + b % WT * 16 + lg * 4, sum);
+        const f32x4 block[1][1] = {{sum}};
+        epilogue_blocks<DT, 1, 1>(go, row_a + b / WT * 16 + lr, row_b + b % WT * 16 + lg * 4, block, whole_cols);
     }
 
     if (blockIdx.x == 0 && threadIdx.x == blockDim.x - 1) {

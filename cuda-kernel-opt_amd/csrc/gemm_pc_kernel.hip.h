@@ -127,59 +127,80 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ void store_b128_nt(void* p, u32x4 v) { asm volatile("global_store_dwordx4 %0, %1, off nt" ::"v"(p), "v"(v) : "memory"); }
 __device__ __forceinline__ void store_b64_nt(void* p, u32x2 v) { asm volatile("global_store_dwordx2 %0, %1, off nt" ::"v"(p), "v"(v) : "memory"); }
 
-// One vector access of C and of D per lane where the four columns lie inside the matrix, on any boundary of their elements (the vector memory path
-// takes 2-byte-aligned addresses: bf16 9472 x 458 x 151 with 16-bit C and D 39.0 us element by element, 22.4 now; fp16 8192 x 8190 x 1024 302, 191); rows past M are skipped, and the lanes on the last columns
-// go element by element.
+// Results block by block: one vector access of C and of D per lane where its four columns lie inside the matrix, on any boundary of their elements (the vector
+// memory path takes 2-byte-aligned addresses: bf16 9472 x 458 x 151 with 16-bit C and D 39.0 us element by element, 22.4 now); rows past M are skipped, and the lanes on the
+// last columns go element by element. whole_cols (of the whole wave): every column of the tile lies inside the matrix. The lanes' own tests of columns are made in the
+// tiles on the edge alone, and what is the same for all blocks is decided once, in front of them: with the tests in every block their masks outgrew
+// the scalar registers and came back from vector lanes, five times a block. 4000 x 8196 x 256 with 16-bit results, fp16 / bf16: without any test of columns (N % 4 == 0 alone)
+// 36.5 / 44.4 us, tested in every block 37.7 / 49.1, now 34.9 / 38.8; 9624 x 8832 x 64 152, 156, 142.
 typedef uint32_t u32x2_a2 __attribute__((ext_vector_type(2), aligned(2)));
-template <typename DT>
-__device__ __forceinline__ void epilogue_block(const GemmArgs& g, int m, int n, f32x4 acc) {
-    const int64_t off = (int64_t)m * g.N + n;
-    const float alpha = g.alpha, beta = g.beta;
-    f32x4 v = acc * alpha;
-    if (m >= g.M || n >= g.N) return;
-    const bool vec = n + 4 <= g.N;
-    if (!g.out16) {
-        if (vec) {
-            if (beta != 0.f) v += *(const f32x4_u*)(g.C + off) * beta;
-            // D is written once and not read again: non-temporal, so that it does not displace the operands in L2
-            // (rows off the 128-byte lines: ordinary stores, whose partial lines are merged in L2 before they reach memory)
-            if (g.nt_store) store_b128_nt(g.D + off, __builtin_bit_cast(u32x4, v));
-            else *(f32x4_u*)(g.D + off) = v;
-        } else {
+template <typename DT, bool OUT16>
+__device__ __forceinline__ void epilogue_four(const GemmArgs& g, int64_t off, f32x4 v, float beta) {
+    if (!OUT16) {
+        if (beta != 0.f) {
+            const f32x4 c = *(const f32x4_u*)(g.C + off);
 #pragma unroll
-            for (int e = 0; e < 3; ++e) {
-                if (n + e < g.N) {
-                    float x = v[e];
-                    if (beta != 0.f) x += g.C[off + e] * beta;
-                    g.D[off + e] = x;
-                }
-            }
+            for (int e = 0; e < 4; ++e) v[e] += c[e] * beta;   // (a vector of four betas takes four scalar registers)
         }
+        // D is written once and not read again: non-temporal, so that it does not displace the operands in L2
+        // (rows off the 128-byte lines: ordinary stores, whose partial lines are merged in L2 before they reach memory)
+        if (g.nt_store) store_b128_nt(g.D + off, __builtin_bit_cast(u32x4, v));
+        else *(f32x4_u*)(g.D + off) = v;
     } else {
-        const unsigned short* c16 = (const unsigned short*)g.C;
+        if (beta != 0.f) {
+            const u32x2_a2 c = *(const u32x2_a2*)((const unsigned short*)g.C + off);
+            v[0] += Out16<DT>::load((unsigned short)(c[0] & 0xffffu)) * beta;
+            v[1] += Out16<DT>::load((unsigned short)(c[0] >> 16)) * beta;
+            v[2] += Out16<DT>::load((unsigned short)(c[1] & 0xffffu)) * beta;
+            v[3] += Out16<DT>::load((unsigned short)(c[1] >> 16)) * beta;
+        }
+        const u32x2 o = {(uint32_t)Out16<DT>::store(v[0]) | ((uint32_t)Out16<DT>::store(v[1]) << 16),
+                         (uint32_t)Out16<DT>::store(v[2]) | ((uint32_t)Out16<DT>::store(v[3]) << 16)};
         unsigned short* d16 = (unsigned short*)g.D;
-        if (vec) {
-            if (beta != 0.f) {
-                const u32x2_a2 c = *(const u32x2_a2*)(c16 + off);
-                v[0] += Out16<DT>::load((unsigned short)(c[0] & 0xffffu)) * beta;
-                v[1] += Out16<DT>::load((unsigned short)(c[0] >> 16)) * beta;
-                v[2] += Out16<DT>::load((unsigned short)(c[1] & 0xffffu)) * beta;
-                v[3] += Out16<DT>::load((unsigned short)(c[1] >> 16)) * beta;
-            }
-            const u32x2 o = {(uint32_t)Out16<DT>::store(v[0]) | ((uint32_t)Out16<DT>::store(v[1]) << 16),
-                             (uint32_t)Out16<DT>::store(v[2]) | ((uint32_t)Out16<DT>::store(v[3]) << 16)};
-            if (g.nt_store) store_b64_nt(d16 + off, o);
-            else *(u32x2_a2*)(d16 + off) = o;
-        } else {
+        if (g.nt_store) store_b64_nt(d16 + off, o);
+        else *(u32x2_a2*)(d16 + off) = o;
+    }
+}
+// a block on the edge: n is the lane's first column
+template <typename DT, bool OUT16>
+__device__ __forceinline__ void epilogue_edge(const GemmArgs& g, int64_t off, int n, f32x4 v) {
+    asm volatile("" : "+v"(n));   // (tested block by block: one mask at a time)
+    if (n + 4 <= g.N) {
+        epilogue_four<DT, OUT16>(g, off, v, g.beta);
+        return;
+    }
+    const unsigned short* c16 = (const unsigned short*)g.C;
+    unsigned short* d16 = (unsigned short*)g.D;
 #pragma unroll
-            for (int e = 0; e < 3; ++e) {
-                if (n + e < g.N) {
-                    float x = v[e];
-                    if (beta != 0.f) x += Out16<DT>::load(c16[off + e]) * beta;
-                    d16[off + e] = Out16<DT>::store(x);
-                }
+    for (int e = 0; e < 3; ++e) {
+        if (n + e < g.N) {
+            float x = v[e];
+            if (g.beta != 0.f) x += (OUT16 ? Out16<DT>::load(c16[off + e]) : g.C[off + e]) * g.beta;
+            if (OUT16) d16[off + e] = Out16<DT>::store(x);
+            else g.D[off + e] = x;
+        }
+    }
+}
+// The blocks of a wave tile, acc[i][j] with its first row in m_base + 16 i and its first column in n_base + 16 j of this lane: one straight line for each of the four forms.
+template <typename DT, int WTR, int WTC>
+__device__ __forceinline__ void epilogue_blocks(const GemmArgs& g, int m_base, int n_base, const f32x4 (&acc)[WTR][WTC], bool whole_cols) {
+    auto each = [&](auto block) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < WTR; ++i) {
+            const int m = m_base + i * 16;
+            if (m < g.M) {
+#pragma unroll
+                for (int j = 0; j < WTC; ++j) block((int64_t)m * g.N + (n_base + j * 16), n_base + j * 16, acc[i][j] * g.alpha);
             }
         }
+    };
+    if (whole_cols) {
+        if (g.out16) each([&](int64_t off, int, f32x4 v) __attribute__((always_inline)) { epilogue_four<DT, true>(g, off, v, g.beta); });
+        else if (g.beta != 0.f) each([&](int64_t off, int, f32x4 v) __attribute__((always_inline)) { epilogue_four<DT, false>(g, off, v, g.beta); });
+        else each([&](int64_t off, int, f32x4 v) __attribute__((always_inline)) { epilogue_four<DT, false>(g, off, v, 0.f); });
+    } else {
+        if (g.out16) each([&](int64_t off, int n, f32x4 v) __attribute__((always_inline)) { epilogue_edge<DT, true>(g, off, n, v); });
+        else each([&](int64_t off, int n, f32x4 v) __attribute__((always_inline)) { epilogue_edge<DT, false>(g, off, n, v); });
     }
 }
 
@@ -745,11 +766,8 @@ __device__ __forceinline__ void consume(const GemmArgs& g, uint32_t flags_base, 
         // fragment as the first MFMA operand a lane holds 4 consecutive columns of one row.
         const int m_base = rc.row * TILE + R * WTR * 16 + (int)(threadIdx.x & 15);
         const int n_base = rc.col * TILE + Cc * WTC * 16 + (int)((threadIdx.x >> 4) & 3) * 4;
-#pragma unroll
-        for (int i = 0; i < WTR; ++i) {
-#pragma unroll
-            for (int j = 0; j < WTC; ++j) epilogue_block<DT>(g, m_base + i * 16, n_base + j * 16, acc[i][j]);
-        }
+        const bool whole_cols = (rc.col + 1) * TILE <= g.N;
+        epilogue_blocks<DT, WTR, WTC>(g, m_base, n_base, acc, whole_cols);
     }
 }
 

@@ -614,11 +614,7 @@ __global__ __launch_bounds__(512) void gemm_stream_kernel(const GemmArgs g) {
                 }
                 }
             } else {
-#pragma unroll
-                for (int i = 0; i < WTR; ++i)
-#pragma unroll
-                    for (int j = 0; j < WTC; ++j)
-                        epilogue_block<DT>(go, m_base + i * 16, n_base + j * 16, acc[i][j]);
+                epilogue_blocks<DT, WTR, WTC>(go, m_base, n_base, acc, vec_cols);
             }
             return interior;
         };

@@ -98,10 +98,8 @@ __global__ __launch_bounds__(CW * 64) void gemm_sync_kernel(const GemmArgs g) {
 
         const int m_base = rc.row * TILE + R * WTR * 16 + lr;
         const int n_base = rc.col * TILE + Cc * WTC * 16 + lg * 4;
-#pragma unroll
-        for (int i = 0; i < WTR; ++i)
-#pragma unroll
-            for (int j = 0; j < WTC; ++j) epilogue_block<DT>(g, m_base + i * 16, n_base + j * 16, acc[i][j]);
+        const bool whole_cols = (rc.col + 1) * TILE <= g.N;
+        epilogue_blocks<DT, WTR, WTC>(g, m_base, n_base, acc, whole_cols);
     }
 
     if (blockIdx.x == 0 && threadIdx.x == blockDim.x - 1) {

@@ -358,6 +358,28 @@ def test_straight_line_kernel_main_loops_hold_no_wait_of_the_compilers(tmp_path)
         assert not waits, "%s %s (%d MFMAs): %s" % (kernel, block, mfmas, waits)
 
 
+def test_block_by_block_results_of_the_straight_line_kernel_keep_scalars_in_registers(tmp_path):
+    """Column tests of the lanes in every block of 16-bit results outgrew the scalar registers: what did not fit came back from vector lanes five
+    times a block (fp16 256 x 256: 341 such reads, bf16 625). In the compiled code of the default instances: no more than two per block of a wave
+    tile, which the edge tiles of the fp32 form need, and 40 in the rest of the kernel."""
+    import importlib.util
+    import subprocess
+    spec = importlib.util.spec_from_file_location("ckopt_build", os.path.join(ROOT, "cuda-kernel-opt_amd", "build.py"))
+    b = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(b)
+    unit = tmp_path / "stream_instances.hip"
+    wanted = [(dt, cols) for dt in ("f16_tag", "bf16_tag") for cols in (8, 6, 4)]
+    unit.write_text('#include "gemm_stream_kernel.hip.h"\nnamespace ck {\n' + "".join("template __global__ void gemm_stream_kernel<%s, false, false, %d>(const GemmArgs);\n" % w for w in wanted) + "}\n")
+    out = str(tmp_path / "stream.s")
+    r = subprocess.run([b.HIPCC] + [f for f in b.DEVICE_FLAGS if f != "-fPIC"] + ["-I", os.path.join(ROOT, "cuda-kernel-opt_amd", "csrc"), "-S", "--cuda-device-only", str(unit), "-o", out],
+                       capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-2000:]
+    kernels = re.findall(r"^_ZN2ck18gemm_stream_kernelINS_\d+(\w+)_tagELb0ELb0ELi(\d)E.*?:(.*?)^\.Lfunc_end", open(out).read(), re.M | re.S)
+    assert len(kernels) == len(wanted)
+    for dt, cols, body in kernels:
+        assert body.count("v_readlane") <= 40 + 2 * 4 * int(cols), (dt, cols, body.count("v_readlane"))   # (wave tiles of 4 x cols blocks)
+
+
 def test_workspace_query_follows_the_launcher_rules(ck):
     # pure host arithmetic (no GPU call): what a launch takes from a caller-owned workspace
     straight = (256, 32, 0, 0, 256, 256, 4, 5, 0, 8, 256)
