@@ -767,24 +767,29 @@ hipError_t add_planes(int dtype, const float* ws, int slices, int64_t count, con
     return hipGetLastError();
 }
 
+bool records_a_graph(hipStream_t s) {   // (the default stream cannot)
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    return s && (hipStreamIsCapturing(s, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone);
+}
+
 // Scratch memory for the fp32 planes of a call on `slices` K slices, NULL where there is no room for them without a new condition on the caller: not while the
 // stream records a graph, which then holds no allocation; not in a provided buffer that is too small; not where the allocation fails.
 float* take_planes(Scratch& sc, int slices, int64_t count, hipStream_t s) {
-    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-    if (sc.mode == Scratch::ALLOCATE && s && (hipStreamIsCapturing(s, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone)) return nullptr;
+    if (sc.mode == Scratch::ALLOCATE && records_a_graph(s)) return nullptr;
     void* ws = nullptr;
     return scratch_take(sc, (size_t)slices * count * sizeof(float), s, &ws) == ck::CK_OK ? static_cast<float*>(ws) : nullptr;
 }
 
 // On a deep K the room that a call finds for the planes decides which kernel the tuples of 64 and 128 tiles run, and the first use of a kernel sets its LDS size,
-// which may not happen while a graph is recorded: the first call makes all of them ready, so that it stands for the later ones whatever their room.
-hipError_t prepare_items(int dtype) {
+// which may not happen while a graph is recorded: the first eager call makes all of them ready, so that it stands for the later ones whatever their room.
+// (A call that is itself recorded leaves it: its own kernel may have been made ready by a call with a shorter K.)
+hipError_t prepare_items(int dtype, hipStream_t s) {
     static std::atomic<bool> ready[MAX_DEV][2] = {};
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess || dev < 0 || dev >= MAX_DEV) return e;
     std::atomic<bool>& done = ready[dev][dtype == ck::CK_DT_BF16];
-    if (done.load(std::memory_order_acquire)) return hipSuccess;
+    if (done.load(std::memory_order_acquire) || records_a_graph(s)) return hipSuccess;
     e = ck::prepare_gemm_direct(dtype == ck::CK_DT_BF16);
     if (e == hipSuccess) e = ck::prepare_gemm_mid(dtype == ck::CK_DT_BF16);
     const auto ring = dtype == ck::CK_DT_F16 ? ck::launch_gemm_fused_f16 : ck::launch_gemm_fused_bf16;
@@ -862,7 +867,7 @@ int gemm_launch(int dtype, const void* A, const void* Bt, const void* C, void* D
     a.producer_nap = opt[OPT_PRODUCER_NAP];
     a.batched_empty_reads = opt[OPT_BATCHED_EMPTY_READS];
     int src = status_ptr_for_current_device(&a.status);
-    if (src == CK_OK && K >= 2 * ITEM_MIN_SLICE && (small_tuple(t, opt) || mid_tuple(t, opt)) && prepare_items(dtype) != hipSuccess) src = CK_ERR_HIP;
+    if (src == CK_OK && K >= 2 * ITEM_MIN_SLICE && (small_tuple(t, opt) || mid_tuple(t, opt)) && prepare_items(dtype, s) != hipSuccess) src = CK_ERR_HIP;
     if (src != CK_OK) {
         if (planes) (void)scratch_release(sc, planes, s);
         return src;

@@ -1926,8 +1926,8 @@ def test_suggested_tuples_keep_their_slices_without_an_allocation(ck):
 
 def test_one_eager_call_stands_for_a_captured_one_with_other_room(tmp_path):
     """The first use of a kernel sets its LDS size, which may not happen while a graph is recorded. One eager call of the same shape, sliced or not, stands for a
-    captured one that finds more or less room for the K planes and so runs another kernel: in a process of its own, no call of
-    hipFuncSetAttribute between the two."""
+    captured one that finds more or less room for the K planes and so runs another kernel; and one of the ring kernel with a short K for a captured one with a longer K
+    that runs it too: in a process of its own, no call of hipFuncSetAttribute between the two."""
     import subprocess
     import sys
     src = tmp_path / "count.cpp"
@@ -1954,6 +1954,20 @@ from tests import gpu_util as G
 from tests.conftest import load_package
 ck = load_package()
 small, mid = (64, 128, 0, 0, 64, 64, 4, 4, 0, 8, 256), (128, 128, 0, 0, 128, 128, 4, 2, 0, 8, 256)
+if sys.argv[1] == "3":
+    d = torch.empty((4096, 4096), device="cuda")
+    short, longer = (torch.zeros((4096, K), dtype=torch.float16, device="cuda") for K in (256, 1024))
+    def product(x, stream):
+        assert ck.gemm_launch_kernel(4096, 4096, x.shape[1], True, *small) == "gemm_fused_kernel"
+        ck.gemm_shmem_tc_async_opt_port(ck.DT_F16, x, x, None, d, 1.0, 0.0, 4096, 4096, x.shape[1], *small, stream)
+    product(short, torch.cuda.current_stream())
+    torch.cuda.synchronize()
+    before = shim.count()
+    assert before > 0
+    kernels, others = G.captured_kernels(lambda s: product(longer, s))
+    assert len(kernels) == 1 and others == 0 and shim.count() == before, (before, shim.count())
+    print("ok")
+    sys.exit()
 dtype, tdt, t, sliced_first = [(ck.DT_F16, torch.float16, small, True), (ck.DT_BF16, torch.bfloat16, small, False), (ck.DT_F16, torch.float16, mid, False)][int(sys.argv[1])]
 M, N, K = (577, 571, 47053) if t is small else (213, 320, 36672)
 off = ck.launch_options(split_k=0)
@@ -1972,6 +1986,6 @@ assert whole != sliced
 assert shim.count() == before, (before, shim.count())
 print("ok")
 ''' % (G.ROOT, str(tmp_path / "count.so")))
-    for which in range(3):
+    for which in range(4):
         r = subprocess.run([sys.executable, str(prog), str(which)], capture_output=True, text=True, timeout=100)
         assert r.returncode == 0 and r.stdout.strip().endswith("ok"), (which, r.stdout[-500:], r.stderr[-1500:])
