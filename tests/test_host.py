@@ -358,6 +358,36 @@ def test_straight_line_kernel_main_loops_hold_no_wait_of_the_compilers(tmp_path)
         assert not waits, "%s %s (%d MFMAs): %s" % (kernel, block, mfmas, waits)
 
 
+def test_straight_line_kernel_main_loops_keep_sums_in_their_registers(tmp_path):
+    """Which registers the compiler gives the results of the main loop hangs on the whole kernel. Where one partly overlapped a fragment that the same MFMA
+    reads, with a wait in front of the next read into that fragment, fp16 8192^3 lost 2 %; results that went into the registers of fragments
+    done with cost one. In the compiled code of the default instances and the K-tail form: no such overlap, at most two sums of a body that leave
+    their registers and come back, and no wait states but the one behind each write of m0."""
+    import importlib.util
+    import subprocess
+    spec = importlib.util.spec_from_file_location("ckopt_build", os.path.join(ROOT, "cuda-kernel-opt_amd", "build.py"))
+    b = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(b)
+    unit, out = tmp_path / "stream_instances.hip", str(tmp_path / "stream.s")
+    wanted = [(dt, tail, cols) for dt in ("f16_tag", "bf16_tag") for tail in ("false", "true") for cols in (8, 6, 4)]
+    unit.write_text('#include "gemm_stream_kernel.hip.h"\nnamespace ck {\n' + "".join("template __global__ void gemm_stream_kernel<%s, false, %s, %d>(const GemmArgs);\n" % w for w in wanted) + "}\n")
+    r = subprocess.run([b.HIPCC] + [f for f in b.DEVICE_FLAGS if f != "-fPIC"] + ["-I", os.path.join(ROOT, "cuda-kernel-opt_amd", "csrc"), "-S", "--cuda-device-only", str(unit), "-o", out],
+                       capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-2000:]
+    loops = 0
+    for kernel, body in re.findall(r"^(_ZN2ck18gemm_stream_kernel\S*):(.*?)^\.Lfunc_end", open(out).read(), re.M | re.S):
+        for block in re.split(r"^\.LBB\d+_\d+:", body, flags=re.M):
+            mfmas = [[range(int(a), int(z) + 1) for a, z in re.findall(r"v\[(\d+):(\d+)\]", line)] for line in block.splitlines() if "v_mfma" in line]
+            if len(mfmas) < 32:   # one loop body: two k-steps of 16, 24 or 32
+                continue
+            loops += 1
+            assert all(len(m) == 4 for m in mfmas)
+            assert not [m for m in mfmas for f in m[1:3] if m[0] != f and m[0].start < f.stop and f.start < m[0].stop], kernel
+            assert sum(m[0] != m[3] for m in mfmas) <= 4, kernel
+            assert sum(1 + int(n) for n in re.findall(r"^\ts_nop (\d+)", block, re.M)) <= len(re.findall(r"s_mov_b32 m0", block)), kernel
+    assert loops == len(wanted)
+
+
 def test_block_by_block_results_of_the_straight_line_kernel_keep_scalars_in_registers(tmp_path):
     """Column tests of the lanes in every block of 16-bit results outgrew the scalar registers: what did not fit came back from vector lanes five
     times a block (fp16 256 x 256: 341 such reads, bf16 625). In the compiled code of the default instances: no more than two per block of a wave
