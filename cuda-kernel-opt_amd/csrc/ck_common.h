@@ -246,33 +246,15 @@ CK_HD int simt_lds_req(int tile_dim, int elem_bytes) {
     // two operands x two buffers x KT x (tile_dim + pad) elements
     return 2 * 2 * SIMT_KT * (tile_dim + SIMT_PAD) * elem_bytes;
 }
-// The instance a launch runs. Every output is one accumulator's ascending-k sum whatever the tile and the micro-tile, so the
-// choice changes no bit of the result. A tuple of 64 or 128 tiles keeps its own instance where that fills the device;
-// on fewer outputs per CU its few workgroups leave most SIMDs with one wave or none, and a wave alone can neither issue
-// fp32 multiply-adds at the full rate (5.4 cycles each against 3.0 with two waves and more) nor hide its LDS reads. There:
-//   up to 8192 outputs per CU: 32 tiles, with 4, 8 or 16 accumulators per thread so that a SIMD has one to two waves
-//     (256 CUs, us, K 1024, f32 / f16 / i32, B transposed, the 64 tile with 16 accumulators against this): 512^2
-//     79 / 95 / 92 -> 29 / 34 / 32, 1024^2 83 / 96 / 96 -> 48 / 50 / 56, 1280^2 87 / 97 / 127 -> 58 / 65 / 84; against the 128
-//     tiles two to seven times; from 1536^2 (9216) on the 32 tiles are level or behind (95 / 106 / 129 against 97 / 95 / 130)
-//   128 tiles, at most one per CU: at most 32 accumulators, in fp16 16 (16 waves on the CU instead of 8 or 4; 2048^3 with 32
-//     accumulators against 16: f16 215 - 244 against 199 - 209, f32 204 - 260 against 217 - 237, i32 307 against 317, with 64
-//     accumulators 329 - 385 in all three); with a second round of tiles 32 are level in f16 too (2304^2: 170 against 168)
-struct SimtInstance { int tile, accs; };
-CK_HD SimtInstance simt_instance(int dtype, int tile_dim, int block_rows, int M, int N, int num_cus) {
-    SimtInstance s{tile_dim, tile_dim / block_rows};
-    const int64_t outputs_per_cu = (int64_t)M * N / num_cus;
-    if (tile_dim == 32) return s;
-    if (outputs_per_cu <= 8192) s = {32, outputs_per_cu <= 1280 ? 4 : outputs_per_cu <= 4608 ? 8 : 16};
-    else if (tile_dim == 128 && (int64_t)(M / 128) * (N / 128) <= num_cus) {
-        const int most = dtype == CK_DT_F16 ? 16 : 32;
-        if (s.accs > most) s.accs = most;
-    }
-    return s;
-}
-// The kernel for few outputs per CU (simt_small_kernel.hip.h) in the place of those instances of the tuples of 64 and 128 tiles, with rm x rn accumulators
-// per thread; tile 0: not taken. Bounds by measurement (256 CUs, us, K 1024 where none is named, the instance above / this, B transposed; K x N differs by
-// a tenth): 512 x 128 x 1248 f32 / f16 / i32 35 / 41 / 38 -> 13 / 15 / 15, 512^2 30 / 35 / 33 -> 19 / 19 / 21, 768^2 43 / 42 / 49 -> 35 / 35 / 42, 1024^2 52 / 52 / 62 -> 39 / 40 / 51.
-// Above the bounds level or behind: f32 1152^2 x 512 27.5 / 31.1; f16 2048 x 1024 66 / 68, K x N 1152^2 x 512 31.7 / 33.0; int32 1280^2 87 / 92, K x N 1152 x 1024 69 / 72.
+// What a launch runs. Every output is one accumulator's ascending-k sum whatever the kernel, the tile and the micro-tile, so the choice
+// changes no bit of the result. A tuple of 64 or 128 tiles keeps its own instance where that fills the device; on fewer outputs per
+// CU its few workgroups leave most SIMDs with one wave or none, and a wave alone can neither issue fp32 multiply-adds at the full rate
+// (5.4 cycles each against 3.0 with two waves and more) nor hide its LDS reads. First the kernel for few outputs per
+// CU (simt_small_kernel.hip.h) with rm x rn accumulators per thread; tile 0: not taken.
+//   256 CUs, us, K 1024 where none is named, f32 / f16 / i32, B transposed (K x N differs by a tenth), 32 tiles of the other kernel -> this: 512 x 128 x 1248
+//     35 / 41 / 38 -> 13 / 15 / 15, 512^2 30 / 35 / 33 -> 19 / 19 / 21, 768^2 43 / 42 / 49 -> 35 / 35 / 42, 1024^2 52 / 52 / 62 -> 39 / 40 / 51
+//   above the bounds level or behind: f32 1152^2 x 512 27.5 / 31.1; f16 2048 x 1024 66 / 68, K x N 1152^2 x 512 31.7 / 33.0; int32 1280^2 87 / 92, K x N
+//     1152 x 1024 69 / 72
 struct SimtSmallInstance { int tile, rm, rn; };
 CK_HD SimtSmallInstance simt_small_instance(int dtype, int tile_dim, bool b_transposed, int M, int N, int num_cus) {
     const int64_t outputs_per_cu = (int64_t)M * N / num_cus;
@@ -281,6 +263,25 @@ CK_HD SimtSmallInstance simt_small_instance(int dtype, int tile_dim, bool b_tran
     if (outputs_per_cu <= 768) return {16, 1, 1};
     if (outputs_per_cu <= 1408) return {32, 2, 1};
     return outputs_per_cu <= 3072 ? SimtSmallInstance{32, 2, 2} : SimtSmallInstance{32, 4, 2};
+}
+// Then, above those bounds, the instance of simt_kernel.hip.h:
+//   up to 8192 outputs per CU: 32 tiles, with 16 accumulators per thread, or 8 up to 4608 (int32 with B as K x N alone, 1024^2 52.5 us), so that a SIMD has one to
+//     two waves (1280^2, f32 / f16 / i32, the 64 tile with 16 accumulators against this: 87 / 97 / 127 -> 58 / 65 / 84; against the 128
+//     tiles two to seven times); from 1536^2 (9216) on the 32 tiles are level or behind (95 / 106 / 129 against 97 / 95 / 130)
+//   128 tiles, at most one per CU: at most 32 accumulators, in fp16 16 (16 waves on the CU instead of 8 or 4; 2048^3 with 32
+//     accumulators against 16: f16 215 - 244 against 199 - 209, f32 204 - 260 against 217 - 237, i32 307 against 317, with 64
+//     accumulators 329 - 385 in all three); with a second round of tiles 32 are level in f16 too (2304^2: 170 against 168)
+struct SimtInstance { int tile, accs; };
+CK_HD SimtInstance simt_instance(int dtype, int tile_dim, int block_rows, int M, int N, int num_cus) {
+    SimtInstance s{tile_dim, tile_dim / block_rows};
+    const int64_t outputs_per_cu = (int64_t)M * N / num_cus;
+    if (tile_dim == 32) return s;
+    if (outputs_per_cu <= 8192) s = {32, outputs_per_cu <= 4608 ? 8 : 16};
+    else if (tile_dim == 128 && (int64_t)(M / 128) * (N / 128) <= num_cus) {
+        const int most = dtype == CK_DT_F16 ? 16 : 32;
+        if (s.accs > most) s.accs = most;
+    }
+    return s;
 }
 CK_HD int check_simt_tuning(int tile_dim, int block_rows) {
     if (!(tile_dim == 32 || tile_dim == 64 || tile_dim == 128)) return CK_ERR_BAD_PARAM;

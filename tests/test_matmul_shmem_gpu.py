@@ -113,14 +113,15 @@ def test_cpp_driver_through_the_matmul_shmem_template(ck):
 
 @pytest.mark.parametrize("name", ["f32", "f16", "i32"])
 def test_every_instance_where_the_grid_keeps_it_and_where_it_is_replaced(ck, oracle, name):
-    # The launcher runs 32 tiles in the place of 64 and 128 ones up to 8192 outputs per CU, and 16 or 32 accumulators in the
-    # place of more where 128 tiles are at most one per CU; neither may change a bit. Outputs per CU (256 CUs): 64; 1280 and 1408, 4608 and
-    # 4736 (either side of the lines between 4, 8 and 16 accumulators); 8192 and 8704; 9216 (144 tiles of 128) and 17408 (272
-    # tiles: every tuple on its own instance). K: one slice, and three.
+    # The launcher runs 32 tiles in the place of 64 and 128 ones up to 8192 outputs per CU (on few of them another kernel, whose bounds the test
+    # below goes by), and 16 or 32 accumulators in the place of more where 128 tiles are at most one per CU; neither may change a bit. Outputs per CU (256
+    # CUs): 64, 1280 and 1408 (the other kernel); 3328, 4608 and 4736 (int32 with B as K x N: eight accumulators, and either side of the line to
+    # 16); 7424 (above every bound of the other kernel), 8192 and 8704; 9216 (144 tiles of 128) and 17408 (272 tiles: every tuple on its own
+    # instance). K: one slice, and three.
     dtype = {"f32": ck.DT_F32, "f16": ck.DT_F16, "i32": ck.DT_I32}[name]
     odt = {"f32": oracle.DT_F32, "f16": oracle.DT_F16, "i32": oracle.DT_I32}[name]
     big = name == "i32"
-    for M, N, K in ((128, 128, 16), (640, 512, 48), (704, 512, 48), (2304, 512, 48), (2368, 512, 16), (2048, 1024, 48), (2176, 1024, 48),
+    for M, N, K in ((128, 128, 16), (640, 512, 48), (704, 512, 48), (1024, 832, 48), (2304, 512, 48), (2368, 512, 16), (1856, 1024, 16), (2048, 1024, 48), (2176, 1024, 48),
                     (1536, 1536, 16), (2176, 2048, 48)):
         for bt in (False, True):
             shape_b = (N, K) if bt else (K, N)
