@@ -1507,9 +1507,9 @@ def test_small_product_kernel_keeps_infinities_to_their_rows(ck):
 
 
 @pytest.mark.parametrize("bf16", [False, True])
-def test_register_staged_128_tiles_exact_at_their_edges(ck, bf16):
-    """The tuple suggested for 128 x 128 tiles (sizes on the ring kernel and on the register-staged one), exact on small integers: ragged edges, one segment of 128 and less, the
-    two stages' parities, K that ends inside a segment's first and second line, more tiles than CUs; C, 16-bit results, a guard
+def test_128_tiles_of_either_kernel_exact_at_their_edges(ck, bf16):
+    """The tuple suggested for 128 x 128 tiles (sizes on the ring kernel and on gemm_mid_kernel), exact on small integers: ragged edges, one segment of 128 and less, an
+    odd and an even number of them, K that ends inside a segment's first and second line, more tiles than CUs; C, 16-bit results, a guard
     behind D; fewer CUs (the persistent ring kernel) give the same."""
     dtype, tdt = (ck.DT_BF16, torch.bfloat16) if bf16 else (ck.DT_F16, torch.float16)
     tup = (128, 128, 0, 0, 128, 128, 4, 2, 0, 8, 256)
@@ -1537,7 +1537,7 @@ MID_TUPLE = (128, 128, 0, 0, 128, 128, 4, 2, 0, 8, 256)   # what the library sug
 
 
 @pytest.mark.parametrize("bf16", [False, True])
-def test_register_staged_kernel_on_its_own_sizes(ck, bf16):
+def test_ring_of_slabs_on_its_own_sizes(ck, bf16):
     """gemm_mid_kernel where the launcher takes it, exact on small integers (sums below 2^24; 16-bit results round the exact value once): K
     that ends in the first and second line of a segment of 128 and on its edge, an odd and an even number of segments, ragged edges, tile
     counts that 8 does not divide, two rounds of tiles. The operands lie in buffers full of NaN, which no lane may multiply; fp32 and
@@ -1568,8 +1568,8 @@ def test_register_staged_kernel_on_its_own_sizes(ck, bf16):
     assert ck.device_status() == 0
 
 
-def test_register_staged_kernel_keeps_infinities_to_their_rows(ck):
-    """Rows past the edge are read as the last row and k past the end as zeros: an infinity or a NaN in the last row, column or k
+def test_ring_of_slabs_keeps_infinities_to_their_rows(ck):
+    """Rows past the edge and k past the end are read as zeros: an infinity or a NaN in the last row, column or k
     reaches the outputs that it belongs to and no other."""
     M, N, K = 140, 150, 584
     assert ck.gemm_launch_kernel(M, N, K, True, *MID_TUPLE) == "gemm_mid_kernel"
@@ -1742,20 +1742,37 @@ def test_kept_scratch_blocks_with_threads_and_given_back(ck):
         before = torch.cuda.mem_get_info()[0]
         ck.trim_scratch_pool()
         assert torch.cuda.mem_get_info()[0] >= before
+    # given back in earnest: the block of a call with planes of tens of MiB is free memory afterwards, and the next call is as exact
+    t, M, N, K = (256, 32, 0, 0, 256, 256, 4, 5, 0, 8, 256), 1024, 1024, 32768
+    planes = ck.gemm_launch_plan(M, N, K, True, *t)["k_slices"] * M * N * 4   # (the workspace query adds what a provided buffer's alignment may take)
+    assert planes >= 32 << 20
+    a = torch.randint(-2, 3, (M, K), device="cuda", generator=gen).half()
+    b = torch.randint(-2, 3, (N, K), device="cuda", generator=gen).half()
+    exact = (a.cpu().float() @ b.cpu().float().t()).cuda()
+    for _ in range(2):
+        d = torch.full((M, N), float("nan"), dtype=torch.float32, device="cuda")
+        ck.gemm_shmem_tc_async_opt_port(ck.DT_F16, a, b, None, d, 1.0, 0.0, M, N, K, *t)
+        torch.cuda.synchronize()
+        assert torch.equal(d, exact)
+        before = torch.cuda.mem_get_info()[0]
+        ck.trim_scratch_pool()
+        assert torch.cuda.mem_get_info()[0] >= before + planes
     assert ck.device_status() == 0
 
 
 @pytest.mark.parametrize("bf16", [False, True])
 def test_16_bit_c_and_d_on_any_two_byte_boundary(ck, bf16):
     """Four 16-bit results go in one access wherever they start: every kernel, N with every remainder by four, C and D one element off each
-    other's and the operands' alignment, edge tiles. Small integers, the exact value rounded once; guards in front of D and behind it."""
+    other's and the operands' alignment, edge tiles; on few CUs the straight-line kernel goes from tile to tile, its loads of the next one counted behind
+    the stores of the last one's interior blocks. Small integers, the exact value rounded once; guards in front of D and behind it."""
     dtype, tdt = (ck.DT_BF16, torch.bfloat16) if bf16 else (ck.DT_F16, torch.float16)
-    tuples = [(256, 32, 0, 0, 256, 256, 4, 5, 0, 8, 256), MID_TUPLE, SMALL_TUPLE, (128, 128, 0, 0, 128, 128, 4, 2, 0, 8, 40), (128, 64, 0, 0, 128, 128, 4, 1, 0, 8, 256),
+    straight_on_8 = (256, 32, 0, 0, 256, 256, 4, 5, 0, 8, 8)
+    tuples = [(256, 32, 0, 0, 256, 256, 4, 5, 0, 8, 256), straight_on_8, MID_TUPLE, SMALL_TUPLE, (128, 128, 0, 0, 128, 128, 4, 2, 0, 8, 40), (128, 64, 0, 0, 128, 128, 4, 1, 0, 8, 256),
               (128, 64, 0, 0, 128, 128, 4, 3, 2, 8, 256), (256, 64, 4, 2, 64, 128, 4, 2, 2, 8, 256), (64, 64, 0, 0, 64, 64, 4, 2, 0, 4, 256)]
     gen = torch.Generator(device="cuda")
     gen.manual_seed(41)
-    seen = set()
-    for M, N, K in [(520, 1030, 128), (300, 517, 576), (256, 1283, 192), (33, 70, 64), (700, 512, 512), (64, 64, 8)]:
+    seen, rounds = set(), set()
+    for M, N, K in [(520, 1030, 128), (520, 1283, 192), (300, 517, 576), (256, 1283, 192), (33, 70, 64), (700, 512, 512), (64, 64, 8)]:
         a = torch.randint(-2, 3, (M, K), device="cuda", generator=gen).to(tdt)
         b = torch.randint(-2, 3, (N, K), device="cuda", generator=gen).to(tdt)
         exact = a.cpu().float() @ b.cpu().float().t()
@@ -1765,6 +1782,10 @@ def test_16_bit_c_and_d_on_any_two_byte_boundary(ck, bf16):
             for t in tuples:
                 for width in (0, 2, 3) if t[1] == 32 else (1,):
                     seen.add(ck.gemm_launch_kernel(M, N, K, True, *t))
+                    if t == straight_on_8:
+                        plan = ck.gemm_launch_plan(M, N, K, True, *t, options=ck.launch_options(half_width=width))
+                        if plan["k_slices"] == 1 and M >= 512 and N % 4 and (M // 256) * (N // plan["tile_cols"]) > plan["grid"]:
+                            rounds.add(plan["tile_cols"])   # a workgroup has a tile behind one without an edge
                     buf = torch.full((M * N + 64,), float("nan"), dtype=tdt, device="cuda")
                     d = buf[16 + d_off:16 + d_off + M * N]
                     for beta in (0.0, -3.0):
@@ -1772,6 +1793,7 @@ def test_16_bit_c_and_d_on_any_two_byte_boundary(ck, bf16):
                         assert torch.equal(d.view(M, N).cpu(), (2 * exact + beta * c.cpu().float()).to(tdt)), (M, N, K, d_off, c_off, t, width, beta)
                     assert torch.isnan(buf[:16 + d_off]).all() and torch.isnan(buf[16 + d_off + M * N:]).all()
     assert seen >= {"gemm_stream_kernel", "gemm_mid_kernel", "gemm_direct_kernel", "gemm_fused_kernel", "gemm_sync_kernel", "gemm_pc_kernel"}
+    assert rounds == {256, 192, 128}
     assert ck.device_status() == 0
 
 

@@ -751,7 +751,7 @@ def test_bench_names_the_kernel_that_runs(ck):
 
 
 def test_kernels_of_the_smaller_tuples_keep_every_value_in_registers(tmp_path):
-    # the small-product and the register-staged kernel are written to the 256 registers of a wave at two waves per SIMD: no scratch memory
+    # the small-product kernel and the ring of slabs are written to the 256 registers of a wave at two waves per SIMD: no scratch memory
     import importlib.util
     import subprocess
     spec = importlib.util.spec_from_file_location("ckopt_build", os.path.join(ROOT, "cuda-kernel-opt_amd", "build.py"))
@@ -767,7 +767,7 @@ def test_kernels_of_the_smaller_tuples_keep_every_value_in_registers(tmp_path):
         sizes, registers = re.findall(r"; ScratchSize: (\d+)", text), re.findall(r"; TotalNumVgprs: (\d+)", text)
         assert sizes and set(sizes) == {"0"} and all(int(v) <= 256 for v in registers), (name, sizes, registers)
         seen += len(sizes)
-    assert seen >= 10   # four instances of the small-product kernel per element type, one of the other
+    assert seen == 20   # per element type eight instances of the small-product kernel (tile, alignment, K slices or none) and two of the other (K a multiple of 64 or not)
 
 
 def test_k_slices_of_the_smaller_tuples(ck, tmp_path):
