@@ -478,32 +478,11 @@ __global__ __launch_bounds__(512) void gemm_stream_kernel(const GemmArgs g) {
                 // exchanged between lanes so that 8 lanes hold the 32 consecutive floats of one row:
                 // store t (0, 1) of a pair writes rows 8t .. 8t+7, lane L the piece L % 8 of row L / 8,
                 // which sits in lane (8t + L / 8) + 16 * (piece % 4) of block piece / 4.
-                // C and D are reached through descriptors of the wave tile, whose extent ends behind its last row inside
-                // the matrix (later rows are not stored and read as zeros): one 32-bit offset per row step, the
-                // columns in the immediate. With 64-bit addresses and a predicate per row step the masks, beta and the
-                // store policy did not fit into the scalar registers and came back from vector lanes at every store;
-                // fp16 16384^3 with C read 6.81 to 6.89 ms, 6.73 to 6.76 now;
-                // 6100 x 6144 x 1024 with C 113.4 us, 111.0; without C 8192^3 797, 796.
                 const int piece = lane & 7;
                 const int src0 = ((lane >> 3) + 16 * (piece & 3)) * 4;  // byte address of the source lane, t = 0
                 const bool second = piece >= 4;
                 const int row0 = __builtin_amdgcn_readfirstlane(rc.row * TILE + R * WTR * 16), col0 = __builtin_amdgcn_readfirstlane(rc.col * TILE_N + Cc * WTC * 16);
-                const int rows = g.M - row0 < WTR * 16 ? g.M - row0 : WTR * 16;
-                const uint32_t extent = rows > 0 ? ((uint32_t)(rows - 1) * (uint32_t)g.N + WTC * 16) * 4u : 0u;
-                auto tile_rsrc = [&](const float* p) __attribute__((always_inline)) {
-                    const uint64_t at = (uint64_t)(uintptr_t)(p + ((int64_t)row0 * g.N + col0));
-                    // (the builtin returns a signed word: unsigned again before it is widened)
-                    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)at), hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(at >> 32));
-                    return __builtin_amdgcn_make_buffer_rsrc((void*)(uintptr_t)((uint64_t)hi << 32 | lo), 0, (int)extent, 0x00020000);
-                };
-                const __amdgpu_buffer_rsrc_t rsrc_d = tile_rsrc(go.D);
-                uint32_t lane_off = ((uint32_t)(lane >> 3) * (uint32_t)g.N + (uint32_t)piece * 4) * 4u;
-                const uint32_t step = (uint32_t)g.N * 32u;
-                // (the offsets do not depend on the tile: opaque, or all sixteen are kept in registers over the main loop)
-                asm volatile("" : "+v"(lane_off));
                 const float alpha = g.alpha, beta = g.beta;
-                // store s of the epilogue: block row i, group of two block columns j, half tt
-                constexpr int GROUPS = WTC / F32_GROUP;
                 auto exchanged = [&](int i, int j, int tt) __attribute__((always_inline)) {
                     f32x4 v;
 #pragma unroll
@@ -515,45 +494,73 @@ __global__ __launch_bounds__(512) void gemm_stream_kernel(const GemmArgs g) {
                     }
                     return v;
                 };
-                auto row_off = [&](int st) { return lane_off + (uint32_t)(st / (GROUPS * STORES_PER_GROUP) * 2 + st % STORES_PER_GROUP) * step; };
-                auto col_off = [](int st) { return ((st / STORES_PER_GROUP) % GROUPS) * F32_GROUP * 64; };
-                auto value = [&](int st) __attribute__((always_inline)) { return exchanged(st / (GROUPS * STORES_PER_GROUP), ((st / STORES_PER_GROUP) % GROUPS) * F32_GROUP, st % STORES_PER_GROUP); };
-                auto put_all = [&](auto policy) __attribute__((always_inline)) {
-                    constexpr int POLICY = decltype(policy)::value;
-                    auto put = [&](int st, f32x4 v) __attribute__((always_inline)) {
-                        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), rsrc_d, (int)(row_off(st) + col_off(st)), 0, POLICY);
+                // Without C: one store at a time behind its exchange, rows past M under a predicate.
+                auto put_without_c = [&](auto policy) __attribute__((always_inline)) {
+                    const int64_t row_lane = (int64_t)row0 + (lane >> 3);
+#pragma unroll
+                    for (int i = 0; i < WTR; ++i)
+#pragma unroll
+                        for (int j = 0; j < WTC; j += F32_GROUP)
+#pragma unroll
+                            for (int tt = 0; tt < STORES_PER_GROUP; ++tt) {
+                                const f32x4 v = exchanged(i, j, tt);
+                                const int64_t row = row_lane + i * 16 + tt * 8;
+                                if (row < g.M) {
+                                    float* at = go.D + (row * g.N + (col0 + piece * 4 + j * 16));
+                                    if (decltype(policy)::value) store_b128_nt(at, __builtin_bit_cast(u32x4, v));
+                                    else *(f32x4_u*)at = v;
+                                }
+                            }
+                };
+                // With C: C and D are reached through descriptors of the wave tile, whose extent ends behind its last row inside
+                // the matrix (later rows are not stored and read as zeros): one 32-bit offset per row step, the
+                // columns in the immediate. With 64-bit addresses and a predicate per row step the masks, beta and the
+                // store policy did not fit into the scalar registers and came back from vector lanes at every store;
+                // 6100 x 6144 x 1024 with C 113.4 us, 111.0 now. (Without C the descriptors' stores left in other order and
+                // were slower on short K: 4096^2 x 512 fp16 29.2 us, bf16 27.6, against 27.4 and 25.5 as above.)
+                auto put_with_c = [&](auto policy) __attribute__((always_inline)) {
+                    const int rows = g.M - row0 < WTR * 16 ? g.M - row0 : WTR * 16;
+                    const uint32_t extent = rows > 0 ? ((uint32_t)(rows - 1) * (uint32_t)g.N + WTC * 16) * 4u : 0u;
+                    auto tile_rsrc = [&](const float* p) __attribute__((always_inline)) {
+                        const uint64_t at = (uint64_t)(uintptr_t)(p + ((int64_t)row0 * g.N + col0));
+                        // (the builtin returns a signed word: unsigned again before it is widened)
+                        const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)at), hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(at >> 32));
+                        return __builtin_amdgcn_make_buffer_rsrc((void*)(uintptr_t)((uint64_t)hi << 32 | lo), 0, (int)extent, 0x00020000);
                     };
-                    if (beta == 0.f) {
+                    const __amdgpu_buffer_rsrc_t rsrc_d = tile_rsrc(go.D), rsrc_c = tile_rsrc(go.C);
+                    uint32_t lane_off = ((uint32_t)(lane >> 3) * (uint32_t)g.N + (uint32_t)piece * 4) * 4u;
+                    const uint32_t step = (uint32_t)g.N * 32u;
+                    // (the offsets do not depend on the tile: opaque, or all sixteen are kept in registers over the main loop)
+                    asm volatile("" : "+v"(lane_off));
+                    // store s of the epilogue: block row i, group of two block columns j, half tt
+                    constexpr int GROUPS = WTC / F32_GROUP;
+                    auto off = [&](int st) { return (int)(lane_off + (uint32_t)(st / (GROUPS * STORES_PER_GROUP) * 2 + st % STORES_PER_GROUP) * step + ((st / STORES_PER_GROUP) % GROUPS) * F32_GROUP * 64); };
+                    // C is read C_DEPTH stores ahead of its use: the loads of a wave would otherwise wait for memory one
+                    // by one between the stores (a load may not pass the store in front of it). Eight fit into the registers
+                    // (252 of 256); four to eight measure the same, twelve spill.
+                    constexpr int C_DEPTH = 8;
+                    f32x4 cv[C_DEPTH];
+                    float factor = beta;   // (in a vector register: as a scalar it is kept four times over and spilled)
+                    asm volatile("" : "+v"(factor));
+                    auto fetch = [&](int st) __attribute__((always_inline)) { return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc_c, off(st), 0, 0)); };
 #pragma unroll
-                        for (int st = 0; st < EPILOGUE_STORES; ++st) put(st, value(st));
-                    } else {
-                        // C is read C_DEPTH stores ahead of its use: the loads of a wave would otherwise wait for memory one
-                        // by one between the stores (a load may not pass the store in front of it). Eight fit into the registers
-                        // (249 of 256); four to eight measure the same, twelve spill.
-                        constexpr int C_DEPTH = 8;
-                        const __amdgpu_buffer_rsrc_t rsrc_c = tile_rsrc(go.C);
-                        f32x4 cv[C_DEPTH];
-                        float factor = beta;   // (in a vector register: as a scalar it is kept four times over and spilled)
-                        asm volatile("" : "+v"(factor));
-                        auto fetch = [&](int st) __attribute__((always_inline)) {
-                            return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc_c, (int)(row_off(st) + col_off(st)), 0, 0));
-                        };
+                    for (int st = 0; st < C_DEPTH; ++st) cv[st] = fetch(st);
 #pragma unroll
-                        for (int st = 0; st < C_DEPTH; ++st) cv[st] = fetch(st);
+                    for (int st = 0; st < EPILOGUE_STORES; ++st) {
+                        f32x4 v = exchanged(st / (GROUPS * STORES_PER_GROUP), ((st / STORES_PER_GROUP) % GROUPS) * F32_GROUP, st % STORES_PER_GROUP);
+                        landed(cv[st % C_DEPTH]);
 #pragma unroll
-                        for (int st = 0; st < EPILOGUE_STORES; ++st) {
-                            f32x4 v = value(st);
-                            landed(cv[st % C_DEPTH]);
-#pragma unroll
-                            for (int e = 0; e < 4; ++e) v[e] += cv[st % C_DEPTH][e] * factor;
-                            put(st, v);
-                            if (st + C_DEPTH < EPILOGUE_STORES) cv[st % C_DEPTH] = fetch(st + C_DEPTH);
-                        }
+                        for (int e = 0; e < 4; ++e) v[e] += cv[st % C_DEPTH][e] * factor;
+                        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), rsrc_d, off(st), 0, decltype(policy)::value);
+                        if (st + C_DEPTH < EPILOGUE_STORES) cv[st % C_DEPTH] = fetch(st + C_DEPTH);
                     }
                 };
-                constexpr int NON_TEMPORAL = 2;   // nt of a buffer access
-                if (nt_store) put_all(std::integral_constant<int, NON_TEMPORAL>{});
-                else put_all(std::integral_constant<int, 0>{});
+                auto put = [&](auto policy) __attribute__((always_inline)) {
+                    if (beta == 0.f) put_without_c(policy);
+                    else put_with_c(policy);
+                };
+                if (nt_store) put(std::integral_constant<int, 2>{});   // nt of a buffer access
+                else put(std::integral_constant<int, 0>{});
             } else if (H16_WHOLE_LINES && interior && g.out16 && d16_misaligned == 0) {
                 if constexpr (H16_WHOLE_LINES) {
                 // 16-bit output in whole 128-byte lines, 16 bytes per lane. A lane's 4 results of a block are
