@@ -264,10 +264,25 @@ __global__ __launch_bounds__(CW * 64) void gemm_fused_kernel(const GemmArgs g) {
             if (has_next_seg) wait_landed(G + 1);
         }
         __builtin_amdgcn_sched_barrier(0);
+        // Behind a column's MFMAs its sums and its fragment, behind the last column all fragments, are named once more in empty statements, so that
+        // results stay in the registers of their sums instead of those of fragments done with (gemm_stream_kernel.hip.h has the reason). Which
+        // ones the compiler picks hangs on the epilogue. us, as it picks / with this: bf16 64 tiles 6354 x 2048 x 960 82.4 / 80.2, 128 tiles on 40
+        // CUs 320 x 1856 x 51968 1124 / 1087; with four waves it is the other way round, 93 x 15808 x 1664 44.3 / 48.4.
+        auto column_done = [&](int j) __attribute__((always_inline)) {
+            if constexpr (CW == 8) {
 #pragma unroll
-        for (int j = 0; j < PRE; ++j)
+                for (int i = 0; i < WTR; ++i) asm volatile("" ::"v"(fb[P][j]), "v"(acc[i][j]));
+                if (j == WTC - 1)
+#pragma unroll
+                    for (int i = 0; i < WTR; ++i) asm volatile("" ::"v"(fa[P][i]), "v"(acc[i][j]));
+            }
+        };
+#pragma unroll
+        for (int j = 0; j < PRE; ++j) {
 #pragma unroll
             for (int i = 0; i < WTR; ++i) acc[i][j] = MfmaOp<DT>::run(fb[P][j], fa[P][i], acc[i][j]);
+            column_done(j);
+        }
         __builtin_amdgcn_sched_barrier(0);
         // chunk of LPK loads this k-step issues: at a segment's last k-step (behind the barrier) chunk 0
         // of the segment that goes into the stage just released, otherwise the next chunk of the
@@ -302,6 +317,7 @@ __global__ __launch_bounds__(CW * 64) void gemm_fused_kernel(const GemmArgs g) {
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int i = 0; i < WTR; ++i) acc[i][j] = MfmaOp<DT>::run(fb[P][j], fa[P][i], acc[i][j]);
+            column_done(j);
             __builtin_amdgcn_sched_barrier(0);
         }
     };
