@@ -66,8 +66,8 @@ struct GemmArgs {
     int out16;      // C and D hold the operands' 16-bit element type instead of fp32 (accumulation stays fp32)
     int nt_store;   // D's rows start on 128-byte lines: vector stores of D are non-temporal (they fill whole lines and need not
                     // stay in L2); otherwise ordinary stores, so that the two parts of a line written by different stores meet in L2
-    int split_k;    // straight-line kernel only: the tiles from whole_tiles on are cut into this many K slices (>= 1), one
-                    // work item per (tile, slice). Without fix_partials slice s writes its partial products to
+    int split_k;    // K slices (>= 1), one work item per (tile, slice): of all tiles in the kernels with one workgroup per tile (direct, mid), of
+                    // the tiles from whole_tiles on in the straight-line kernel, of none in the others. Without fix_partials slice s writes its partial products to
                     // D + s * M * N (a workspace; alpha 1, beta 0, fp32) and a second kernel adds the planes.
     int split_chunk;  // consecutive work items that belong to one slice (32 = one XCD round, or all sliced tiles if fewer)
     int whole_tiles;  // straight-line kernel only: tile counts [0, whole_tiles) are work items over all of K; the K-sliced

@@ -10,13 +10,17 @@
  *   - "warps" are 64-lane wavefronts and "SMs" are compute units.
  * All pointers are device memory owned by the caller. Nothing is synchronised; launches are asynchronous on `stream`.
  * Device memory beyond the operands is needed in two cases only (zero-padded operand copies when K % 8 != 0 or an
- * operand is off a 16-byte boundary; partial planes when the straight-line kernel cuts K into slices). The reference's
+ * operand is off a 16-byte boundary; partial planes when a launch cuts K into slices). The reference's
  * launcher needs none and allocates nothing (port_2.cu:1088-1168; its drivers own all memory, :1200-1203). Here the
  * plain entry points take it from stream-ordered allocations on `stream`, out of a memory pool the library keeps per
  * device (freed blocks stay in the pool for the next launch, and two of up to 256 MiB are kept for the launches on the device's default
  * stream; ckopt_trim_scratch_pool hands them back);
  * ckopt_gemm_shmem_tc_async_opt_port_2_ws takes it from a workspace the caller owns and allocates nothing;
  * ckopt_gemm_shmem_tc_async_opt_port_2_noalloc takes it from a static array inside the library.
+ * Bits: the same call again - entry point, arguments, options, workspace size, default stream or another, recorded or not, with its scratch memory
+ * found - gives the same bits. Between such conditions they may differ, within the rounding of fp32 sums: where K is cut into slices, which key 7 of
+ * ckopt_set_option describes, its sums are added slice by slice. And gemm_mid_kernel begins K at another place on each of the device's
+ * XCDs, so that equal rows of A in different tiles need not give equal rows of D.
  */
 #ifndef CKOPT_H
 #define CKOPT_H
@@ -85,7 +89,8 @@ int ckopt_gemm_shmem_tc_async_opt_port_2_lp(int dtype, const void* A, const void
  * works on the caller's device memory only, port_2.cu:1088-1168, :1200-1203) for the launches that need memory beyond
  * the operands. cd_dtype is CKOPT_DT_F32 (the port_2 entry) or equal to dtype (the _lp entry). `workspace` is device
  * memory of `workspace_bytes` bytes, any alignment, used only during the call's work on `stream`; it may be NULL when
- * the launch needs none. ckopt_gemm_workspace_bytes returns how much the launch with these sizes and this tuning
+ * the launch needs none. Calls whose work may overlap (other streams, other threads) must not be given the same workspace: any call may write all of
+ * it, also one whose tuple makes no operand copies (K slices of every tuple that cuts K). ckopt_gemm_workspace_bytes returns how much the launch with these sizes and this tuning
  * needs under the process's current options (0: none; negative: the error the launch would give);
  * operands_aligned != 0 promises A and Bt on 16-byte boundaries. A workspace that is too small gives
  * CKOPT_ERR_TOO_LARGE and D is not written, also where the kernel that runs makes no use of it (gemm_direct_kernel on rows off a 16-byte
